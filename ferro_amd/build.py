@@ -7,7 +7,8 @@ import sys
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
-SRC = os.path.join(PKG, "csrc", "sampler_kernels.hip")
+# the kernel files, compiled side by side and linked into one library
+SRCS = [os.path.join(PKG, "csrc", f) for f in ("sampler_kernels.hip", "small_k_kernel.hip", "history_kernels.hip")]
 LIB = os.path.join(PKG, "libferro_sampler.so")
 # the same source with phase timestamps compiled in (-DFS_TRACE, fs_trace_set): read by ferro_amd/trace_phases.py
 TRACE_LIB = os.path.join(PKG, "libferro_sampler_trace.so")
@@ -48,14 +49,16 @@ def _run(cmd, what, verbose):
 
 
 def build(verbose: bool = False, trace: bool = False) -> str:
-    jobs = [([HIPCC, *FLAGS, "-o", LIB, SRC], LIB)]
+    """Compiles every source to an object (all at once), then links the library, and with `trace` the trace library."""
+    libs = [(LIB, "", [])] + ([(TRACE_LIB, ".trace", ["-DFS_TRACE"])] if trace else [])
+    objs = {lib: [os.path.splitext(s)[0] + tag + ".o" for s in SRCS] for lib, tag, _ in libs}
+    cflags = [f for f in FLAGS if f != "-shared"]
+    jobs = [([HIPCC, *cflags, *more, "-c", "-o", o, s], o)
+            for lib, _, more in libs for s, o in zip(SRCS, objs[lib])]
     if os.path.exists(FLOOR_SRC):
-        jobs.append(([HIPCC, *[f for f in FLAGS if f not in ("-shared", "-fPIC")], "-o", FLOOR_BIN, FLOOR_SRC],
-                     FLOOR_BIN))
-    if trace:
-        jobs.append(([HIPCC, *FLAGS, "-DFS_TRACE", "-o", TRACE_LIB, SRC], TRACE_LIB))
+        jobs.append(([HIPCC, *[f for f in cflags if f != "-fPIC"], "-o", FLOOR_BIN, FLOOR_SRC], FLOOR_BIN))
     procs = []
-    for cmd, what in jobs:                         # the two libraries compile side by side
+    for cmd, what in jobs:
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True), cmd, what))
@@ -64,6 +67,8 @@ def build(verbose: bool = False, trace: bool = False) -> str:
         if p.returncode != 0:
             sys.stderr.write(out)
             raise RuntimeError(f"{cmd[0]} failed ({p.returncode}) building {what}")
+    for lib, _, _ in libs:
+        _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib, *objs[lib]], lib, verbose)
     for src, out, rpath in ((SHIM_SRC, SHIM_BIN, "$ORIGIN/../../ferro_amd"), (DROPIN_SRC, DROPIN_BIN, "$ORIGIN")):
         if os.path.exists(src):
             _run(["g++", "-O2", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROOT, "include"),

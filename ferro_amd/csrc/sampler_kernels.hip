@@ -27,640 +27,10 @@
 // sums. Rows with k > 2048 are sampled here by whole-row passes. Verify windows (server.cpp:627-637): the last
 // row of a stream to finish (agent-scope sc1 stores, a vmcnt drain and an agent-scope counter, no L2 write-back)
 // computes the accepted prefix.
-#include <hip/hip_runtime.h>
-#include <stdint.h>
-
-#include <algorithm>
-#include <cstring>
-#include <mutex>
-#include <new>
-#include <random>
-#include <vector>
-
-#include "../../include/ferro_sampler.h"
-
-#if !defined(__gfx950__) && defined(__HIP_DEVICE_COMPILE__)
-#error "ferro sampler kernels are written for gfx950 only"
-#endif
+#include "sampler_device.hpp"
+#include "sampler_launch.hpp"
 
 namespace fs {
-
-constexpr int BLOCK = 512;                // threads per workgroup: 8 wave64s, two workgroups per CU
-constexpr int WAVE = 64;
-constexpr int NWAVES = BLOCK / WAVE;
-constexpr int TPT = 8;                    // logits per thread per tile
-constexpr int NV = TPT / 4;               // float4 loads per thread per tile
-constexpr int TILE = BLOCK * TPT;         // 4096 logits per tile
-constexpr int PF = 2;                     // tiles in flight per workgroup
-constexpr int KMAX = 2048;                // largest k on the fused select path
-constexpr int KPT = KMAX / BLOCK;         // candidates per thread in the softmax / draw phase
-constexpr int CAP = KMAX + TILE;          // candidate buffer (LDS), per-segment list in the workspace, merge gather
-constexpr int HBITS = 11;
-constexpr int NBINS = 1 << HBITS;         // threshold histograms
-constexpr int SMALL = 512;                // rank-sort capacity of the merge
-constexpr int MAX_SEGS = 1024;            // segments per row
-constexpr int SPEC = 2;                   // merge gather: loads in flight per thread per round
-constexpr int FAST_SEGS = 64;             // merge fast path: a wave reads every list's bound and count
-static_assert(SPEC * BLOCK + SMALL + 2 * WAVE + 4 * 2 * WAVE / 2 <= CAP, "merge fast path: list, ranks and finish buffers fit");
-constexpr int RBITS = 12;                 // row histogram: bins of the top key bits, shared by a row's segments
-constexpr int RBINS = 1 << RBITS;
-constexpr int RSHIFT = 32 - RBITS;
-constexpr int XCDS = 8;                   // MI355X: 8 XCDs, workgroups dealt round-robin by index
-constexpr int WIDS = 2048;                // penalty-window ids of one segment kept in LDS (longer: rescanned per tile)
-
-enum Mode : int { MODE_SAMPLE = 0, MODE_ARGMAX = 1, MODE_VERIFY = 2 };
-
-struct Args {
-    const float* logits;
-    int64_t ld;
-    int B;            // rows
-    int V;
-    const int32_t* hist;
-    const int64_t* hist_off;
-    const fs_row_params* params;   // NULL: no penalties (argmax mode only)
-    const double* u;
-    int32_t* tok;
-    int kcap;
-    int32_t* cand_ids;
-    double* cand_probs;
-    int32_t* keep;
-    const int32_t* rows;           // verify: tokens fed per row
-    const int64_t* row_off;        // verify: stream -> rows
-    int n_streams;
-    int eos;
-    int32_t* accepted;
-    int mode;
-    int nseg;                      // segments per row (the default layout)
-    int balance;                   // nonzero: each XCD splits its workgroups among its rows by the rows' cost
-    int seg_tiles;                 // tiles per segment
-    uint64_t* cand;                // [B*nseg][CAP]
-    uint32_t* meta;                // [B*nseg][2]: lower bound of the k-th key, count
-    uint32_t* rhist;               // [B][RBINS] row histograms of the segments' candidates, left at 0
-    uint64_t* rmass;               // [B][4096] fixed-point mass histograms of large rows' candidates, left at 0
-    uint32_t* stream_cnt;          // [n_streams] verify completion counters, left at 0
-    int32_t* err;                  // device error bits
-    int32_t* dirty;                // nonzero: a merge gave up waiting; the row histograms and counters may be stale
-    uint32_t merge_spins;          // bounded wait of the merge role (polls); 0: give up without waiting
-    uint64_t* trace;               // FS_TRACE builds: per-workgroup phase timestamps (NULL: none)
-    // one-launch decode step (fs_decode_step): the draws come from device streams (row r = stream r) instead of u,
-    // and each row's token is appended to its stream's history, out of place
-    uint64_t* dmt;                 // [B][312] mt19937_64 states (NULL: draws from u)
-    int32_t* didx;                 // [B] their next indices
-    int32_t* out_hist;             // the histories with the tokens appended (NULL: no append)
-    int64_t* out_hist_off;         // [B + 1]
-    int64_t out_cap;               // ids out_hist holds
-};
-
-constexpr int MT_N = 312, MT_M = 156;
-constexpr uint64_t MT_A = 0xB5026F5AA96619E9ull, MT_UPPER = 0xFFFFFFFF80000000ull, MT_LOWER = 0x7FFFFFFFull;
-
-__device__ __forceinline__ uint64_t mt_temper(uint64_t y) {
-    y ^= (y >> 29) & 0x5555555555555555ull;
-    y ^= (y << 17) & 0x71D67FFFEDA60000ull;
-    y ^= (y << 37) & 0xFFF7EEE000000000ull;
-    y ^= y >> 43;
-    return y;
-}
-__device__ __forceinline__ uint64_t mt_twist_one(uint64_t cur, uint64_t next, uint64_t far) {
-    const uint64_t x = (cur & MT_UPPER) | (next & MT_LOWER);
-    return far ^ (x >> 1) ^ ((x & 1ull) ? MT_A : 0ull);
-}
-__device__ void mt_twist(uint64_t* mt) {
-    for (int k = 0; k < MT_N; ++k) mt[k] = mt_twist_one(mt[k], mt[(k + 1) % MT_N], mt[(k + MT_M) % MT_N]);
-}
-__device__ __forceinline__ double mt_canonical(uint64_t x) {
-    const double r = __ull2double_rn(x) * 0x1p-64;
-    return r < 1.0 ? r : 0x1.fffffffffffffp-1;
-}
-__device__ __forceinline__ bool samples(const fs_row_params& p) { return p.temperature > 0.0f && p.top_k != 1; }
-
-// The draw of row `row` (sampler.cpp:45-46): u from the caller, or, in a decode step, the next value of the row's
-// device stream, read without advancing it (the row's merge commits it after every reader is done).
-__device__ __forceinline__ double row_u(const Args& a, int row) {
-    if (a.dmt) {
-        const uint64_t* mt = a.dmt + (int64_t)row * MT_N;
-        const int idx = a.didx[row];
-        const uint64_t y = idx < MT_N ? mt[idx] : mt_twist_one(mt[0], mt[1], mt[MT_M]);
-        return mt_canonical(mt_temper(y));
-    }
-    return a.u ? a.u[row] : 0.0;
-}
-
-// Phase timestamps (FS_TRACE builds only; the product library compiles these to nothing): thread 0 of a workgroup
-// keeps the constant 100 MHz clock (s_memrealtime) of phase i in LDS (no memory store, so no wait on the memory
-// counter in the middle of the kernel) and writes them to trace[blockIdx * TRACE_W + i] at its end; slots 13-15 hold
-// the role (1 segment, 2 merge), the row and the segment.
-[[maybe_unused]] constexpr int TRACE_W = 16;
-#ifdef FS_TRACE
-#define FS_MARK(i)                                                                                        \
-    do {                                                                                                  \
-        if (threadIdx.x == 0) s.trace_t[(i)] = __builtin_amdgcn_s_memrealtime();                          \
-    } while (0)
-#define FS_TAG(i, v)                                                                                      \
-    do {                                                                                                  \
-        if (threadIdx.x == 0) s.trace_t[(i)] = (uint64_t)(v);                                            \
-    } while (0)
-// the latest of the workgroup's waves to reach phase i (lane 0 of each wave)
-#define FS_MARKW(i)                                                                                       \
-    do {                                                                                                  \
-        if (lane_id() == 0) atomicMax((unsigned long long*)&s.trace_t[(i)],                               \
-                                      (unsigned long long)__builtin_amdgcn_s_memrealtime());              \
-    } while (0)
-#define FS_FLUSH()                                                                                        \
-    do {                                                                                                  \
-        if (threadIdx.x == 0 && a.trace)                                                                  \
-            for (int i_ = 0; i_ < TRACE_W; ++i_) a.trace[(int64_t)blockIdx.x * TRACE_W + i_] = s.trace_t[i_]; \
-    } while (0)
-#else
-#define FS_MARK(i) do {} while (0)
-#define FS_TAG(i, v) do {} while (0)
-#define FS_MARKW(i) do {} while (0)
-#define FS_FLUSH() do {} while (0)
-#endif
-
-// ------------------------------------------------------------------------------------------------ keys
-// Order-preserving map fp32 -> u32: larger float -> larger key; -0 and +0 share a key (sampler.cpp:30 compares
-// with == and >, under which they are equal); NaN maps below every number.
-__device__ __forceinline__ uint32_t key_of(float x) {
-    uint32_t u = __float_as_uint(x);
-    if (x != x) return 0u;
-    if (u == 0x80000000u) u = 0u;
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float val_of(uint32_t k) {
-    const uint32_t u = (k & 0x80000000u) ? (k & 0x7fffffffu) : ~k;
-    return __uint_as_float(u);
-}
-// Composite: ordered like ferro's candidate order (value desc, id asc) when compared as integers, descending.
-__device__ __forceinline__ uint64_t comp_of(uint32_t key, uint32_t id) {
-    return ((uint64_t)key << 32) | (uint64_t)(0xFFFFFFFFu - id);
-}
-__device__ __forceinline__ uint32_t comp_id(uint64_t c) { return 0xFFFFFFFFu - (uint32_t)c; }
-__device__ __forceinline__ uint32_t comp_key(uint64_t c) { return (uint32_t)(c >> 32); }
-
-// ------------------------------------------------------------------------------------------------ hand-off I/O
-// Agent-scope relaxed accesses compile to sc1 loads/stores: coherent across the XCDs' L2s without a write-back.
-__device__ __forceinline__ void st_agent(uint64_t* p, uint64_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_agent(uint32_t* p, uint32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_agent(int32_t* p, int32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint64_t ld_agent(const uint64_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint32_t ld_agent(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ int32_t ld_agent(const int32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Wait until this wave's vector memory operations (the sc1 stores above) have completed.
-__device__ __forceinline__ void vm_drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// Invalidate the CU's L1 (vector cache): later loads are served by the XCD's L2, which holds what other workgroups
-// of this XCD stored or added (stores write through the L1; atomics execute in the L2).
-__device__ __forceinline__ void l1_invalidate() { asm volatile("buffer_inv sc0" ::: "memory"); }
-
-// ------------------------------------------------------------------------------------------------ wave/block
-__device__ __forceinline__ int lane_id() { return __lane_id(); }
-__device__ __forceinline__ uint32_t mbcnt(uint64_t m) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-// Cross-lane moves for whole waves (every call site runs with all 64 lanes active). DPP moves and lane reads stay
-// in the VALU; the LDS permute path (__shfl*) costs an LDS round trip per step.
-template <int CTRL, int ROWMASK = 0xF>
-__device__ __forceinline__ uint32_t dpp32(uint32_t v) {        // lanes without a source read 0
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWMASK, 0xF, false);
-}
-template <int CTRL, class T>
-__device__ __forceinline__ T dpp_move(T v) {
-    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "32- or 64-bit lanes");
-    if constexpr (sizeof(T) == 4) {
-        return __builtin_bit_cast(T, dpp32<CTRL>(__builtin_bit_cast(uint32_t, v)));
-    } else {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        const uint64_t lo = dpp32<CTRL>((uint32_t)u), hi = dpp32<CTRL>((uint32_t)(u >> 32));
-        return __builtin_bit_cast(T, (hi << 32) | lo);
-    }
-}
-template <class T>
-__device__ __forceinline__ T read_lane(T v, int lane) {
-    if constexpr (sizeof(T) == 4) {
-        return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
-    } else {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
-        const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
-        return __builtin_bit_cast(T, (hi << 32) | lo);
-    }
-}
-// op over the wave, result uniform: butterflies within each row of 16 lanes (quad swaps, half-row and row
-// mirrors), then the four rows' lane 0
-template <class T, class Op>
-__device__ __forceinline__ T wave_allreduce(T v, Op op) {
-    v = op(v, dpp_move<0xB1>(v));     // quad_perm [1,0,3,2]
-    v = op(v, dpp_move<0x4E>(v));     // quad_perm [2,3,0,1]
-    v = op(v, dpp_move<0x141>(v));    // row_half_mirror
-    v = op(v, dpp_move<0x140>(v));    // row_mirror
-    return op(op(read_lane(v, 0), read_lane(v, 16)), op(read_lane(v, 32), read_lane(v, 48)));
-}
-template <class T>
-__device__ __forceinline__ T wave_max(T v) {
-    return wave_allreduce(v, [](T x, T y) { return y > x ? y : x; });
-}
-template <class T>
-__device__ __forceinline__ T wave_min(T v) {
-    return wave_allreduce(v, [](T x, T y) { return y < x ? y : x; });
-}
-// The verification rule (server.cpp:627-637) over a stream's m >= 1 tokens, read by the whole wave at once (agent
-// scope: the stream's rows ran on several XCDs): 1 + the leading rows whose token equals the next row's draft, the
-// walk ending after an eos token. Uniform over the wave.
-__device__ __forceinline__ int accepted_prefix(const int32_t* tok, const int32_t* rows, int64_t r0, int m, int eos) {
-    for (int c0 = 0; c0 < m; c0 += WAVE) {
-        const int r = c0 + lane_id();
-        bool stop = false;
-        if (r < m) {
-            const int t = ld_agent(&tok[r0 + r]);
-            stop = (eos >= 0 && t == eos) || r + 1 >= m || t != rows[r0 + r + 1];
-        }
-        const uint64_t b = __ballot(stop);
-        if (b) return c0 + __ffsll((unsigned long long)b);    // 1-based: the row that ends the walk, plus one
-    }
-    return m;
-}
-// inclusive sum over lanes 0..lane (32-bit integers): row shifts 1, 2, 4, 8, then row broadcasts 15 and 31
-__device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t x) {
-    x += dpp32<0x111>(x);
-    x += dpp32<0x112>(x);
-    x += dpp32<0x114>(x);
-    x += dpp32<0x118>(x);
-    x += dpp32<0x142, 0xA>(x);
-    x += dpp32<0x143, 0xC>(x);
-    return x;
-}
-__device__ __forceinline__ double wave_sum_f64(double v) {
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
-// Small shared scratch for block-wide reductions and broadcasts.
-struct Red {
-    uint64_t u64[NWAVES];
-    uint64_t u64b[NWAVES];
-    double f64[NWAVES];
-    int i32[NWAVES];
-    uint32_t u32[NWAVES];
-    uint32_t misc[8];
-    double dmisc[4];
-};
-
-__device__ __forceinline__ uint64_t block_max_u64(uint64_t v, Red& r) {
-    v = wave_max(v);
-    if (lane_id() == 0) r.u64[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    uint64_t m = r.u64[0];
-#pragma unroll
-    for (int w = 1; w < NWAVES; ++w) m = r.u64[w] > m ? r.u64[w] : m;
-    __syncthreads();
-    return m;
-}
-__device__ __forceinline__ uint64_t block_min_u64(uint64_t v, Red& r) {
-    v = wave_min(v);
-    if (lane_id() == 0) r.u64[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    uint64_t m = r.u64[0];
-#pragma unroll
-    for (int w = 1; w < NWAVES; ++w) m = r.u64[w] < m ? r.u64[w] : m;
-    __syncthreads();
-    return m;
-}
-__device__ __forceinline__ uint32_t block_max_u32(uint32_t v, Red& r) {
-    v = wave_max(v);
-    if (lane_id() == 0) r.u32[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    uint32_t m = r.u32[0];
-#pragma unroll
-    for (int w = 1; w < NWAVES; ++w) m = r.u32[w] > m ? r.u32[w] : m;
-    __syncthreads();
-    return m;
-}
-// max and min in one round
-__device__ __forceinline__ void block_minmax_u32(uint32_t& mn, uint32_t& mx, Red& r) {
-    uint32_t a = wave_max(mx), b = wave_min(mn);
-    if (lane_id() == 0) { r.u32[threadIdx.x / WAVE] = a; r.i32[threadIdx.x / WAVE] = (int)b; }
-    __syncthreads();
-    a = r.u32[0];
-    b = (uint32_t)r.i32[0];
-#pragma unroll
-    for (int w = 1; w < NWAVES; ++w) {
-        a = r.u32[w] > a ? r.u32[w] : a;
-        b = (uint32_t)r.i32[w] < b ? (uint32_t)r.i32[w] : b;
-    }
-    __syncthreads();
-    mx = a;
-    mn = b;
-}
-__device__ __forceinline__ int block_min_i32(int v, Red& r) {
-    v = wave_min(v);
-    if (lane_id() == 0) r.i32[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    int m = r.i32[0];
-#pragma unroll
-    for (int w = 1; w < NWAVES; ++w) m = r.i32[w] < m ? r.i32[w] : m;
-    __syncthreads();
-    return m;
-}
-__device__ __forceinline__ int block_max_i32(int v, Red& r) {
-    v = wave_max(v);
-    if (lane_id() == 0) r.i32[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    int m = r.i32[0];
-#pragma unroll
-    for (int w = 1; w < NWAVES; ++w) m = r.i32[w] > m ? r.i32[w] : m;
-    __syncthreads();
-    return m;
-}
-// Deterministic double sum: fixed butterfly in each wave, waves added in order.
-__device__ __forceinline__ double block_sum_f64(double v, Red& r) {
-    v = wave_sum_f64(v);
-    if (lane_id() == 0) r.f64[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    double s = r.f64[0];
-#pragma unroll
-    for (int w = 1; w < NWAVES; ++w) s += r.f64[w];
-    __syncthreads();
-    return s;
-}
-// DPP moves of a double (two 32-bit halves); lanes without a source read 0 (bound_ctrl off, old = 0).
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const uint64_t u = (uint64_t)__double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWMASK, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROWMASK, 0xF, false);
-    return __longlong_as_double((long long)(((uint64_t)(uint32_t)hi << 32) | (uint64_t)(uint32_t)lo));
-}
-// Inclusive wave scan: row_shr 1, 2, 4, 8 inside each 16-lane row, then row_bcast 15 / 31 across rows.
-__device__ __forceinline__ double wave_scan_f64(double v) {
-    v += dpp_f64<0x111, 0xF>(v);
-    v += dpp_f64<0x112, 0xF>(v);
-    v += dpp_f64<0x114, 0xF>(v);
-    v += dpp_f64<0x118, 0xF>(v);
-    v += dpp_f64<0x142, 0xA>(v);
-    v += dpp_f64<0x143, 0xC>(v);
-    return v;
-}
-// Exclusive prefix over threads (thread order), deterministic; *total = the sum over the block.
-template <class T>
-__device__ __forceinline__ T block_excl_scan(T v, T* wsum /*NWAVES*/, T* total) {
-    const int lane = lane_id(), w = threadIdx.x / WAVE;
-    T x, ex;
-    if constexpr (sizeof(T) == 4 && T(-1) > T(0)) {            // 32-bit unsigned: DPP scan (exact in any order)
-        x = wave_incl_scan_u32(v);
-        ex = x - v;
-    } else if constexpr (sizeof(T) == 8 && T(0.5) > T(0)) {    // double: DPP scan, then wave_shr:1 (lane 0 reads 0)
-        x = wave_scan_f64(v);
-        ex = dpp_f64<0x138, 0xF>(x);
-    } else {                                                   // the fixed shuffle order of the sums
-        x = v;
-#pragma unroll
-        for (int o = 1; o < WAVE; o <<= 1) {
-            const T y = __shfl_up(x, o);
-            if (lane >= o) x += y;
-        }
-        ex = __shfl_up(x, 1);
-        if (lane == 0) ex = T(0);
-    }
-    if (lane == WAVE - 1) wsum[w] = x;
-    __syncthreads();
-    T off = T(0), tot = T(0);
-#pragma unroll
-    for (int q = 0; q < NWAVES; ++q) {
-        if (q < w) off += wsum[q];
-        tot += wsum[q];
-    }
-    __syncthreads();
-    *total = tot;
-    return off + ex;
-}
-
-// Append `pred` lanes' values to an LDS list (one LDS atomic per wave); entries past cap are counted, not stored.
-__device__ __forceinline__ void wave_append(bool pred, uint64_t v, uint64_t* list, uint32_t* count, uint32_t cap) {
-    const uint64_t m = __ballot(pred);
-    if (m == 0) return;
-    uint32_t base = 0;
-    const int leader = __ffsll((unsigned long long)m) - 1;
-    if (lane_id() == leader) base = atomicAdd(count, (uint32_t)__popcll(m));
-    base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);   // a scalar read, no LDS round trip
-    if (pred) {
-        const uint32_t pos = base + mbcnt(m);
-        if (pos < cap) list[pos] = v;
-    }
-}
-
-// wave_append for a register element: the 64-bit composite is formed only when some lane of the wave appends.
-__device__ __forceinline__ void wave_append_kv(bool pred, uint32_t key, uint32_t id, uint64_t* list, uint32_t* count,
-                                               uint32_t cap) {
-    const uint64_t m = __ballot(pred);
-    if (m == 0) return;
-    uint32_t base = 0;
-    const int leader = __ffsll((unsigned long long)m) - 1;
-    if (lane_id() == leader) base = atomicAdd(count, (uint32_t)__popcll(m));
-    base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);   // a scalar read, no LDS round trip
-    if (pred) {
-        const uint32_t pos = base + mbcnt(m);
-        if (pos < cap) list[pos] = comp_of(key, id);
-    }
-}
-
-// Histogram helpers over keys in [base, base + (NBINS << shift)): bin = (key - base) >> shift.
-__device__ __forceinline__ int range_shift(uint32_t lo, uint32_t hi) {
-    const uint32_t span = hi - lo;                       // keys lo..hi map to bins 0..span>>shift < NBINS
-    int s = 0;
-    while ((span >> s) >= (uint32_t)NBINS) ++s;
-    return s;
-}
-// From a filled histogram, the bin b holding the kk-th largest entry: count(bins > b) < kk <= count(bins >= b).
-// *above = count(bins > b), *atb = count(bins >= b). Requires 1 <= kk <= total.
-__device__ __forceinline__ int hist_locate(const uint32_t* bins, int kk, uint32_t* above_out, uint32_t* atb_out, uint32_t* wsum,
-                           Red& r) {
-    constexpr int BPT = NBINS / BLOCK;
-    const int tid = threadIdx.x;
-    uint32_t mine = 0;
-#pragma unroll
-    for (int i = 0; i < BPT; ++i) mine += bins[NBINS - 1 - (tid * BPT + i)];
-    uint32_t tot;
-    const uint32_t above = block_excl_scan<uint32_t>(mine, wsum, &tot);
-    if (above < (uint32_t)kk && above + mine >= (uint32_t)kk) {
-        uint32_t c = above;
-        for (int i = 0; i < BPT; ++i) {
-            const int bin = NBINS - 1 - (tid * BPT + i);
-            const uint32_t nb = bins[bin];
-            if (c + nb >= (uint32_t)kk) { r.misc[4] = (uint32_t)bin; r.misc[5] = c; r.misc[6] = c + nb; break; }
-            c += nb;
-        }
-    }
-    __syncthreads();
-    const int b = (int)r.misc[4];
-    *above_out = r.misc[5];
-    *atb_out = r.misc[6];
-    __syncthreads();
-    return b;
-}
-
-// From a filled histogram: the largest bin b such that count(bins >= b) >= k. Returns T = base + (b << shift) and
-// *cnt = count(bins >= b); T = 0 and *cnt = total when the histogram holds fewer than k entries.
-__device__ __forceinline__ uint32_t hist_threshold(const uint32_t* bins, uint32_t base, int shift, int k, uint32_t* cnt,
-                                   uint32_t* wsum, Red& r) {
-    constexpr int BPT = NBINS / BLOCK;
-    const int tid = threadIdx.x;
-    uint32_t mine = 0;
-#pragma unroll
-    for (int i = 0; i < BPT; ++i) mine += bins[NBINS - 1 - (tid * BPT + i)];
-    uint32_t tot;
-    const uint32_t above = block_excl_scan<uint32_t>(mine, wsum, &tot);
-    if (tid == 0) { r.misc[4] = 0u; r.misc[5] = tot; }
-    __syncthreads();
-    if (tot >= (uint32_t)k && above < (uint32_t)k && above + mine >= (uint32_t)k) {
-        uint32_t c = above;
-        for (int i = 0; i < BPT; ++i) {
-            const int bin = NBINS - 1 - (tid * BPT + i);
-            c += bins[bin];
-            if (c >= (uint32_t)k) { r.misc[4] = base + ((uint32_t)bin << shift); r.misc[5] = c; break; }
-        }
-    }
-    __syncthreads();
-    *cnt = r.misc[5];
-    const uint32_t T = r.misc[4];
-    __syncthreads();
-    return T;
-}
-
-// Exact k-th largest composite among the candidates a visitor yields (all distinct, 0 = absent; 1 <= k <= count).
-// Radix select from the top byte: 8 passes of a 256-bin LDS histogram. each(f) calls f(c) for every candidate the
-// calling thread holds. With last_shift = 32 it stops after the key bytes: the result is the k-th largest key (low
-// word 0), which at least k candidates reach.
-template <class Each>
-__device__ __forceinline__ uint64_t radix_kth(Each each, int k, uint32_t* hist256, uint32_t* wsum, Red& r,
-                                              int last_shift = 0) {
-    uint64_t prefix = 0, mask = 0;
-    int kk = k;
-    const int tid = threadIdx.x;
-    for (int shift = 56; shift >= last_shift; shift -= 8) {
-        if (tid < 256) hist256[tid] = 0;
-        __syncthreads();
-        each([&](uint64_t c) {
-            if (c != 0 && (c & mask) == prefix) atomicAdd(&hist256[(c >> shift) & 255], 1u);
-        });
-        __syncthreads();
-        const uint32_t cnt = tid < 256 ? hist256[255 - tid] : 0u;   // thread t owns bin 255 - t: scan from the top
-        uint32_t tot;
-        const uint32_t above = block_excl_scan<uint32_t>(cnt, wsum, &tot);
-        if (tid < 256 && above < (uint32_t)kk && above + cnt >= (uint32_t)kk) {
-            r.misc[0] = 255 - tid;
-            r.misc[1] = above;
-        }
-        __syncthreads();
-        const uint64_t d = r.misc[0];
-        kk -= (int)r.misc[1];
-        prefix |= d << shift;
-        mask |= (uint64_t)255 << shift;
-        __syncthreads();
-    }
-    return prefix;
-}
-
-// Descending bitonic sort of n (a power of two, n <= 4 * BLOCK) composites in LDS, whole block. The stages of the
-// network are taken two at a time: for a pair of strides 2^p1, 2^p2 thread t loads the four entries whose indices
-// are t with zero bits inserted at p1 and p2, plus 0/1 in those bits, applies both stages in registers and stores
-// them back. While both bits are below 8 the four entries lie in the 256-entry block of the thread's wave
-// (index bits 8.. = wave id), and a wave's LDS accesses complete in order, so such rounds need no barrier; a
-// barrier is placed only on each side of a round that crosses blocks.
-__device__ __forceinline__ void bitonic_desc(uint64_t* a, int n) {
-    static_assert(4 * BLOCK >= KMAX && 4 * WAVE == 256, "four entries per thread; a wave spans 256 entries");
-    const int tid = threadIdx.x;
-    if (n < 4) {
-        if (n == 2 && tid == 0) {
-            const uint64_t x = a[0], y = a[1];
-            if (x < y) { a[0] = y; a[1] = x; }
-        }
-        __syncthreads();
-        return;
-    }
-    int lg = 0;
-    while ((1 << lg) < n) ++lg;
-    const bool act = tid < (n >> 2);
-    int m = 1, p = 0;                               // next stage: merge size 2^m, stride 2^p
-    bool prev_cross = false;
-    while (m <= lg) {
-        // this round: the stage (m, p), the next one, and a third while its stride is one of the two
-        int sm[3], sp[3], ns = 0;
-        int b0 = p, b1 = -1;
-        while (m <= lg && ns < 3) {
-            if (p != b0 && p != b1) {
-                if (b1 >= 0) break;
-                b1 = p;
-            }
-            sm[ns] = m; sp[ns] = p; ++ns;
-            if (p == 0) { ++m; p = m - 1; } else { --p; }
-        }
-        if (b1 < 0) b1 = b0 == 0 ? 1 : 0;           // a lone last stage: any second bit
-        const int hi = b0 > b1 ? b0 : b1, lo = b0 > b1 ? b1 : b0;
-        const bool cross = hi >= 8;
-        if (cross || prev_cross) __syncthreads();
-        prev_cross = cross;
-        if (act) {
-            const int t = tid;
-            const int base = (t & ((1 << lo) - 1)) | (((t >> lo) & ((1 << (hi - lo - 1)) - 1)) << (lo + 1)) |
-                             ((t >> (hi - 1)) << (hi + 1));
-            const int ix[4] = {base, base + (1 << lo), base + (1 << hi), base + (1 << hi) + (1 << lo)};
-            uint64_t e[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) e[j] = a[ix[j]];
-            auto cx = [](uint64_t& x, uint64_t& y, bool desc) {
-                const uint64_t lo_v = x < y ? x : y, hi_v = x < y ? y : x;
-                x = desc ? hi_v : lo_v;
-                y = desc ? lo_v : hi_v;
-            };
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                if (q >= ns) break;
-                const int sh = sm[q];
-                if (sp[q] == hi) {                      // partners two registers apart
-                    cx(e[0], e[2], ((ix[0] >> sh) & 1) == 0);
-                    cx(e[1], e[3], ((ix[1] >> sh) & 1) == 0);
-                } else {
-                    cx(e[0], e[1], ((ix[0] >> sh) & 1) == 0);
-                    cx(e[2], e[3], ((ix[2] >> sh) & 1) == 0);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) a[ix[j]] = e[j];
-        }
-    }
-    __syncthreads();
-}
-
-// Rank sort of n <= SMALL distinct composites: out[rank] = in[i] for ranks < k.
-__device__ __forceinline__ void rank_sort(const uint64_t* in, int n, uint64_t* out, int k) {
-    for (int i = threadIdx.x; i < n; i += BLOCK) {
-        const uint64_t c = in[i];
-        int rank = 0;
-        for (int m = 0; m < n; ++m) rank += in[m] > c ? 1 : 0;
-        if (rank < k) out[rank] = c;
-    }
-    __syncthreads();
-}
-
-__device__ __forceinline__ int64_t window_begin(int64_t len, const fs_row_params& p) {
-    int64_t b = (p.repeat_last_n > 0 && (int64_t)p.repeat_last_n < len) ? len - (int64_t)p.repeat_last_n : 0;
-    if (p.penalty_from > 0 && (int64_t)p.penalty_from > b) b = p.penalty_from;
-    return b;
-}
 
 // ------------------------------------------------------------------------------------------------ kernel
 struct Shared {
@@ -779,89 +149,6 @@ __device__ __forceinline__ uint32_t bin_sort_desc(int m, Shared& s) {
 }
 static_assert((TILE / 2 + NBINS) / 2 >= KMAX, "the stage holds a compacted top k");
 
-// Per-row view of the arguments: params, greedy/k, and the two history segments (a verify row sees its stream's
-// base history followed by the drafts fed before it).
-struct RowCtx {
-    int row, pidx;
-    fs_row_params p;
-    bool greedy, large, pen, rep_on, fp_on, capped;
-    int k;
-    int64_t hA0, lenA, lenB, b, len;     // window [b, len) over the concatenated history
-    const int32_t* segB;
-    // the row's segments: nseg of st tiles each (the last may be shorter); segment s publishes in list slot
-    // lx + XCDS * (lbase + s) (the index of the segment workgroup that streams it)
-    int nseg, st, lbase, lx;
-};
-__device__ __forceinline__ int64_t slot_of(const RowCtx& rc, int seg) {
-    return (int64_t)rc.lx + (int64_t)XCDS * (int64_t)(rc.lbase + seg);
-}
-
-// Inputs that no kernel writes (params, history offsets, verify row offsets) are read through the constant address
-// space, so uniform indices become scalar loads (lgkmcnt) and never wait behind the vector loads in flight.
-template <class T>
-__device__ __forceinline__ T ld_const(const T* p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return *(const __attribute__((address_space(4))) T*)(p);
-#else
-    return *p;                                  // the host pass never runs device code
-#endif
-}
-
-__device__ __forceinline__ RowCtx row_ctx(const Args& a, int row) {
-    RowCtx rc;
-    rc.row = row;
-    rc.pidx = row;
-    rc.nseg = a.nseg;
-    rc.st = a.seg_tiles;
-    rc.lx = row % XCDS;
-    rc.lbase = (row / XCDS) * a.nseg;
-    rc.hA0 = 0; rc.lenA = 0; rc.lenB = 0;
-    rc.segB = nullptr;
-    if (a.mode == MODE_VERIFY) {
-        int s0 = 0, s1 = a.n_streams;           // largest s with row_off[s] <= row
-        while (s1 - s0 > 1) {
-            const int m = (s0 + s1) >> 1;
-            if (ld_const(a.row_off + m) <= row) s0 = m; else s1 = m;
-        }
-        rc.pidx = s0;
-        const int64_t r0 = ld_const(a.row_off + s0);
-        rc.segB = a.rows + r0 + 1;
-        rc.lenB = row - r0;
-    }
-    if (a.hist_off && a.hist) {
-        rc.hA0 = ld_const(a.hist_off + rc.pidx);
-        rc.lenA = ld_const(a.hist_off + rc.pidx + 1) - rc.hA0;
-    }
-    if (a.params) {                           // dword by dword: scalar loads (a struct copy becomes vector loads)
-        static_assert(sizeof(fs_row_params) % 4 == 0, "fs_row_params is a sequence of dwords");
-        uint32_t w[sizeof(fs_row_params) / 4];
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(a.params + rc.pidx);
-#pragma unroll
-        for (int i = 0; i < (int)(sizeof(fs_row_params) / 4); ++i) w[i] = ld_const(src + i);
-        __builtin_memcpy(&rc.p, w, sizeof(fs_row_params));
-    } else {
-        rc.p.temperature = 0.f; rc.p.top_k = 1; rc.p.top_p = 1.f; rc.p.min_p = 0.f; rc.p.repetition_penalty = 1.f;
-        rc.p.frequency_penalty = 0.f; rc.p.presence_penalty = 0.f; rc.p.repeat_last_n = 0; rc.p.penalty_from = 0;
-        rc.p.softcap = 0.f;
-    }
-    const int V = a.V;
-    rc.greedy = a.mode == MODE_ARGMAX || rc.p.temperature <= 0.0f || rc.p.top_k == 1;
-    rc.k = rc.greedy ? 1 : ((rc.p.top_k > 0 && rc.p.top_k < V) ? rc.p.top_k : V);
-    rc.large = rc.k > KMAX;                 // not on the segment path: sampled by large_row in the merge kernel
-    rc.capped = rc.p.softcap > 0.0f;
-    rc.rep_on = rc.p.repetition_penalty != 1.0f;
-    rc.fp_on = rc.p.frequency_penalty != 0.0f || rc.p.presence_penalty != 0.0f;
-    rc.len = rc.lenA + rc.lenB;
-    rc.pen = (rc.rep_on || rc.fp_on) && rc.p.repeat_last_n != 0 && rc.len > 0;
-    rc.b = rc.pen ? window_begin(rc.len, rc.p) : rc.len;
-    if (rc.b >= rc.len) rc.pen = false;
-    return rc;
-}
-
-__device__ __forceinline__ int hist_at(const Args& a, const RowCtx& rc, int64_t i) {
-    return i < rc.lenA ? a.hist[rc.hA0 + i] : rc.segB[i - rc.lenA];
-}
-
 // Issue the loads of one tile (TPT logits per thread: float4 j at element lo + (j*BLOCK + t)*4) without waiting.
 // Lanes past the row's end read a clamped in-bounds address and are zeroed. The float4 holding element V-1 may
 // extend up to 12 bytes past it, inside the same 16-byte-aligned block (never into another page); masked too.
@@ -877,104 +164,12 @@ __device__ __forceinline__ void load_tile(float (&x)[TPT], const float* rowp, in
 // Tile t of a segment through its buffer resource: a tile past the segment's end reads zeros without a memory
 // access, so the tile loop requests its next tiles unconditionally (straight-line loads keep the compiler's
 // memory-counter waits exact: consuming a tile waits for that tile only).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-__device__ f32x4 raw_buffer_load_f32x4(__amdgpu_buffer_rsrc_t rs, int voffset, int soffset, int aux)
-    __asm("llvm.amdgcn.raw.ptr.buffer.load.v4f32");
 template <int AUX = 0>
 __device__ __forceinline__ void load_seg_tile(float (&x)[TPT], __amdgpu_buffer_rsrc_t rs, int t) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const f32x4 v = raw_buffer_load_f32x4(rs, (j * BLOCK + (int)threadIdx.x) * 16, t * TILE * 4, AUX);
         x[4 * j + 0] = v.x; x[4 * j + 1] = v.y; x[4 * j + 2] = v.z; x[4 * j + 3] = v.w;
-    }
-}
-// tanhf as the host C library computes it where ferro runs (glibc's float tanh, which follows Sun's fdlibm
-// s_tanh.c / s_expm1.c in single precision): tanh(x) = -e/(e+2) with e = expm1(-2|x|) for |x| < 1,
-// 1 - 2/(expm1(2|x|)+2) for 1 <= |x| < 22, +-1 beyond; expm1 reduces x = k ln2 + r (ln2 split into a 24-bit-exact
-// hi part and a lo part), approximates expm1(r) by fdlibm's rational scheme (the degree-5 polynomial in r^2/2 with
-// fdlibm's Q1..Q5 rounded to float) and rescales by 2^k. Every operation is a separately rounded IEEE fp32 add,
-// multiply or divide (no contraction), so the result is bit-identical to the host's: the GPU test checks all 2^32
-// inputs against the C library.
-__device__ __forceinline__ float f_of(uint32_t u) { return __uint_as_float(u); }
-// Straight-line form (every case computed, the result selected): no branches, so the eight-wide unrolled reads
-// that call it stay one basic block each. Selecting between separately computed IEEE results changes none of them.
-__device__ __forceinline__ float host_tanhf(float x) {
-    const float ln2_hi = f_of(0x3f317180u), ln2_lo = f_of(0x3717f7d1u), invln2 = f_of(0x3fb8aa3bu);
-    const float Q1 = f_of(0xbd088889u), Q2 = f_of(0x3ad00d01u), Q3 = f_of(0xb8a670cdu), Q4 = f_of(0x36867e54u),
-                Q5 = f_of(0xb457edbbu);
-    const uint32_t jx = __float_as_uint(x), ix = jx & 0x7fffffffu;
-    const bool neg = (jx >> 31) != 0u;
-    const float ax = __uint_as_float(ix);
-    const bool big = ix >= 0x3f800000u;                     // |x| >= 1: tanh = 1 - 2/(expm1(2|x|)+2)
-    const float y = big ? __fmul_rn(2.0f, ax) : __fmul_rn(-2.0f, ax);   // expm1's argument, in (-2, 44) for |x| < 22
-    const uint32_t hy = __float_as_uint(y) & 0x7fffffffu;
-    const bool yneg = !big;
-    // expm1(y): y = k ln2 + r (|y| > ln2 / 2; k = +-1 below 1.5 ln2)
-    const bool red = hy > 0x3eb17218u;
-    const bool near = hy < 0x3F851592u;
-    const float hiA = yneg ? __fadd_rn(y, ln2_hi) : __fsub_rn(y, ln2_hi);
-    const float loA = yneg ? -ln2_lo : ln2_lo;
-    const int kB = (int)__fadd_rn(__fmul_rn(invln2, y), yneg ? -0.5f : 0.5f);   // truncation toward zero
-    const float tB = (float)kB;
-    const float hiB = __fsub_rn(y, __fmul_rn(tB, ln2_hi));   // tB * ln2_hi is exact
-    const float loB = __fmul_rn(tB, ln2_lo);
-    const int k = red ? (near ? (yneg ? -1 : 1) : kB) : 0;
-    const float hi = near ? hiA : hiB, lo = near ? loA : loB;
-    const float xr = red ? __fsub_rn(hi, lo) : y;
-    const float c = red ? __fsub_rn(__fsub_rn(hi, xr), lo) : 0.0f;
-    const float hfx = __fmul_rn(0.5f, xr);
-    const float hxs = __fmul_rn(xr, hfx);
-    const float r1 = __fadd_rn(1.0f, __fmul_rn(hxs, __fadd_rn(Q1, __fmul_rn(hxs, __fadd_rn(Q2, __fmul_rn(hxs,
-                     __fadd_rn(Q3, __fmul_rn(hxs, __fadd_rn(Q4, __fmul_rn(hxs, Q5))))))))));
-    const float t = __fsub_rn(3.0f, __fmul_rn(r1, hfx));
-    const float e = __fmul_rn(hxs, __fdiv_rn(__fsub_rn(r1, t), __fsub_rn(6.0f, __fmul_rn(xr, t))));
-    const float R0 = __fsub_rn(xr, __fsub_rn(__fmul_rn(xr, e), hxs));                       // k = 0
-    const float e2 = __fsub_rn(__fsub_rn(__fmul_rn(xr, __fsub_rn(e, c)), c), hxs);
-    const float Rm1 = __fsub_rn(__fmul_rn(0.5f, __fsub_rn(xr, e2)), 0.5f);                 // k = -1
-    const float R1 = xr < -0.25f ? __fmul_rn(-2.0f, __fsub_rn(e2, __fadd_rn(xr, 0.5f)))    // k = 1
-                                 : __fadd_rn(1.0f, __fmul_rn(2.0f, __fsub_rn(xr, e2)));
-    const int kc = k < -126 ? -126 : (k > 127 ? 127 : k);
-    const float twopk = f_of(0x3f800000u + ((uint32_t)kc << 23));
-    const float RL = __fsub_rn(__fmul_rn(__fsub_rn(1.0f, __fsub_rn(e2, xr)), twopk), 1.0f);  // k <= -2 or k > 56
-    const int ks = k < 0 ? 0 : (k > 31 ? 31 : k);
-    const float RS = __fmul_rn(__fsub_rn(f_of(0x3f800000u - (0x1000000u >> ks)), __fsub_rn(e2, xr)), twopk);   // 1 - 2^-k
-    const int kt = k < 0 ? 0 : (k > 126 ? 126 : k);
-    const float RB = __fmul_rn(__fadd_rn(__fsub_rn(xr, __fadd_rn(e2, f_of((uint32_t)(0x7f - kt) << 23))), 1.0f), twopk);
-    float em = k == 0 ? R0 : k == -1 ? Rm1 : k == 1 ? R1 : (k <= -2 || k > 56) ? RL : k < 23 ? RS : RB;
-    const float huge = 1.0e+30f;
-    if (hy < 0x33000000u) em = __fsub_rn(y, __fsub_rn(__fadd_rn(huge, y), __fadd_rn(huge, y)));   // |y| < 2^-25
-    // tanh from expm1
-    float z = big ? __fsub_rn(1.0f, __fdiv_rn(2.0f, __fadd_rn(em, 2.0f))) : __fdiv_rn(-em, __fadd_rn(em, 2.0f));
-    if (ix >= 0x41b00000u) z = __fsub_rn(1.0f, 1.0e-30f);      // |x| >= 22: +-1 (inexact)
-    float r = neg ? -z : z;
-    if (ix < 0x24000000u) r = __fmul_rn(x, __fadd_rn(1.0f, x));  // |x| < 2^-55
-    if (ix >= 0x7f800000u)                                       // +-inf, NaN
-        r = neg ? __fsub_rn(__fdiv_rn(1.0f, x), 1.0f) : __fadd_rn(__fdiv_rn(1.0f, x), 1.0f);
-    return r;
-}
-// The model's final-logit softcap, moved into the read: l = cap * tanhf(l / cap) (model_gemma4_gpu.cpp:282-283:
-// fp32 divide, the host C library's tanhf, fp32 multiply), before the penalties as in ferro, where the model caps
-// the row first. Bit-identical to the host loop.
-__device__ __forceinline__ float softcap_one(float l, float cap) { return __fmul_rn(cap, host_tanhf(__fdiv_rn(l, cap))); }
-// Unrolled, for the streaming loop of the segment path (its three call sites): a rolled loop there changes the
-// allocation of the tile registers and slows every row, capped or not.
-template <int N>
-__device__ __forceinline__ void softcap_vals_unrolled(float (&x)[N], float cap) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = softcap_one(x[i], cap);
-}
-// A rolled loop: one copy of the cap per call site (there are dozens, all unrolled eight-wide otherwise), for capped
-// rows only; the element is picked and put back by index.
-template <int N>
-__device__ __forceinline__ void softcap_vals(float (&x)[N], float cap) {
-#pragma unroll 1
-    for (int i = 0; i < N; ++i) {
-        float v = x[0];
-#pragma unroll
-        for (int j = 1; j < N; ++j) v = i == j ? x[j] : v;
-        v = softcap_one(v, cap);
-#pragma unroll
-        for (int j = 0; j < N; ++j) x[j] = i == j ? v : x[j];
     }
 }
 // element id of this thread's i-th logit of the tile starting at lo
@@ -1895,13 +1090,6 @@ __device__ __forceinline__ void row_abandon(const Args& a, int row) {
 // softmax / min-p / top-p / draw of sampler.cpp:37-49, the sums as DPP wave scans in candidate order. LDS accesses
 // of one wave are ordered, so no further block barrier is needed: the other waves go straight to the epilogue.
 
-__device__ __forceinline__ double lane_f64(double v, int lane) {   // lane: wave-uniform
-    const uint64_t u = (uint64_t)__double_as_longlong(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
 // Ranks of the c1 <= 128 candidates in[0, c1) (whole block, one barrier): thread t compares candidate t % 128
 // with a quarter of the list; rk[q*128 + e] is candidate e's count of larger entries in quarter q. Pads in[c1, 128)
 // with 0 first. Returns after a barrier.
@@ -2008,53 +1196,6 @@ __device__ __forceinline__ void prefetch_lists(const Args& a, const RowCtx& rc, 
     }
 #pragma unroll
     for (int q = 0; q < SPEC; ++q) pre.v[q] = nseg > 0 ? lst[pre.act ? pre.r_me + q * pre.tps : 0] : 0ull;
-}
-
-// Softmax at temperature, min-p, top-p and the draw (sampler.cpp:37-49) over k <= WAVE candidates held by one wave:
-// lane i holds candidate i in ferro's order (0 past k). Sums are DPP wave scans in candidate order. Writes the
-// optional candidate outputs; returns the token and the kept count.
-__device__ __forceinline__ void wave_softmax(const Args& a, const RowCtx& rc, uint64_t v, int k, double u, int& tok_out,
-                                             int& keep_out) {
-    const int lane = lane_id();
-    const int row = rc.row;
-    const fs_row_params& p = rc.p;
-    const float mx = val_of(comp_key(read_lane(v, 0)));
-    const double Td = (double)p.temperature;
-    double e = 0.0;
-    if (lane < k) {
-        const float d = val_of(comp_key(v)) - mx;        // fp32 subtraction, as ferro
-        e = exp((double)d / Td);
-    }
-    const double sum = lane_f64(wave_scan_f64(e), WAVE - 1);   // lanes >= k hold 0
-    const double pr = e / sum;
-    const double cum = wave_scan_f64(pr);                 // ferro's running c (sampler.cpp:44,47)
-    int keep_m = k;
-    if (p.min_p > 0.0f) {                                 // keep = 1 + the last index not below pr[0]*min_p (NaN masses stay)
-        const double thr = lane_f64(pr, 0) * (double)p.min_p;
-        const uint64_t mm = __ballot(lane < k && !(pr < thr));
-        keep_m = mm ? 64 - __clzll((long long)mm) : 1;
-    }
-    int keep = keep_m;
-    if (p.top_p < 1.0f) {
-        const uint64_t mm = __ballot(lane < keep_m && cum >= (double)p.top_p);
-        if (mm) {
-            const int first = __ffsll((unsigned long long)mm) - 1;
-            keep = first + 1 < keep_m ? first + 1 : keep_m;
-        }
-    }
-    const double tot = lane_f64(cum, keep - 1);
-    const double rr = u * tot + 0.0;
-    const uint64_t hm = __ballot(lane < keep && rr <= cum);
-    const int at = hm ? __ffsll((unsigned long long)hm) - 1 : keep - 1;
-    tok_out = (int)comp_id(read_lane(v, at));
-    keep_out = keep;
-    if (a.mode != MODE_VERIFY) {
-        const int m = k < a.kcap ? k : a.kcap;
-        if (lane < m) {
-            if (a.cand_ids) a.cand_ids[(int64_t)row * a.kcap + lane] = (int32_t)comp_id(v);
-            if (a.cand_probs) a.cand_probs[(int64_t)row * a.kcap + lane] = pr;
-        }
-    }
 }
 
 // The short merge: rows with no partial tail tile whose segment lists lie inside the prefetched windows.
@@ -4631,114 +3772,6 @@ __global__ __launch_bounds__(PEN_BLOCK) void penalize_kernel(float* logits, int6
     }
 }
 
-// ------------------------------------------------------------------------------------------------ prompt lookup
-// Prompt-lookup drafting (server.cpp:552-564), one workgroup per stream: for n = min(4, L-1) down to min_n, every
-// thread tests its positions p for h[p, p+n) == the history's last n tokens with a non-eos token after the match
-// (the reference skips a match whose continuation is empty); the largest such p (the most recent occurrence) wins,
-// and the tokens after it, up to kmax and stopping before eos, are the draft.
-constexpr int LD_BLOCK = 256;
-
-// History append (the per-stream hist.push_back of each consumed token, server.cpp:342, as the decode loop at
-// server.cpp:603-606 and the verify window at server.cpp:627-637 feed them), on CSR histories and out of place: stream
-// s keeps its old ids and gains tok[row_off[s] + i], i < n_s, where n_s is count[s] (NULL: 1) clamped to its rows
-// [0, row_off[s+1] - row_off[s]]. The new offsets are old (rebased to 0) + the exclusive prefix of the n_s.
-__device__ __forceinline__ int64_t app_n(const int64_t* row_off, const int32_t* count, int s, bool* bad) {
-    const int64_t r0 = row_off ? row_off[s] : (int64_t)s;
-    const int64_t nr = row_off ? row_off[s + 1] - r0 : 1;
-    int64_t n = count ? (int64_t)count[s] : 1;
-    if (n < 0 || n > nr) {
-        *bad = true;
-        n = n < 0 ? 0 : nr;
-    }
-    return n;
-}
-
-// One workgroup: the new offsets, streams in chunks of BLOCK (carry in int64).
-__global__ __launch_bounds__(BLOCK) void hist_offsets_kernel(int S, const int64_t* hist_off, const int64_t* row_off,
-                                                             const int32_t* count, int64_t* out_off, int64_t out_cap,
-                                                             int32_t* err) {
-    __shared__ uint32_t wsum[NWAVES];
-    const int tid = threadIdx.x;
-    const int64_t h0 = hist_off[0];
-    int64_t carry = 0;
-    bool bad = false;
-    for (int c0 = 0; c0 < S; c0 += BLOCK) {
-        const int s = c0 + tid;
-        const uint32_t n = s < S ? (uint32_t)app_n(row_off, count, s, &bad) : 0u;
-        uint32_t tot;
-        const uint32_t ex = block_excl_scan<uint32_t>(n, wsum, &tot);
-        if (s < S) out_off[s] = hist_off[s] - h0 + carry + ex;
-        carry += tot;
-        __syncthreads();                                 // wsum is reused by the next chunk
-    }
-    if (tid == 0) {
-        const int64_t end = hist_off[S] - h0 + carry;
-        out_off[S] = end;
-        if (end > out_cap) atomicOr(err, FS_DEVERR_HIST_APPEND);
-    }
-    if (bad) atomicOr(err, FS_DEVERR_HIST_APPEND);
-}
-
-// One workgroup per stream: its old ids, then its appended tokens (positions >= out_cap are not written).
-__global__ __launch_bounds__(LD_BLOCK) void hist_append_kernel(const int32_t* hist, const int64_t* hist_off,
-                                                               const int32_t* tok, const int64_t* row_off,
-                                                               const int32_t* count, const int64_t* out_off,
-                                                               int32_t* out, int64_t out_cap) {
-    const int s = (int)blockIdx.x;
-    bool bad = false;
-    const int64_t n = app_n(row_off, count, s, &bad);
-    const int64_t a = hist_off[s], L = hist_off[s + 1] - a;
-    const int64_t o = out_off[s];
-    const int64_t r0 = row_off ? row_off[s] : (int64_t)s;
-    for (int64_t i = threadIdx.x; i < L + n; i += LD_BLOCK) {
-        const int64_t d = o + i;
-        if (d < out_cap) out[d] = i < L ? hist[a + i] : tok[r0 + (i - L)];
-    }
-}
-
-__global__ __launch_bounds__(LD_BLOCK) void lookup_draft_kernel(const int32_t* hist, const int64_t* hist_off,
-                                                                const int32_t* kmax_arr, const int32_t* min_n_arr,
-                                                                int eos, int32_t* draft, int draft_ld,
-                                                                int32_t* ndraft) {
-    __shared__ int64_t wbest[LD_BLOCK / WAVE];
-    const int st = (int)blockIdx.x;
-    const int tid = threadIdx.x;
-    const int64_t h0 = hist_off[st];
-    const int64_t L = hist_off[st + 1] - h0;
-    const int32_t* h = hist + h0;
-    int kmax = kmax_arr ? kmax_arr[st] : draft_ld;
-    kmax = kmax < draft_ld ? kmax : draft_ld;
-    const int min_n = min_n_arr ? min_n_arr[st] : 2;
-    int d = 0;
-    for (int64_t n = (L - 1 < 4 ? L - 1 : 4); n >= min_n && kmax > 0; --n) {
-        int32_t t[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) t[q] = q < n ? h[L - n + q] : 0;
-        int64_t best = -1;
-        for (int64_t p = tid; p <= L - n - 1; p += LD_BLOCK) {
-            bool eq = true;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) eq = eq && (q >= n || h[p + q] == t[q]);
-            if (eq && h[p + n] != eos) best = p;               // p grows: the last hit is this thread's largest
-        }
-        best = wave_max(best);
-        if (lane_id() == 0) wbest[tid / WAVE] = best;
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < LD_BLOCK / WAVE; ++w) best = wbest[w] > best ? wbest[w] : best;
-        __syncthreads();
-        if (best >= 0) {
-            if (tid == 0)
-                for (int64_t k = best + n; k < L && d < kmax; ++k) {
-                    if (h[k] == eos) break;
-                    draft[(int64_t)st * draft_ld + d++] = h[k];
-                }
-            break;
-        }
-    }
-    if (tid == 0) ndraft[st] = d;
-}
-
 // ------------------------------------------------------------------------------------------------ draw streams
 // std::mt19937_64 (the standard's parameters: n = 312, m = 156, r = 31, a = 0xB5026F5AA96619E9, tempering
 // u = 29 / d = 0x5555555555555555, s = 17 / b = 0x71D67FFFEDA60000, t = 37 / c = 0xFFF7EEE000000000, l = 43) per
@@ -4793,855 +3826,6 @@ __global__ __launch_bounds__(64) void drng_skip_kernel(uint64_t* mts, int32_t* i
         c -= take;
     }
     idxs[sidx] = idx;
-}
-
-// ------------------------------------------------------------------------------------------------ small-k kernel
-// A separate kernel for batches whose every row is greedy or samples from k <= SK_K candidates with at most a
-// repetition penalty (no frequency / presence counts) - the serving batches of ferro's decode loop (server.cpp:603-606:
-// top-k 40-64 on every row). The host picks it from a host copy of the parameters (fs_sample_batch_hp). It has its own
-// register budget (it shares no code path with the fused kernel above), which lets it stream a row differently:
-//   - one workgroup of SK_LT threads per (row, segment): every load of the segment (NL float4 per thread) is issued at
-//     once, so the whole batch is requested at the start. The memory system serves the requests roughly in dispatch
-//     order, so a row's segments (consecutive workgroups) receive their data together, and rows finish one after
-//     another: the merge of an early row overlaps the streaming of later rows;
-//   - per group of four logits only a maximum and, later, one compare: the bound is the ceil(k / waves)-th largest
-//     lane maximum of each wave, the smallest over the waves (each lane maximum is a distinct logit of the segment, so
-//     at least k logits of the segment reach it). Groups whose maximum reaches it are written to LDS, expanded to the
-//     candidates at or above it (about 1.5 k per segment on heavy-tailed rows), and sorted exactly into the segment's
-//     top k by a bitonic network in registers (DPP and permlane moves: no LDS round trips);
-//   - the last segment of a row to finish (an L2 ticket) merges the row's sorted lists by a tree of bitonic merges and
-//     finishes the row in one wave (softmax at temperature, min-p, top-p, draw: the merge path's wave_softmax).
-// A segment with more than SK_CAP candidates (ties at its bound) selects its exact top k by a radix select over the
-// composites held in registers instead (slow, exact).
-constexpr int SK_LT = 256;                 // threads per segment workgroup
-constexpr int SK_NW = SK_LT / WAVE;
-constexpr int SK_K = 64;                   // largest k (one candidate per lane of the finishing wave)
-constexpr int SK_GCAP = 128;               // groups of four a wave can hand to the expansion
-constexpr int SK_CAP = 512;                // candidates a segment ranks in LDS
-constexpr int SK_MAX_SEGS = 64;            // segments per row
-
-struct SkArgs {
-    const float* logits;
-    int64_t ld;
-    int B, V, nseg;
-    const int32_t* hist;
-    const int64_t* hist_off;
-    const fs_row_params* params;
-    const double* u;
-    int32_t* tok;
-    int kcap;
-    int32_t* cand_ids;
-    double* cand_probs;
-    int32_t* keep;
-    uint64_t* lists;                       // [B * nseg][SK_K]: each segment's top k, sorted, 0-padded
-    uint32_t* ticket;                      // [B]: segments finished (left at 0)
-    int32_t* err;
-    uint64_t* trace;                       // FS_TRACE builds: per-workgroup phase timestamps (NULL: none)
-    // verification windows (mode MODE_VERIFY; the host sends only windows without an active penalty here)
-    int mode;
-    const int32_t* rows;                   // token fed at each row
-    const int64_t* row_off;                // stream -> rows
-    int n_streams, eos;
-    int32_t* accepted;
-    uint32_t* stream_cnt;                  // [3 n_streams]: 64-bit counts + stop bits, 32-bit counts (left at 0)
-    // a decode step (fs_decode_step_hp; NULL otherwise): draw streams and the histories with the tokens appended
-    uint64_t* dmt;
-    int32_t* didx;
-    int32_t* out_hist;
-    int64_t* out_hist_off;
-    int64_t out_cap;
-};
-
-// lane ^ D over the wave, in the VALU: DPP for D < 16 (both shifts in full exec, then an arithmetic select: a branch
-// would run each DPP move on half the lanes), permlane swaps for 16 and 32 (gfx950)
-template <int D>
-__device__ __forceinline__ uint32_t xor_lane32(uint32_t v) {
-    if constexpr (D == 1) {
-        return dpp32<0xB1>(v);                                  // quad_perm [1,0,3,2]
-    } else if constexpr (D == 2) {
-        return dpp32<0x4E>(v);                                  // quad_perm [2,3,0,1]
-    } else if constexpr (D == 4 || D == 8) {
-        const uint32_t up = dpp32<0x100 + D>(v), dn = dpp32<0x110 + D>(v);   // row_shl: lane + D; row_shr: lane - D
-        const uint32_t m = 0u - (((uint32_t)lane_id() / D) & 1u);
-        return up ^ ((up ^ dn) & m);
-    } else if constexpr (D == 16) {
-        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-        return (lane_id() & 16) ? r[0] : r[1];
-    } else {
-        static_assert(D == 32, "xor distances 1..32");
-        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-        return (lane_id() & 32) ? r[0] : r[1];
-    }
-}
-template <int D>
-__device__ __forceinline__ uint64_t xor_lane64(uint64_t v) {
-    return ((uint64_t)xor_lane32<D>((uint32_t)(v >> 32)) << 32) | (uint64_t)xor_lane32<D>((uint32_t)v);
-}
-// Bitonic compare-exchange at distance D: the lane keeps the larger of its pair iff (its bit D is clear) == up.
-template <int D>
-__device__ __forceinline__ uint64_t bcx(uint64_t v, bool up) {
-    const uint64_t o = xor_lane64<D>(v);
-    const bool keep_max = ((lane_id() & D) == 0) == up;
-    return keep_max ? (v > o ? v : o) : (v < o ? v : o);
-}
-// 32-bit compare-exchange and descending sort of the wave's 64 values (lane 0 the largest), VALU only.
-template <int D>
-__device__ __forceinline__ uint32_t bcx32(uint32_t v, bool up) {
-    const uint32_t o = xor_lane32<D>(v);
-    const bool keep_max = ((lane_id() & D) == 0) == up;
-    const uint32_t hi = v > o ? v : o, lo = v > o ? o : v;
-    return keep_max ? hi : lo;
-}
-__device__ __forceinline__ uint32_t sort64_desc_u32(uint32_t v) {
-    const int lane = lane_id();
-    { const bool up = (lane & 2) == 0; v = bcx32<1>(v, up); }
-    { const bool up = (lane & 4) == 0; v = bcx32<2>(v, up); v = bcx32<1>(v, up); }
-    { const bool up = (lane & 8) == 0; v = bcx32<4>(v, up); v = bcx32<2>(v, up); v = bcx32<1>(v, up); }
-    { const bool up = (lane & 16) == 0;
-      v = bcx32<8>(v, up); v = bcx32<4>(v, up); v = bcx32<2>(v, up); v = bcx32<1>(v, up); }
-    { const bool up = (lane & 32) == 0;
-      v = bcx32<16>(v, up); v = bcx32<8>(v, up); v = bcx32<4>(v, up); v = bcx32<2>(v, up); v = bcx32<1>(v, up); }
-    v = bcx32<32>(v, true); v = bcx32<16>(v, true); v = bcx32<8>(v, true); v = bcx32<4>(v, true);
-    v = bcx32<2>(v, true);
-    return bcx32<1>(v, true);
-}
-
-// The wave's 64 values sorted, descending (lane 0 the largest) or ascending.
-template <bool DESC>
-__device__ __forceinline__ uint64_t sort64(uint64_t v) {
-    const int lane = lane_id();
-    { const bool up = ((lane & 2) == 0) == DESC; v = bcx<1>(v, up); }
-    { const bool up = ((lane & 4) == 0) == DESC; v = bcx<2>(v, up); v = bcx<1>(v, up); }
-    { const bool up = ((lane & 8) == 0) == DESC; v = bcx<4>(v, up); v = bcx<2>(v, up); v = bcx<1>(v, up); }
-    { const bool up = ((lane & 16) == 0) == DESC;
-      v = bcx<8>(v, up); v = bcx<4>(v, up); v = bcx<2>(v, up); v = bcx<1>(v, up); }
-    { const bool up = ((lane & 32) == 0) == DESC;
-      v = bcx<16>(v, up); v = bcx<8>(v, up); v = bcx<4>(v, up); v = bcx<2>(v, up); v = bcx<1>(v, up); }
-    v = bcx<32>(v, DESC); v = bcx<16>(v, DESC); v = bcx<8>(v, DESC); v = bcx<4>(v, DESC); v = bcx<2>(v, DESC);
-    return bcx<1>(v, DESC);
-}
-// The top 64 of a (sorted descending) and b (sorted ascending), sorted descending (DESC) or ascending: the lane-wise
-// maximum is a bitonic sequence holding them, then a bitonic merge.
-template <bool DESC = true>
-__device__ __forceinline__ uint64_t merge_top64(uint64_t a_desc, uint64_t b_asc) {
-    uint64_t v = a_desc > b_asc ? a_desc : b_asc;
-    v = bcx<32>(v, DESC); v = bcx<16>(v, DESC); v = bcx<8>(v, DESC); v = bcx<4>(v, DESC); v = bcx<2>(v, DESC);
-    return bcx<1>(v, DESC);
-}
-
-// fs_decode_step_hp on the small-k kernel (the fused kernel's decode_hist_copy / row_u / decode_commit for this
-// kernel's merging workgroup): the stream's history copied to the new histories by the whole workgroup before the
-// merge; the draw read from the stream without advancing it; after the token, wave 0 appends it and advances the
-// stream (greedy rows draw nothing).
-__device__ __forceinline__ void sk_hist_copy(const SkArgs& a, int row) {
-    const int64_t h0 = a.hist_off ? a.hist_off[0] : 0, b = a.hist_off ? a.hist_off[row] : 0;
-    const int64_t e = a.hist_off ? a.hist_off[row + 1] : 0;
-    const int64_t nb = b - h0 + row;
-    for (int64_t i = threadIdx.x; i < e - b; i += SK_LT)
-        if (nb + i < a.out_cap) a.out_hist[nb + i] = a.hist[b + i];
-    if (threadIdx.x == 0) {
-        a.out_hist_off[row] = nb;
-        if (row == a.B - 1) a.out_hist_off[a.B] = e - h0 + a.B;
-        if (nb + (e - b) + 1 > a.out_cap) atomicOr(a.err, FS_DEVERR_HIST_APPEND);
-    }
-}
-__device__ __forceinline__ double sk_row_u(const SkArgs& a, int row) {
-    if (a.dmt) {
-        const uint64_t* mt = a.dmt + (int64_t)row * MT_N;
-        const int idx = a.didx[row];
-        const uint64_t y = idx < MT_N ? mt[idx] : mt_twist_one(mt[0], mt[1], mt[MT_M]);
-        return mt_canonical(mt_temper(y));
-    }
-    return a.u ? ld_const(a.u + row) : 0.0;
-}
-// Wave 0 alone: w is LDS scratch of MT_N entries. The twist in three passes, each reading every value it needs
-// before it writes: entries below N - M from old values only (all computed, then written); the rest in ascending
-// chunks of one wave (each reads its own and the next old entry and a new one below N - M; entry N - 1 the new
-// entry 0), so no entry is overwritten before it is read.
-__device__ __forceinline__ void sk_decode_commit(const SkArgs& a, int row, bool sampled, int tok, uint64_t* w) {
-    const int lane = lane_id();
-    if (a.out_hist_off && lane == 0) {
-        const int64_t h0 = a.hist_off ? a.hist_off[0] : 0, b = a.hist_off ? a.hist_off[row] : 0;
-        const int64_t e = a.hist_off ? a.hist_off[row + 1] : 0;
-        const int64_t at = b - h0 + row + (e - b);
-        if (at < a.out_cap) a.out_hist[at] = tok;
-    }
-    if (!a.dmt || !sampled) return;
-    uint64_t* mt = a.dmt + (int64_t)row * MT_N;
-    const int idx = a.didx[row];
-    if (idx < MT_N) {
-        if (lane == 0) a.didx[row] = idx + 1;
-        return;
-    }
-    auto wave_sync = []() {
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    };
-    for (int t = lane; t < MT_N; t += WAVE) w[t] = mt[t];
-    wave_sync();
-    constexpr int LO = MT_N - MT_M, NLO = (LO + WAVE - 1) / WAVE;
-    uint64_t nv[NLO];
-#pragma unroll
-    for (int c = 0; c < NLO; ++c) {
-        const int t = c * WAVE + lane;
-        nv[c] = t < LO ? mt_twist_one(w[t], w[t + 1], w[t + MT_M]) : 0ull;
-    }
-    wave_sync();
-#pragma unroll
-    for (int c = 0; c < NLO; ++c) {
-        const int t = c * WAVE + lane;
-        if (t < LO) w[t] = nv[c];
-    }
-    wave_sync();
-    for (int t0 = LO; t0 < MT_N; t0 += WAVE) {
-        const int t = t0 + lane;
-        uint64_t v = 0ull;
-        if (t < MT_N) v = mt_twist_one(w[t], w[(t + 1) % MT_N], w[t - LO]);
-        wave_sync();
-        if (t < MT_N) w[t] = v;
-        wave_sync();
-    }
-    for (int t = lane; t < MT_N; t += WAVE) mt[t] = w[t];
-    if (lane == 0) a.didx[row] = 1;
-}
-
-struct SkShared {
-    float4 gval[SK_NW][SK_GCAP + 1];       // groups of four whose maximum reaches the bound (+ a dummy slot)
-    int32_t gidx[SK_NW][SK_GCAP + 1];      //   and the segment offset of their first logit
-    uint64_t cand[SK_CAP];                 // the segment's candidates (composites)
-    uint64_t wl[SK_NW][SK_K];              // per-wave sorted lists (segment sort, row merge)
-    uint32_t bmp[SK_LT * 16 * 4 / 32];     // repetition window ids in the segment (largest segment: NL = 16)
-    uint32_t hist[16];                     // radix select digits (exact fallback)
-    uint32_t wb[SK_NW];
-    uint32_t wcnt[SK_NW];
-    uint32_t tscan[SK_NW];
-    uint32_t misc[4];
-#ifdef FS_TRACE
-    uint64_t trace_t[16];
-#endif
-};
-static_assert(offsetof(SkShared, cand) % 16 == 0, "the rank loops read the candidates in 16-byte pairs");
-// Phase timestamps of the small-k kernel (FS_TRACE builds only; thread 0, after the barrier that closes a phase):
-// 0 start, 11 the segment's logits in and transformed, 12 lane maxima sorted, 2 bound, 3 groups handed over,
-// 4 candidates expanded, 5 list ranked and published, 6 ticket taken; merging workgroup: 7 lists folded, 8 row
-// finished (greedy rows set only 0, 5-8). Slots 9-10: candidates and groups of the segment; 13-15: role (3 segment,
-// 4 segment + merge), row, segment. ferro_amd/trace_phases.py --route host reads them.
-#ifdef FS_TRACE
-#define SK_MARK(i) do { if (threadIdx.x == 0) s.trace_t[(i)] = __builtin_amdgcn_s_memrealtime(); } while (0)
-#define SK_TAG(i, v) do { if (threadIdx.x == 0) s.trace_t[(i)] = (uint64_t)(v); } while (0)
-#define SK_FLUSH() do { if (threadIdx.x == 0 && a.trace) \
-    for (int i_ = 0; i_ < TRACE_W; ++i_) a.trace[(int64_t)blockIdx.x * TRACE_W + i_] = s.trace_t[i_]; } while (0)
-#else
-#define SK_MARK(i) do {} while (0)
-#define SK_TAG(i, v) do {} while (0)
-#define SK_FLUSH() do {} while (0)
-#endif
-
-// The exact path, for segments whose candidates at the bound overflow SK_CAP (ties at the bound): the segment's
-// logits are re-read from memory (the L2 holds them by then) in batches of SK_EB per thread, sixteen loads in flight,
-// and transformed again (softcap, then the repetition penalty from the segment's bitmap; past n: NaN).
-constexpr int SK_EB = 16;
-template <bool CAP, class F>
-__device__ __forceinline__ void sk_each(const float* segp, int n, int nseg_elems, float cap, bool pen, float rep,
-                                        const uint32_t* bmp, F f) {
-    const int tid = threadIdx.x;
-#pragma unroll 1
-    for (int i0 = 0; i0 < nseg_elems; i0 += SK_LT * SK_EB) {
-        float x[SK_EB];
-#pragma unroll
-        for (int j = 0; j < SK_EB; ++j) {
-            const int i = i0 + j * SK_LT + tid;
-            x[j] = i < n ? segp[i] : 0.0f;
-        }
-        if (CAP && cap > 0.0f) softcap_vals(x, cap);
-#pragma unroll
-        for (int j = 0; j < SK_EB; ++j) {
-            const int i = i0 + j * SK_LT + tid;
-            float l = x[j];
-            if (pen && i < n && ((bmp[i >> 5] >> (i & 31)) & 1u)) l = l > 0.0f ? __fdiv_rn(l, rep) : __fmul_rn(l, rep);
-            f(i, i < n ? key_of(l) : 0u);
-        }
-    }
-}
-// The exact k-th largest composite of the segment (every composite is distinct: the id is part of it), by a radix
-// select over 4-bit digits. Slow, and rare.
-template <bool CAP>
-__device__ __forceinline__ uint64_t sk_kth_exact(const float* segp, int seg_lo, int n, int nseg_elems, float cap,
-                                                 bool pen, float rep, int k, SkShared& s) {
-    const int tid = threadIdx.x;
-    uint64_t prefix = 0ull;
-    int need = k;
-#pragma unroll 1
-    for (int sh = 60; sh >= 0; sh -= 4) {
-        if (tid < 16) s.hist[tid] = 0u;
-        __syncthreads();
-        const uint64_t hi_mask = sh + 4 >= 64 ? 0ull : (~0ull << (sh + 4));
-        sk_each<CAP>(segp, n, nseg_elems, cap, pen, rep, s.bmp, [&](int i, uint32_t key) {
-            const uint64_t cm = comp_of(key, (uint32_t)(seg_lo + i));
-            if (key != 0u && (cm & hi_mask) == prefix) atomicAdd(&s.hist[(uint32_t)(cm >> sh) & 15u], 1u);
-        });
-        __syncthreads();
-        if (tid == 0) {
-            int d = 15;
-            for (; d > 0; --d) {
-                const int c = (int)s.hist[d];
-                if (c >= need) break;
-                need -= c;
-            }
-            s.misc[2] = (uint32_t)d;
-            s.misc[3] = (uint32_t)need;
-        }
-        __syncthreads();
-        prefix |= (uint64_t)s.misc[2] << sh;
-        need = (int)s.misc[3];
-        __syncthreads();
-    }
-    return prefix;
-}
-
-// CAP: some row of the batch has a softcap (the cap's code is left out of batches without one).
-struct Ids16 {
-    int32_t v[16];
-};
-
-// small_k_kernel's argument list as a struct: the argument segment follows the same layout rules
-struct SkKernargs {
-    const float* logits;
-    int64_t ld;
-    int B, V, nseg, may_pen;
-    const fs_row_params* params;
-    const int64_t* hist_off;
-    const int32_t* hist;
-    SkArgs a;
-};
-constexpr size_t SK_ARGS_OFF = offsetof(SkKernargs, a);
-
-// Dynamic LDS a launch requests beyond SkShared (unused): with it a CU holds 4 workgroups (≈35 KB each of its 160 KB),
-// as the kernel's 96 VGPRs would otherwise allow 5. Measured on MI355X with this instantiation: a 272-row call of 1088
-// workgroups 21.3 -> 20.6 us with the limit, the headline's 1024 workgroups unchanged. (All-greedy batches run the
-// greedy-only instantiation without it.)
-constexpr unsigned SK_PAD_LDS = 16384;
-
-// GREEDY: every row of the batch is greedy (the selection code is left out: fewer registers, more workgroups per CU).
-template <int NL, bool CAP, bool GREEDY>
-__global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int64_t ld, int B, int V, int nseg,
-                                                        int may_pen, const fs_row_params* params,
-                                                        const int64_t* hist_off, const int32_t* hist, SkArgs a_) {
-    // The leading arguments arrive in SGPRs at wave launch (kernel-argument preloading), so the logits are requested
-    // before any scalar memory round trip. A call with a repetition window (may_pen, set by the host from its copy of
-    // the parameters) then reads the row's window bounds and requests its ids behind the logits.
-    constexpr int SEG = SK_LT * NL * 4;
-    static_assert(NL <= 16, "the repetition bitmap covers NL <= 16");
-    __shared__ __align__(16) SkShared s;
-    const int tid = threadIdx.x, lane = lane_id(), w = tid / WAVE;
-    // workgroup i: XCD slot i % XCDS takes rows x, x + XCDS, ...: a row's segments are consecutive workgroups of one
-    // index class mod XCDS, so they share an XCD and its L2 (the ticket and the lists)
-    const int x = (int)(blockIdx.x % (unsigned)XCDS);
-    const int j = (int)(blockIdx.x / (unsigned)XCDS);
-    const int q_row = __builtin_amdgcn_readfirstlane(j / nseg);
-    const int seg = j - q_row * nseg;
-    const int row = x + XCDS * q_row;
-    if (row >= B) return;
-    SK_MARK(0);
-    for (int i_ = 1; i_ < 13; ++i_) SK_TAG(i_, 0);
-    SK_TAG(13, 3); SK_TAG(14, row); SK_TAG(15, seg);
-    const int seg_lo = seg * SEG;
-    const int n_in = V - seg_lo < SEG ? V - seg_lo : SEG;             // logits of this segment (>= 1)
-
-    // every load of the segment at once; past the row's end (rounded up to four, inside ld) reads are zeros, masked
-    const float* rowp = logits + (int64_t)row * ld;
-    const int nrec = ((n_in + 3) & ~3) * 4;
-    const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(rowp + seg_lo), (short)0, nrec, 0x00020000);
-    float4 v[NL];
-#pragma unroll
-    for (int q = 0; q < NL; ++q) {
-        const f32x4 t = raw_buffer_load_f32x4(rs, (q * SK_LT + tid) * 16, 0, 2);    // nontemporal: read once
-        v[q] = make_float4(t.x, t.y, t.z, t.w);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-
-    // the repetition window [wb0, len) over the row's history (sampling rows only: verification windows reach this
-    // kernel only without an active penalty); its first 512 ids are requested behind the logits, two per thread
-    bool pen = false, cnt_on = false;
-    float rep = 1.0f, fq = 0.0f, pres = 0.0f;
-    int64_t h0 = 0, len = 0, wb0 = 0;
-    int wid[2] = {-1, -1};
-    if (may_pen) {
-        const fs_row_params* pr = params + row;
-        rep = ld_const(&pr->repetition_penalty);
-        fq = ld_const(&pr->frequency_penalty);
-        pres = ld_const(&pr->presence_penalty);
-        fs_row_params pw;
-        pw.repeat_last_n = ld_const(&pr->repeat_last_n);
-        pw.penalty_from = ld_const(&pr->penalty_from);
-        h0 = ld_const(hist_off + row);
-        len = ld_const(hist_off + row + 1) - h0;
-        // frequency / presence penalties (greedy rows only, segments of 4096 logits: the host checks both) need
-        // each window id's count in the segment
-        cnt_on = NL == 4 && (fq != 0.0f || pres != 0.0f);
-        pen = (rep != 1.0f || cnt_on) && pw.repeat_last_n != 0 && len > 0;
-        wb0 = window_begin(len, pw);                           // unconditionally: all five loads in one round trip
-        if (!pen || wb0 >= len) { pen = false; wb0 = len; }
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const int64_t i = wb0 + r * SK_LT + tid;
-            wid[r] = (pen && i < len) ? hist[h0 + i] : -1;
-        }
-    }
-    // The remaining arguments are read from here on, through a pointer the compiler cannot trace back to the argument
-    // segment: otherwise it loads some of them early and, short of scalar registers, spills them to vector lanes,
-    // which waits for those loads before the logits are requested.
-    const __attribute__((address_space(4))) char* kseg =
-        (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(kseg) : : "memory");
-    const SkArgs& a = *(const SkArgs*)(kseg + SK_ARGS_OFF);
-    (void)a_;
-
-    // verification: the row's stream (its parameters); sampling: the row's own
-    int pidx = row;
-    if (a.mode == MODE_VERIFY) {
-        int s0 = 0, s1 = a.n_streams;                          // the largest s with row_off[s] <= row
-        while (s1 - s0 > 1) {
-            const int m = (s0 + s1) >> 1;
-            if (ld_const(a.row_off + m) <= row) s0 = m; else s1 = m;
-        }
-        pidx = s0;
-    }
-    const fs_row_params* pp = params + pidx;
-    const float temp = ld_const(&pp->temperature);
-    const int top_k = ld_const(&pp->top_k);
-    const float cap = CAP ? ld_const(&pp->softcap) : 0.0f;
-    const bool greedy = GREEDY || temp <= 0.0f || top_k == 1;
-    const int k = greedy ? 1 : ((top_k > 0 && top_k < V) ? top_k : V);
-
-    // repetition penalty: an exact bitmap of the window's ids in this segment (each distinct id once: sampler.cpp:14-17).
-    // rep >= 1 never raises a logit (l > 0: l / rep <= l; l <= 0: l * rep <= l), so the bound is taken over the raw
-    // logits, the bitmap is filled while the bound is sorted (the ids arrive right behind the logits), and the penalty
-    // is applied to the handed-over logits only; the bound then needs a check (below). rep < 1 raises the flagged
-    // logits: they are penalised before the bound (the bitmap first).
-    // greedy rows take the penalty before their maximum (no bound to protect), with its counts when cnt_on
-    const bool pen_late = pen && rep >= 1.0f && !greedy;
-    const bool pen_early = pen && !pen_late;
-    cnt_on = cnt_on && pen;
-    // cnt_on: 16-bit counts of the window's ids per logit of the segment, in the group buffer (unused on this path)
-    uint32_t* cnt = reinterpret_cast<uint32_t*>(&s.gval[0][0]);
-    static_assert(sizeof(SkShared::gval) >= SK_LT * 4 * 4 / 2 * sizeof(uint32_t),
-                  "a 4096-logit segment's 16-bit counts fit the group buffer");
-    bool ovf = false;
-    auto mark = [&](int id) {
-        const uint32_t rel = (uint32_t)(id - seg_lo);
-        if (id >= 0 && id < V && rel < (uint32_t)SEG) {
-            atomicOr(&s.bmp[rel >> 5], 1u << (rel & 31u));
-            if (cnt_on) {
-                const uint32_t sh = (rel & 1u) * 16u;
-                const uint32_t old = atomicAdd(&cnt[rel >> 1], 1u << sh);
-                ovf |= ((old >> sh) & 0xFFFFu) == 0xFFFFu;
-            }
-        }
-    };
-    auto mark_window = [&]() {
-        // the ids arrive behind the logits: an empty asm keeps the compiler from hoisting their first use (and the
-        // wait for every load it needs) above the branch that calls this
-        int i0 = wid[0], i1 = wid[1];
-        asm volatile("" : "+v"(i0), "+v"(i1));
-        mark(i0);
-        mark(i1);
-        for (int64_t i = wb0 + 2 * SK_LT + tid; i < len; i += SK_LT) mark(a.hist[h0 + i]);
-    };
-    if (pen) {
-        for (int i = tid; i < SEG / 32; i += SK_LT) s.bmp[i] = 0u;
-        if (cnt_on)
-            for (int i = tid; i < SEG / 2; i += SK_LT) cnt[i] = 0u;
-        __syncthreads();
-    }
-    uint64_t pm = 0ull;                        // rep < 1 or greedy: 4 bits per group of this thread
-    if (pen_early) {
-        mark_window();
-        if (ovf) atomicOr(a.err, FS_DEVERR_COUNT_OVERFLOW);
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < NL; ++q) {
-            const uint32_t rel = (uint32_t)(q * SK_LT + tid) * 4u;
-            pm |= (uint64_t)((s.bmp[rel >> 5] >> (rel & 31u)) & 0xFu) << (4 * q);
-        }
-    }
-    const bool wpen = __ballot(pm != 0ull) != 0ull;
-    const bool tail = n_in < SEG;
-
-    // the logits as ferro's sampler sees them (softcap; rep < 1: the penalty; past the row's end: NaN, never a
-    // candidate) and the lane maximum (NaN-free: fmaxf drops NaN; NaN when every logit of the lane is NaN)
-    float lm = __builtin_nanf("");
-#pragma unroll
-    for (int q = 0; q < NL; ++q) {
-        float e[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-        if (CAP && cap > 0.0f) softcap_vals(e, cap);       // a rolled loop: one copy of the cap per group
-        if (wpen) {
-            const uint32_t nib = (uint32_t)(pm >> (4 * q)) & 0xFu;
-            if (__ballot(nib != 0u)) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    if ((nib >> c) & 1u) {
-                        float l = e[c] > 0.0f ? __fdiv_rn(e[c], rep) : __fmul_rn(e[c], rep);
-                        if (cnt_on) {                      // l - (count * frequency + presence), as the fused kernel
-                            const uint32_t rel = (uint32_t)(q * SK_LT + tid) * 4u + (uint32_t)c;
-                            const float cc = (float)((cnt[rel >> 1] >> ((rel & 1u) * 16u)) & 0xFFFFu);
-                            l = __fsub_rn(l, __fadd_rn(__fmul_rn(cc, fq), pres));
-                        }
-                        e[c] = l;
-                    }
-            }
-        }
-        if (tail) {
-            const int e0 = (q * SK_LT + tid) * 4;
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (e0 + c >= n_in) e[c] = __builtin_nanf("");
-        }
-        v[q] = make_float4(e[0], e[1], e[2], e[3]);
-        lm = fmaxf(lm, fmaxf(fmaxf(e[0], e[1]), fmaxf(e[2], e[3])));
-    }
-    // Greedy rows (their penalties already applied above): the segment's list is its first maximum alone (ferro's
-    // scan, sampler.cpp:19-23, takes a larger logit only: the lowest index among equal maxima; NaN never), so the
-    // bound, the candidates and their ranks are skipped: a lane's first index holding its maximum, then the largest
-    // composite of the workgroup (value first, then the lower id). The rest of the list is zeros, which every merge
-    // reads as empty.
-    uint64_t* myl = a.lists + ((int64_t)row * a.nseg + seg) * SK_K;
-    const bool gfast = greedy;
-    if (gfast) {
-        uint64_t best = 0ull;
-        if (lm == lm) {                                        // NaN: every logit of the lane is NaN
-            uint32_t first = 0u;
-#pragma unroll
-            for (int q = NL - 1; q >= 0; --q) {
-                const uint32_t e0 = (uint32_t)(seg_lo + (q * SK_LT + tid) * 4);
-                first = v[q].w == lm ? e0 + 3u : first;
-                first = v[q].z == lm ? e0 + 2u : first;
-                first = v[q].y == lm ? e0 + 1u : first;
-                first = v[q].x == lm ? e0 : first;
-            }
-            best = comp_of(key_of(lm), first);
-        }
-        best = wave_max(best);
-        if (lane == 0) s.wl[w][0] = best;
-        __syncthreads();
-        if (w == 0) {
-            const uint64_t m = wave_max(lane < SK_NW ? s.wl[lane][0] : 0ull);
-            myl[lane] = lane == 0 ? m : 0ull;
-        }
-    } else {
-        // the bound: each wave sorts its lane maxima in registers (no scalar round trips per step); lane kq - 1 holds
-        // its kq-th largest, and the smallest over the waves counts SK_NW kq >= k distinct logits (one lane more per
-        // wave when the penalty comes later: the raw logits counted may be among the penalised ones)
-        const uint32_t kq = (uint32_t)((k + SK_NW - 1) / SK_NW) + (pen_late ? 1u : 0u);
-        SK_MARK(11);
-        {
-            const uint32_t srt = sort64_desc_u32(key_of(lm));
-            if (lane == (int)kq - 1) s.wb[w] = srt;
-        }
-        if (pen_late) mark_window();                               // completed by the barrier below
-        SK_MARK(12);
-        __syncthreads();
-        SK_MARK(2);
-        uint32_t tau = s.wb[0];
-#pragma unroll
-        for (int q = 1; q < SK_NW; ++q) tau = s.wb[q] < tau ? s.wb[q] : tau;
-        if (tau == 0u) tau = 1u;                                   // NaN (key 0) is never a candidate
-        const float tf = tau > 0x007FFFFFu ? val_of(tau) : -__builtin_huge_valf();
-        // groups whose maximum reaches the bound: this wave's region of the group buffer, in lane order
-        uint32_t gmask = 0u;
-#pragma unroll
-        for (int q = 0; q < NL; ++q)                     // the group's raw maximum (recomputed: no register array)
-            gmask |= (fmaxf(fmaxf(v[q].x, v[q].y), fmaxf(v[q].z, v[q].w)) >= tf ? 1u : 0u) << q;
-        const uint32_t gn = (uint32_t)__popc(gmask);
-        const uint32_t gincl = wave_incl_scan_u32(gn);
-        const uint32_t wtot = (uint32_t)__builtin_amdgcn_readlane((int)gincl, WAVE - 1);
-        uint32_t go = gincl - gn;
-        // the groups any lane of the wave hands over (one scalar mask); per such group every lane writes, those without
-        // it into the region's dummy slot, so no per-lane branch waits on a compare
-        const uint32_t wmask = (uint32_t)__builtin_amdgcn_readfirstlane(
-            (int)wave_allreduce(gmask, [](uint32_t x, uint32_t y) { return x | y; }));
-#pragma unroll
-        for (int q = 0; q < NL; ++q) {
-            if ((wmask >> q) & 1u) {
-                const bool mine = ((gmask >> q) & 1u) != 0u && go < (uint32_t)SK_GCAP;
-                const uint32_t slot = mine ? go : (uint32_t)SK_GCAP;
-                s.gval[w][slot] = v[q];
-                s.gidx[w][slot] = (int32_t)((uint32_t)(q * SK_LT + tid) * 4u);
-                go += (gmask >> q) & 1u;
-            }
-        }
-        if (lane == 0) s.wcnt[w] = wtot;
-        __syncthreads();
-        SK_MARK(3);
-        // expansion: thread t takes group t of the concatenated regions, its logits at or above the bound become
-        // candidates
-        uint32_t goff[SK_NW + 1];
-        goff[0] = 0u;
-        bool gover = false;
-#pragma unroll
-        for (int q = 0; q < SK_NW; ++q) {
-            const uint32_t c = s.wcnt[q];
-            gover |= c > (uint32_t)SK_GCAP;
-            goff[q + 1] = goff[q] + (c < (uint32_t)SK_GCAP ? c : (uint32_t)SK_GCAP);
-        }
-        const uint32_t G = goff[SK_NW];
-        uint64_t cm[4] = {0ull, 0ull, 0ull, 0ull};
-        bool cp[4] = {false, false, false, false};
-        uint32_t nc = 0u;
-        if (!gover && (uint32_t)tid < G) {
-            int r = 0;
-            uint32_t gb = 0u;
-#pragma unroll
-            for (int q = 1; q < SK_NW; ++q) {
-                const bool past = (uint32_t)tid >= goff[q];
-                r += past ? 1 : 0;
-                gb = past ? goff[q] : gb;
-            }
-            const uint32_t gi = (uint32_t)tid - gb;
-            const float4 gv = s.gval[r][gi];
-            const uint32_t gw = (uint32_t)s.gidx[r][gi];
-            const int e0 = (int)gw;
-            // rep >= 1: the group's penalised logits, from the bitmap (its 4 bits share a word: e0 % 4 == 0)
-            float e[4] = {gv.x, gv.y, gv.z, gv.w};
-            if (pen_late) {
-                const uint32_t nib = (s.bmp[(uint32_t)e0 >> 5] >> ((uint32_t)e0 & 31u)) & 0xFu;
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    if ((nib >> c) & 1u) e[c] = e[c] > 0.0f ? __fdiv_rn(e[c], rep) : __fmul_rn(e[c], rep);
-            }
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                cp[c] = e[c] >= tf;
-                cm[c] = comp_of(key_of(e[c]), (uint32_t)(seg_lo + e0 + c));
-                nc += cp[c] ? 1u : 0u;
-            }
-        }
-        if (G > (uint32_t)SK_LT) gover = true;                     // more groups than threads: the exact path
-        // block exclusive scan of the candidate counts
-        const uint32_t cincl = wave_incl_scan_u32(nc);
-        if (lane == WAVE - 1) s.tscan[w] = cincl;
-        __syncthreads();
-        SK_MARK(4);
-        uint32_t cbase = 0u, ntot = 0u;
-#pragma unroll
-        for (int q = 0; q < SK_NW; ++q) {
-            const uint32_t t = s.tscan[q];
-            cbase += q < w ? t : 0u;
-            ntot += t;
-        }
-        // With the penalty applied after the bound, fewer than k logits may stay at or above it: the segment's top k
-        // may then hold a logit below the bound, which was not handed over (never expected with the spare lane per
-        // wave)
-        const bool short_k = pen_late && ntot < (uint32_t)k && tf > -__builtin_huge_valf();
-        const bool exact = gover || short_k || ntot > (uint32_t)SK_CAP;   // uniform
-        if (!exact) {
-            uint32_t pos = cbase + cincl - nc;
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (cp[c]) s.cand[pos++] = cm[c];
-        }
-        if (exact) {
-            // ties at the bound: the exact k-th composite of the segment, then the (exactly k) composites at or above
-            // it
-            const float* segp = rowp + seg_lo;
-            const uint64_t kth = sk_kth_exact<CAP>(segp, seg_lo, n_in, SEG, cap, pen, rep, k, s);
-            if (tid == 0) s.misc[0] = 0u;
-            __syncthreads();
-            sk_each<CAP>(segp, n_in, SEG, cap, pen, rep, s.bmp, [&](int i, uint32_t key) {
-                const uint64_t c64 = comp_of(key, (uint32_t)(seg_lo + i));
-                if (key != 0u && c64 >= kth) {
-                    const uint32_t p = atomicAdd(&s.misc[0], 1u);
-                    if (p < (uint32_t)SK_K) s.cand[p] = c64;
-                }
-            });
-            __syncthreads();
-            ntot = s.misc[0] < (uint32_t)SK_K ? s.misc[0] : (uint32_t)SK_K;
-        }
-        __syncthreads();
-        // the segment's top k, sorted by rank: P threads per candidate each count the larger entries in 1/P of the list
-        // (LDS reads of one address per wave: broadcasts), the partial counts are summed and the first k placed by rank
-        uint64_t* sorted = &s.wl[0][0];
-        uint32_t* rk = reinterpret_cast<uint32_t*>(&s.wl[1][0]);    // [P][per] partial ranks (SK_LT words)
-        {
-            const int n = (int)ntot;
-            if (n <= SK_LT) {
-                const int P = n <= SK_LT / 4 ? 4 : (n <= SK_LT / 2 ? 2 : 1);
-                const int per = SK_LT / P;
-                const int c = tid % per, qq = tid / per;
-                const int span = (((n + P - 1) / P) + 1) & ~1;     // even: every part starts on a 16-byte pair
-                if (c < n) {
-                    const uint64_t me = s.cand[c];
-                    const int j0 = qq * span, j1 = j0 + span < n ? j0 + span : n;
-                    uint32_t r = 0u;
-                    int jj = j0;
-                    const ulonglong2* c2 = reinterpret_cast<const ulonglong2*>(s.cand);
-                    for (; jj + 8 <= j1; jj += 8) {                // eight entries per step: four 16-byte LDS reads
-                        const ulonglong2 e0 = c2[jj >> 1], e1 = c2[(jj >> 1) + 1], e2 = c2[(jj >> 1) + 2],
-                                         e3 = c2[(jj >> 1) + 3];
-                        r += (e0.x > me ? 1u : 0u) + (e0.y > me ? 1u : 0u) + (e1.x > me ? 1u : 0u) +
-                             (e1.y > me ? 1u : 0u) + (e2.x > me ? 1u : 0u) + (e2.y > me ? 1u : 0u) +
-                             (e3.x > me ? 1u : 0u) + (e3.y > me ? 1u : 0u);
-                    }
-                    for (; jj < j1; ++jj) r += s.cand[jj] > me ? 1u : 0u;
-                    rk[qq * per + c] = r;
-                }
-                __syncthreads();
-                if (tid < n) {                                     // placed straight into the published list
-                    uint32_t r = 0u;
-                    for (int p2 = 0; p2 < P; ++p2) r += rk[p2 * per + tid];
-                    if (r < (uint32_t)k) myl[r] = s.cand[tid];
-                }
-            } else {                                               // 256 < n <= SK_CAP: two candidates per thread
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int c = tid + h * SK_LT;
-                    if (c < n) {
-                        const uint64_t me = s.cand[c];
-                        uint32_t r = 0u;
-                        int jj = 0;
-                        const ulonglong2* c2 = reinterpret_cast<const ulonglong2*>(s.cand);
-                        for (; jj + 8 <= n; jj += 8) {
-                            const ulonglong2 e0 = c2[jj >> 1], e1 = c2[(jj >> 1) + 1], e2 = c2[(jj >> 1) + 2],
-                                             e3 = c2[(jj >> 1) + 3];
-                            r += (e0.x > me ? 1u : 0u) + (e0.y > me ? 1u : 0u) + (e1.x > me ? 1u : 0u) +
-                                 (e1.y > me ? 1u : 0u) + (e2.x > me ? 1u : 0u) + (e2.y > me ? 1u : 0u) +
-                                 (e3.x > me ? 1u : 0u) + (e3.y > me ? 1u : 0u);
-                        }
-                        for (; jj < n; ++jj) r += s.cand[jj] > me ? 1u : 0u;
-                        if (r < (uint32_t)k) myl[r] = me;
-                    }
-                }
-            }
-            if (tid >= (n < k ? n : k) && tid < SK_K) myl[tid] = 0ull;   // slots past the segment's top k
-        }
-        (void)sorted;
-        SK_TAG(9, ntot);
-        SK_TAG(10, G);
-    }
-    vm_drain();                                                // the list is in the L2
-    __syncthreads();
-    SK_MARK(5);
-    if (tid == 0) {
-        const uint32_t t = __hip_atomic_fetch_add(a.ticket + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        s.misc[1] = t == (uint32_t)a.nseg - 1u ? 1u : 0u;
-    }
-    __syncthreads();
-    SK_MARK(6);
-    if (s.misc[1] == 0u) {
-        SK_FLUSH();
-        return;
-    }
-    SK_TAG(13, 4);
-    if (a.out_hist_off) sk_hist_copy(a, row);                  // a decode step: every thread, before the merge
-    // ---- the row's merge (the last of its segments): wave w folds lists w, w + SK_NW, ... (the first as stored,
-    // the rest reversed: ascending), then wave 0 folds the waves' lists
-    const uint64_t* rl = a.lists + (int64_t)row * a.nseg * SK_K;
-    uint64_t acc = 0ull;
-    if (greedy) {
-        // k = 1: every list holds its segment's top composite first; wave 0 takes the largest of the nseg heads
-        if (w != 0) return;
-        SK_MARK(7);
-        if (tid == 0) a.ticket[row] = 0u;                     // all segments have counted: reset for the next call
-        acc = wave_max(lane < a.nseg ? rl[lane * SK_K] : 0ull);
-    } else {
-        for (int L0 = w; L0 < a.nseg; L0 += 4 * SK_NW) {
-            // four lists per wave, requested together: lists 0 and 2 as stored (descending), 1 and 3 reversed
-            uint64_t b[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int L = L0 + r * SK_NW;
-                b[r] = L < a.nseg ? rl[L * SK_K + ((r & 1) ? WAVE - 1 - lane : lane)] : 0ull;
-            }
-            // two independent merges (their latencies overlap), then one
-            const uint64_t m01 = merge_top64<true>(b[0], b[1]);
-            const uint64_t m23 = merge_top64<false>(b[2], b[3]);
-            if (L0 == w) acc = merge_top64<true>(m01, m23);
-            else acc = merge_top64<true>(acc, merge_top64<false>(m01, m23));
-        }
-        // across the waves: waves 0 and 2 fold 1 and 3 (in parallel), then wave 0 folds wave 2's
-        s.wl[w][lane] = acc;
-        __syncthreads();
-        if (w == 0 || w == 2) acc = merge_top64(acc, s.wl[w + 1][WAVE - 1 - lane]);
-        if (w == 2) s.wl[2][lane] = acc;
-        __syncthreads();
-        if (w != 0) return;
-        SK_MARK(7);
-        if (tid == 0) a.ticket[row] = 0u;                     // all segments have counted: reset for the next call
-        acc = merge_top64(acc, s.wl[2][WAVE - 1 - lane]);
-    }
-    // the row's candidates: lane i holds the i-th in ferro's order (value desc, id asc); NaN never is one
-    const int kk = __popcll(__ballot(lane < k && acc != 0ull));
-    Args fa = {};
-    fa.mode = MODE_SAMPLE; fa.kcap = a.kcap; fa.cand_ids = a.cand_ids; fa.cand_probs = a.cand_probs;
-    RowCtx rc = {};
-    rc.row = row;
-    rc.p.temperature = temp; rc.p.top_k = top_k;
-    rc.p.top_p = ld_const(&pp->top_p); rc.p.min_p = ld_const(&pp->min_p);
-    int tok = 0, keep = 1;
-    if (greedy) {
-        // ferro's scan (sampler.cpp:19-23) keeps index 0 when its logit is NaN; otherwise the first maximum
-        float l0 = ld_const(rowp);
-        if (CAP && cap > 0.0f) l0 = softcap_one(l0, cap);
-        tok = (l0 != l0 || kk == 0) ? 0 : (int)comp_id(read_lane(acc, 0));
-        if (lane == 0 && a.kcap > 0) {
-            if (a.cand_ids) a.cand_ids[(int64_t)row * a.kcap] = tok;
-            if (a.cand_probs) a.cand_probs[(int64_t)row * a.kcap] = 1.0;
-        }
-    } else if (kk == 0) {
-        tok = 0; keep = 0;                                     // every logit NaN: token 0, nothing kept
-    } else {
-        wave_softmax(fa, rc, lane < kk ? acc : 0ull, kk, sk_row_u(a, row), tok, keep);
-    }
-    if (a.mode != MODE_VERIFY) {
-        if (lane == 0) {
-            a.tok[row] = tok;
-            if (a.keep) a.keep[row] = keep;
-        }
-        if (a.out_hist_off || a.dmt) sk_decode_commit(a, row, !greedy, tok, &s.cand[0]);
-    } else {
-        // the last row of a stream to finish computes its accepted prefix (server.cpp:627-637): the stream's rows
-        // run on several XCDs, so the exchange is agent-scope.
-        const int64_t r0 = ld_const(a.row_off + pidx);
-        const int m = (int)(ld_const(a.row_off + pidx + 1) - r0);
-        if (m <= 32) {
-            // Streams of up to 32 rows: one 64-bit atomic per row carries everything - the count of rows done in its
-            // high word, in its low word a bit for each row that ends the walk (an eos token, the last row, or a
-            // token other than the next row's draft). The last row's fetched value holds every other row's bit, so
-            // its accepted prefix is the lowest set bit + 1, with no token exchanged and no wait for stores.
-            if (lane == 0) {
-                a.tok[row] = tok;
-                const int rr = row - (int)r0;
-                const bool stop = (a.eos >= 0 && tok == a.eos) || rr + 1 >= m || tok != ld_const(a.rows + row + 1);
-                const uint64_t mine = stop ? (1ull << rr) : 0ull;
-                uint64_t* cnt = reinterpret_cast<uint64_t*>(a.stream_cnt) + pidx;
-                const uint64_t old = __hip_atomic_fetch_add(cnt, (1ull << 32) | mine, __ATOMIC_RELAXED,
-                                                            __HIP_MEMORY_SCOPE_AGENT);
-                if ((uint32_t)(old >> 32) == (uint32_t)m - 1u) {
-                    __hip_atomic_store(cnt, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    a.accepted[pidx] = __ffs((int)((uint32_t)old | (uint32_t)mine));
-                }
-            }
-            SK_MARK(8);
-            SK_FLUSH();
-            return;
-        }
-        // longer streams: the token at agent scope, a row counter (after the 64-bit words), the last row walks
-        uint32_t* cnt32 = a.stream_cnt + 2 * (int64_t)a.n_streams + pidx;
-        uint32_t old = 0u;
-        if (lane == 0) {
-            st_agent(&a.tok[row], (int32_t)tok);
-            vm_drain();
-            old = __hip_atomic_fetch_add(cnt32, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (read_lane(old, 0) == (uint32_t)m - 1u) {
-            if (lane == 0) st_agent(cnt32, 0u);
-            const int acc = accepted_prefix(a.tok, a.rows, r0, m, a.eos);
-            if (lane == 0) a.accepted[pidx] = acc;
-        }
-    }
-    SK_MARK(8);
-    SK_FLUSH();
 }
 
 }  // namespace fs
@@ -6022,33 +4206,7 @@ int launch_small(fs_context* ctx, const fs::Args& a_in, const fs_row_params* h_p
     bool may_pen = ch.may_pen;
     // a verification window reaches this kernel only without an active penalty (small_k_windows)
     may_pen = may_pen && !verify && a.hist && a.hist_off;
-    const dim3 gd((unsigned)grid), bd(fs::SK_LT);
-    // all-greedy batches: the greedy-only kernel, without the LDS pad (its registers allow more workgroups per CU)
-    auto go = [&](auto kern, unsigned pad) {
-        hipLaunchKernelGGL(kern, gd, bd, pad, st, a.logits, a.ld, a.B, a.V, nseg, may_pen ? 1 : 0, a.params,
-                           a.hist_off, a.hist, k);
-    };
-    const unsigned pad = fs::SK_PAD_LDS;
-    if (all_greedy) {
-        if (capped) {
-            if (nl == 16) go(fs::small_k_kernel<16, true, true>, 0u);
-            else if (nl == 8) go(fs::small_k_kernel<8, true, true>, 0u);
-            else go(fs::small_k_kernel<4, true, true>, 0u);
-        } else {
-            if (nl == 16) go(fs::small_k_kernel<16, false, true>, 0u);
-            else if (nl == 8) go(fs::small_k_kernel<8, false, true>, 0u);
-            else go(fs::small_k_kernel<4, false, true>, 0u);
-        }
-    } else if (capped) {
-        if (nl == 16) go(fs::small_k_kernel<16, true, false>, pad);
-        else if (nl == 8) go(fs::small_k_kernel<8, true, false>, pad);
-        else go(fs::small_k_kernel<4, true, false>, pad);
-    } else {
-        if (nl == 16) go(fs::small_k_kernel<16, false, false>, pad);
-        else if (nl == 8) go(fs::small_k_kernel<8, false, false>, pad);
-        else go(fs::small_k_kernel<4, false, false>, pad);
-    }
-    if (hipGetLastError() != hipSuccess) return FS_E_HIP;
+    if (fs::launch_small_k(nl, capped, all_greedy, (unsigned)grid, may_pen ? 1 : 0, k, st) != hipSuccess) return FS_E_HIP;
     used = true;
     return FS_OK;
 }
@@ -6402,9 +4560,8 @@ int fs_lookup_draft(fs_context* ctx, int32_t n_streams, const int32_t* d_hist, c
                     int32_t* d_ndraft, void* stream) {
     if (!ctx || n_streams < 0 || !d_hist_off || !d_draft || !d_ndraft || draft_ld < 1) return FS_E_INVALID;
     if (n_streams == 0) return FS_OK;
-    hipLaunchKernelGGL(fs::lookup_draft_kernel, dim3((unsigned)n_streams), dim3(fs::LD_BLOCK), 0, (hipStream_t)stream,
-                       d_hist, d_hist_off, d_kmax, d_min_n, eos_id, d_draft, draft_ld, d_ndraft);
-    return hipGetLastError() == hipSuccess ? FS_OK : FS_E_HIP;
+    return fs::launch_lookup_draft(n_streams, d_hist, d_hist_off, d_kmax, d_min_n, eos_id, d_draft, draft_ld, d_ndraft,
+                                   (hipStream_t)stream) == hipSuccess ? FS_OK : FS_E_HIP;
 }
 
 int fs_hist_append(fs_context* ctx, int32_t n_streams, const int32_t* d_hist, const int64_t* d_hist_off,
@@ -6419,14 +4576,8 @@ int fs_hist_append(fs_context* ctx, int32_t n_streams, const int32_t* d_hist, co
         const int rc = grow(ctx, 1, 1, 1);               // the device error word
         if (rc != FS_OK) return rc;
     }
-    const hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(fs::hist_offsets_kernel, dim3(1), dim3(fs::BLOCK), 0, st, (int)n_streams, d_hist_off,
-                       d_row_off, d_count, d_out_hist_off, out_cap, ctx->err);
-    if (hipGetLastError() != hipSuccess) return FS_E_HIP;
-    if (n_streams == 0) return FS_OK;
-    hipLaunchKernelGGL(fs::hist_append_kernel, dim3((unsigned)n_streams), dim3(fs::LD_BLOCK), 0, st, d_hist,
-                       d_hist_off, d_tok, d_row_off, d_count, d_out_hist_off, d_out_hist, out_cap);
-    return hipGetLastError() == hipSuccess ? FS_OK : FS_E_HIP;
+    return fs::launch_hist_append(n_streams, d_hist, d_hist_off, d_tok, d_row_off, d_count, d_out_hist, d_out_hist_off,
+                                  out_cap, ctx->err, (hipStream_t)stream) == hipSuccess ? FS_OK : FS_E_HIP;
 }
 
 int fs_device_error(fs_context* ctx, void* stream, int32_t* bits) {
