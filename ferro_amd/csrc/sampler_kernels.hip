@@ -4206,7 +4206,8 @@ int launch_small(fs_context* ctx, const fs::Args& a_in, const fs_row_params* h_p
     bool may_pen = ch.may_pen;
     // a verification window reaches this kernel only without an active penalty (small_k_windows)
     may_pen = may_pen && !verify && a.hist && a.hist_off;
-    if (fs::launch_small_k(nl, capped, all_greedy, (unsigned)grid, may_pen ? 1 : 0, k, st) != hipSuccess) return FS_E_HIP;
+    const int flags = (may_pen ? fs::SK_MAY_PEN : 0) | (a.out_hist_off ? fs::SK_COPY : 0);
+    if (fs::launch_small_k(nl, capped, all_greedy, (unsigned)grid, flags, k, st) != hipSuccess) return FS_E_HIP;
     used = true;
     return FS_OK;
 }

@@ -48,8 +48,10 @@ struct SkArgs {
     int64_t out_cap;
 };
 
+// flags of a launch: some row has an active penalty window; a decode step (the histories are copied)
+constexpr int SK_MAY_PEN = 1, SK_COPY = 2;
 // nl: float4 loads per thread (4, 8 or 16); the grid and k's layout come from the small-k plan.
-hipError_t launch_small_k(int nl, bool capped, bool all_greedy, unsigned grid, int may_pen, const SkArgs& k,
+hipError_t launch_small_k(int nl, bool capped, bool all_greedy, unsigned grid, int flags, const SkArgs& k,
                           hipStream_t st);
 
 hipError_t launch_lookup_draft(int n_streams, const int32_t* hist, const int64_t* hist_off, const int32_t* kmax,

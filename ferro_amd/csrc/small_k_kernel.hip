@@ -2,6 +2,8 @@
 #include "sampler_device.hpp"
 #include "sampler_launch.hpp"
 
+#include <type_traits>
+
 namespace fs {
 
 // ------------------------------------------------------------------------------------------------ small-k kernel
@@ -23,45 +25,89 @@ namespace fs {
 // A segment with more than SK_CAP candidates (ties at its bound) selects its exact top k by a radix select over the
 // composites held in registers instead (slow, exact).
 // fs_decode_step_hp on the small-k kernel (the fused kernel's decode_hist_copy / row_u / decode_commit for this
-// kernel's merging workgroup): the stream's history copied to the new histories by the whole workgroup before the
-// merge; the draw read from the stream without advancing it; after the token, wave 0 appends it and advances the
+// kernel): each segment's workgroup copies its share of the stream's history to the new histories; the draw is read
+// from the stream without advancing it; after the token, wave 0 of the merging workgroup appends it and advances the
 // stream (greedy rows draw nothing).
-__device__ __forceinline__ void sk_hist_copy(const SkArgs& a, int row) {
-    const int64_t h0 = a.hist_off ? a.hist_off[0] : 0, b = a.hist_off ? a.hist_off[row] : 0;
-    const int64_t e = a.hist_off ? a.hist_off[row + 1] : 0;
-    const int64_t nb = b - h0 + row;
-    for (int64_t i = threadIdx.x; i < e - b; i += SK_LT)
-        if (nb + i < a.out_cap) a.out_hist[nb + i] = a.hist[b + i];
-    if (threadIdx.x == 0) {
-        a.out_hist_off[row] = nb;
-        if (row == a.B - 1) a.out_hist_off[a.B] = e - h0 + a.B;
-        if (nb + (e - b) + 1 > a.out_cap) atomicOr(a.err, FS_DEVERR_HIST_APPEND);
+// The share of segment seg: ids [seg * n, (seg + 1) * n) of the row's history, n = its length over the row's segments,
+// rounded up. The first SK_CP ids per thread are requested with the window's (cp_load) and stored once the logits are
+// spent (cp_store), so the copy costs no round trip of its own. (Before, the merging workgroup copied the row's whole
+// history, one id per thread and round trip: a decode step of 32 rows with 175 to 1225 ids each 13.1 us -> 12.5, the
+// draw's early reads included.)
+constexpr int SK_CP = 2;
+struct SkCopy {
+    int64_t b, e, nb;                      // this segment's ids [b, e) of the histories; the row's new offset
+    int64_t h0, len;                       // the row's first id, its history's length
+    int id[SK_CP];
+};
+__device__ __forceinline__ SkCopy sk_cp_load(const int64_t* hist_off, const int32_t* hist, int row, int seg, int nseg) {
+    SkCopy c;
+    const int64_t base = hist_off ? ld_const(hist_off) : 0;
+    c.h0 = hist_off ? ld_const(hist_off + row) : 0;
+    const int64_t e = hist_off ? ld_const(hist_off + row + 1) : 0;
+    c.len = e - c.h0;
+    const int64_t n = (c.len + nseg - 1) / nseg;
+    c.b = c.h0 + n * seg < e ? c.h0 + n * seg : e;
+    c.e = c.b + n < e ? c.b + n : e;
+    c.nb = c.h0 - base + row;
+#pragma unroll
+    for (int r = 0; r < SK_CP; ++r) {
+        const int64_t i = c.b + r * SK_LT + (int)threadIdx.x;
+        c.id[r] = i < c.e ? hist[i] : 0;
+    }
+    return c;
+}
+__device__ __forceinline__ void sk_cp_store(const SkArgs& a, const SkCopy& c, int row, int seg) {
+    const int64_t d = c.nb - c.h0;                          // new position minus old
+#pragma unroll
+    for (int r = 0; r < SK_CP; ++r) {
+        const int64_t i = c.b + r * SK_LT + (int)threadIdx.x;
+        if (i < c.e && i + d < a.out_cap) a.out_hist[i + d] = c.id[r];
+    }
+    constexpr int U = 8;                                   // a longer share: eight loads in flight
+    for (int64_t i0 = c.b + SK_CP * SK_LT + (int)threadIdx.x; i0 < c.e; i0 += U * SK_LT) {
+        int v[U];
+#pragma unroll
+        for (int r = 0; r < U; ++r) v[r] = i0 + r * SK_LT < c.e ? a.hist[i0 + r * SK_LT] : 0;
+#pragma unroll
+        for (int r = 0; r < U; ++r) {
+            const int64_t i = i0 + r * SK_LT;
+            if (i < c.e && i + d < a.out_cap) a.out_hist[i + d] = v[r];
+        }
+    }
+    if (seg == 0 && threadIdx.x == 0) {
+        const int64_t end = c.nb + c.len + 1;
+        a.out_hist_off[row] = c.nb;
+        if (row == a.B - 1) a.out_hist_off[a.B] = end;
+        if (end > a.out_cap) atomicOr(a.err, FS_DEVERR_HIST_APPEND);
     }
 }
-__device__ __forceinline__ double sk_row_u(const SkArgs& a, int row) {
+struct SkDraw {
+    double u;
+    int idx;                               // a decode step: the stream's next index, before this draw
+};
+__device__ __forceinline__ SkDraw sk_draw(const SkArgs& a, int row) {
+    SkDraw d;
+    d.idx = 0;
     if (a.dmt) {
         const uint64_t* mt = a.dmt + (int64_t)row * MT_N;
-        const int idx = a.didx[row];
-        const uint64_t y = idx < MT_N ? mt[idx] : mt_twist_one(mt[0], mt[1], mt[MT_M]);
-        return mt_canonical(mt_temper(y));
+        d.idx = a.didx[row];
+        const uint64_t y = d.idx < MT_N ? mt[d.idx] : mt_twist_one(mt[0], mt[1], mt[MT_M]);
+        d.u = mt_canonical(mt_temper(y));
+    } else {
+        d.u = a.u ? ld_const(a.u + row) : 0.0;              // (a scalar load: no wait before it is used)
     }
-    return a.u ? ld_const(a.u + row) : 0.0;
+    return d;
 }
 // Wave 0 alone: w is LDS scratch of MT_N entries. The twist in three passes, each reading every value it needs
 // before it writes: entries below N - M from old values only (all computed, then written); the rest in ascending
 // chunks of one wave (each reads its own and the next old entry and a new one below N - M; entry N - 1 the new
 // entry 0), so no entry is overwritten before it is read.
-__device__ __forceinline__ void sk_decode_commit(const SkArgs& a, int row, bool sampled, int tok, uint64_t* w) {
+__device__ __forceinline__ void sk_decode_commit(const SkArgs& a, int row, bool sampled, int tok, const SkCopy& c,
+                                                 int idx, uint64_t* w) {
     const int lane = lane_id();
-    if (a.out_hist_off && lane == 0) {
-        const int64_t h0 = a.hist_off ? a.hist_off[0] : 0, b = a.hist_off ? a.hist_off[row] : 0;
-        const int64_t e = a.hist_off ? a.hist_off[row + 1] : 0;
-        const int64_t at = b - h0 + row + (e - b);
-        if (at < a.out_cap) a.out_hist[at] = tok;
-    }
+    if (a.out_hist_off && lane == 0 && c.nb + c.len < a.out_cap) a.out_hist[c.nb + c.len] = tok;
     if (!a.dmt || !sampled) return;
     uint64_t* mt = a.dmt + (int64_t)row * MT_N;
-    const int idx = a.didx[row];
     if (idx < MT_N) {
         if (lane == 0) a.didx[row] = idx + 1;
         return;
@@ -192,6 +238,92 @@ __device__ __forceinline__ uint64_t sk_kth_exact(const float* segp, int seg_lo, 
     return prefix;
 }
 
+// Ranks of the n <= SK_LT composites s.cand[0, n), all distinct: P threads per candidate each count the larger entries
+// in 1/P of the list (LDS reads of one address per wave: broadcasts), the partial counts are summed and place(rank,
+// composite) runs once per candidate. Whole workgroup; uses s.wl[1..].
+template <class F>
+__device__ __forceinline__ void sk_rank(SkShared& s, int n, F place) {
+    const int tid = threadIdx.x;
+    uint32_t* rk = reinterpret_cast<uint32_t*>(&s.wl[1][0]);       // [P][per] partial ranks (SK_LT words)
+    const int P = n <= SK_LT / 4 ? 4 : (n <= SK_LT / 2 ? 2 : 1);
+    const int per = SK_LT / P;
+    const int c = tid % per, qq = tid / per;
+    const int span = (((n + P - 1) / P) + 1) & ~1;                 // even: every part starts on a 16-byte pair
+    if (c < n) {
+        const uint64_t me = s.cand[c];
+        const int j0 = qq * span, j1 = j0 + span < n ? j0 + span : n;
+        uint32_t r = 0u;
+        int jj = j0;
+        const ulonglong2* c2 = reinterpret_cast<const ulonglong2*>(s.cand);
+        for (; jj + 8 <= j1; jj += 8) {                            // eight entries per step: four 16-byte LDS reads
+            const ulonglong2 e0 = c2[jj >> 1], e1 = c2[(jj >> 1) + 1], e2 = c2[(jj >> 1) + 2], e3 = c2[(jj >> 1) + 3];
+            r += (e0.x > me ? 1u : 0u) + (e0.y > me ? 1u : 0u) + (e1.x > me ? 1u : 0u) + (e1.y > me ? 1u : 0u) +
+                 (e2.x > me ? 1u : 0u) + (e2.y > me ? 1u : 0u) + (e3.x > me ? 1u : 0u) + (e3.y > me ? 1u : 0u);
+        }
+        for (; jj < j1; ++jj) r += s.cand[jj] > me ? 1u : 0u;
+        rk[qq * per + c] = r;
+    }
+    __syncthreads();
+    if (tid < n) {
+        uint32_t r = 0u;
+        for (int p2 = 0; p2 < P; ++p2) r += rk[p2 * per + tid];
+        place(r, s.cand[tid]);
+    }
+}
+
+// The merge of a row with many lists (more than 4 * SK_NW: the tree of bitonic merges then takes several rounds of
+// list reads). Thread t reads entries 4 (t % 4) .. + 3 of list t / 4: the first 16 of every list in one round trip. The
+// q-th entries of the lists, q = ceil(2 k / nseg), bound the row's k-th: m = ceil(k / q) of them at or above a value
+// make q m >= k entries that reach it. The entries at or above the m-th largest (about 1.5 k) are ranked at once.
+// 8 rows of 64 lists, k 50, a whole call: 18.6 us with the tree, 14.8 with this.
+// Returns false, with nothing placed, when a list may hold more than its first 16 entries above the bound or more than
+// SK_LT entries reach it (the tree then runs). The row's sorted top goes to s.wl[0]. Whole workgroup.
+constexpr int SK_HEAD = 16;
+__device__ __forceinline__ bool sk_merge_many(const uint64_t* rl, int nseg, int k, SkShared& s) {
+    const int tid = threadIdx.x, lane = lane_id(), w = tid / WAVE;
+    const int L = tid >> 2, part = tid & 3;
+    uint64_t e[4] = {0ull, 0ull, 0ull, 0ull};
+    if (L < nseg) {
+        const ulonglong2* p2 = reinterpret_cast<const ulonglong2*>(rl + (int64_t)L * SK_K + 4 * part);
+        const ulonglong2 x = p2[0], y = p2[1];
+        e[0] = x.x; e[1] = x.y; e[2] = y.x; e[3] = y.y;
+    }
+    const int q = (2 * k + nseg - 1) / nseg, m = (k + q - 1) / q;
+    uint32_t* hq = reinterpret_cast<uint32_t*>(&s.wl[0][0]);       // [SK_MAX_SEGS] keys of the q-th entries
+    if (part == (q - 1) >> 2) {
+        const int j = (q - 1) & 3;
+        hq[L] = comp_key(j == 0 ? e[0] : j == 1 ? e[1] : j == 2 ? e[2] : e[3]);
+    }
+    __syncthreads();
+    uint32_t T = (uint32_t)__builtin_amdgcn_readlane((int)sort64_desc_u32(hq[lane]), m - 1);
+    if (T == 0u) T = 1u;                                           // fewer than m lists reach q entries: every entry
+    uint32_t n = 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) n += comp_key(e[j]) >= T ? 1u : 0u;
+    const uint32_t incl = wave_incl_scan_u32(n);
+    const bool more = part == 3 && n == 4u && k > SK_HEAD;         // the list may go on above the bound
+    const uint64_t mo = __ballot(more);
+    if (lane == WAVE - 1) s.tscan[w] = incl;
+    if (lane == 0) s.wcnt[w] = mo != 0ull ? 1u : 0u;
+    __syncthreads();
+    uint32_t base = 0u, tot = 0u, ovf = 0u;
+#pragma unroll
+    for (int v = 0; v < SK_NW; ++v) {
+        base += v < w ? s.tscan[v] : 0u;
+        tot += s.tscan[v];
+        ovf |= s.wcnt[v];
+    }
+    if (ovf != 0u || tot > (uint32_t)SK_LT) return false;          // uniform
+    uint32_t pos = base + incl - n;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (comp_key(e[j]) >= T) s.cand[pos++] = e[j];
+    if (tid < SK_K) s.wl[0][tid] = 0ull;                           // (hq is spent)
+    __syncthreads();
+    sk_rank(s, (int)tot, [&](uint32_t r, uint64_t c) { if (r < (uint32_t)SK_K) s.wl[0][r] = c; });
+    return true;
+}
+
 // CAP: some row of the batch has a softcap (the cap's code is left out of batches without one).
 struct Ids16 {
     int32_t v[16];
@@ -201,7 +333,7 @@ struct Ids16 {
 struct SkKernargs {
     const float* logits;
     int64_t ld;
-    int B, V, nseg, may_pen;
+    int B, V, nseg, flags;
     const fs_row_params* params;
     const int64_t* hist_off;
     const int32_t* hist;
@@ -215,16 +347,18 @@ constexpr size_t SK_ARGS_OFF = offsetof(SkKernargs, a);
 // greedy-only instantiation without it.)
 constexpr unsigned SK_PAD_LDS = 16384;
 
+// MANY: more than 4 * SK_NW lists per row (sk_merge_many; left out of the others, which it cost 0.2 us of 8.4).
 // GREEDY: every row of the batch is greedy (the selection code is left out: fewer registers, more workgroups per CU).
-template <int NL, bool CAP, bool GREEDY>
-__global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int64_t ld, int B, int V, int nseg,
-                                                        int may_pen, const fs_row_params* params,
+template <int NL, bool CAP, bool GREEDY, bool MANY>
+__global__ __launch_bounds__(SK_LT, 4) void small_k_kernel(const float* logits, int64_t ld, int B, int V, int nseg,
+                                                        int flags, const fs_row_params* params,
                                                         const int64_t* hist_off, const int32_t* hist, SkArgs a_) {
     // The leading arguments arrive in SGPRs at wave launch (kernel-argument preloading), so the logits are requested
-    // before any scalar memory round trip. A call with a repetition window (may_pen, set by the host from its copy of
+    // before any scalar memory round trip. A call with a repetition window (SK_MAY_PEN, set by the host from its copy of
     // the parameters) then reads the row's window bounds and requests its ids behind the logits.
     constexpr int SEG = SK_LT * NL * 4;
     static_assert(NL <= 16, "the repetition bitmap covers NL <= 16");
+    constexpr int SK_WL = NL <= 8 ? 8 : 2;                     // 16-byte loads of a long window in flight (registers)
     __shared__ __align__(16) SkShared s;
     const int tid = threadIdx.x, lane = lane_id(), w = tid / WAVE;
     // workgroup i: XCD slot i % XCDS takes rows x, x + XCDS, ...: a row's segments are consecutive workgroups of one
@@ -260,7 +394,7 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
     float rep = 1.0f, fq = 0.0f, pres = 0.0f;
     int64_t h0 = 0, len = 0, wb0 = 0;
     int wid[2] = {-1, -1};
-    if (may_pen) {
+    if (flags & SK_MAY_PEN) {
         const fs_row_params* pr = params + row;
         rep = ld_const(&pr->repetition_penalty);
         fq = ld_const(&pr->frequency_penalty);
@@ -282,6 +416,9 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
             wid[r] = (pen && i < len) ? hist[h0 + i] : -1;
         }
     }
+    const bool cp_on = (flags & SK_COPY) != 0;                 // a decode step: this segment's share of the history
+    SkCopy cp = {};
+    if (cp_on) cp = sk_cp_load(hist_off, hist, row, seg, nseg);
     // The remaining arguments are read from here on, through a pointer the compiler cannot trace back to the argument
     // segment: otherwise it loads some of them early and, short of scalar registers, spills them to vector lanes,
     // which waits for those loads before the logits are requested.
@@ -317,6 +454,11 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
     const bool pen_late = pen && rep >= 1.0f && !greedy;
     const bool pen_early = pen && !pen_late;
     cnt_on = cnt_on && pen;
+    // The softcap never decreases (tanhf does not, over every float, and the divide and multiply around it round a
+    // monotone result), so sampled rows without an early penalty find their bound over the raw logits and cap only the
+    // handed-over ones: a tanhf for about 100 logits of a segment instead of all of them (64 rows of 262144 logits,
+    // k 64: 68.4 us -> 28.3).
+    const bool cap_late = CAP && cap > 0.0f && !greedy && !pen_early;
     // cnt_on: 16-bit counts of the window's ids per logit of the segment, in the group buffer (unused on this path)
     uint32_t* cnt = reinterpret_cast<uint32_t*>(&s.gval[0][0]);
     static_assert(sizeof(SkShared::gval) >= SK_LT * 4 * 4 / 2 * sizeof(uint32_t),
@@ -325,11 +467,34 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
     auto mark = [&](int id) {
         const uint32_t rel = (uint32_t)(id - seg_lo);
         if (id >= 0 && id < V && rel < (uint32_t)SEG) {
-            atomicOr(&s.bmp[rel >> 5], 1u << (rel & 31u));
+            const uint32_t bit = 1u << (rel & 31u);
+            atomicOr(&s.bmp[rel >> 5], bit);
             if (cnt_on) {
                 const uint32_t sh = (rel & 1u) * 16u;
                 const uint32_t old = atomicAdd(&cnt[rel >> 1], 1u << sh);
                 ovf |= ((old >> sh) & 0xFFFFu) == 0xFFFFu;
+            }
+        }
+    };
+    // four ids of a long window. Most segments hold few of them: one compare sorts those out. Its ids repeat, and a
+    // wave's atomics on one word run one after another, so a bit that already reads set is left (a stale read only sets
+    // it again); the four reads are in flight together.
+    const uint32_t in_seg = (uint32_t)n_in;                    // ids of this segment, from seg_lo
+    auto mark4 = [&](const int4& id) {
+        const uint32_t rel[4] = {(uint32_t)(id.x - seg_lo), (uint32_t)(id.y - seg_lo), (uint32_t)(id.z - seg_lo),
+                                 (uint32_t)(id.w - seg_lo)};
+        const uint32_t m01 = rel[0] < rel[1] ? rel[0] : rel[1], m23 = rel[2] < rel[3] ? rel[2] : rel[3];
+        if ((m01 < m23 ? m01 : m23) < in_seg) {
+            if (cnt_on) {
+                mark(id.x); mark(id.y); mark(id.z); mark(id.w);
+            } else {
+                uint32_t word[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) word[c] = *(volatile uint32_t*)&s.bmp[rel[c] < in_seg ? rel[c] >> 5 : 0u];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (rel[c] < in_seg && ((word[c] >> (rel[c] & 31u)) & 1u) == 0u)
+                        atomicOr(&s.bmp[rel[c] >> 5], 1u << (rel[c] & 31u));
             }
         }
     };
@@ -340,7 +505,34 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
         asm volatile("" : "+v"(i0), "+v"(i1));
         mark(i0);
         mark(i1);
-        for (int64_t i = wb0 + 2 * SK_LT + tid; i < len; i += SK_LT) mark(a.hist[h0 + i]);
+        // the rest of a long window: 16 bytes per load from the first 16-byte block on, SK_WL loads in flight (with one
+        // id per load and round trip, decode steps of 8 rows of 262144 logits with 4096 to 28672 ids each, the copy
+        // included: 49 us; now 22)
+        const int64_t i = wb0 + 2 * SK_LT;
+        if (i < len) {
+            const int32_t* hp = a.hist + h0;
+            const int64_t ab = i + (int64_t)((0u - (unsigned)((uintptr_t)(hp + i) >> 2)) & 3u);
+            if (i + tid < ab && i + tid < len) mark(hp[i + tid]);      // at most three ids before it
+            const int4* hv = reinterpret_cast<const int4*>(hp + ab);
+            const int64_t nv = ab < len ? (len - ab) >> 2 : 0;
+            int64_t j0 = 0;
+            for (; j0 + SK_WL * SK_LT <= nv; j0 += SK_WL * SK_LT) {
+                int4 w4[SK_WL];
+#pragma unroll
+                for (int r = 0; r < SK_WL; ++r) w4[r] = hv[j0 + r * SK_LT + tid];
+#pragma unroll
+                for (int r = 0; r < SK_WL; ++r) mark4(w4[r]);
+            }
+            for (int64_t j = j0 + tid; j < nv; j += 2 * SK_LT) {       // the last ones, two in flight
+                const int4 x = hv[j];
+                const bool more = j + SK_LT < nv;
+                const int4 y = more ? hv[j + SK_LT] : x;
+                mark4(x);
+                if (more) mark4(y);
+            }
+            const int64_t rest = ab + 4 * nv;
+            if (rest + tid < len) mark(hp[rest + tid]);                // at most three ids after the last block
+        }
     };
     if (pen) {
         for (int i = tid; i < SEG / 32; i += SK_LT) s.bmp[i] = 0u;
@@ -368,7 +560,7 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
 #pragma unroll
     for (int q = 0; q < NL; ++q) {
         float e[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-        if (CAP && cap > 0.0f) softcap_vals(e, cap);       // a rolled loop: one copy of the cap per group
+        if (CAP && cap > 0.0f && !cap_late) softcap_vals(e, cap);   // a rolled loop: one copy of the cap per group
         if (wpen) {
             const uint32_t nib = (uint32_t)(pm >> (4 * q)) & 0xFu;
             if (__ballot(nib != 0u)) {
@@ -441,11 +633,27 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
         for (int q = 1; q < SK_NW; ++q) tau = s.wb[q] < tau ? s.wb[q] : tau;
         if (tau == 0u) tau = 1u;                                   // NaN (key 0) is never a candidate
         const float tf = tau > 0x007FFFFFu ? val_of(tau) : -__builtin_huge_valf();
+        // cap_late: the candidates are the logits whose capped value reaches the capped bound tc; tr is a raw value that
+        // every one of them reaches: lane j < 32 caps the value 2^j keys below the bound (lane 32 the bound itself), and the first that falls
+        // below tc (the cap is flat where it saturates) ends the range.
+        float tc = tf, tr = tf;
+        if (cap_late) {
+            const uint32_t kb = tau > 0x007FFFFFu ? tau : 0x007FFFFFu;          // (the key of -inf is the lowest)
+            const uint32_t step = lane < 32 ? 1u << lane : 0u, room = kb - 0x007FFFFFu;
+            const float c = softcap_one(val_of(room > step ? kb - step : 0x007FFFFFu + (lane < 32 ? 0u : room)), cap);
+            tc = read_lane(c, 32);
+            const uint64_t below = __ballot(lane < 32 && c < tc);
+            tr = -__builtin_huge_valf();
+            if (below) {
+                const uint32_t st = 1u << (__ffsll((unsigned long long)below) - 1);
+                tr = room > st ? val_of(kb - st) : tr;
+            }
+        }
         // groups whose maximum reaches the bound: this wave's region of the group buffer, in lane order
         uint32_t gmask = 0u;
 #pragma unroll
         for (int q = 0; q < NL; ++q)                     // the group's raw maximum (recomputed: no register array)
-            gmask |= (fmaxf(fmaxf(v[q].x, v[q].y), fmaxf(v[q].z, v[q].w)) >= tf ? 1u : 0u) << q;
+            gmask |= (fmaxf(fmaxf(v[q].x, v[q].y), fmaxf(v[q].z, v[q].w)) >= tr ? 1u : 0u) << q;
         const uint32_t gn = (uint32_t)__popc(gmask);
         const uint32_t gincl = wave_incl_scan_u32(gn);
         const uint32_t wtot = (uint32_t)__builtin_amdgcn_readlane((int)gincl, WAVE - 1);
@@ -497,6 +705,14 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
             const int e0 = (int)gw;
             // rep >= 1: the group's penalised logits, from the bitmap (its 4 bits share a word: e0 % 4 == 0)
             float e[4] = {gv.x, gv.y, gv.z, gv.w};
+            if (CAP && cap_late) {
+#pragma unroll 1
+                for (int c = 0; c < 4; c += 2) {
+                    float e2[2] = {c ? e[2] : e[0], c ? e[3] : e[1]};
+                    softcap_vals_unrolled(e2, cap);
+                    if (c) { e[2] = e2[0]; e[3] = e2[1]; } else { e[0] = e2[0]; e[1] = e2[1]; }
+                }
+            }
             if (pen_late) {
                 const uint32_t nib = (s.bmp[(uint32_t)e0 >> 5] >> ((uint32_t)e0 & 31u)) & 0xFu;
 #pragma unroll
@@ -505,7 +721,7 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
             }
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                cp[c] = e[c] >= tf;
+                cp[c] = e[c] >= tc;
                 cm[c] = comp_of(key_of(e[c]), (uint32_t)(seg_lo + e0 + c));
                 nc += cp[c] ? 1u : 0u;
             }
@@ -552,39 +768,11 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
             ntot = s.misc[0] < (uint32_t)SK_K ? s.misc[0] : (uint32_t)SK_K;
         }
         __syncthreads();
-        // the segment's top k, sorted by rank: P threads per candidate each count the larger entries in 1/P of the list
-        // (LDS reads of one address per wave: broadcasts), the partial counts are summed and the first k placed by rank
-        uint64_t* sorted = &s.wl[0][0];
-        uint32_t* rk = reinterpret_cast<uint32_t*>(&s.wl[1][0]);    // [P][per] partial ranks (SK_LT words)
+        // the segment's top k, sorted by rank
         {
             const int n = (int)ntot;
             if (n <= SK_LT) {
-                const int P = n <= SK_LT / 4 ? 4 : (n <= SK_LT / 2 ? 2 : 1);
-                const int per = SK_LT / P;
-                const int c = tid % per, qq = tid / per;
-                const int span = (((n + P - 1) / P) + 1) & ~1;     // even: every part starts on a 16-byte pair
-                if (c < n) {
-                    const uint64_t me = s.cand[c];
-                    const int j0 = qq * span, j1 = j0 + span < n ? j0 + span : n;
-                    uint32_t r = 0u;
-                    int jj = j0;
-                    const ulonglong2* c2 = reinterpret_cast<const ulonglong2*>(s.cand);
-                    for (; jj + 8 <= j1; jj += 8) {                // eight entries per step: four 16-byte LDS reads
-                        const ulonglong2 e0 = c2[jj >> 1], e1 = c2[(jj >> 1) + 1], e2 = c2[(jj >> 1) + 2],
-                                         e3 = c2[(jj >> 1) + 3];
-                        r += (e0.x > me ? 1u : 0u) + (e0.y > me ? 1u : 0u) + (e1.x > me ? 1u : 0u) +
-                             (e1.y > me ? 1u : 0u) + (e2.x > me ? 1u : 0u) + (e2.y > me ? 1u : 0u) +
-                             (e3.x > me ? 1u : 0u) + (e3.y > me ? 1u : 0u);
-                    }
-                    for (; jj < j1; ++jj) r += s.cand[jj] > me ? 1u : 0u;
-                    rk[qq * per + c] = r;
-                }
-                __syncthreads();
-                if (tid < n) {                                     // placed straight into the published list
-                    uint32_t r = 0u;
-                    for (int p2 = 0; p2 < P; ++p2) r += rk[p2 * per + tid];
-                    if (r < (uint32_t)k) myl[r] = s.cand[tid];
-                }
+                sk_rank(s, n, [&](uint32_t r, uint64_t c) { if (r < (uint32_t)k) myl[r] = c; });   // the published list
             } else {                                               // 256 < n <= SK_CAP: two candidates per thread
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -608,10 +796,10 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
             }
             if (tid >= (n < k ? n : k) && tid < SK_K) myl[tid] = 0ull;   // slots past the segment's top k
         }
-        (void)sorted;
         SK_TAG(9, ntot);
         SK_TAG(10, G);
     }
+    if (cp_on) sk_cp_store(a, cp, row, seg);
     vm_drain();                                                // the list is in the L2
     __syncthreads();
     SK_MARK(5);
@@ -626,7 +814,9 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
         return;
     }
     SK_TAG(13, 4);
-    if (a.out_hist_off) sk_hist_copy(a, row);                  // a decode step: every thread, before the merge
+    // a decode step's draw takes two dependent reads: requested before the lists, so that they overlap the merge
+    SkDraw dr = {0.0, 0};
+    if (!greedy && a.dmt) dr = sk_draw(a, row);
     // ---- the row's merge (the last of its segments): wave w folds lists w, w + SK_NW, ... (the first as stored,
     // the rest reversed: ascending), then wave 0 folds the waves' lists
     const uint64_t* rl = a.lists + (int64_t)row * a.nseg * SK_K;
@@ -637,6 +827,12 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
         SK_MARK(7);
         if (tid == 0) a.ticket[row] = 0u;                     // all segments have counted: reset for the next call
         acc = wave_max(lane < a.nseg ? rl[lane * SK_K] : 0ull);
+    } else if (MANY && sk_merge_many(rl, a.nseg, k, s)) {
+        __syncthreads();
+        if (w != 0) return;
+        SK_MARK(7);
+        if (tid == 0) a.ticket[row] = 0u;                     // all segments have counted: reset for the next call
+        acc = s.wl[0][lane];
     } else {
         for (int L0 = w; L0 < a.nseg; L0 += 4 * SK_NW) {
             // four lists per wave, requested together: lists 0 and 2 as stored (descending), 1 and 3 reversed
@@ -684,14 +880,15 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
     } else if (kk == 0) {
         tok = 0; keep = 0;                                     // every logit NaN: token 0, nothing kept
     } else {
-        wave_softmax(fa, rc, lane < kk ? acc : 0ull, kk, sk_row_u(a, row), tok, keep);
+        if (!a.dmt) dr = sk_draw(a, row);
+        wave_softmax(fa, rc, lane < kk ? acc : 0ull, kk, dr.u, tok, keep);
     }
     if (a.mode != MODE_VERIFY) {
         if (lane == 0) {
             a.tok[row] = tok;
             if (a.keep) a.keep[row] = keep;
         }
-        if (a.out_hist_off || a.dmt) sk_decode_commit(a, row, !greedy, tok, &s.cand[0]);
+        if (a.out_hist_off || a.dmt) sk_decode_commit(a, row, !greedy, tok, cp, dr.idx, &s.cand[0]);
     } else {
         // the last row of a stream to finish computes its accepted prefix (server.cpp:627-637): the stream's rows
         // run on several XCDs, so the exchange is agent-scope.
@@ -737,33 +934,32 @@ __global__ __launch_bounds__(SK_LT) void small_k_kernel(const float* logits, int
     SK_FLUSH();
 }
 
-hipError_t launch_small_k(int nl, bool capped, bool all_greedy, unsigned grid, int may_pen, const SkArgs& k,
+hipError_t launch_small_k(int nl, bool capped, bool all_greedy, unsigned grid, int flags, const SkArgs& k,
                           hipStream_t st) {
     const dim3 gd(grid), bd(SK_LT);
     // all-greedy batches: the greedy-only kernel, without the LDS pad (its registers allow more workgroups per CU)
     auto go = [&](auto kern, unsigned pad) {
-        hipLaunchKernelGGL(kern, gd, bd, pad, st, k.logits, k.ld, k.B, k.V, k.nseg, may_pen, k.params, k.hist_off,
+        hipLaunchKernelGGL(kern, gd, bd, pad, st, k.logits, k.ld, k.B, k.V, k.nseg, flags, k.params, k.hist_off,
                            k.hist, k);
     };
-    const unsigned pad = SK_PAD_LDS;
+    auto by_nl = [&](auto cap, auto greedy, auto many) {
+        constexpr bool C = decltype(cap)::value, G = decltype(greedy)::value, M = decltype(many)::value;
+        const unsigned pad = G ? 0u : SK_PAD_LDS;
+        if (nl == 16) go(small_k_kernel<16, C, G, M>, pad);
+        else if (nl == 8) go(small_k_kernel<8, C, G, M>, pad);
+        else go(small_k_kernel<4, C, G, M>, pad);
+    };
+    const std::true_type yes;
+    const std::false_type no;
     if (all_greedy) {
-        if (capped) {
-            if (nl == 16) go(small_k_kernel<16, true, true>, 0u);
-            else if (nl == 8) go(small_k_kernel<8, true, true>, 0u);
-            else go(small_k_kernel<4, true, true>, 0u);
-        } else {
-            if (nl == 16) go(small_k_kernel<16, false, true>, 0u);
-            else if (nl == 8) go(small_k_kernel<8, false, true>, 0u);
-            else go(small_k_kernel<4, false, true>, 0u);
-        }
-    } else if (capped) {
-        if (nl == 16) go(small_k_kernel<16, true, false>, pad);
-        else if (nl == 8) go(small_k_kernel<8, true, false>, pad);
-        else go(small_k_kernel<4, true, false>, pad);
+        if (capped) by_nl(yes, yes, no);
+        else by_nl(no, yes, no);
+    } else if (k.nseg > 4 * SK_NW) {
+        if (capped) by_nl(yes, no, yes);
+        else by_nl(no, no, yes);
     } else {
-        if (nl == 16) go(small_k_kernel<16, false, false>, pad);
-        else if (nl == 8) go(small_k_kernel<8, false, false>, pad);
-        else go(small_k_kernel<4, false, false>, pad);
+        if (capped) by_nl(yes, no, no);
+        else by_nl(no, no, no);
     }
     return hipGetLastError();
 }

@@ -64,3 +64,62 @@ def test_lookup_draft_tile_edges(L):
         want = O.lookup_draft(h, 70, eos=E, min_n=min_n[s])
         assert nd[s] == len(want), (L, s)
         np.testing.assert_array_equal(draft[s, :nd[s]], want)
+
+
+@pytest.mark.parametrize("H,V", [(511, 65536), (512, 65536), (513, 65536), (515, 262144), (516 + 8192, 262144),
+                                 (517 + 8192 + 2048 + 3, 262144), (20011, 100004)])
+def test_long_windows_and_history_copies(H, V):
+    """Decode steps whose histories end before, at and after the prefetched ids, at every offset from a 16-byte
+    boundary, and shares of a row's copy longer than the prefetched part."""
+    rng = np.random.default_rng(H)
+    S = 5
+    p = W.make_params(S, temperature=0.7, top_k=50, repetition_penalty=1.3)
+    p["repeat_last_n"][1] = H - 3
+    p["penalty_from"][2] = 5
+    p["softcap"][3] = 30.0
+    hist0 = [list(W.zipf_ids(rng, V, H + s)) for s in range(S)]
+    rows = [W.mixture_logits(rng, S, V) for _ in range(2)]
+    seeds = list(range(1, S + 1))
+    want, want_hist, want_off = oracle_decode_loop(rows, p, seeds, hist0)
+    d = F.DeviceRng(np.asarray(seeds, np.uint64))
+    hist, off = (torch.from_numpy(a).cuda() for a in csr(hist0))
+    for k, x in enumerate(rows):
+        tok, _, hist, off = F.decode_step(torch.from_numpy(x).cuda(), p, d, hist=hist, hist_off=off)
+        np.testing.assert_array_equal(tok.cpu().numpy(), want[k])
+    np.testing.assert_array_equal(off.cpu().numpy(), want_off)
+    np.testing.assert_array_equal(hist[:int(off[-1])].cpu().numpy(), want_hist)
+    assert F.device_error() == 0
+
+
+@pytest.mark.parametrize("V,k", [(65537, 64), (65537, 1 + 16), (262144, 64), (262144, 5), (262144, 16), (150000, 40)])
+def test_rows_with_many_segment_lists(V, k):
+    """17 to 64 lists per row: even rows, every top candidate in one segment (its list alone holds them: past its
+    prefetched head), one candidate per segment, ties across segments, fewer candidates than k."""
+    rng = np.random.default_rng(V + k)
+    x = (rng.standard_normal((6, V)) * 2).astype(np.float32)
+    x[1, 4096:4096 + 200] += 30.0
+    x[2, ::4096] += 30.0
+    x[3] = bf16_valued(x[3])
+    x[4, :] = 1.0
+    x[5, :] = np.nan
+    x[5, rng.choice(V, 7, replace=False)] = 2.0
+    p = W.make_params(6, temperature=0.8, top_k=k, top_p=0.97, repetition_penalty=1.0)
+    check(x, p, [[]] * 6, rng.random(6))
+
+
+@pytest.mark.parametrize("cap,scale", [(30.0, 1.0), (30.0, 40.0), (0.5, 1.0), (30.0, 300.0)])
+def test_softcap_where_it_saturates(cap, scale):
+    """Capped rows from unclipped to wholly saturated (every top logit caps to the same value: ties by id), with and
+    without a repetition penalty above and below 1."""
+    rng = np.random.default_rng(int(cap * 10 + scale))
+    V = 70000
+    x = (rng.standard_normal((6, V)) * scale).astype(np.float32)
+    x[0, 5] = np.inf
+    x[1, 6] = -np.inf
+    x[2, 7] = np.nan
+    x[3] = np.abs(x[3]) + np.float32(20 * cap)             # saturated everywhere
+    p = W.make_params(6, temperature=0.9, top_k=40, repetition_penalty=1.2)
+    p["softcap"] = cap
+    p["repetition_penalty"][4] = 0.8
+    p["repetition_penalty"][5] = 1.0
+    check(x, p, [list(W.zipf_ids(rng, V, 900)) for _ in range(6)], rng.random(6))
