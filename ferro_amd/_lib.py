@@ -45,6 +45,7 @@ SIGNATURES = {
     "fs_sample_batch_hp": (ctypes.c_int, [_P, _P, _I64, _I32, _I32, _P, _P, _P, _P, _P, _P, _I32, _P, _P, _P, _P]),
     "fs_small_k_plan": (ctypes.c_int, [_I32, _I32, _I32, _P, _P]),
     "fs_route_plan": (ctypes.c_int, [_I32, _P, _I32, _I32, _I32, _I32, _P, _P, _P, _P]),
+    "fs_mid_k_plan": (ctypes.c_int, [_I32, _P, _I32, _I32, _I32, _P, _P]),
     "fs_argmax_batch": (ctypes.c_int, [_P, _P, _I64, _I32, _I32, _P, _P, _P, _P, _P]),
     "fs_verify": (ctypes.c_int, [_P, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _P, _P, _P, _I32, _P, _P, _P]),
     "fs_verify_hp": (ctypes.c_int, [_P, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _I32, _P, _P, _P]),
@@ -131,3 +132,15 @@ def route_plan(cus: int, params, V: int, total_rows: int = None, verify: bool = 
                              1 if verify else 0, ctypes.byref(k), ctypes.byref(nl), ctypes.byref(ns), ctypes.byref(pc))
     check(rc, "fs_route_plan")
     return k.value, nl.value, ns.value, pc.value
+
+
+def mid_k_plan(cus: int, params, V: int, total_rows: int = None):
+    """fs_mid_k_plan: (nl, nseg) of the mid-k kernel for these host parameter records, None when it does not fit."""
+    p = np.ascontiguousarray(params)
+    nl, ns = ctypes.c_int32(), ctypes.c_int32()
+    rc = lib().fs_mid_k_plan(cus, p.ctypes.data_as(ctypes.c_void_p), len(p), total_rows if total_rows else len(p), V,
+                             ctypes.byref(nl), ctypes.byref(ns))
+    if rc == FS_E_LIMIT:
+        return None
+    check(rc, "fs_mid_k_plan")
+    return nl.value, ns.value

@@ -8,7 +8,8 @@ import sys
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 # the kernel files, compiled side by side and linked into one library
-SRCS = [os.path.join(PKG, "csrc", f) for f in ("sampler_kernels.hip", "small_k_kernel.hip", "history_kernels.hip")]
+SRCS = [os.path.join(PKG, "csrc", f) for f in ("fused_kernel.hip", "sampler_kernels.hip", "small_k_kernel.hip",
+                                                  "mid_k_kernel.hip", "history_kernels.hip")]
 LIB = os.path.join(PKG, "libferro_sampler.so")
 # the same source with phase timestamps compiled in (-DFS_TRACE, fs_trace_set): read by ferro_amd/trace_phases.py
 TRACE_LIB = os.path.join(PKG, "libferro_sampler_trace.so")

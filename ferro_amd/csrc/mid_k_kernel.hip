@@ -1,0 +1,1029 @@
+// mid_k_kernel.hip - the kernel of batches that mix rows: greedy rows and rows that sample from k <= 2048 candidates,
+// with every penalty, and verification windows with penalties.
+//
+// One workgroup of SK_LT threads per (row, segment), the segment's logits requested at once and kept in registers, as in
+// the small-k kernel. A row's segments agree on one bound before any of them writes a candidate:
+//   - the window's ids in the segment are a bitmap laid out by thread (and 16-bit counts, frequency / presence): each
+//     wave moves its flagged logits to a list in LDS (a long window's to memory) and penalises them while the row's
+//     segments meet, one entry per lane, so the rest of the segment needs no penalty arithmetic;
+//   - each wave sorts its 64 lane maxima in registers and publishes them at 16 ranks (1, 2, 3, ... 64, weights adding up
+//     to 64); the row's segments meet (an L2 counter), and every one takes the same bound from the row's published keys:
+//     the largest T such that the ranks published at or above T add up to k. k distinct logits of the row then reach T,
+//     whatever the other segments hold;
+//   - the logits at or above T (about 1.05 k to 1.4 k per row) go to the row's list, one L2 atomic per wave for its
+//     places; the last segment to finish (an L2 ticket) sorts the list and samples the row.
+// The waiting is bounded and a row's segments are consecutive workgroups of one XCD, dispatched in order; a segment that
+// gives up (or a list that overflows: thousands of equal logits at the bound) marks the row, and its last segment then
+// selects the row's exact top k from the logits alone (mk_slow).
+// Bound: HBM, one read of the logits, then the chain behind a row's last logits.
+// Measured against the fused kernel (running bounds, per-row merges of the segments' lists): 256 rows of 262144 logits
+// with k from 1 to 2048 and every penalty 124 us -> 79; 24 rows of 100003 logits, k 200, frequency / presence 35 -> 19.4;
+// 40 rows of a verification window over 262144 logits, k 50, repetition 26.5 -> 24.3.
+#include "row_device.hpp"
+
+#include <type_traits>
+
+namespace fs {
+
+constexpr int MK_K = 2048;                 // largest k
+constexpr int MK_LCAP = MK_LIST;           // entries of a row's list
+constexpr int MK_TOP = 2560;               // sorted candidates: k plus the rest of the bin that holds the k-th
+constexpr int MK_BINS = 2048;              // bins of the merge's counting sort
+constexpr int MK_H = 1024;                 // bins of the bound's histograms and of mk_slow's digits
+constexpr int MK_PC = 512;                 // penalised logits of a segment kept in LDS
+constexpr int MK_W = 4;                    // window ids per thread requested behind the logits
+// published ranks of a wave's 64 sorted lane maxima, and what each adds to the rank before it
+constexpr uint64_t MK_RANK_LO = 0x0A08060504030201ull, MK_RANK_HI = 0x403028201814100Cull;   // 1..6, 8, 10; 12..64
+__device__ __forceinline__ uint32_t mk_rank(int j) {
+    return (uint32_t)((j < 8 ? MK_RANK_LO >> (8 * j) : MK_RANK_HI >> (8 * (j - 8))) & 0xFFu);
+}
+
+struct MkShared {
+    // in turn: the window's 16-bit counts per logit of the segment (frequency / presence); the merge's sorted candidates
+    // and its bins
+    union {
+        uint32_t cnt[SK_LT * 16 * 4 / 2];
+        struct {
+            uint64_t top[MK_TOP];
+            uint32_t bins[MK_BINS + 1];
+        } m;
+        struct {
+            uint64_t top[MK_K];            // (u.m.top's head)
+            double e[MK_K];                // their masses, then probabilities
+        } w;
+    } u;
+    union {
+        uint32_t hist[MK_H];               // the bound's histograms; mk_slow's digits
+        uint32_t rk[SK_LT];                // partial ranks of a short list
+        uint32_t srt[SK_NW][WAVE];         // the waves' sorted lane maxima
+    } h;
+    union {
+        uint32_t bmp[SK_LT * 2];           // one bit per logit of the window's ids: 64 bits per thread; mk_slow: by id
+        float pv[MK_PC];                   // (the bits are read) the flagged logits, raw, then penalised
+    } b;
+    uint16_t prel[MK_PC];                  //   and their places in the segment
+    uint32_t np;                           //   places given out
+    uint64_t w64[SK_NW];
+    double wf[SK_NW];
+    uint32_t w32[SK_NW];
+    uint32_t misc[6];
+    double dmisc;
+#ifdef FS_TRACE
+    uint64_t trace_t[16];
+#endif
+};
+
+// ---- block reductions of SK_LT threads (each starts after and ends with a barrier)
+__device__ __forceinline__ uint32_t mk_excl_u32(uint32_t v, MkShared& s, uint32_t& total) {
+    const int w = threadIdx.x / WAVE;
+    const uint32_t x = wave_incl_scan_u32(v);
+    if (lane_id() == WAVE - 1) s.w32[w] = x;
+    __syncthreads();
+    uint32_t off = 0u, tot = 0u;
+#pragma unroll
+    for (int q = 0; q < SK_NW; ++q) {
+        off += q < w ? s.w32[q] : 0u;
+        tot += s.w32[q];
+    }
+    __syncthreads();
+    total = tot;
+    return off + x - v;
+}
+__device__ __forceinline__ double mk_excl_f64(double v, MkShared& s, double& total) {
+    const int w = threadIdx.x / WAVE;
+    const double x = wave_scan_f64(v);
+    const double ex = dpp_f64<0x138, 0xF>(x);                  // wave_shr:1 (lane 0 reads 0)
+    if (lane_id() == WAVE - 1) s.wf[w] = x;
+    __syncthreads();
+    double off = 0.0, tot = 0.0;
+#pragma unroll
+    for (int q = 0; q < SK_NW; ++q) {
+        if (q < w) off += s.wf[q];
+        tot += s.wf[q];
+    }
+    __syncthreads();
+    total = tot;
+    return off + ex;
+}
+template <class Op>
+__device__ __forceinline__ uint64_t mk_reduce_u64(uint64_t v, MkShared& s, Op op) {
+    v = wave_allreduce(v, op);
+    if (lane_id() == 0) s.w64[threadIdx.x / WAVE] = v;
+    __syncthreads();
+    uint64_t m = s.w64[0];
+#pragma unroll
+    for (int w = 1; w < SK_NW; ++w) m = op(m, s.w64[w]);
+    __syncthreads();
+    return m;
+}
+__device__ __forceinline__ uint64_t mk_max_u64(uint64_t v, MkShared& s) {
+    return mk_reduce_u64(v, s, [](uint64_t x, uint64_t y) { return y > x ? y : x; });
+}
+__device__ __forceinline__ uint64_t mk_min_u64(uint64_t v, MkShared& s) {
+    return mk_reduce_u64(v, s, [](uint64_t x, uint64_t y) { return y < x ? y : x; });
+}
+
+// From s.h.hist: the bin b with count(bins > b) < kk <= count(bins >= b) and the count above it; false when the
+// histogram holds fewer than kk. Whole workgroup, after a barrier; ends with one.
+__device__ __forceinline__ bool mk_locate(MkShared& s, uint32_t kk, uint32_t& b, uint32_t& above) {
+    static_assert(MK_H == 4 * SK_LT, "four bins per thread");
+    const int tid = threadIdx.x;
+    const uint4 c = *reinterpret_cast<const uint4*>(&s.h.hist[MK_H - 4 - 4 * tid]);   // descending: w, z, y, x
+    const uint32_t mine = c.x + c.y + c.z + c.w;
+    uint32_t tot;
+    const uint32_t ex = mk_excl_u32(mine, s, tot);
+    if (tot < kk) return false;                                // uniform
+    if (ex < kk && ex + mine >= kk) {
+        uint32_t a = ex, j = 0u;
+        if (a + c.w < kk) { a += c.w; j = 1u;
+            if (a + c.z < kk) { a += c.z; j = 2u;
+                if (a + c.y < kk) { a += c.y; j = 3u; } } }
+        s.misc[0] = (uint32_t)(MK_H - 1 - 4 * tid) - j;
+        s.misc[1] = a;
+    }
+    __syncthreads();
+    b = s.misc[0];
+    above = s.misc[1];
+    return true;
+}
+
+// The row's bound from its segments' published keys (nseg * SK_NW lists of 16): the largest 20-bit prefix T (sign,
+// exponent, 11 mantissa bits) such that the weights of the keys at or above it add up to k, 1 when they do not. Two
+// histograms of ten key bits each in LDS. Whole workgroup; s.h.hist is zero on entry.
+template <int NQ>
+__device__ __forceinline__ uint32_t mk_bound(const uint32_t* qk, int nseg, int k, MkShared& s) {
+    const int tid = threadIdx.x;
+    const int n4 = nseg * SK_NW * 4;                           // 16-byte quarters of the lists
+    uint4 e[NQ];
+#pragma unroll
+    for (int r = 0; r < NQ; ++r) {
+        const int i = r * SK_LT + tid;
+        e[r] = i < n4 ? reinterpret_cast<const uint4*>(qk)[i] : make_uint4(0u, 0u, 0u, 0u);
+    }
+    // weights of quarter (tid & 3) of a list: 1 1 1 1 | 1 1 2 2 | 2 4 4 4 | 8 8 8 16
+    const uint32_t pk = (tid & 3) == 0 ? 0x01010101u : (tid & 3) == 1 ? 0x02020101u : (tid & 3) == 2 ? 0x04040402u : 0x10080808u;
+    auto add = [&](uint32_t key, uint32_t wgt, uint32_t hi, int level) {
+        if (key == 0u) return;
+        if (level == 0) atomicAdd(&s.h.hist[key >> 22], wgt);
+        else if (key >> 22 == hi) atomicAdd(&s.h.hist[(key >> 12) & 1023u], wgt);
+    };
+    uint32_t hi = 0u, lo = 0u, above = 0u, above2 = 0u;
+#pragma unroll
+    for (int r = 0; r < NQ; ++r) {
+        add(e[r].x, pk & 255u, 0u, 0);
+        add(e[r].y, (pk >> 8) & 255u, 0u, 0);
+        add(e[r].z, (pk >> 16) & 255u, 0u, 0);
+        add(e[r].w, pk >> 24, 0u, 0);
+    }
+    __syncthreads();
+    if (!mk_locate(s, (uint32_t)k, hi, above)) return 1u;
+    *reinterpret_cast<uint4*>(&s.h.hist[4 * tid]) = make_uint4(0u, 0u, 0u, 0u);   // (mk_locate's reads are over)
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < NQ; ++r) {
+        add(e[r].x, pk & 255u, hi, 1);
+        add(e[r].y, (pk >> 8) & 255u, hi, 1);
+        add(e[r].z, (pk >> 16) & 255u, hi, 1);
+        add(e[r].w, pk >> 24, hi, 1);
+    }
+    __syncthreads();
+    (void)mk_locate(s, (uint32_t)k - above, lo, above2);
+    const uint32_t T = (hi << 22) | (lo << 12);
+    return T ? T : 1u;
+}
+
+// The row's window of history ids: na ids of the stream's history, then nb of the drafts fed before this row.
+struct MkWin {
+    const int32_t* pa;
+    const int32_t* pb;
+    int64_t na;
+    int nb;
+    __device__ __forceinline__ int at(int64_t i) const { return i < na ? pa[i] : pb[i - na]; }
+    __device__ __forceinline__ int64_t n() const { return na + nb; }
+};
+struct MkPen {
+    float rep, fq, pres, cap;
+    bool rep_on, fp_on;
+    // ferro's penalties on one raw logit with c occurrences in the window (sampler.cpp:11-18 and the extension)
+    __device__ __forceinline__ float apply(float l, uint32_t c) const {
+        if (rep_on) l = l > 0.0f ? __fdiv_rn(l, rep) : __fmul_rn(l, rep);
+        if (fp_on) l = __fsub_rn(l, __fadd_rn(__fmul_rn((float)c, fq), pres));
+        return l;
+    }
+};
+
+// The exact top k of a row, from its logits alone, by one workgroup: a radix select over the composites, ten bits at a
+// time (it stops where a digit's bin is wholly inside), then the composites at or above the k-th to the row's list.
+// The penalties are counted again chunk by chunk. Returns the list's length. For rows with thousands of equal logits at
+// the bound, and rows whose segments gave up waiting.
+template <bool CAP>
+__device__ __forceinline__ uint32_t mk_slow(const float* rowp, int V, int k, bool pen, const MkWin& win, const MkPen& pn,
+                                            uint64_t* list, MkShared& s) {
+    constexpr int CH = SK_LT * 16 * 4;                         // logits per chunk
+    const int tid = threadIdx.x;
+    uint64_t prefix = 0ull, mask = 0ull;
+    uint32_t need = (uint32_t)k;
+    int sh = 54;
+    bool gather = false;
+    if (tid == 0) s.misc[2] = 0u;
+#pragma unroll 1
+    for (;;) {                                                 // a pass: one digit's counts, at last the gather
+        const int sft = sh < 0 ? 0 : sh;
+        const uint64_t dm = sh < 0 ? 0x3FFull >> -sh : 0x3FFull;
+        __syncthreads();
+        *reinterpret_cast<uint4*>(&s.h.hist[4 * tid]) = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();
+#pragma unroll 1
+        for (int lo = 0; lo < V; lo += CH) {
+            const int n = V - lo < CH ? V - lo : CH;
+            if (pen) {
+                __syncthreads();
+                for (int i = tid; i < CH / 32; i += SK_LT) s.b.bmp[i] = 0u;
+                if (pn.fp_on)
+                    for (int i = tid; i < CH / 2; i += SK_LT) s.u.cnt[i] = 0u;
+                __syncthreads();
+#pragma unroll 1
+                for (int64_t i = tid; i < win.n(); i += SK_LT) {
+                    const uint32_t rel = (uint32_t)win.at(i) - (uint32_t)lo;
+                    if (rel < (uint32_t)n) {
+                        atomicOr(&s.b.bmp[rel >> 5], 1u << (rel & 31u));
+                        if (pn.fp_on) atomicAdd(&s.u.cnt[rel >> 1], 1u << ((rel & 1u) * 16u));
+                    }
+                }
+                __syncthreads();
+            }
+#pragma unroll 1
+            for (int i = tid; i < n; i += SK_LT) {
+                float l = rowp[lo + i];
+                if (CAP && pn.cap > 0.0f) l = softcap_one(l, pn.cap);
+                if (pen && ((s.b.bmp[i >> 5] >> (i & 31)) & 1u))
+                    l = pn.apply(l, pn.fp_on ? (s.u.cnt[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu : 0u);
+                const uint32_t key = key_of(l);
+                const uint64_t c = comp_of(key, (uint32_t)(lo + i));
+                if (key == 0u) continue;
+                if (gather) {
+                    if ((c & mask) >= prefix) {
+                        const uint32_t pos = atomicAdd(&s.misc[2], 1u);
+                        if (pos < (uint32_t)MK_LCAP) st_agent(&list[pos], (c << 32) | (uint64_t)__float_as_uint(l));
+                    }
+                } else if ((c & mask) == prefix) {
+                    atomicAdd(&s.h.hist[(uint32_t)(c >> sft) & (uint32_t)dm], 1u);
+                }
+            }
+        }
+        __syncthreads();
+        if (gather) break;
+        uint32_t b, above;
+        if (!mk_locate(s, need, b, above)) {                   // (the first digit only) fewer than k candidates: all
+            prefix = mask = 0ull;
+            gather = true;
+            continue;
+        }
+        const uint32_t in = s.h.hist[b];
+        need -= above;
+        prefix |= (uint64_t)b << sft;
+        mask |= dm << sft;
+        gather = in == need || sh < 0;                         // the whole bin is inside
+        sh -= 10;
+    }
+    vm_drain();
+    __syncthreads();
+    return s.misc[2];
+}
+
+// Sorts the row's list (n <= MK_LCAP composites in registers, 0: none) into s.u.m.top[0, min(n, k)), descending: a
+// counting sort over the span of the composites, of which only the bins that hold the first k are placed; entries rank
+// themselves within their bin. Returns false when those bins hold more than MK_TOP entries (hundreds of ties at the
+// k-th). Whole workgroup.
+template <int EPT>
+__device__ __forceinline__ bool mk_sort(const uint64_t (&v)[EPT], int n, int k, MkShared& s) {
+    const int tid = threadIdx.x;
+    uint64_t cmn = ~0ull, cmx = 0ull;
+#pragma unroll
+    for (int q = 0; q < EPT; ++q) {
+        if (q * SK_LT + tid < n) {
+            cmn = v[q] < cmn ? v[q] : cmn;
+            cmx = v[q] > cmx ? v[q] : cmx;
+        }
+    }
+    for (int i = tid; i < MK_BINS; i += SK_LT) s.u.m.bins[i] = 0u;
+    cmn = mk_min_u64(cmn, s);
+    cmx = mk_max_u64(cmx, s);
+    const uint64_t span = cmx - cmn;
+    const int lz = span ? __clzll((long long)span) : 64;
+    const int sh = 64 - lz > 11 ? 64 - lz - 11 : 0;
+    static_assert(MK_BINS == 1 << 11, "span >> sh fits eleven bits");
+    uint32_t place[EPT];                                    // bin << 16 | slot
+#pragma unroll
+    for (int q = 0; q < EPT; ++q) {
+        place[q] = 0u;
+        if (q * SK_LT + tid < n) {
+            const uint32_t b = (uint32_t)((cmx - v[q]) >> sh);
+            place[q] = (b << 16) | atomicAdd(&s.u.m.bins[b], 1u);
+        }
+    }
+    __syncthreads();
+    constexpr int BPT = MK_BINS / SK_LT;
+    uint32_t c[BPT], sum = 0u;
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+        c[j] = s.u.m.bins[BPT * tid + j];
+        sum += c[j];
+    }
+    uint32_t tot;
+    uint32_t off = mk_excl_u32(sum, s, tot);
+    if (tid == 0) s.misc[3] = (uint32_t)n;                     // entries in the bins that start before k
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+        s.u.m.bins[BPT * tid + j] = off;
+        if (off < (uint32_t)k && off + c[j] >= (uint32_t)k) s.misc[4] = off + c[j];
+        off += c[j];
+    }
+    if (tid == SK_LT - 1) s.u.m.bins[MK_BINS] = off;
+    __syncthreads();
+    const int m = n <= k ? n : (int)s.misc[4];
+    if (m > MK_TOP) return false;
+#pragma unroll
+    for (int q = 0; q < EPT; ++q) {
+        if (q * SK_LT + tid < n) {
+            const uint32_t pos = s.u.m.bins[place[q] >> 16] + (place[q] & 0xFFFFu);
+            if (pos < (uint32_t)m) s.u.m.top[pos] = v[q];
+        }
+    }
+    __syncthreads();
+    constexpr int TPT_ = EPT < MK_TOP / SK_LT ? EPT : MK_TOP / SK_LT;
+    uint64_t e[TPT_];
+    uint32_t r[TPT_];
+#pragma unroll
+    for (int q = 0; q < TPT_; ++q) {
+        const int i = q * SK_LT + tid;
+        e[q] = 0ull;
+        r[q] = 0xFFFFFFFFu;
+        if (i < m) {
+            e[q] = s.u.m.top[i];
+            const uint32_t b = (uint32_t)((cmx - e[q]) >> sh);
+            const uint32_t lo = s.u.m.bins[b], hi = s.u.m.bins[b + 1];
+            uint32_t x = lo;
+            for (uint32_t j = lo; j < hi; ++j) x += s.u.m.top[j] > e[q] ? 1u : 0u;
+            r[q] = x;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < TPT_; ++q)
+        if (r[q] < (uint32_t)k) s.u.m.top[r[q]] = e[q];
+    __syncthreads();
+    return true;
+}
+
+// Softmax at temperature, min-p, top-p and the draw (sampler.cpp:37-49) over the k <= MK_K sorted candidates in
+// s.u.w.top; the optional candidate outputs. Masses are taken strided, prefixes over ceil(k / SK_LT) neighbours per
+// thread. Whole workgroup; the results are uniform.
+__device__ __forceinline__ void mk_softmax(const SkArgs& a, const fs_row_params& p, int row, int k, double u, MkShared& s,
+                                           int& tok, int& keep) {
+    const int tid = threadIdx.x, per = (k + SK_LT - 1) / SK_LT, i0 = tid * per;
+    const int i1 = i0 + per < k ? i0 + per : k;
+    const uint64_t* top = s.u.w.top;
+    double* E = s.u.w.e;
+    const float mx = val_of(comp_key(top[0]));
+    const double Td = (double)p.temperature;
+    double run = 0.0, sum;
+#pragma unroll 1
+    for (int i = tid; i < k; i += SK_LT) {
+        const float d = val_of(comp_key(top[i])) - mx;         // fp32 subtraction, as ferro
+        const double m = exp((double)d / Td);
+        E[i] = m;
+        run += m;
+    }
+    (void)mk_excl_f64(run, s, sum);                            // (its barriers publish E)
+    run = 0.0;
+    uint64_t last = 0ull;                                      // min-p: 1 + the last index not below pr[0] * min_p
+    const double thr = (1.0 / sum) * (double)p.min_p;
+#pragma unroll 1
+    for (int i = i0; i < i1; ++i) {
+        const double pr = E[i] / sum;
+        E[i] = pr;
+        run += pr;
+        if (!(pr < thr)) last = (uint64_t)(i + 1);
+    }
+    int keep_m = k;
+    if (p.min_p > 0.0f) {
+        last = mk_max_u64(last, s);
+        keep_m = last > 1ull ? (int)last : 1;
+    }
+    double all;
+    const double off = mk_excl_f64(run, s, all);
+    keep = keep_m;
+    if (p.top_p < 1.0f) {
+        uint64_t first = ~0ull;
+        run = 0.0;
+#pragma unroll 1
+        for (int i = i0; i < i1; ++i) {
+            run += E[i];
+            if (first == ~0ull && i < keep_m && run + off >= (double)p.top_p) first = (uint64_t)i;
+        }
+        first = mk_min_u64(first, s);
+        if (first != ~0ull) keep = (int)first + 1 < keep_m ? (int)first + 1 : keep_m;
+        if (keep < 1) keep = 1;
+    }
+    if (i0 < keep && keep <= i0 + per) {                       // tot: the kept prefix's sum
+        run = 0.0;
+        for (int i = i0; i < keep; ++i) run += E[i];
+        s.dmisc = run + off;
+    }
+    __syncthreads();
+    const double rr = u * s.dmisc + 0.0;
+    uint64_t hit = ~0ull;
+    run = 0.0;
+#pragma unroll 1
+    for (int i = i0; i < i1; ++i) {
+        run += E[i];
+        if (hit == ~0ull && i < keep && rr <= run + off) hit = (uint64_t)i;
+    }
+    hit = mk_min_u64(hit, s);
+    tok = (int)comp_id(top[hit == ~0ull ? keep - 1 : (int)hit]);
+    if (a.mode != MODE_VERIFY) {
+        const int m = k < a.kcap ? k : a.kcap;
+        for (int i = tid; i < m; i += SK_LT) {
+            if (a.cand_ids) a.cand_ids[(int64_t)row * a.kcap + i] = (int32_t)comp_id(top[i]);
+            if (a.cand_probs) a.cand_probs[(int64_t)row * a.kcap + i] = E[i];
+        }
+    }
+}
+
+struct MkKernargs {
+    const float* logits;
+    int64_t ld;
+    int B, V, nseg, flags;
+    const fs_row_params* params;
+    const int64_t* hist_off;
+    const int32_t* hist;
+    MkArgs m;
+};
+constexpr size_t MK_ARGS_OFF = offsetof(MkKernargs, m);
+
+// CAP: some row of the batch has a softcap. It never decreases, so the bound is taken over raw logits and the merge caps
+// the list (an entry whose value is final already, a penalised one, has its id word's top bit cleared).
+template <int NL, bool CAP>
+__global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, int64_t ld, int B, int V, int nseg,
+                                                         int flags, const fs_row_params* params,
+                                                         const int64_t* hist_off, const int32_t* hist, MkArgs m_) {
+    constexpr int SEG = SK_LT * NL * 4;
+    __shared__ __align__(16) MkShared s;
+    const int tid = threadIdx.x, lane = lane_id(), w = tid / WAVE;
+    // a row's segments are consecutive workgroups of one index class mod XCDS: they share an XCD and its L2
+    const int x = (int)(blockIdx.x % (unsigned)XCDS);
+    const int j = (int)(blockIdx.x / (unsigned)XCDS);
+    const int q_row = __builtin_amdgcn_readfirstlane(j / nseg);
+    const int seg = j - q_row * nseg;
+    const int row = x + XCDS * q_row;
+    if (row >= B) return;
+    SK_MARK(0);
+    for (int i_ = 1; i_ < 13; ++i_) SK_TAG(i_, 0);
+    SK_TAG(13, 3); SK_TAG(14, row); SK_TAG(15, seg);
+    const int seg_lo = seg * SEG;
+    const int n_in = V - seg_lo < SEG ? V - seg_lo : SEG;      // logits of this segment (>= 1)
+    const float* rowp = logits + (int64_t)row * ld;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(rowp + seg_lo), (short)0, ((n_in + 3) & ~3) * 4, 0x00020000);
+    float v[NL][4];
+    auto load = [&](int q) {
+        const f32x4 t = raw_buffer_load_f32x4(rs, (q * SK_LT + tid) * 16, 0, 2);    // nontemporal: read once
+        v[q][0] = t.x; v[q][1] = t.y; v[q][2] = t.z; v[q][3] = t.w;
+    };
+    // the first half, then the window's ids, then the rest: a wave's loads return in order, and so the bitmap is built
+    // while the rest streams in (segments of 4096 logits are all requested at once: their ids come last anyway)
+    constexpr int NL0 = NL > 4 ? NL / 2 : NL;
+#pragma unroll
+    for (int q = 0; q < NL0; ++q) load(q);
+    __builtin_amdgcn_sched_barrier(0);
+    // the other arguments through a pointer the compiler cannot trace (it would load some of them before the logits)
+    const __attribute__((address_space(4))) char* kseg =
+        (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(kseg) : : "memory");
+    const MkArgs& mk = *(const MkArgs*)(kseg + MK_ARGS_OFF);
+    const SkArgs& a = mk.a;
+    (void)m_;
+
+    // the row's parameters (verification: its stream's) and its window; its first ids requested behind the logits
+    int pidx = row, fed = 0;
+    MkWin win = {hist, nullptr, 0, 0};
+    if (flags & MK_VERIFY) {
+        // the largest s with row_off[s] <= row: where it lies if every stream has as many rows, else by bisection
+        int s0 = (int)((int64_t)row * a.n_streams / B), s1 = s0 + 1;
+        if (ld_const(a.row_off + s0) > row || ld_const(a.row_off + s1) <= row) { s0 = 0; s1 = a.n_streams; }
+        while (s1 - s0 > 1) {
+            const int m = (s0 + s1) >> 1;
+            if (ld_const(a.row_off + m) <= row) s0 = m; else s1 = m;
+        }
+        pidx = s0;
+        const int64_t r0 = ld_const(a.row_off + s0);
+        win.pb = a.rows + r0 + 1;
+        fed = row - (int)r0;
+    }
+    fs_row_params p;
+    {
+        uint32_t pw[sizeof(fs_row_params) / 4];
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(params + pidx);
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(fs_row_params) / 4); ++i) pw[i] = ld_const(src + i);
+        __builtin_memcpy(&p, pw, sizeof(p));
+    }
+    bool pen = false;
+    MkPen pn;
+    pn.rep = p.repetition_penalty; pn.fq = p.frequency_penalty; pn.pres = p.presence_penalty; pn.cap = p.softcap;
+    pn.rep_on = pn.rep != 1.0f;
+    pn.fp_on = pn.fq != 0.0f || pn.pres != 0.0f;
+    int wid[MK_W];
+#pragma unroll
+    for (int r = 0; r < MK_W; ++r) wid[r] = -1;
+    if (flags & SK_MAY_PEN) {
+        int64_t h0 = 0, lenA = 0;
+        if (hist_off && hist) {
+            h0 = ld_const(hist_off + pidx);
+            lenA = ld_const(hist_off + pidx + 1) - h0;
+        }
+        const int64_t len = lenA + fed;
+        pen = (pn.rep_on || pn.fp_on) && p.repeat_last_n != 0 && len > 0;
+        const int64_t b = window_begin(len, p);
+        if (b >= len) pen = false;
+        if (pen) {
+            win.pa = hist + h0 + (b < lenA ? b : lenA);
+            win.na = b < lenA ? lenA - b : 0;
+            win.nb = fed - (b > lenA ? (int)(b - lenA) : 0);
+            win.pb += fed - win.nb;
+#pragma unroll
+            for (int r = 0; r < MK_W; ++r)
+                if (r * SK_LT + tid < win.na) wid[r] = win.pa[r * SK_LT + tid];
+        }
+    }
+    const bool cp_on = (flags & SK_COPY) != 0;
+    SkCopy cp = {};
+    if (cp_on) cp = sk_cp_load(hist_off, hist, row, seg, nseg);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = NL0; q < NL; ++q) load(q);
+    __builtin_amdgcn_sched_barrier(0);
+    const bool greedy = p.temperature <= 0.0f || p.top_k == 1;
+    const bool scan = greedy && !(CAP && pn.cap > 0.0f);       // (a capped greedy row goes the sampled rows' way, k = 1)
+    const int k = greedy ? 1 : ((p.top_k > 0 && p.top_k < V) ? p.top_k : V);
+
+    // the window's ids of this segment: a bit per logit, 64 bits per thread (its own logits), and counts
+    uint32_t* ctr = mk.ctr + (int64_t)row * MK_CTR;            // [0] barrier; [32] ticket, [33] list length, [34] slow, [35] spill
+    uint64_t* list = mk.list + (int64_t)row * MK_LCAP;
+    uint64_t* spill = mk.spill + (int64_t)row * MK_SPILL;
+    // this wave's flagged logits: nf of them, in LDS from place pb on, or in the row's spill list (far; over: it is full)
+    uint32_t nf = 0u, pb = 0u;
+    bool far = false, over = false;
+    if (pen) {
+        uint32_t m0 = 0u, m1 = 0u;
+        bool ovf = false;
+        for (int i = tid; i < SK_LT * 2; i += SK_LT) s.b.bmp[i] = 0u;
+        if (tid == 0) s.np = 0u;
+        if (pn.fp_on)
+            for (int i = tid; i < SEG / 8; i += SK_LT) reinterpret_cast<uint4*>(s.u.cnt)[i] = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();
+        auto set = [&](uint32_t rel) {
+            const uint32_t g = rel >> 2;
+            atomicOr(&s.b.bmp[(g % SK_LT) * 2 + g / (SK_LT * 8)], 1u << (4u * ((g / SK_LT) & 7u) + (rel & 3u)));
+        };
+        auto mark4 = [&](int i0, int i1, int i2, int i3) {     // (the counts' old values are in flight together)
+            const uint32_t lo = (uint32_t)seg_lo;
+            const uint32_t rel[4] = {(uint32_t)i0 - lo, (uint32_t)i1 - lo, (uint32_t)i2 - lo, (uint32_t)i3 - lo};
+            const uint32_t m01 = rel[0] < rel[1] ? rel[0] : rel[1], m23 = rel[2] < rel[3] ? rel[2] : rel[3];
+            if ((m01 < m23 ? m01 : m23) >= (uint32_t)n_in) return;   // (most hold no id of the segment)
+            if (pn.fp_on) {
+                uint32_t old[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    old[c] = rel[c] < (uint32_t)n_in ? atomicAdd(&s.u.cnt[rel[c] >> 1], 1u << ((rel[c] & 1u) * 16u)) : 0u;
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (rel[c] < (uint32_t)n_in) {
+                        const uint32_t had = (old[c] >> ((rel[c] & 1u) * 16u)) & 0xFFFFu;
+                        ovf |= had == 0xFFFFu;
+                        if (had == 0u) set(rel[c]);
+                    }
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (rel[c] < (uint32_t)n_in) set(rel[c]);
+            }
+        };
+#pragma unroll
+        for (int r = 0; r < MK_W; ++r) asm volatile("" : "+v"(wid[r]));   // (no wait for the ids above this branch)
+        static_assert(MK_W == 4, "one batch of prefetched ids");
+        // batches of four ids per thread: the prefetched ones, the drafts and the ends of the rest, then the rest's 16-byte
+        // blocks, four loads in flight
+        const int32_t* hp = win.pa + MK_W * SK_LT;
+        const int64_t n = win.na - MK_W * SK_LT;               // ids past the prefetched ones
+        const int ab = (int)((0u - (unsigned)((uintptr_t)hp >> 2)) & 3u);
+        const int64_t nv = n > ab ? (n - ab) >> 2 : 0;
+        const int64_t rest = ab + 4 * nv;
+        const int4* hv = reinterpret_cast<const int4*>(hp + ab);
+        int4 w4[4];
+        w4[0] = make_int4(wid[0], wid[1], wid[2], wid[3]);
+        w4[1] = make_int4(tid < win.nb ? win.pb[tid] : -1, tid < ab && tid < n ? hp[tid] : -1,
+                          rest + tid < n ? hp[rest + tid] : -1, SK_LT + tid < win.nb ? win.pb[SK_LT + tid] : -1);
+        w4[2] = w4[3] = make_int4(-1, -1, -1, -1);
+        int nr = win.nb > 0 || n > 0 ? 2 : 1;
+        int64_t d0 = 2 * SK_LT;
+#pragma unroll 1
+        for (int64_t j0 = 0;;) {
+#pragma unroll 1
+            for (int r = 0; r < nr; ++r) {
+                // (unary plus: selects of values, not of addresses, which would put the array in memory)
+                const int i0 = r == 0 ? +w4[0].x : r == 1 ? +w4[1].x : r == 2 ? +w4[2].x : +w4[3].x;
+                const int i1 = r == 0 ? +w4[0].y : r == 1 ? +w4[1].y : r == 2 ? +w4[2].y : +w4[3].y;
+                const int i2 = r == 0 ? +w4[0].z : r == 1 ? +w4[1].z : r == 2 ? +w4[2].z : +w4[3].z;
+                const int i3 = r == 0 ? +w4[0].w : r == 1 ? +w4[1].w : r == 2 ? +w4[2].w : +w4[3].w;
+                mark4(i0, i1, i2, i3);
+            }
+            if (j0 < nv) {
+                nr = 4;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    w4[r] = j0 + r * SK_LT + tid < nv ? hv[j0 + r * SK_LT + tid] : make_int4(-1, -1, -1, -1);
+                j0 += 4 * SK_LT;
+            } else if (d0 < win.nb) {                          // (a stream of more than 512 rows)
+                nr = 1;
+                w4[0] = make_int4(d0 + tid < win.nb ? win.pb[d0 + tid] : -1, -1, -1, -1);
+                d0 += SK_LT;
+            } else {
+                break;
+            }
+        }
+        if (ovf) atomicOr(a.err, FS_DEVERR_COUNT_OVERFLOW);
+        __syncthreads();
+        m0 = s.b.bmp[2 * tid];
+        m1 = NL > 8 ? s.b.bmp[2 * tid + 1] : 0u;
+        // the flagged logits to the wave's list, and out of the registers (NaN: no comparison takes it)
+        const uint32_t mine = (uint32_t)(__popc(m0) + __popc(m1));
+        const uint32_t incl = wave_incl_scan_u32(mine);
+        nf = (uint32_t)__builtin_amdgcn_readlane((int)incl, WAVE - 1);
+        __syncthreads();                                       // every thread has read its bits
+        if (nf != 0u) {
+            if (lane == 0) pb = atomicAdd(&s.np, nf);
+            pb = (uint32_t)__builtin_amdgcn_readfirstlane((int)pb);
+            far = pb + nf > (uint32_t)MK_PC;
+            if (far) {
+                if (lane == 0) pb = __hip_atomic_fetch_add(ctr + 35, nf, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                pb = (uint32_t)__builtin_amdgcn_readfirstlane((int)pb);
+                over = pb + nf > (uint32_t)MK_SPILL;
+                if (over) nf = 0u;
+            }
+            uint32_t at = pb + incl - mine;
+#pragma unroll
+            for (int q = 0; q < NL; ++q) {
+                const uint32_t nib = ((q < 8 ? m0 : m1) >> (4 * (q & 7))) & 15u;
+                if (__ballot(nib != 0u) != 0ull) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        if ((nib >> c) & 1u) {
+                            const uint32_t rel = (uint32_t)((q * SK_LT + tid) * 4 + c);
+                            if (!far) {
+                                s.b.pv[at] = v[q][c];
+                                s.prel[at] = (uint16_t)rel;
+                            } else if (!over) {
+                                spill[at] = ((uint64_t)rel << 32) | __float_as_uint(v[q][c]);
+                            }
+                            ++at;
+                            v[q][c] = __builtin_nanf("");
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if (n_in < SEG) {                                          // past the row's end: NaN, no comparison takes it
+#pragma unroll
+        for (int q = 0; q < NL; ++q)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if ((q * SK_LT + tid) * 4 + c >= n_in) v[q][c] = __builtin_nanf("");
+    }
+    float lm = __builtin_nanf("");                             // the lane maximum (fmaxf drops NaN)
+#pragma unroll
+    for (int q = 0; q < NL; ++q) lm = fmaxf(lm, fmaxf(fmaxf(v[q][0], v[q][1]), fmaxf(v[q][2], v[q][3])));
+    const bool capped = CAP && pn.cap > 0.0f;
+    // the wave's flagged logits, penalised in place; afterwards entry i as ~id above the value (far: read past the L1)
+    auto penalise = [&]() {
+        if (far) vm_drain();
+#pragma unroll 1
+        for (uint32_t i = (uint32_t)lane; i < nf; i += WAVE) {
+            const uint64_t e = far ? ld_agent(&spill[pb + i]) : 0ull;
+            const uint32_t rel = far ? (uint32_t)(e >> 32) : s.prel[pb + i];
+            float l = far ? __uint_as_float((uint32_t)e) : s.b.pv[pb + i];
+            if (CAP && pn.cap > 0.0f) l = softcap_one(l, pn.cap);
+            l = pn.apply(l, pn.fp_on ? (s.u.cnt[rel >> 1] >> ((rel & 1u) * 16u)) & 0xFFFFu : 0u);
+            if (far) st_agent(&spill[pb + i], (e & 0xFFFFFFFF00000000ull) | __float_as_uint(l));
+            else s.b.pv[pb + i] = l;
+        }
+        if (far) vm_drain();
+    };
+    auto pen_at = [&](uint32_t i) {
+        const uint64_t e = far ? ld_agent(&spill[pb + i]) : 0ull;
+        uint32_t nid = ~((uint32_t)seg_lo + (far ? (uint32_t)(e >> 32) : (uint32_t)s.prel[pb + i]));
+        if (CAP && pn.cap > 0.0f) nid &= 0x7FFFFFFFu;          // (its value is capped already)
+        return ((uint64_t)nid << 32) | (far ? (uint32_t)e : __float_as_uint(s.b.pv[pb + i]));
+    };
+    SK_MARK(1);
+    float tr = 0.0f, tc = 0.0f;                                // the bound: raw, capped
+    bool go = true;
+    if (!scan) {
+        // the lane maxima, sorted in each wave, published at 16 ranks
+        const uint32_t srt = sort64_desc_u32(key_of(lm));
+        s.h.srt[w][lane] = srt;
+        uint32_t* qk = mk.qk + (int64_t)row * nseg * (SK_NW * 16);
+        if (lane < 16) qk[(seg * SK_NW + w) * 16 + lane] = s.h.srt[w][mk_rank(lane) - 1];
+        SK_MARK(2);
+        vm_drain();
+        __syncthreads();
+        if (tid == 0) __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        penalise();                                            // (while the other segments arrive)
+        if (tid == 0) {
+            uint32_t ok = 1u, spins = 0u;
+            for (;;) {                                         // (a poll that adds: it executes in the L2)
+                const uint32_t c = __hip_atomic_fetch_add(ctr, 0x10000u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if ((c & 0xFFFFu) >= (uint32_t)nseg && mk.spins != 0u) break;
+                if (++spins >= mk.spins) { ok = 0u; break; }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            s.misc[5] = ok;
+            if (!ok) __hip_atomic_fetch_or(ctr + 34, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        *reinterpret_cast<uint4*>(&s.h.hist[4 * tid]) = make_uint4(0u, 0u, 0u, 0u);   // (the ranks are read)
+        __syncthreads();
+        SK_MARK(3);
+        go = s.misc[5] != 0u;
+        if (go) {
+            const uint32_t T = mk_bound<NL == 16 ? 1 : NL == 8 ? 2 : 4>(qk, nseg, k, s);
+            SK_MARK(4);
+            tc = T > 0x007FFFFFu ? val_of(T) : -__builtin_huge_valf();
+            tr = tc;
+            if (CAP && pn.cap > 0.0f) {
+                // tc: the capped bound; tr: a raw value that every logit whose capped value reaches tc reaches. Lane
+                // l < 32 caps the value 2^l keys below the bound (lane 32 the bound): the first that falls below tc
+                const uint32_t kb = T > 0x007FFFFFu ? T : 0x007FFFFFu, room = kb - 0x007FFFFFu;
+                const uint32_t step = lane < 32 ? 1u << lane : 0u;
+                const float c = softcap_one(val_of(room > step ? kb - step : 0x007FFFFFu + (lane < 32 ? 0u : room)), pn.cap);
+                tc = read_lane(c, 32);
+                const uint64_t below = __ballot(lane < 32 && c < tc);
+                tr = -__builtin_huge_valf();
+                if (below) {
+                    const uint32_t st = 1u << (__ffsll((unsigned long long)below) - 1);
+                    tr = room > st ? val_of(kb - st) : tr;
+                }
+            }
+        }
+    }
+    if (scan) {
+        // the segment's first maximum (ferro's scan, sampler.cpp:19-23)
+        uint64_t best = 0ull;
+        if (lm == lm) {
+            uint32_t first = 0u;
+#pragma unroll
+            for (int q = NL - 1; q >= 0; --q)
+#pragma unroll
+                for (int c = 3; c >= 0; --c)
+                    first = v[q][c] == lm ? (uint32_t)(q * SK_LT * 4 + c) : first;
+            best = comp_of(key_of(lm), (uint32_t)(seg_lo + tid * 4) + first);
+        }
+        penalise();
+        for (uint32_t i = (uint32_t)lane; i < nf; i += WAVE) {    // and the penalised ones
+            const uint64_t e = pen_at(i);
+            const uint32_t key = key_of(__uint_as_float((uint32_t)e));
+            const uint64_t c = ((uint64_t)key << 32) | (e >> 32);
+            if (key != 0u && c > best) best = c;
+        }
+        best = mk_max_u64(best, s);
+        if (tid == 0) list[seg] = best;
+    } else {
+        if (go) {
+            // the logits at or above the bound to the row's list, the penalised ones against the capped bound
+            uint32_t np = 0u;
+            for (uint32_t i = (uint32_t)lane; i < nf; i += WAVE) np += __uint_as_float((uint32_t)pen_at(i)) >= tc ? 1u : 0u;
+            uint64_t gm = 0ull;
+#pragma unroll
+            for (int q = 0; q < NL; ++q)                       // (most groups hold none)
+                if (__ballot(fmaxf(fmaxf(v[q][0], v[q][1]), fmaxf(v[q][2], v[q][3])) >= tr) != 0ull) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) gm |= (uint64_t)(v[q][c] >= tr ? 1u : 0u) << (4 * q + c);
+                }
+            if (tr == -__builtin_huge_valf()) {
+                // fewer than k finite lane maxima (a masked vocabulary): of the logits at -inf only this wave's first
+                // k ids can be among the row's top k
+                uint64_t eq = 0ull;
+#pragma unroll
+                for (int q = 0; q < NL; ++q)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) eq |= (uint64_t)(v[q][c] == tr ? 1u : 0u) << (4 * q + c);
+                gm &= ~eq;
+                uint32_t seen = 0u;
+#pragma unroll 1
+                for (int q = 0; q < NL && seen < (uint32_t)k; ++q) {
+                    uint32_t nib = (uint32_t)(eq >> (4 * q)) & 15u;
+                    const uint32_t incl = wave_incl_scan_u32((uint32_t)__popc(nib));
+                    uint32_t before = seen + incl - (uint32_t)__popc(nib);
+                    for (int c = 0; c < 4; ++c)
+                        if ((nib >> c) & 1u) {
+                            if (before < (uint32_t)k) gm |= 1ull << (4 * q + c);
+                            ++before;
+                        }
+                    seen += (uint32_t)__builtin_amdgcn_readlane((int)incl, WAVE - 1);
+                }
+            }
+            const uint32_t n = (uint32_t)__popcll(gm) + np;
+            const uint32_t incl = wave_incl_scan_u32(n);
+            const uint32_t nw = (uint32_t)__builtin_amdgcn_readlane((int)incl, WAVE - 1);
+            if (nw != 0u) {
+                uint32_t base = 0u;
+                if (lane == 0) base = __hip_atomic_fetch_add(ctr + 33, nw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
+                if (base + nw <= (uint32_t)MK_LCAP) {          // (else the list's length shows it)
+                    uint64_t* at = list + (base + incl - n);
+                    if (np != 0u)
+                        for (uint32_t i = (uint32_t)lane; i < nf; i += WAVE) {
+                            const uint64_t e = pen_at(i);
+                            if (__uint_as_float((uint32_t)e) >= tc) *at++ = e;
+                        }
+#pragma unroll
+                    for (int q = 0; q < NL; ++q) {
+                        const uint32_t nib = (uint32_t)(gm >> (4 * q)) & 15u;
+                        if (__ballot(nib != 0u) != 0ull) {
+                            const uint32_t id0 = ~(uint32_t)(seg_lo + (q * SK_LT + tid) * 4);   // ~(x + c) = ~x - c
+#pragma unroll
+                            for (int c = 0; c < 4; ++c)
+                                if ((nib >> c) & 1u) *at++ = ((uint64_t)(id0 - (uint32_t)c) << 32) | __float_as_uint(v[q][c]);
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if (over && lane == 0)                                     // too many penalised ids: the row is selected alone
+        __hip_atomic_fetch_or(ctr + 34, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (cp_on) sk_cp_store(a, cp, row, seg);
+    SK_MARK(5);
+    vm_drain();                                                // the candidates are in the L2
+    __syncthreads();
+    if (tid == 0)
+        s.misc[0] = __hip_atomic_fetch_add(ctr + 32, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) ==
+                    (uint32_t)nseg - 1u ? 1u : 0u;
+    __syncthreads();
+    SK_MARK(6);
+    if (s.misc[0] == 0u) {
+        SK_FLUSH();
+        return;
+    }
+    SK_TAG(13, 4);
+    // ---- the row's end, by its last segment. (The lists are read at agent scope: past this CU's L1.)
+    SkDraw dr = {0.0, 0};
+    if (!greedy) dr = sk_draw(a, row);
+    int tok = 0, keep = 1;
+    // a greedy row's token (ferro keeps index 0 when its logit is NaN)
+    auto greedy_end = [&](uint64_t top) {
+        tok = (rowp[0] != rowp[0] || top == 0ull) ? 0 : (int)comp_id(top);
+        if (lane == 0 && a.mode != MODE_VERIFY && a.kcap > 0) {
+            if (a.cand_ids) a.cand_ids[(int64_t)row * a.kcap] = tok;
+            if (a.cand_probs) a.cand_probs[(int64_t)row * a.kcap] = 1.0;
+        }
+    };
+    const uint32_t slow = ld_agent(ctr + 34);                  // uniform
+    if (scan && slow == 0u) {
+        if (w != 0) return;
+        greedy_end(wave_max(lane < nseg ? ld_agent(&list[lane]) : 0ull));
+        if (lane == 0) {
+            ctr[32] = 0u;
+            ctr[35] = 0u;
+        }
+    } else {
+        uint32_t C = ld_agent(ctr + 33);
+        bool capped_list = capped;
+        const bool again = slow != 0u || C > (uint32_t)MK_LCAP;   // uniform
+        __syncthreads();
+        if (tid == 0) {                                        // every segment has met and counted: left at 0
+            ctr[0] = 0u;
+            ctr[32] = 0u;
+            ctr[33] = 0u;
+            ctr[34] = 0u;
+            ctr[35] = 0u;
+            if (slow & 2u) atomicOr(a.err, FS_DEVERR_INTERNAL);
+        }
+        bool select = again;
+        for (;;) {
+            if (select) {
+                C = mk_slow<CAP>(rowp, V, k, pen, win, pn, list, s);
+                capped_list = false;
+            }
+            if (C == 0u) {                                     // every logit NaN: token 0, nothing kept
+                keep = greedy ? 1 : 0;
+                if (greedy && w == 0) greedy_end(0ull);
+                break;
+            }
+            const int kk = (uint32_t)k < C ? k : (int)C;
+            // the list's entries (~id above the logit's bits) as the composites ferro ranks; raw logits are capped here
+            auto entry = [&](uint64_t c) {
+                uint32_t nid = (uint32_t)(c >> 32);
+                float l = __uint_as_float((uint32_t)c);
+                if (CAP) {
+                    if (capped_list && (nid & 0x80000000u)) l = softcap_one(l, pn.cap);
+                    nid |= 0x80000000u;
+                }
+                return c == 0ull ? 0ull : ((uint64_t)key_of(l) << 32) | nid;
+            };
+            if (k <= WAVE && C <= (uint32_t)SK_LT) {
+                uint64_t* cand = s.u.m.top;
+                if ((uint32_t)tid < C) cand[tid] = entry(ld_agent(&list[tid]));
+                if (tid < WAVE) cand[SK_LT + tid] = 0ull;
+                __syncthreads();
+                sk_rank(cand, s.h.rk, (int)C, [&](uint32_t r, uint64_t c) { if (r < (uint32_t)WAVE) cand[SK_LT + r] = c; });
+                __syncthreads();
+                if (w != 0) return;
+                SK_MARK(7);
+                if (greedy) {
+                    greedy_end(read_lane(cand[SK_LT + lane], 0));
+                    break;
+                }
+                Args fa = {};
+                fa.mode = a.mode; fa.kcap = a.kcap; fa.cand_ids = a.cand_ids; fa.cand_probs = a.cand_probs;
+                RowCtx rc = {};
+                rc.row = row;
+                rc.p = p;
+                wave_softmax(fa, rc, lane < kk ? cand[SK_LT + lane] : 0ull, kk, dr.u, tok, keep);
+                break;
+            }
+            // the list in registers, as many entries per thread as it needs
+            auto sort_list = [&](auto ept) {
+                constexpr int EPT = decltype(ept)::value;
+                uint64_t e[EPT];
+#pragma unroll
+                for (int q = 0; q < EPT; ++q)
+                    e[q] = (uint32_t)(q * SK_LT + tid) < C ? ld_agent(&list[q * SK_LT + tid]) : 0ull;
+                if (CAP) {                                     // (a rolled loop: one copy of the cap)
+#pragma unroll 1
+                    for (int q = 0; q < EPT; ++q) {
+                        uint64_t c = e[0];
+#pragma unroll
+                        for (int t = 1; t < EPT; ++t) c = q == t ? e[t] : c;
+                        c = entry(c);
+#pragma unroll
+                        for (int t = 0; t < EPT; ++t) e[t] = q == t ? c : e[t];
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < EPT; ++q) e[q] = entry(e[q]);
+                }
+                __syncthreads();
+                return mk_sort(e, (int)C, k, s);
+            };
+            bool sorted = true;
+            if (C <= (uint32_t)SK_LT) {
+                uint64_t* cand = s.u.m.top + MK_TOP - SK_LT;
+                if ((uint32_t)tid < C) cand[tid] = entry(ld_agent(&list[tid]));
+                __syncthreads();
+                sk_rank(cand, s.h.rk, (int)C, [&](uint32_t r, uint64_t c) { if (r < (uint32_t)k) s.u.m.top[r] = c; });
+                __syncthreads();
+            } else if (C <= 4u * SK_LT) sorted = sort_list(std::integral_constant<int, 4>{});
+            else sorted = sort_list(std::integral_constant<int, MK_LCAP / SK_LT>{});
+            SK_MARK(7);
+            if (sorted && greedy) {
+                if (w == 0) greedy_end(s.u.m.top[0]);
+                break;
+            }
+            if (sorted) {
+                mk_softmax(a, p, row, kk, dr.u, s, tok, keep);
+                break;
+            }
+            if (select) {                                      // (never: mk_slow leaves at most k <= MK_TOP entries)
+                if (tid == 0) atomicOr(a.err, FS_DEVERR_INTERNAL);
+                break;
+            }
+            select = true;
+        }
+        if (w != 0) return;
+    }
+    SK_TAG(9, k);
+    sk_finish(a, row, pidx, !greedy, tok, keep, cp, dr.idx, &s.u.m.top[0]);
+    SK_MARK(8);
+    SK_FLUSH();
+}
+
+hipError_t launch_mid_k(int nl, bool capped, unsigned grid, int flags, const MkArgs& m, hipStream_t st) {
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_LT), 0, st, m.a.logits, m.a.ld, m.a.B, m.a.V, m.a.nseg, flags,
+                           m.a.params, m.a.hist_off, m.a.hist, m);
+    };
+    if (capped) {
+        if (nl == 16) go(mid_k_kernel<16, true>);
+        else if (nl == 8) go(mid_k_kernel<8, true>);
+        else go(mid_k_kernel<4, true>);
+    } else {
+        if (nl == 16) go(mid_k_kernel<16, false>);
+        else if (nl == 8) go(mid_k_kernel<8, false>);
+        else go(mid_k_kernel<4, false>);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace fs

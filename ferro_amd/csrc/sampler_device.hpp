@@ -44,6 +44,9 @@ constexpr int RSHIFT = 32 - RBITS;
 constexpr int XCDS = 8;                   // MI355X: 8 XCDs, workgroups dealt round-robin by index
 constexpr int WIDS = 2048;                // penalty-window ids of one segment kept in LDS (longer: rescanned per tile)
 
+constexpr int LB = 4096;                    // coarse key bins of the large-k path
+constexpr uint32_t MERGE_SPINS = 1u << 20;   // bounded wait of the merge role (far above any segment's time)
+
 enum Mode : int { MODE_SAMPLE = 0, MODE_ARGMAX = 1, MODE_VERIFY = 2 };
 
 struct Args {

@@ -9,6 +9,11 @@
 
 namespace fs {
 
+struct Args;
+// The fused kernel's grid (segments, then merges), and its merge alone (alone != 0: each row from its logits).
+hipError_t launch_segments(const Args& a, unsigned grid, hipStream_t st);
+hipError_t launch_merges(const Args& a, unsigned rows, int nseg, int alone, hipStream_t st);
+
 constexpr int SK_LT = 256;                 // threads per segment workgroup
 constexpr int SK_NW = SK_LT / 64;
 constexpr int SK_K = 64;                   // largest k (one candidate per lane of the finishing wave)
@@ -48,11 +53,26 @@ struct SkArgs {
     int64_t out_cap;
 };
 
-// flags of a launch: some row has an active penalty window; a decode step (the histories are copied)
-constexpr int SK_MAY_PEN = 1, SK_COPY = 2;
+// flags of a launch: some row has an active penalty window; a decode step (the histories are copied); a verification
+// window (mid-k kernel)
+constexpr int SK_MAY_PEN = 1, SK_COPY = 2, MK_VERIFY = 4;
 // nl: float4 loads per thread (4, 8 or 16); the grid and k's layout come from the small-k plan.
 hipError_t launch_small_k(int nl, bool capped, bool all_greedy, unsigned grid, int flags, const SkArgs& k,
                           hipStream_t st);
+
+// The mid-k kernel: the small-k kernel's arguments (lists and ticket unused) and its own workspace.
+constexpr int MK_LIST = 4096;              // entries of a row's candidate list
+constexpr int MK_SPILL = 16384;            // entries of a row's list of penalised logits past those its segments keep in LDS
+constexpr int MK_CTR = 64;                 // words of a row's counters
+struct MkArgs {
+    SkArgs a;
+    uint32_t* ctr;                         // [B][MK_CTR], left at 0
+    uint32_t* qk;                          // [B][nseg][SK_NW][16] published lane maxima
+    uint64_t* list;                        // [B][MK_LIST]
+    uint64_t* spill;                       // [B][MK_SPILL]
+    uint32_t spins;                        // bounded wait for a row's segments (polls)
+};
+hipError_t launch_mid_k(int nl, bool capped, unsigned grid, int flags, const MkArgs& m, hipStream_t st);
 
 hipError_t launch_lookup_draft(int n_streams, const int32_t* hist, const int64_t* hist_off, const int32_t* kmax,
                                const int32_t* min_n, int eos, int32_t* draft, int draft_ld, int32_t* ndraft,

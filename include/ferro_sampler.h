@@ -41,7 +41,8 @@ extern "C" {
                                         segments (workgroups not dispatched round-robin over the XCDs by index, or
                                         a wait limit below the segments' time). The row was then computed alone from
                                         its logits (the token is exact). The next sampling call on the context (or
-                                        fs_device_error) clears the workspace; that call returns FS_W_RECOVERED */
+                                        fs_device_error) clears the workspace; that call returns FS_W_RECOVERED (the mid-k
+                                        kernel's rows leave nothing to clear) */
 #define FS_DEVERR_HIST_APPEND 4      /* fs_hist_append: the new histories exceed out_cap (ids past it are not
                                         written), or a count lies outside [0, its stream's rows] (clamped) */
 
@@ -92,9 +93,11 @@ int fs_sample_batch(fs_context* ctx, const float* d_logits, int64_t ld, int32_t 
  * greedy (frequency / presence penalties only where rows split into segments of 4096 logits) or samples from at
  * most 64 candidates (k = top_k, or V when top_k is 0) with no frequency / presence penalty run on a kernel made for
  * them (every segment's loads issued at once, bitonic sorts in registers; all-greedy batches a greedy-only form);
- * batches mixing rows of 64 < k <= 2048 with cheaper rows run fs_sample_batch's kernel with about twice its segments;
- * other batches, and h_params = NULL, run fs_sample_batch. fs_route_plan reports the choice. Same outputs as
- * fs_sample_batch. h_params is read before the call returns. */
+ * other batches whose every row is greedy or samples from at most 2048 candidates, with any penalty, run on the mid-k
+ * kernel (fs_mid_k_plan); of the rest, batches mixing rows of 64 < k <= 2048 with cheaper rows run fs_sample_batch's
+ * kernel with about twice its segments; other batches, and h_params = NULL, run fs_sample_batch. fs_route_plan reports
+ * the choice between the small-k kernel and the others. Same outputs as fs_sample_batch. h_params is read before the
+ * call returns. Under HIP graph capture a batch whose mid-k workspace would have to grow runs fs_sample_batch's kernel. */
 int fs_sample_batch_hp(fs_context* ctx, const float* d_logits, int64_t ld, int32_t B, int32_t V,
                        const int32_t* d_hist, const int64_t* d_hist_off, const fs_row_params* d_params,
                        const fs_row_params* h_params, const double* d_u, int32_t* d_tok, int32_t kcap,
@@ -107,11 +110,18 @@ int fs_small_k_plan(int32_t cus, int32_t B, int32_t V, int32_t* nl, int32_t* nse
 
 /* Host-only: the kernel fs_sample_batch_hp (verify = 0: n = total_rows = B row records) or fs_verify_hp (verify != 0:
  * n stream records over total_rows rows) launches for these host parameters, on a device with `cus` compute units
- * whose XCD count divides 8: *kernel 0 the fused kernel (*nseg segments per row, *per_cu segments per CU of its
- * layout), 1 the small-k kernel, 2 its greedy-only form (*nl float4 loads per thread, *nseg segments per row). No
+ * whose XCD count divides 8: *kernel 0 the mid-k kernel where fs_mid_k_plan gives it a layout, else the fused kernel
+ * (*nseg segments per row, *per_cu segments per CU of the fused kernel's layout), 1 the small-k kernel, 2 its greedy-only form (*nl float4 loads per thread, *nseg segments per row). No
  * counterpart in the reference (a routing check for callers and tests). */
 int fs_route_plan(int32_t cus, const fs_row_params* h_params, int32_t n, int32_t total_rows, int32_t V,
                   int32_t verify, int32_t* kernel, int32_t* nl, int32_t* nseg, int32_t* per_cu);
+
+/* Host-only: the mid-k kernel's layout for a batch the small-k kernel does not take (arguments as fs_route_plan's): *nl
+ * float4 loads per thread (segments of 1024 * nl logits) and *nseg segments per row; FS_E_LIMIT, and zeros, when the
+ * batch does not fit it (a row of more than 2048 candidates, more than 262144 logits per row, or too few logits for the
+ * largest k). No counterpart in the reference (a planner check). */
+int fs_mid_k_plan(int32_t cus, const fs_row_params* h_params, int32_t n, int32_t total_rows, int32_t V, int32_t* nl,
+                  int32_t* nseg);
 
 /* fs_sample_batch without any allocation. No counterpart in the reference: it is for callers that cannot allocate
  * device memory during a call - code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.
@@ -150,7 +160,9 @@ int fs_verify(fs_context* ctx, const float* d_logits, int64_t ld, int32_t n_stre
 /* fs_verify with the stream parameters also in host memory (h_params: the same n_streams records as d_params). Windows
  * whose every stream is greedy or samples from at most 64 candidates, with no active penalty (repetition 1, or
  * repeat_last_n 0, and no frequency / presence penalty: a row's history then does not matter), run on the small-k
- * kernel of fs_sample_batch_hp; other windows, and h_params = NULL, run fs_verify. Same outputs as fs_verify. */
+ * kernel of fs_sample_batch_hp; other windows whose every stream is greedy or samples from at most 2048 candidates run on
+ * its mid-k kernel (each row's window is the stream's history and the drafts fed before it); the rest, and h_params =
+ * NULL, run fs_verify. Same outputs as fs_verify. */
 int fs_verify_hp(fs_context* ctx, const float* d_logits, int64_t ld, int32_t n_streams, int32_t total_rows,
                  int32_t V, const int32_t* d_rows, const int64_t* d_row_off, const int32_t* d_hist,
                  const int64_t* d_hist_off, const fs_row_params* d_params, const fs_row_params* h_params,
@@ -221,7 +233,7 @@ int fs_decode_step(fs_context* ctx, fs_drng* r, const float* d_logits, int64_t l
                    int32_t* d_keep, int32_t* d_out_hist, int64_t* d_out_hist_off, int64_t out_cap, void* stream);
 
 /* fs_decode_step with a host copy of the parameters too (h_params: B records, as fs_sample_batch_hp): batches the
- * small-k kernel fits run on it, with the same three additions in each row's merge; others run fs_decode_step.
+ * small-k or the mid-k kernel fits run on it, with the same three additions; others run fs_decode_step.
  * Same outputs and stream semantics. No counterpart call in the reference (the server holds its SamplerParams on
  * the host, server.cpp:603-606). */
 int fs_decode_step_hp(fs_context* ctx, fs_drng* r, const float* d_logits, int64_t ld, int32_t B, int32_t V,

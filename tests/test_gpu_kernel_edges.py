@@ -123,3 +123,126 @@ def test_softcap_where_it_saturates(cap, scale):
     p["repetition_penalty"][4] = 0.8
     p["repetition_penalty"][5] = 1.0
     check(x, p, [list(W.zipf_ids(rng, V, 900)) for _ in range(6)], rng.random(6))
+
+
+def mid_params(B, k, **kw):
+    p = W.make_params(B, temperature=0.9, top_k=k, top_p=0.97, repetition_penalty=1.0)
+    for f, v in kw.items():
+        p[f] = v
+    return p
+
+
+@pytest.mark.parametrize("B,V,k", [(1, 4096, 65), (3, 33000, 1000), (2, 65537, 2048), (9, 100003, 66), (2, 262144, 2048),
+                                   (70, 65536, 300), (33, 262144, 257)])
+def test_mid_k_rows(B, V, k):
+    """k past the small-k kernel's 64 on every segment size: heavy tails, bf16 values (ties at the k-th), every top
+    logit in one segment, a masked vocabulary (fewer finite logits than k), an all-equal row, a row without a number."""
+    rng = np.random.default_rng(V + k)
+    x = W.mixture_logits(rng, B, V)
+    if B > 1:
+        x[1] = bf16_valued(x[1])
+        x[B - 1, V // 3:V // 3 + 900] += 40.0
+    if B > 2:
+        m = np.full(V, -np.inf, np.float32)
+        at = rng.choice(V, min(50, k // 2), replace=False)
+        m[at] = x[2, at]
+        x[2] = m
+    if B > 8:
+        x[3, :] = 2.5
+        x[4, :] = np.nan
+        x[5, rng.choice(V, V // 2, replace=False)] = np.nan
+        x[6, 7] = np.inf
+        x[7] = np.round(x[7])                        # thousands of equal logits at the bound
+    check(x, mid_params(B, k), [[]] * B, rng.random(B), kcap=2048)
+
+
+@pytest.mark.parametrize("V,B,H", [(100003, 6, 3000), (262144, 66, 2500), (70000, 4, 1), (70000, 4, 1025), (262144, 65, 9)])
+def test_mid_k_penalties(V, B, H):
+    """Every penalty mix, raising ones too; windows past the prefetched ids and histories whose distinct ids of one
+    segment leave LDS for the spill list; every fourth row greedy, every fifth capped."""
+    rng = np.random.default_rng(V + H)
+    x = W.mixture_logits(rng, B, V)
+    p = mid_params(B, 200, repetition_penalty=rng.choice([0.7, 1.0, 1.3], B), frequency_penalty=rng.choice([-0.2, 0.0, 0.3], B),
+                   presence_penalty=rng.choice([0.0, 0.4], B))
+    p["frequency_penalty"][0] = 0.1                  # at least one row past the small-k kernel
+    p["temperature"][3::4] = 0.0
+    p["softcap"][4::5] = 30.0
+    p["repeat_last_n"][2::7] = max(1, H // 2)
+    hists = [list(W.zipf_ids(rng, V, H)) if b % 3 else list(rng.integers(0, V, H)) for b in range(B)]
+    hists[1] = list(rng.permutation(16384)[:H]) if H <= 16384 else hists[1]     # one segment's ids alone
+    check(x, p, hists, rng.random(B), kcap=256)
+
+
+def test_mid_k_more_penalised_ids_than_the_spill_list():
+    rng = np.random.default_rng(5)
+    V, H = 262144, 40000
+    x = W.mixture_logits(rng, 2, V)
+    p = mid_params(2, 100, frequency_penalty=0.3, repetition_penalty=1.1)
+    p["temperature"][1] = 0.0
+    check(x, p, [list(rng.permutation(V)[:H]) for _ in range(2)], rng.random(2), kcap=100)
+
+
+@pytest.mark.parametrize("M,S,V", [(5, 8, 262144), (17, 3, 65537), (40, 2, 40000), (600, 1, 6000)])
+def test_verify_windows_with_penalties(M, S, V):
+    """Windows whose rows see their stream's history and the drafts fed before them, of equal and of ragged lengths."""
+    rng = np.random.default_rng(M)
+    for ragged in (False, True):
+        m = np.full(S, M) if not ragged else np.maximum(1, M - np.arange(S) * 2 - 1)
+        off = np.concatenate([[0], np.cumsum(m)]).astype(np.int64)
+        R = int(off[-1])
+        x = W.mixture_logits(rng, R, V)
+        rows = x.argmax(axis=1).astype(np.int32)
+        rows = np.where(rng.random(R) < 0.8, np.roll(rows, 1), rng.integers(0, V, R)).astype(np.int32)
+        p = mid_params(S, 50, temperature=0.05, repetition_penalty=1.3)
+        p["frequency_penalty"][::2] = 0.2
+        p["repeat_last_n"][-1] = M // 2 + 1
+        hist, hoff = csr([list(rng.integers(0, V, 5 + 7 * s)) for s in range(S)])
+        u = rng.random(R)
+        tok, acc = F.verify(torch.from_numpy(x).cuda(), rows, off, p, u=u, hist=hist, hist_off=hoff, eos_id=3)
+        otok, oacc = O.verify(x, rows, off, hist, hoff, p, u, eos_id=3)
+        np.testing.assert_array_equal(tok.cpu().numpy(), otok)
+        np.testing.assert_array_equal(acc.cpu().numpy(), oacc)
+        assert F.device_error() == 0
+
+
+def test_mid_k_give_up_is_exact():
+    """Segments that do not wait for each other: every sampled row is selected by its last segment alone, the tokens
+    are the same and the give-up is reported; the next call finds clean counters."""
+    from ferro_amd._lib import FS_DEVERR_INTERNAL, FS_WAIT_GIVE_UP
+    rng = np.random.default_rng(9)
+    B, V = 5, 65537
+    x = W.mixture_logits(rng, B, V)
+    p = mid_params(B, 300, repetition_penalty=1.2)
+    p["frequency_penalty"][1] = 0.2
+    p["temperature"][2] = 0.0
+    hists = [list(W.zipf_ids(rng, V, 700)) for _ in range(B)]
+    hist, off = csr(hists)
+    u = rng.random(B)
+    o = O.sample_batch(x, hist, off, p, u, kcap=300, nthreads=NT)
+    ctx = F.sampler.Context()
+    for limit, bits in ((FS_WAIT_GIVE_UP, FS_DEVERR_INTERNAL), (0, 0)):
+        ctx.set_wait_limit(limit)
+        out = F.sample_batch(torch.from_numpy(x).cuda(), p, u, hist=hist, hist_off=off, kcap=300, ctx=ctx)
+        torch.cuda.synchronize()
+        g = {k: v.cpu().numpy() for k, v in out.items() if v is not None and not k.startswith("_")}
+        compare(g, o, p, u, 300)
+        assert F.device_error(ctx) == bits
+
+
+def test_mid_k_decode_steps():
+    """Decode steps the mid-k kernel takes: history copies, draws and appends beside k > 64 and frequency penalties."""
+    rng = np.random.default_rng(12)
+    S, V = 6, 100004
+    p = mid_params(S, 150, repetition_penalty=1.1, frequency_penalty=0.2)
+    p["temperature"][1] = 0.0
+    hist0 = [list(W.zipf_ids(rng, V, 300 * s)) for s in range(S)]
+    rows = [W.mixture_logits(rng, S, V) for _ in range(4)]
+    seeds = list(range(1, S + 1))
+    want, want_hist, want_off = oracle_decode_loop(rows, p, seeds, hist0)
+    d = F.DeviceRng(np.asarray(seeds, np.uint64))
+    hist, off = (torch.from_numpy(a).cuda() for a in csr(hist0))
+    for k, x in enumerate(rows):
+        tok, _, hist, off = F.decode_step(torch.from_numpy(x).cuda(), p, d, hist=hist, hist_off=off)
+        np.testing.assert_array_equal(tok.cpu().numpy(), want[k])
+    np.testing.assert_array_equal(off.cpu().numpy(), want_off)
+    np.testing.assert_array_equal(hist[:int(off[-1])].cpu().numpy(), want_hist)
