@@ -1,5 +1,5 @@
-// mid_k_kernel.hip - the kernel of batches that mix rows: greedy rows and rows that sample from k <= 2048 candidates,
-// with every penalty, and verification windows with penalties.
+// mid_k_kernel.hip - the kernel of batches that mix rows: greedy rows, rows that sample from k <= 2048 candidates and rows
+// with every token a candidate (top_k = 0), with every penalty, and verification windows with penalties.
 //
 // One workgroup of SK_LT threads per (row, segment), the segment's logits requested at once and kept in registers, as in
 // the small-k kernel. A row's segments agree on one bound before any of them writes a candidate:
@@ -19,6 +19,9 @@
 // Measured against the fused kernel (running bounds, per-row merges of the segments' lists): 256 rows of 262144 logits
 // with k from 1 to 2048 and every penalty 124 us -> 79; 24 rows of 100003 logits, k 200, frequency / presence 35 -> 19.4;
 // 40 rows of a verification window over 262144 logits, k 50, repetition 26.5 -> 24.3.
+// Rows with every token a candidate (ak_segment, ak_finish) stay in registers through all their passes; the fused kernel
+// reads such a row again for each, and gave flat ones to one workgroup: 32 rows of 65536 N(0, 2) logits at temperature 1
+// 51.4 us -> 23.0, 3 rows of 178740 507 -> 21, 64 rows of 262144 heavy-tailed logits with top-p 0.95 37.5 -> 35.1.
 #include "row_device.hpp"
 
 #include <type_traits>
@@ -38,6 +41,12 @@ __device__ __forceinline__ uint32_t mk_rank(int j) {
     return (uint32_t)((j < 8 ? MK_RANK_LO >> (8 * j) : MK_RANK_HI >> (8 * (j - 8))) & 0xFFu);
 }
 
+constexpr int AK_BINS = 2048;              // every token a candidate: mass bins of a row
+constexpr int AK_STAGE = 1024;             // logits of the searched bins that a segment stages, per list
+constexpr int AK_LIST = MK_LCAP / 2;       // entries of a row's two lists of such logits
+constexpr float AK_DEPTH = 32.0f;          // temperatures below the maximum that the bins reach
+constexpr double AK_FX = 17592186044416.0; // 2^44: fixed-point mass scale (a mass is <= 1)
+
 struct MkShared {
     // in turn: the window's 16-bit counts per logit of the segment (frequency / presence); the merge's sorted candidates
     // and its bins
@@ -51,6 +60,14 @@ struct MkShared {
             uint64_t top[MK_K];            // (u.m.top's head)
             double e[MK_K];                // their masses, then probabilities
         } w;
+        uint64_t mass[AK_BINS];            // every token a candidate: fixed-point masses by bin
+        struct {
+            uint64_t l[2][AK_STAGE];       //   this segment's logits of the bins searched, ~id above the value
+        } g;
+        struct {
+            uint32_t cnt[SK_LT * 8 * 4 / 2];   // ak_slow: a chunk's counts beside a digit's masses
+            uint64_t mass[MK_H];
+        } z;
     } u;
     union {
         uint32_t hist[MK_H];               // the bound's histograms; mk_slow's digits
@@ -68,6 +85,9 @@ struct MkShared {
     uint32_t w32[SK_NW];
     uint32_t misc[6];
     double dmisc;
+    uint64_t umisc[2];
+    uint32_t gn[4];
+    double pow2[64];                       // every token a candidate: 2^(j/64)
 #ifdef FS_TRACE
     uint64_t trace_t[16];
 #endif
@@ -451,6 +471,606 @@ __device__ __forceinline__ void mk_softmax(const SkArgs& a, const fs_row_params&
     }
 }
 
+// ---- every token a candidate (top_k = 0: k = V)
+// 2^(j/64), correctly rounded.
+__constant__ double ak_pow2[64] = {
+    0x1.0000000000000p+0, 0x1.02c9a3e778061p+0, 0x1.059b0d3158574p+0, 0x1.0874518759bc8p+0,
+    0x1.0b5586cf9890fp+0, 0x1.0e3ec32d3d1a2p+0, 0x1.11301d0125b51p+0, 0x1.1429aaea92de0p+0,
+    0x1.172b83c7d517bp+0, 0x1.1a35beb6fcb75p+0, 0x1.1d4873168b9aap+0, 0x1.2063b88628cd6p+0,
+    0x1.2387a6e756238p+0, 0x1.26b4565e27cddp+0, 0x1.29e9df51fdee1p+0, 0x1.2d285a6e4030bp+0,
+    0x1.306fe0a31b715p+0, 0x1.33c08b26416ffp+0, 0x1.371a7373aa9cbp+0, 0x1.3a7db34e59ff7p+0,
+    0x1.3dea64c123422p+0, 0x1.4160a21f72e2ap+0, 0x1.44e086061892dp+0, 0x1.486a2b5c13cd0p+0,
+    0x1.4bfdad5362a27p+0, 0x1.4f9b2769d2ca7p+0, 0x1.5342b569d4f82p+0, 0x1.56f4736b527dap+0,
+    0x1.5ab07dd485429p+0, 0x1.5e76f15ad2148p+0, 0x1.6247eb03a5585p+0, 0x1.6623882552225p+0,
+    0x1.6a09e667f3bcdp+0, 0x1.6dfb23c651a2fp+0, 0x1.71f75e8ec5f74p+0, 0x1.75feb564267c9p+0,
+    0x1.7a11473eb0187p+0, 0x1.7e2f336cf4e62p+0, 0x1.82589994cce13p+0, 0x1.868d99b4492edp+0,
+    0x1.8ace5422aa0dbp+0, 0x1.8f1ae99157736p+0, 0x1.93737b0cdc5e5p+0, 0x1.97d829fde4e50p+0,
+    0x1.9c49182a3f090p+0, 0x1.a0c667b5de565p+0, 0x1.a5503b23e255dp+0, 0x1.a9e6b5579fdbfp+0,
+    0x1.ae89f995ad3adp+0, 0x1.b33a2b84f15fbp+0, 0x1.b7f76f2fb5e47p+0, 0x1.bcc1e904bc1d2p+0,
+    0x1.c199bdd85529cp+0, 0x1.c67f12e57d14bp+0, 0x1.cb720dcef9069p+0, 0x1.d072d4a07897cp+0,
+    0x1.d5818dcfba487p+0, 0x1.da9e603db3285p+0, 0x1.dfc97337b9b5fp+0, 0x1.e502ee78b3ff6p+0,
+    0x1.ea4afa2a490dap+0, 0x1.efa1bee615a27p+0, 0x1.f50765b6e4540p+0, 0x1.fa7c1819e90d8p+0};
+// exp(z), -40 < z <= 0, within 2.3e-16 (Tang's table method: z = n ln2/64 + r, the degree-5 polynomial of e^r - 1 on
+// |r| < ln2/128, the table's 2^(j/64)); the ocml function takes twice the instructions. pow2: the table in LDS.
+__device__ __forceinline__ double ak_exp(double z, const double* pow2) {
+    const double n = __builtin_rint(z * 0x1.71547652b82fep+6);
+    const int i = (int)n;
+    double r = __builtin_fma(-n, 0x1.62e42fee00000p-7, z);
+    r = __builtin_fma(-n, 0x1.a39ef35793c76p-39, r);
+    double q = __builtin_fma(r, 1.0 / 120.0, 1.0 / 24.0);
+    q = __builtin_fma(r, q, 1.0 / 6.0);
+    q = __builtin_fma(r, q, 0.5);
+    q = __builtin_fma(r * r, q, r);
+    const double t = pow2[i & 63];
+    return __builtin_ldexp(__builtin_fma(t, q, t), i >> 6);
+}
+__device__ __forceinline__ double ak_mass(float x, float mx, double Td) { return exp((double)(x - mx) / Td); }
+
+// A row's segments meet: arrive, then wait (bounded) for `target` arrivals. What the caller published is drained first.
+// Whole workgroup; returns false when the row gave up.
+__device__ __forceinline__ bool mk_meet(uint32_t* ctr, uint32_t target, uint32_t spins_max, MkShared& s) {
+    vm_drain();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        uint32_t ok = 1u, spins = 0u;
+        for (;;) {
+            const uint32_t c = __hip_atomic_fetch_add(ctr, 0x10000u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if ((c & 0xFFFFu) >= target && spins_max != 0u) break;
+            if (++spins >= spins_max) { ok = 0u; break; }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        s.misc[5] = ok;
+        if (!ok) __hip_atomic_fetch_or(ctr + 34, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __syncthreads();
+    return s.misc[5] != 0u;
+}
+
+// The bin that holds the target-th unit of the row's mass, and the mass before it: cum (LDS) holds the mass up to and
+// with bins 8t .. 8t + 7, rm the bins. Each wave finds it by itself, the same in all (no barrier); false when the row's
+// mass does not reach the target.
+__device__ __forceinline__ bool ak_locate(const uint64_t* cum, const uint64_t* rm, uint64_t target, int& bin,
+                                          uint64_t& before) {
+    const int lane = lane_id();
+    if (target == 0ull) target = 1ull;
+    const uint64_t m4 = __ballot(cum[4 * lane + 3] >= target);
+    if (m4 == 0ull) return false;
+    const int g4 = 4 * (__ffsll((unsigned long long)m4) - 1);  // four groups of eight bins
+    const uint64_t m1 = __ballot(lane < 4 && cum[g4 + (lane & 3)] >= target);
+    const int g = g4 + __ffsll((unsigned long long)m1) - 1;
+    const uint64_t at = g > 0 ? cum[g - 1] : 0ull;
+    uint64_t h = lane < 8 ? rm[8 * g + lane] : 0ull, inc = h;
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+        const uint64_t y = __shfl_up(inc, o);
+        if (lane >= o) inc += y;
+    }
+    const int j = __ffsll((unsigned long long)__ballot(lane < 8 && at + inc >= target)) - 1;
+    bin = 8 * g + j;
+    before = at + read_lane(inc, j) - read_lane(h, j);
+    return true;
+}
+
+// The first of the n sorted candidates in s.u.w.top at which above + the masses so far reach the target, -1 when they do
+// not; *cum: the sum there. Whole workgroup.
+__device__ __forceinline__ int ak_walk(int n, double above, double target, float mx, double Td, MkShared& s, double& cum) {
+    const int tid = threadIdx.x, per = (n + SK_LT - 1) / SK_LT, i0 = tid * per, i1 = i0 + per < n ? i0 + per : n;
+    double* E = s.u.w.e;
+#pragma unroll 1
+    for (int i = tid; i < n; i += SK_LT) E[i] = ak_mass(val_of(comp_key(s.u.w.top[i])), mx, Td);
+    __syncthreads();
+    double run = 0.0, all;
+#pragma unroll 1
+    for (int i = i0; i < i1; ++i) run += E[i];
+    const double off = mk_excl_f64(run, s, all) + above;
+    uint64_t first = ~0ull;
+    double at = 0.0;
+    run = 0.0;
+#pragma unroll 1
+    for (int i = i0; i < i1; ++i) {
+        run += E[i];
+        if (first == ~0ull && run + off >= target) { first = (uint64_t)i; at = run + off; }
+    }
+    const uint64_t hit = mk_min_u64(first, s);
+    if (first == hit && first != ~0ull) s.dmisc = at;
+    __syncthreads();
+    cum = s.dmisc;
+    __syncthreads();
+    return hit == ~0ull ? -1 : (int)hit;
+}
+
+// A row with every token a candidate from its logits alone, by one workgroup: extremes and the mass total in one pass,
+// then for top-p's crossing and for the draw a radix select by mass over the composites, ten bits at a time. Exact, and
+// slow (about 20 passes): rows whose mass no single bin narrows down (all logits equal), infinite maxima, give-ups.
+template <bool CAP>
+__device__ __forceinline__ void ak_slow(const float* rowp, int V, bool pen, const MkWin& win, const MkPen& pn,
+                                        const fs_row_params& p, double u, MkShared& s, int& tok, int& keep) {
+    constexpr int CH = SK_LT * 8 * 4;                          // logits per chunk
+    const int tid = threadIdx.x;
+    const double Td = (double)p.temperature;
+    float mx = 0.0f;
+    double S = 0.0, target = 0.0, cum = 0.0, top_cum = 0.0;
+    uint64_t cmax = 0ull, cmin = ~0ull, nv = 0ull, prefix = 0ull, mask = 0ull, before = 0ull, xc = 0ull;
+    int phase = 0, sh = 54;                                    // 0 extremes, 1 total, 2 top-p's select, 3 its count, 4 the draw's
+    tok = 0;
+    keep = 0;
+#pragma unroll 1
+    for (;;) {
+        const int sft = sh < 0 ? 0 : sh;
+        const uint64_t dm = sh < 0 ? 0x3FFull >> -sh : 0x3FFull;
+        __syncthreads();
+        for (int i = tid; i < MK_H; i += SK_LT) s.u.z.mass[i] = 0ull;
+        __syncthreads();
+        uint64_t mxc = 0ull, mnc = ~0ull, n_ = 0ull;
+        double part = 0.0;
+#pragma unroll 1
+        for (int lo = 0; lo < V; lo += CH) {
+            const int n = V - lo < CH ? V - lo : CH;
+            if (pen) {
+                __syncthreads();
+                for (int i = tid; i < CH / 32; i += SK_LT) s.b.bmp[i] = 0u;
+                if (pn.fp_on)
+                    for (int i = tid; i < CH / 2; i += SK_LT) s.u.z.cnt[i] = 0u;
+                __syncthreads();
+#pragma unroll 1
+                for (int64_t i = tid; i < win.n(); i += SK_LT) {
+                    const uint32_t rel = (uint32_t)win.at(i) - (uint32_t)lo;
+                    if (rel < (uint32_t)n) {
+                        atomicOr(&s.b.bmp[rel >> 5], 1u << (rel & 31u));
+                        if (pn.fp_on) atomicAdd(&s.u.z.cnt[rel >> 1], 1u << ((rel & 1u) * 16u));
+                    }
+                }
+                __syncthreads();
+            }
+#pragma unroll 1
+            for (int i = tid; i < n; i += SK_LT) {
+                float l = rowp[lo + i];
+                if (CAP && pn.cap > 0.0f) l = softcap_one(l, pn.cap);
+                if (pen && ((s.b.bmp[i >> 5] >> (i & 31)) & 1u))
+                    l = pn.apply(l, pn.fp_on ? (s.u.z.cnt[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu : 0u);
+                const uint32_t key = key_of(l);
+                if (key == 0u) continue;
+                const uint64_t c = comp_of(key, (uint32_t)(lo + i));
+                if (phase == 0) {
+                    mxc = c > mxc ? c : mxc;
+                    mnc = c < mnc ? c : mnc;
+                    ++n_;
+                } else if (phase == 3) {
+                    n_ += c >= xc ? 1ull : 0ull;
+                } else {
+                    const double m = ak_mass(l, mx, Td);
+                    if (phase == 1) part += m;
+                    else if ((c & mask) == prefix)
+                        atomicAdd(reinterpret_cast<unsigned long long*>(&s.u.z.mass[(uint32_t)(c >> sft) & (uint32_t)dm]),
+                                  (unsigned long long)(m * AK_FX + 0.5));
+                }
+            }
+        }
+        __syncthreads();
+        if (phase == 0) {
+            cmax = mk_max_u64(mxc, s);
+            cmin = mk_min_u64(mnc, s);
+            nv = mk_reduce_u64(n_, s, [](uint64_t x, uint64_t y) { return x + y; });
+            if (nv == 0ull) return;                            // no number in the row: token 0, nothing kept
+            mx = val_of(comp_key(cmax));
+            keep = (int)nv;
+            phase = 1;
+            continue;
+        }
+        if (phase == 1) {
+            (void)mk_excl_f64(part, s, S);
+            if (S != S) {                                      // an infinite maximum: nothing is cut, and the draw falls
+                tok = (int)comp_id(cmin);                      // through to the last candidate (sampler.cpp:43-49)
+                return;
+            }
+            cum = S;
+            phase = p.top_p < 1.0f ? 2 : 4;
+            target = phase == 2 ? (double)p.top_p * S : u * S;
+            continue;
+        }
+        if (phase == 3) {
+            keep = (int)mk_reduce_u64(n_, s, [](uint64_t x, uint64_t y) { return x + y; });
+            phase = 4;
+            target = u * top_cum;
+            prefix = mask = before = 0ull;
+            sh = 54;
+            continue;
+        }
+        // the digit's bin, from the top: thread t sums bins 1023 - 4t .. 1020 - 4t
+        uint64_t h[4], mine = 0ull;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            h[j] = s.u.z.mass[MK_H - 1 - 4 * tid - j];
+            mine += h[j];
+        }
+        uint64_t inc = mine;
+#pragma unroll
+        for (int o = 1; o < WAVE; o <<= 1) {
+            const uint64_t y = __shfl_up(inc, o);
+            if (lane_id() >= o) inc += y;
+        }
+        if (lane_id() == WAVE - 1) s.w64[tid / WAVE] = inc;
+        __syncthreads();
+        uint64_t ex = before + inc - mine;
+#pragma unroll
+        for (int w = 0; w < SK_NW; ++w) ex += w < tid / WAVE ? s.w64[w] : 0ull;
+        uint64_t want = (uint64_t)(target * AK_FX);
+        want = want ? want : 1ull;
+        if (tid == 0) s.umisc[0] = ~0ull;
+        __syncthreads();
+        if (ex < want && ex + mine >= want) {
+            uint64_t b = ex;
+            int at = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (b + h[j] < want && at == j) { b += h[j]; at = j + 1; }
+            s.umisc[0] = (uint64_t)(MK_H - 1 - 4 * tid - at);
+            s.umisc[1] = b;
+        }
+        __syncthreads();
+        const bool none = s.umisc[0] == ~0ull;                 // past the last candidate (the sums' rounding)
+        if (!none) {
+            prefix |= s.umisc[0] << sft;
+            mask |= dm << sft;
+            before = s.umisc[1];
+            sh -= 10;
+            if (sh > -10) continue;
+        }
+        const uint64_t c = none ? (phase == 2 || xc == 0ull ? cmin : xc) : prefix;
+        if (phase == 2) {
+            xc = c;
+            top_cum = none ? cum : (double)before / AK_FX + ak_mass(val_of(comp_key(c)), mx, Td);
+            phase = 3;
+            continue;
+        }
+        tok = (int)comp_id(xc != 0ull && c < xc ? xc : c);
+        return;
+    }
+}
+
+// What a row's segments agree on: the maximum, the mass total S, the draw; top-p's crossing bin bc with the mass above it
+// (cut), the bins d0 .. d1 that hold the draw; plain: nothing to search (no number, an infinite maximum, all logits equal).
+struct AkRow {
+    float mx;
+    uint32_t nv;
+    double S, u, above_c, above_d;
+    int bc, d0, d1;
+    bool cut, plain;
+};
+// One segment of such a row: extremes, meet, masses into the row's 2048 bins (linear in the logit from the row's maximum
+// down to its minimum, or 32 temperatures below: about 500 logits in the fullest bin of a normal row of 262144 whatever
+// its width), meet, and the logits of the bins that top-p's crossing and the draw fall in to the row's lists. The logits
+// stay in registers throughout. Returns false when the row gave up.
+template <int NL, bool CAP, class P, class E>
+__device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, const fs_row_params& p, int row, int seg,
+                                           int nseg, int seg_lo, uint32_t* ctr, uint64_t* list, P penalise, E pen_at,
+                                           uint32_t nf, double u, AkRow& r, MkShared& s) {
+    const int tid = threadIdx.x, lane = lane_id(), w = tid / WAVE;
+    const double Td = (double)p.temperature, inv = 1.0 / Td;
+    const float invf = 1.0f / p.temperature;
+    r.u = u;
+    if (tid < 64) s.pow2[tid] = ak_pow2[tid];
+    penalise();
+    if (CAP && p.softcap > 0.0f) {
+#pragma unroll
+        for (int q = 0; q < NL; ++q) softcap_vals(v[q], p.softcap);
+    }
+    float hi = __builtin_nanf(""), lo = hi;                    // (fmaxf and fminf drop NaN)
+    uint32_t n = NL * 4;                                       // the lane's numbers
+    bool nans = false;
+#pragma unroll
+    for (int q = 0; q < NL; ++q) {
+        hi = fmaxf(hi, fmaxf(fmaxf(v[q][0], v[q][1]), fmaxf(v[q][2], v[q][3])));
+        lo = fminf(lo, fminf(fminf(v[q][0], v[q][1]), fminf(v[q][2], v[q][3])));
+        nans |= __builtin_isunordered(v[q][0], v[q][1]) || __builtin_isunordered(v[q][2], v[q][3]);
+    }
+    if (__ballot(nans) != 0ull) {
+        n = 0u;
+#pragma unroll
+        for (int q = 0; q < NL; ++q)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) n += v[q][c] == v[q][c] ? 1u : 0u;
+    }
+    for (uint32_t i = (uint32_t)lane; i < nf; i += WAVE) {
+        const float x = __uint_as_float((uint32_t)pen_at(i));
+        hi = fmaxf(hi, x);
+        lo = fminf(lo, x);
+        n += x == x ? 1u : 0u;
+    }
+    auto add_u = [](uint32_t x, uint32_t y) { return x + y; };
+    auto add_d = [](double x, double y) { return x + y; };
+    uint32_t kx = wave_max(key_of(hi)), kn = wave_min(lo == lo ? key_of(lo) : 0xFFFFFFFFu);
+    n = wave_allreduce(n, add_u);
+    if (lane == 0) {
+        s.w64[w] = ((uint64_t)kx << 32) | kn;
+        s.w32[w] = n;
+    }
+    __syncthreads();
+    // two 128-byte lines per segment, one per meeting (a line is read by others only after the meeting it is written for)
+    uint64_t* line = reinterpret_cast<uint64_t*>(mk.qk) + ((int64_t)row * nseg) * 32;
+    if (tid == 0) {
+#pragma unroll
+        for (int q = 1; q < SK_NW; ++q) {
+            const uint32_t a = (uint32_t)(s.w64[q] >> 32), b = (uint32_t)s.w64[q];
+            kx = a > kx ? a : kx;
+            kn = b < kn ? b : kn;
+            n += s.w32[q];
+        }
+        line[seg * 32] = ((uint64_t)kx << 32) | kn;
+        line[seg * 32 + 1] = n;
+    }
+    if (!mk_meet(ctr, (uint32_t)nseg, mk.spins, s)) return false;
+    SK_MARK(2);
+    {
+        const uint64_t e = lane < nseg ? line[lane * 32] : 0xFFFFFFFFull;
+        r.nv = wave_allreduce(lane < nseg ? (uint32_t)line[lane * 32 + 1] : 0u, add_u);
+        kx = wave_max((uint32_t)(e >> 32));
+        kn = wave_min((uint32_t)e);
+    }
+    const float mx = val_of(kx), mn = val_of(kn);
+    r.mx = mx;
+    float depth = (mx - mn) * invf;
+    const bool tail = !(depth < AK_DEPTH);
+    depth = tail ? AK_DEPTH : depth;
+    const float scale = (float)AK_BINS / (depth * p.temperature);
+    r.plain = r.nv == 0u || !(mx < __builtin_huge_valf()) || !(mx > -__builtin_huge_valf()) || !(mn < mx) || !(scale > 0.0f) ||
+              !(scale < __builtin_huge_valf());
+    if (r.plain) return true;                                  // uniform over the row
+    for (int i = tid; i < AK_BINS / 2; i += SK_LT) reinterpret_cast<ulonglong2*>(s.u.mass)[i] = make_ulonglong2(0ull, 0ull);
+    __syncthreads();
+    // a logit's place below the maximum, in bins, and its bin (AK_BINS: none), the same function of its value in both
+    // passes; it never falls as the logit falls (NaN: not a candidate)
+    auto place_of = [&](float x) { return (mx - x) * scale; };
+    auto bin_at = [&](float t) {
+        const int b = (int)fminf(t, (float)AK_BINS);
+        return t == t ? (tail ? b : (b < AK_BINS ? b : AK_BINS - 1)) : AK_BINS;
+    };
+    auto bin_of = [&](float x) { return bin_at(place_of(x)); };
+    // Sixteen logits of the segment at a time, taken from the registers by a uniform index: the bodies below are not
+    // repeated 64 times (unrolled, the kernel outgrew the instruction cache and its registers: 69 us on the nucleus rows)
+    // (by masks: the compiler turns selects between array elements into an array in memory)
+    auto pick16 = [&](float (&x)[4][4], int h) {
+        uint32_t m[NL / 4];
+#pragma unroll
+        for (int g = 0; g < NL / 4; ++g) m[g] = (uint32_t)__builtin_amdgcn_readfirstlane(h == g ? -1 : 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                uint32_t y = __float_as_uint(v[q][c]) & m[0];
+#pragma unroll
+                for (int g = 1; g < NL / 4; ++g) y |= __float_as_uint(v[4 * g + q][c]) & m[g];
+                x[q][c] = __uint_as_float(y);
+            }
+    };
+    // the groups of sixteen in which some lane of the wave has a logit at or above x
+    auto groups_above = [&](float x) {
+        uint32_t m = 0u;
+#pragma unroll
+        for (int h = 0; h < NL / 4; ++h) {
+            float g = __builtin_nanf("");
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                g = fmaxf(g, fmaxf(fmaxf(v[4 * h + q][0], v[4 * h + q][1]), fmaxf(v[4 * h + q][2], v[4 * h + q][3])));
+            m |= __ballot(g >= x) != 0ull ? 1u << h : 0u;
+        }
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
+    };
+    // the value `bins` bins below the maximum, a little lower (the place's roundings are below 1e-6 of it)
+    auto value_at = [&](float bins) { return mx - bins * 1.00001f / scale - fabsf(mx) * 1e-6f; };
+    double part = 0.0;
+    float rest = 0.0f;                                         // masses below e^-32 (see the fused kernel's large rows)
+    const float faint = (float)AK_BINS * (104.0f / AK_DEPTH);  // from here on expf is 0
+    auto add = [&](float x, int b) {
+        if (b < AK_BINS) {
+            const double d = (double)(x - mx);                 // fp32 subtraction, as ferro; then d / Td, correctly rounded
+            double z = d * inv;
+            z = __builtin_fma(__builtin_fma(-z, Td, d), inv, z);
+            const double m = ak_exp(z, s.pow2);
+            part += m;
+            const uint64_t f = (uint64_t)__double_as_longlong(__builtin_fma(m, AK_FX, 0x1p52)) - 0x4330000000000000ull;
+            atomicAdd(reinterpret_cast<unsigned long long*>(&s.u.mass[b]), (unsigned long long)f);
+        } else if (x == x) {
+            rest += __expf((x - mx) * invf);
+        }
+    };
+#pragma unroll 1
+    for (uint32_t todo = groups_above(value_at(faint)); todo != 0u; todo &= todo - 1u) {
+        const int h = __ffs((int)todo) - 1;
+        float x[4][4];
+        pick16(x, h);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float at[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) at[c] = place_of(x[q][c]);
+            const float first = fminf(fminf(at[0], at[1]), fminf(at[2], at[3]));
+            if (__ballot(first < (tail ? (float)AK_BINS : __builtin_huge_valf())) != 0ull) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) add(x[q][c], bin_at(at[c]));
+            } else if (__ballot(first < faint) != 0ull) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) rest += x[q][c] == x[q][c] ? __expf((x[q][c] - mx) * invf) : 0.0f;
+            }
+        }
+    }
+    for (uint32_t i = (uint32_t)lane; i < nf; i += WAVE) {
+        const float x = __uint_as_float((uint32_t)pen_at(i));
+        add(x, bin_of(x));
+    }
+    SK_MARK(3);
+    double sum;
+    (void)mk_excl_f64(part + (double)rest, s, sum);            // (its barriers complete the bins)
+    uint64_t* rm = mk.mass + (int64_t)row * AK_BINS;
+#pragma unroll
+    for (int j = 0; j < AK_BINS / SK_LT; ++j) {
+        const uint64_t h = s.u.mass[j * SK_LT + tid];
+        if (h != 0ull) __hip_atomic_fetch_add(rm + j * SK_LT + tid, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    if (tid == 0) line[seg * 32 + 16] = (uint64_t)__double_as_longlong(sum);
+    if (!mk_meet(ctr, 2u * (uint32_t)nseg, mk.spins, s)) return false;
+    SK_MARK(4);
+    r.S = wave_allreduce(lane < nseg ? __longlong_as_double((long long)line[lane * 32 + 16]) : 0.0, add_d);
+    {
+        uint64_t mine = 0ull;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const ulonglong2 x = reinterpret_cast<const ulonglong2*>(rm)[4 * tid + j];
+            mine += x.x + x.y;
+        }
+        uint64_t inc = mine;
+#pragma unroll
+        for (int o = 1; o < WAVE; o <<= 1) {
+            const uint64_t y = __shfl_up(inc, o);
+            if (lane >= o) inc += y;
+        }
+        if (lane == WAVE - 1) s.w64[w] = inc;
+        if (tid < 4) s.gn[tid] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < SK_NW; ++q) inc += q < w ? s.w64[q] : 0ull;
+        uint64_t* cum = s.u.mass;                              // (the segment's own bins are spent)
+        cum[tid] = inc;
+        __syncthreads();
+        uint64_t before = 0ull;
+        r.cut = p.top_p < 1.0f;
+        r.bc = -1;
+        bool ok = true;
+        if (r.cut) {
+            // top-p keeps through its crossing candidate (sampler.cpp:44), so the kept total lies in [tgt, tgt + the
+            // largest mass of bin bc]: the draw's bin at both ends
+            const double tgt = (double)p.top_p * r.S;
+            ok = ak_locate(cum, rm, (uint64_t)(tgt * AK_FX), r.bc, before);
+            r.above_c = (double)before / AK_FX;
+            const double most = ak_exp(-(double)(ok ? r.bc : 0) * (double)depth * (1.0 / AK_BINS), s.pow2) * (1.0 + 1e-4);
+            const double thi = tgt + most < r.S ? tgt + most : r.S;
+            if (ok) ok = ak_locate(cum, rm, (uint64_t)(u * tgt * (1.0 - 1e-12) * AK_FX), r.d0, before);
+            r.above_d = (double)before / AK_FX;
+            if (ok && !ak_locate(cum, rm, (uint64_t)(u * thi * (1.0 + 1e-12) * AK_FX), r.d1, before)) r.d1 = r.bc;
+            if (r.d1 > r.bc) r.d1 = r.bc;
+        } else {
+            ok = ak_locate(cum, rm, (uint64_t)(u * r.S * AK_FX), r.d0, before);
+            r.above_d = (double)before / AK_FX;
+            r.d1 = r.d0;
+        }
+        r.plain = !ok;                                         // past the binned mass: the row is selected alone
+        if (!ok) return true;
+        __syncthreads();                                       // every wave has read cum (the lists below take its place)
+    }
+    // the searched bins' logits, staged in LDS (the bins there are spent), then to the row's lists
+    uint32_t above = 0u;
+    auto stage = [&](float x, int b, uint32_t nid) {
+        if (b == r.bc) {
+            const uint32_t at = atomicAdd(&s.gn[0], 1u);
+            if (at < (uint32_t)AK_STAGE) s.u.g.l[0][at] = ((uint64_t)nid << 32) | __float_as_uint(x);
+        }
+        if (b >= r.d0 && b <= r.d1) {
+            const uint32_t at = atomicAdd(&s.gn[1], 1u);
+            if (at < (uint32_t)AK_STAGE) s.u.g.l[1][at] = ((uint64_t)nid << 32) | __float_as_uint(x);
+        }
+    };
+    const int deepest = r.bc > r.d1 ? r.bc : r.d1;
+#pragma unroll 1
+    for (uint32_t todo = groups_above(value_at((float)(deepest + 1))); todo != 0u; todo &= todo - 1u) {
+        const int h = __ffs((int)todo) - 1;
+        float x[4][4];
+        pick16(x, h);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            bool any = false;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int b = bin_of(x[q][c]);
+                above += b < r.bc ? 1u : 0u;
+                any |= b == r.bc || (b >= r.d0 && b <= r.d1);
+            }
+            if (__ballot(any) != 0ull) {
+                const uint32_t own = ~(uint32_t)(seg_lo + ((4 * h + q) * SK_LT + tid) * 4);
+#pragma unroll 1
+                for (int c = 0; c < 4; ++c) {
+                    const float y = c == 0 ? +x[q][0] : c == 1 ? +x[q][1] : c == 2 ? +x[q][2] : +x[q][3];
+                    stage(y, bin_of(y), own - (uint32_t)c);
+                }
+            }
+        }
+    }
+    for (uint32_t i = (uint32_t)lane; i < nf; i += WAVE) {
+        const uint64_t e = pen_at(i);
+        const float x = __uint_as_float((uint32_t)e);
+        const int b = bin_of(x);
+        above += b < r.bc ? 1u : 0u;
+        stage(x, b, (uint32_t)(e >> 32) | 0x80000000u);
+    }
+    above = wave_allreduce(above, add_u);
+    if (lane == 0 && above != 0u) atomicAdd(&s.gn[2], above);
+    __syncthreads();
+    const uint32_t n0 = s.gn[0], n1 = s.gn[1];
+    if (tid == 0) {
+        s.misc[0] = n0 ? __hip_atomic_fetch_add(ctr + 33, n0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
+        s.misc[1] = n1 ? __hip_atomic_fetch_add(ctr + 36, n1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
+        if (s.gn[2]) __hip_atomic_fetch_add(ctr + 37, s.gn[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (n0 > (uint32_t)AK_STAGE || n1 > (uint32_t)AK_STAGE)
+            __hip_atomic_fetch_or(ctr + 34, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __syncthreads();
+    const uint32_t b0 = s.misc[0], b1 = s.misc[1];
+    for (uint32_t i = (uint32_t)tid; i < n0 && i < (uint32_t)AK_STAGE; i += SK_LT)
+        if (b0 + i < (uint32_t)AK_LIST) list[b0 + i] = s.u.g.l[0][i];
+    for (uint32_t i = (uint32_t)tid; i < n1 && i < (uint32_t)AK_STAGE; i += SK_LT)
+        if (b1 + i < (uint32_t)AK_LIST) list[AK_LIST + b1 + i] = s.u.g.l[1][i];
+    return true;
+}
+
+// The row's end, by its last segment: top-p's crossing and the draw located exactly in their bins' sorted logits. Returns
+// false when a target lies outside its bin's exact masses (a rounding step at the edge).
+__device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uint32_t n1, uint32_t above, const AkRow& r,
+                                          const fs_row_params& p, MkShared& s, int& tok, int& keep) {
+    const int tid = threadIdx.x;
+    const double Td = (double)p.temperature;
+    uint64_t xc = 0ull;
+    double tot = r.S;
+    keep = (int)r.nv;
+#pragma unroll 1
+    for (int pass = r.cut ? 0 : 1; pass < 2; ++pass) {
+        const int n = (int)(pass == 0 ? n0 : n1);
+        if (n == 0) return false;
+        constexpr int EPT = AK_LIST / SK_LT;
+        auto entry = [&](int i) {
+            const uint64_t c = i < n ? ld_agent(&list[pass * AK_LIST + i]) : 0ull;
+            return c == 0ull ? 0ull : ((uint64_t)key_of(__uint_as_float((uint32_t)c)) << 32) | (c >> 32);
+        };
+        if (n <= SK_LT) {
+            uint64_t* cand = s.u.m.top + MK_TOP - SK_LT;
+            const uint64_t c = entry(tid);
+            __syncthreads();                                   // (the first pass's lists are spent)
+            cand[tid] = c;
+            __syncthreads();
+            sk_rank(cand, s.h.rk, n, [&](uint32_t rank, uint64_t e) { s.u.m.top[rank] = e; });
+            __syncthreads();
+        } else {
+            uint64_t e[EPT];
+#pragma unroll
+            for (int q = 0; q < EPT; ++q) e[q] = entry(q * SK_LT + tid);
+            __syncthreads();
+            if (!mk_sort(e, n, n, s)) return false;
+        }
+        double cum;
+        const double target = pass == 0 ? (double)p.top_p * r.S : r.u * tot + 0.0;
+        const int at = ak_walk(n, pass == 0 ? r.above_c : r.above_d, target, r.mx, Td, s, cum);
+        if (at < 0) return false;
+        const uint64_t c = s.u.w.top[at];
+        if (pass == 0) {
+            xc = c;
+            tot = cum;
+            keep = (int)above + at + 1;
+        } else {
+            tok = (int)comp_id(c < xc ? xc : c);
+        }
+    }
+    return true;
+}
+
 struct MkKernargs {
     const float* logits;
     int64_t ld;
@@ -464,7 +1084,8 @@ constexpr size_t MK_ARGS_OFF = offsetof(MkKernargs, m);
 
 // CAP: some row of the batch has a softcap. It never decreases, so the bound is taken over raw logits and the merge caps
 // the list (an entry whose value is final already, a penalised one, has its id word's top bit cleared).
-template <int NL, bool CAP>
+// ALL: some row samples with every token a candidate.
+template <int NL, bool CAP, bool ALL>
 __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, int64_t ld, int B, int V, int nseg,
                                                          int flags, const fs_row_params* params,
                                                          const int64_t* hist_off, const int32_t* hist, MkArgs m_) {
@@ -728,9 +1349,13 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
         return ((uint64_t)nid << 32) | (far ? (uint32_t)e : __float_as_uint(s.b.pv[pb + i]));
     };
     SK_MARK(1);
+    const bool every = ALL && k > MK_K;                        // every token a candidate
     float tr = 0.0f, tc = 0.0f;                                // the bound: raw, capped
     bool go = true;
-    if (!scan) {
+    AkRow ak = {};
+    if (ALL && every) {
+        go = ak_segment<NL, CAP>(v, mk, p, row, seg, nseg, seg_lo, ctr, list, penalise, pen_at, nf, sk_draw(a, row).u, ak, s);
+    } else if (!scan) {
         // the lane maxima, sorted in each wave, published at 16 ranks
         const uint32_t srt = sort64_desc_u32(key_of(lm));
         s.h.srt[w][lane] = srt;
@@ -798,7 +1423,7 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
         }
         best = mk_max_u64(best, s);
         if (tid == 0) list[seg] = best;
-    } else {
+    } else if (!every) {
         if (go) {
             // the logits at or above the bound to the row's list, the penalised ones against the capped bound
             uint32_t np = 0u;
@@ -897,6 +1522,20 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
             ctr[32] = 0u;
             ctr[35] = 0u;
         }
+    } else if (ALL && every) {
+        const uint32_t n0 = ld_agent(ctr + 33), n1 = ld_agent(ctr + 36), above = ld_agent(ctr + 37);
+        __syncthreads();
+        if (tid == 0) {                                        // every segment has met and counted: left at 0
+            ctr[0] = 0u;
+            for (int i = 32; i < 38; ++i) ctr[i] = 0u;
+            if (slow & 2u) atomicOr(a.err, FS_DEVERR_INTERNAL);
+        }
+        ulonglong2* rm = reinterpret_cast<ulonglong2*>(mk.mass + (int64_t)row * AK_BINS);
+        for (int i = tid; i < AK_BINS / 2; i += SK_LT) rm[i] = make_ulonglong2(0ull, 0ull);
+        if (slow != 0u || ak.plain || n0 > (uint32_t)AK_LIST || n1 > (uint32_t)AK_LIST ||
+            !ak_finish(list, n0, n1, above, ak, p, s, tok, keep))
+            ak_slow<CAP>(rowp, V, pen, win, pn, p, dr.u, s, tok, keep);
+        if (w != 0) return;
     } else {
         uint32_t C = ld_agent(ctr + 33);
         bool capped_list = capped;
@@ -1009,19 +1648,25 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
     SK_FLUSH();
 }
 
-hipError_t launch_mid_k(int nl, bool capped, unsigned grid, int flags, const MkArgs& m, hipStream_t st) {
+hipError_t launch_mid_k(int nl, bool capped, bool all, unsigned grid, int flags, const MkArgs& m, hipStream_t st) {
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(grid), dim3(SK_LT), 0, st, m.a.logits, m.a.ld, m.a.B, m.a.V, m.a.nseg, flags,
                            m.a.params, m.a.hist_off, m.a.hist, m);
     };
+    auto by_nl = [&](auto cap, auto every) {
+        constexpr bool C = decltype(cap)::value, A = decltype(every)::value;
+        if (nl == 16) go(mid_k_kernel<16, C, A>);
+        else if (nl == 8) go(mid_k_kernel<8, C, A>);
+        else go(mid_k_kernel<4, C, A>);
+    };
+    const std::true_type yes;
+    const std::false_type no;
     if (capped) {
-        if (nl == 16) go(mid_k_kernel<16, true>);
-        else if (nl == 8) go(mid_k_kernel<8, true>);
-        else go(mid_k_kernel<4, true>);
+        if (all) by_nl(yes, yes);
+        else by_nl(yes, no);
     } else {
-        if (nl == 16) go(mid_k_kernel<16, false>);
-        else if (nl == 8) go(mid_k_kernel<8, false>);
-        else go(mid_k_kernel<4, false>);
+        if (all) by_nl(no, yes);
+        else by_nl(no, no);
     }
     return hipGetLastError();
 }

@@ -139,6 +139,7 @@ struct fs_context {
     uint32_t* mk_ctr = nullptr;     // mid-k kernel: [mk_rows][MK_CTR] counters, left at 0
     uint64_t* mk_list = nullptr;    //   [mk_rows][MK_LIST] candidate lists
     uint64_t* mk_spill = nullptr;   //   [mk_rows][MK_SPILL] penalised logits
+    uint64_t* mk_mass = nullptr;    //   [mk_rows][2048] mass bins, left at 0
     size_t mk_rows = 0;
     uint32_t* mk_qk = nullptr;      //   [mk_segs][SK_NW][16] published lane maxima
     size_t mk_segs = 0;
@@ -515,15 +516,21 @@ int launch_small(fs_context* ctx, const fs::Args& a_in, const fs_row_params* h_p
 // segments publish at most 64 lists of 16 per 4 * nl loads, which the bound's search reads in one round.
 struct MidKChoice {
     int nl = 0, nseg = 0;
-    bool capped = false, may_pen = false;
+    bool capped = false, may_pen = false, all = false;
 };
-bool mid_k_choice(int cus, const fs_row_params* h, int64_t n, int64_t rows, int32_t V, MidKChoice& c) {
+bool mid_k_choice(int cus, const fs_row_params* h, int64_t n, int64_t rows, int32_t V, bool outputs, MidKChoice& c) {
     int64_t kmax = 1;
     for (int64_t b = 0; b < n; ++b) {
         const fs_row_params& p = h[b];
         const bool greedy = !(p.temperature > 0.0f && p.top_k != 1);
         const int64_t k = greedy ? 1 : ((p.top_k > 0 && p.top_k < V) ? p.top_k : V);
-        kmax = std::max(kmax, k);
+        if (k == V && k > fs::KMAX) {
+            // every token a candidate: no candidate outputs and no min-p (its count and sum over the kept logits)
+            if (outputs || p.min_p > 0.0f) return false;
+            c.all = true;
+        } else {
+            kmax = std::max(kmax, k);
+        }
         c.capped |= p.softcap > 0.0f;
         c.may_pen |= (p.repetition_penalty != 1.0f || p.frequency_penalty != 0.0f || p.presence_penalty != 0.0f) &&
                      p.repeat_last_n != 0;
@@ -555,11 +562,15 @@ int grow_mid(fs_context* c, size_t segs, size_t rows) {
         release(c, c->mk_ctr);
         release(c, c->mk_list);
         release(c, c->mk_spill);
+        release(c, c->mk_mass);
+        c->mk_mass = nullptr;
         c->mk_ctr = nullptr; c->mk_list = nullptr; c->mk_spill = nullptr; c->mk_rows = 0;
         if (hipMalloc(&c->mk_ctr, rows * fs::MK_CTR * sizeof(uint32_t)) != hipSuccess) return FS_E_NOMEM;
         if (hipMemset(c->mk_ctr, 0, rows * fs::MK_CTR * sizeof(uint32_t)) != hipSuccess) return FS_E_HIP;
         if (hipMalloc(&c->mk_list, rows * fs::MK_LIST * sizeof(uint64_t)) != hipSuccess) return FS_E_NOMEM;
         if (hipMalloc(&c->mk_spill, rows * fs::MK_SPILL * sizeof(uint64_t)) != hipSuccess) return FS_E_NOMEM;
+        if (hipMalloc(&c->mk_mass, rows * 2048 * sizeof(uint64_t)) != hipSuccess) return FS_E_NOMEM;
+        if (hipMemset(c->mk_mass, 0, rows * 2048 * sizeof(uint64_t)) != hipSuccess) return FS_E_HIP;
         c->mk_rows = rows;
     }
     return FS_OK;
@@ -576,7 +587,9 @@ int launch_mid(fs_context* ctx, const fs::Args& a, const fs_row_params* h_params
     if (!ctx->seg_layout) return FS_OK;
     const bool verify = a.mode == fs::MODE_VERIFY;
     MidKChoice ch;
-    if (!mid_k_choice(ctx->cus, h_params, verify ? (int64_t)a.n_streams : (int64_t)a.B, a.B, a.V, ch)) return FS_OK;
+    if (!mid_k_choice(ctx->cus, h_params, verify ? (int64_t)a.n_streams : (int64_t)a.B, a.B, a.V,
+                      a.cand_ids || a.cand_probs, ch))
+        return FS_OK;
     const size_t segs = (size_t)a.B * ch.nseg, streams = verify ? 3 * (size_t)a.n_streams : 0;
     const bool cap = capturing(st);
     if (cap && (segs > ctx->mk_segs || (size_t)a.B > ctx->mk_rows || streams > ctx->stream_cap || !ctx->err))
@@ -588,14 +601,14 @@ int launch_mid(fs_context* ctx, const fs::Args& a, const fs_row_params* h_params
     if (cap) ctx->captured = true;
     fs::MkArgs m = {};
     m.a = row_args(ctx, a, ch.nseg);
-    m.ctr = ctx->mk_ctr; m.qk = ctx->mk_qk; m.list = ctx->mk_list; m.spill = ctx->mk_spill; m.spins = ctx->merge_spins;
+    m.ctr = ctx->mk_ctr; m.qk = ctx->mk_qk; m.list = ctx->mk_list; m.spill = ctx->mk_spill; m.mass = ctx->mk_mass; m.spins = ctx->merge_spins;
     const int64_t grid = (int64_t)fs::XCDS * ch.nseg * (((int64_t)a.B + fs::XCDS - 1) / fs::XCDS);
 #ifdef FS_TRACE
     if (ctx->trace && grid * fs::TRACE_W <= ctx->trace_cap) m.a.trace = ctx->trace;
 #endif
     const int flags = (ch.may_pen ? fs::SK_MAY_PEN : 0) | (a.out_hist_off ? fs::SK_COPY : 0) |
                       (verify ? fs::MK_VERIFY : 0);
-    if (fs::launch_mid_k(ch.nl, ch.capped, (unsigned)grid, flags, m, st) != hipSuccess) return FS_E_HIP;
+    if (fs::launch_mid_k(ch.nl, ch.capped, ch.all, (unsigned)grid, flags, m, st) != hipSuccess) return FS_E_HIP;
     used = true;
     return FS_OK;
 }
@@ -725,6 +738,7 @@ int fs_destroy(fs_context* c) {
     (void)hipFree(c->mk_ctr);
     (void)hipFree(c->mk_list);
     (void)hipFree(c->mk_spill);
+    (void)hipFree(c->mk_mass);
     (void)hipFree(c->mk_qk);
     (void)hipFree(c->cand);
     (void)hipFree(c->meta);
@@ -839,7 +853,7 @@ int fs_mid_k_plan(int32_t cus, const fs_row_params* h_params, int32_t n, int32_t
                   int32_t* nseg) {
     if (cus < 1 || !h_params || n < 1 || total_rows < 1 || V < 1 || V > FS_MAX_VOCAB || !nl || !nseg) return FS_E_INVALID;
     MidKChoice c;
-    const bool fits = mid_k_choice(cus, h_params, n, total_rows, V, c);
+    const bool fits = mid_k_choice(cus, h_params, n, total_rows, V, false, c);
     *nl = fits ? c.nl : 0;
     *nseg = fits ? c.nseg : 0;
     return fits ? FS_OK : FS_E_LIMIT;

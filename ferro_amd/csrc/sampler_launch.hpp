@@ -70,9 +70,11 @@ struct MkArgs {
     uint32_t* qk;                          // [B][nseg][SK_NW][16] published lane maxima
     uint64_t* list;                        // [B][MK_LIST]
     uint64_t* spill;                       // [B][MK_SPILL]
+    uint64_t* mass;                        // [B][2048] mass bins of rows with every token a candidate, left at 0
     uint32_t spins;                        // bounded wait for a row's segments (polls)
 };
-hipError_t launch_mid_k(int nl, bool capped, unsigned grid, int flags, const MkArgs& m, hipStream_t st);
+// all: some row samples with every token a candidate
+hipError_t launch_mid_k(int nl, bool capped, bool all, unsigned grid, int flags, const MkArgs& m, hipStream_t st);
 
 hipError_t launch_lookup_draft(int n_streams, const int32_t* hist, const int64_t* hist_off, const int32_t* kmax,
                                const int32_t* min_n, int eos, int32_t* draft, int draft_ld, int32_t* ndraft,

@@ -93,8 +93,8 @@ int fs_sample_batch(fs_context* ctx, const float* d_logits, int64_t ld, int32_t 
  * greedy (frequency / presence penalties only where rows split into segments of 4096 logits) or samples from at
  * most 64 candidates (k = top_k, or V when top_k is 0) with no frequency / presence penalty run on a kernel made for
  * them (every segment's loads issued at once, bitonic sorts in registers; all-greedy batches a greedy-only form);
- * other batches whose every row is greedy or samples from at most 2048 candidates, with any penalty, run on the mid-k
- * kernel (fs_mid_k_plan); of the rest, batches mixing rows of 64 < k <= 2048 with cheaper rows run fs_sample_batch's
+ * other batches whose every row is greedy, samples from at most 2048 candidates or, without min-p and candidate outputs,
+ * from every token (k = V), with any penalty, run on the mid-k kernel (fs_mid_k_plan); of the rest, batches mixing rows of 64 < k <= 2048 with cheaper rows run fs_sample_batch's
  * kernel with about twice its segments; other batches, and h_params = NULL, run fs_sample_batch. fs_route_plan reports
  * the choice between the small-k kernel and the others. Same outputs as fs_sample_batch. h_params is read before the
  * call returns. Under HIP graph capture a batch whose mid-k workspace would have to grow runs fs_sample_batch's kernel. */
@@ -118,8 +118,8 @@ int fs_route_plan(int32_t cus, const fs_row_params* h_params, int32_t n, int32_t
 
 /* Host-only: the mid-k kernel's layout for a batch the small-k kernel does not take (arguments as fs_route_plan's): *nl
  * float4 loads per thread (segments of 1024 * nl logits) and *nseg segments per row; FS_E_LIMIT, and zeros, when the
- * batch does not fit it (a row of more than 2048 candidates, more than 262144 logits per row, or too few logits for the
- * largest k). No counterpart in the reference (a planner check). */
+ * batch does not fit it (a row of more than 2048 candidates that are not every token or with min-p, more than 262144
+ * logits per row, or too few logits for the largest k). No counterpart in the reference (a planner check). */
 int fs_mid_k_plan(int32_t cus, const fs_row_params* h_params, int32_t n, int32_t total_rows, int32_t V, int32_t* nl,
                   int32_t* nseg);
 
@@ -160,8 +160,8 @@ int fs_verify(fs_context* ctx, const float* d_logits, int64_t ld, int32_t n_stre
 /* fs_verify with the stream parameters also in host memory (h_params: the same n_streams records as d_params). Windows
  * whose every stream is greedy or samples from at most 64 candidates, with no active penalty (repetition 1, or
  * repeat_last_n 0, and no frequency / presence penalty: a row's history then does not matter), run on the small-k
- * kernel of fs_sample_batch_hp; other windows whose every stream is greedy or samples from at most 2048 candidates run on
- * its mid-k kernel (each row's window is the stream's history and the drafts fed before it); the rest, and h_params =
+ * kernel of fs_sample_batch_hp; other windows whose every stream is greedy or samples from at most 2048 candidates or
+ * (without min-p) from every token run on its mid-k kernel (each row's window is the stream's history and the drafts fed before it); the rest, and h_params =
  * NULL, run fs_verify. Same outputs as fs_verify. */
 int fs_verify_hp(fs_context* ctx, const float* d_logits, int64_t ld, int32_t n_streams, int32_t total_rows,
                  int32_t V, const int32_t* d_rows, const int64_t* d_row_off, const int32_t* d_hist,

@@ -246,3 +246,88 @@ def test_mid_k_decode_steps():
         np.testing.assert_array_equal(tok.cpu().numpy(), want[k])
     np.testing.assert_array_equal(off.cpu().numpy(), want_off)
     np.testing.assert_array_equal(hist[:int(off[-1])].cpu().numpy(), want_hist)
+
+
+@pytest.mark.parametrize("B,V", [(1, 4096), (3, 33001), (5, 65536), (24, 100003), (9, 262144), (70, 65537), (66, 262144)])
+@pytest.mark.parametrize("top_p", [1.0, 0.95, 0.4])
+def test_every_token_a_candidate(B, V, top_p):
+    """top_k = 0 on every segment size: flat and spiky rows, bf16 values, narrow and wide spreads, all-equal and two-valued
+    rows (no bin narrows them down), a masked vocabulary, infinities, NaN, a row without a number; penalties, a softcap,
+    greedy and k <= 2048 rows among them."""
+    rng = np.random.default_rng(V + B)
+    x = (rng.standard_normal((B, V)) * 2).astype(np.float32)
+    x[::2] = W.mixture_logits(rng, len(x[::2]), V)
+    p = mid_params(B, 0, temperature=rng.uniform(0.5, 1.3, B))
+    p["top_p"] = top_p
+    p["repetition_penalty"][::3] = 1.2
+    p["frequency_penalty"][1::4] = 0.2
+    if B > 3:
+        x[1] = bf16_valued(x[1])
+        p["temperature"][2] = 0.0
+        p["top_k"][3] = 80
+    if B > 8:
+        x[4, :] = 1.5                                # all equal
+        x[5] = np.where(rng.random(V) < 0.5, 1.0, 2.0)
+        x[6, rng.choice(V, V - 40, replace=False)] = -np.inf
+        x[7] *= 1e-3
+        x[8] = x[8] * 30 + 5
+    if B > 20:
+        x[9, 11] = np.inf
+        x[10, :] = np.nan
+        x[11, ::3] = np.nan
+        x[12, :] = -np.inf
+        x[13, 100] += 60.0                           # one token holds the whole mass
+        p["softcap"][14:16] = 30.0
+        x[15] *= 20
+    u = rng.random(B)
+    u[0] = 0.0
+    hists = [list(W.zipf_ids(rng, V, int(rng.integers(0, 1500)))) for _ in range(B)]
+    hist, off = csr(hists)
+    out = F.sample_batch(torch.from_numpy(x).cuda(), p, u, hist=hist, hist_off=off)
+    torch.cuda.synchronize()
+    o = O.sample_batch(x, hist, off, p, u, kcap=1, nthreads=NT)
+    np.testing.assert_array_equal(out["tok"].cpu().numpy(), o["tok"])
+    np.testing.assert_array_equal(out["keep"].cpu().numpy(), o["keep"])
+    assert F.device_error() == 0
+
+
+def test_every_token_give_up_and_decode():
+    """Rows whose segments do not wait for each other are selected alone; decode steps and verification windows with
+    top_k = 0."""
+    from ferro_amd._lib import FS_DEVERR_INTERNAL, FS_WAIT_GIVE_UP
+    rng = np.random.default_rng(3)
+    S, V = 4, 40000
+    p = mid_params(S, 0, temperature=0.8, repetition_penalty=1.1)
+    p["top_p"][::2] = 0.9
+    p["top_p"][1::2] = 1.0
+    x = W.mixture_logits(rng, S, V)
+    hists = [list(W.zipf_ids(rng, V, 400)) for _ in range(S)]
+    hist, off = csr(hists)
+    u = rng.random(S)
+    o = O.sample_batch(x, hist, off, p, u, kcap=1, nthreads=NT)
+    ctx = F.sampler.Context()
+    for limit, bits in ((FS_WAIT_GIVE_UP, FS_DEVERR_INTERNAL), (0, 0)):
+        ctx.set_wait_limit(limit)
+        out = F.sample_batch(torch.from_numpy(x).cuda(), p, u, hist=hist, hist_off=off, ctx=ctx)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out["tok"].cpu().numpy(), o["tok"])
+        np.testing.assert_array_equal(out["keep"].cpu().numpy(), o["keep"])
+        assert F.device_error(ctx) == bits
+    rows = [W.mixture_logits(rng, S, V) for _ in range(3)]
+    seeds = list(range(1, S + 1))
+    want, want_hist, want_off = oracle_decode_loop(rows, p, seeds, hists)
+    d = F.DeviceRng(np.asarray(seeds, np.uint64))
+    h, ho = torch.from_numpy(hist).cuda(), torch.from_numpy(off).cuda()
+    for k, r in enumerate(rows):
+        tok, _, h, ho = F.decode_step(torch.from_numpy(r).cuda(), p, d, hist=h, hist_off=ho)
+        np.testing.assert_array_equal(tok.cpu().numpy(), want[k])
+    np.testing.assert_array_equal(h[:int(ho[-1])].cpu().numpy(), want_hist)
+    R = 12
+    xv = W.mixture_logits(rng, R, V)
+    fed = xv.argmax(axis=1).astype(np.int32)
+    ro = np.array([0, 3, 4, 9, 12], np.int64)
+    uv = rng.random(R)
+    tok, acc = F.verify(torch.from_numpy(xv).cuda(), fed, ro, p, u=uv, hist=hist, hist_off=off)
+    otok, oacc = O.verify(xv, fed, ro, hist, off, p, uv)
+    np.testing.assert_array_equal(tok.cpu().numpy(), otok)
+    np.testing.assert_array_equal(acc.cpu().numpy(), oacc)

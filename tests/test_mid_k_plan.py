@@ -20,10 +20,15 @@ def test_layouts(B, V, k, want):
     assert _lib.mid_k_plan(256, W.make_params(B, temperature=0.8, top_k=k, frequency_penalty=0.1), V) == want
 
 
-def test_largest_k_counts_and_whole_rows_do_not_fit():
+def test_which_rows_fit():
     p = W.make_params(8, temperature=0.8, top_k=70)
     assert _lib.mid_k_plan(256, p, 65536) == (4, 16)
-    p["top_k"][3] = 0                   # every token a candidate
+    p["top_k"][3] = 3000                # between the largest k and every token
     assert _lib.mid_k_plan(256, p, 65536) is None
     p["temperature"][3] = 0.0           # greedy: top_k does not matter
     assert _lib.mid_k_plan(256, p, 65536) == (4, 16)
+    p["temperature"][3] = 0.8
+    p["top_k"][3] = 0                   # every token a candidate: without min-p
+    assert _lib.mid_k_plan(256, p, 65536) == (4, 16)
+    p["min_p"][3] = 0.05
+    assert _lib.mid_k_plan(256, p, 65536) is None
