@@ -60,7 +60,10 @@ struct MkShared {
             uint64_t top[MK_K];            // (u.m.top's head)
             double e[MK_K];                // their masses, then probabilities
         } w;
-        uint64_t mass[AK_BINS];            // every token a candidate: fixed-point masses by bin
+        struct {
+            uint64_t mass[AK_BINS];        // every token a candidate: fixed-point masses by bin, the segment's, then
+            uint64_t cum[SK_LT];           //   the row's, and the mass up to and with each eight
+        } a;
         struct {
             uint64_t l[2][AK_STAGE];       //   this segment's logits of the bins searched, ~id above the value
         } g;
@@ -473,7 +476,7 @@ __device__ __forceinline__ void mk_softmax(const SkArgs& a, const fs_row_params&
 
 // ---- every token a candidate (top_k = 0: k = V)
 // 2^(j/64), correctly rounded.
-__constant__ double ak_pow2[64] = {
+__device__ double ak_pow2[64] = {
     0x1.0000000000000p+0, 0x1.02c9a3e778061p+0, 0x1.059b0d3158574p+0, 0x1.0874518759bc8p+0,
     0x1.0b5586cf9890fp+0, 0x1.0e3ec32d3d1a2p+0, 0x1.11301d0125b51p+0, 0x1.1429aaea92de0p+0,
     0x1.172b83c7d517bp+0, 0x1.1a35beb6fcb75p+0, 0x1.1d4873168b9aap+0, 0x1.2063b88628cd6p+0,
@@ -528,7 +531,7 @@ __device__ __forceinline__ bool mk_meet(uint32_t* ctr, uint32_t target, uint32_t
 }
 
 // The bin that holds the target-th unit of the row's mass, and the mass before it: cum (LDS) holds the mass up to and
-// with bins 8t .. 8t + 7, rm the bins. Each wave finds it by itself, the same in all (no barrier); false when the row's
+// with bins 8t .. 8t + 7, rm (LDS) the bins. Each wave finds it by itself, the same in all (no barrier); false when the row's
 // mass does not reach the target.
 __device__ __forceinline__ bool ak_locate(const uint64_t* cum, const uint64_t* rm, uint64_t target, int& bin,
                                           uint64_t& before) {
@@ -750,7 +753,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     const double Td = (double)p.temperature, inv = 1.0 / Td;
     const float invf = 1.0f / p.temperature;
     r.u = u;
-    if (tid < 64) s.pow2[tid] = ak_pow2[tid];
+    const uint64_t pow2 = ld_agent(reinterpret_cast<const uint64_t*>(ak_pow2) + lane);   // (it arrives behind the meeting)
     penalise();
     if (CAP && p.softcap > 0.0f) {
 #pragma unroll
@@ -802,6 +805,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     }
     if (!mk_meet(ctr, (uint32_t)nseg, mk.spins, s)) return false;
     SK_MARK(2);
+    if (tid < 64) s.pow2[tid] = __longlong_as_double((long long)pow2);   // (the barrier before the masses publishes it)
     {
         const uint64_t e = lane < nseg ? line[lane * 32] : 0xFFFFFFFFull;
         r.nv = wave_allreduce(lane < nseg ? (uint32_t)line[lane * 32 + 1] : 0u, add_u);
@@ -817,7 +821,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     r.plain = r.nv == 0u || !(mx < __builtin_huge_valf()) || !(mx > -__builtin_huge_valf()) || !(mn < mx) || !(scale > 0.0f) ||
               !(scale < __builtin_huge_valf());
     if (r.plain) return true;                                  // uniform over the row
-    for (int i = tid; i < AK_BINS / 2; i += SK_LT) reinterpret_cast<ulonglong2*>(s.u.mass)[i] = make_ulonglong2(0ull, 0ull);
+    for (int i = tid; i < AK_BINS / 2; i += SK_LT) reinterpret_cast<ulonglong2*>(s.u.a.mass)[i] = make_ulonglong2(0ull, 0ull);
     __syncthreads();
     // a logit's place below the maximum, in bins, and its bin (AK_BINS: none), the same function of its value in both
     // passes; it never falls as the logit falls (NaN: not a candidate)
@@ -870,7 +874,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
             const double m = ak_exp(z, s.pow2);
             part += m;
             const uint64_t f = (uint64_t)__double_as_longlong(__builtin_fma(m, AK_FX, 0x1p52)) - 0x4330000000000000ull;
-            atomicAdd(reinterpret_cast<unsigned long long*>(&s.u.mass[b]), (unsigned long long)f);
+            atomicAdd(reinterpret_cast<unsigned long long*>(&s.u.a.mass[b]), (unsigned long long)f);
         } else if (x == x) {
             rest += __expf((x - mx) * invf);
         }
@@ -905,7 +909,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     uint64_t* rm = mk.mass + (int64_t)row * AK_BINS;
 #pragma unroll
     for (int j = 0; j < AK_BINS / SK_LT; ++j) {
-        const uint64_t h = s.u.mass[j * SK_LT + tid];
+        const uint64_t h = s.u.a.mass[j * SK_LT + tid];
         if (h != 0ull) __hip_atomic_fetch_add(rm + j * SK_LT + tid, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     if (tid == 0) line[seg * 32 + 16] = (uint64_t)__double_as_longlong(sum);
@@ -915,8 +919,9 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     {
         uint64_t mine = 0ull;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < 4; ++j) {                          // (the segment's own bins are spent)
             const ulonglong2 x = reinterpret_cast<const ulonglong2*>(rm)[4 * tid + j];
+            reinterpret_cast<ulonglong2*>(s.u.a.mass)[4 * tid + j] = x;
             mine += x.x + x.y;
         }
         uint64_t inc = mine;
@@ -930,8 +935,8 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < SK_NW; ++q) inc += q < w ? s.w64[q] : 0ull;
-        uint64_t* cum = s.u.mass;                              // (the segment's own bins are spent)
-        cum[tid] = inc;
+        const uint64_t *cum = s.u.a.cum, *row_mass = s.u.a.mass;
+        s.u.a.cum[tid] = inc;
         __syncthreads();
         uint64_t before = 0ull;
         r.cut = p.top_p < 1.0f;
@@ -941,22 +946,22 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
             // top-p keeps through its crossing candidate (sampler.cpp:44), so the kept total lies in [tgt, tgt + the
             // largest mass of bin bc]: the draw's bin at both ends
             const double tgt = (double)p.top_p * r.S;
-            ok = ak_locate(cum, rm, (uint64_t)(tgt * AK_FX), r.bc, before);
+            ok = ak_locate(cum, row_mass, (uint64_t)(tgt * AK_FX), r.bc, before);
             r.above_c = (double)before / AK_FX;
             const double most = ak_exp(-(double)(ok ? r.bc : 0) * (double)depth * (1.0 / AK_BINS), s.pow2) * (1.0 + 1e-4);
             const double thi = tgt + most < r.S ? tgt + most : r.S;
-            if (ok) ok = ak_locate(cum, rm, (uint64_t)(u * tgt * (1.0 - 1e-12) * AK_FX), r.d0, before);
+            if (ok) ok = ak_locate(cum, row_mass, (uint64_t)(u * tgt * (1.0 - 1e-12) * AK_FX), r.d0, before);
             r.above_d = (double)before / AK_FX;
-            if (ok && !ak_locate(cum, rm, (uint64_t)(u * thi * (1.0 + 1e-12) * AK_FX), r.d1, before)) r.d1 = r.bc;
+            if (ok && !ak_locate(cum, row_mass, (uint64_t)(u * thi * (1.0 + 1e-12) * AK_FX), r.d1, before)) r.d1 = r.bc;
             if (r.d1 > r.bc) r.d1 = r.bc;
         } else {
-            ok = ak_locate(cum, rm, (uint64_t)(u * r.S * AK_FX), r.d0, before);
+            ok = ak_locate(cum, row_mass, (uint64_t)(u * r.S * AK_FX), r.d0, before);
             r.above_d = (double)before / AK_FX;
             r.d1 = r.d0;
         }
         r.plain = !ok;                                         // past the binned mass: the row is selected alone
         if (!ok) return true;
-        __syncthreads();                                       // every wave has read cum (the lists below take its place)
+        __syncthreads();                                       // every wave has read the bins (the lists below take their place)
     }
     // the searched bins' logits, staged in LDS (the bins there are spent), then to the row's lists
     uint32_t above = 0u;
@@ -1007,8 +1012,12 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     __syncthreads();
     const uint32_t n0 = s.gn[0], n1 = s.gn[1];
     if (tid == 0) {
-        s.misc[0] = n0 ? __hip_atomic_fetch_add(ctr + 33, n0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
-        s.misc[1] = n1 ? __hip_atomic_fetch_add(ctr + 36, n1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
+        uint64_t at = 0ull;                                    // both lists' places in one round trip
+        if ((n0 | n1) != 0u)
+            at = __hip_atomic_fetch_add(reinterpret_cast<uint64_t*>(ctr + 38), ((uint64_t)n1 << 32) | n0, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_WORKGROUP);
+        s.misc[0] = (uint32_t)at;
+        s.misc[1] = (uint32_t)(at >> 32);
         if (s.gn[2]) __hip_atomic_fetch_add(ctr + 37, s.gn[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (n0 > (uint32_t)AK_STAGE || n1 > (uint32_t)AK_STAGE)
             __hip_atomic_fetch_or(ctr + 34, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1023,14 +1032,41 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
 }
 
 // The row's end, by its last segment: top-p's crossing and the draw located exactly in their bins' sorted logits. Returns
-// false when a target lies outside its bin's exact masses (a rounding step at the edge).
-__device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uint32_t n1, uint32_t above, const AkRow& r,
-                                          const fs_row_params& p, MkShared& s, int& tok, int& keep) {
-    const int tid = threadIdx.x;
+// false when a target lies outside its bin's exact masses (a rounding step at the edge). c0, c1: the lists' first WAVE
+// entries; lists no longer than that (most are: a spiky row's bins hold a few logits) are sorted and summed in registers,
+// by every wave for itself, without a barrier.
+__device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uint32_t n1, uint64_t c0, uint64_t c1,
+                                          uint32_t above, const AkRow& r, const fs_row_params& p, MkShared& s, int& tok,
+                                          int& keep) {
+    const int tid = threadIdx.x, lane = lane_id();
     const double Td = (double)p.temperature;
     uint64_t xc = 0ull;
     double tot = r.S;
     keep = (int)r.nv;
+    if (n0 <= (uint32_t)WAVE && n1 <= (uint32_t)WAVE) {
+#pragma unroll 1
+        for (int pass = r.cut ? 0 : 1; pass < 2; ++pass) {
+            const uint32_t n = pass == 0 ? n0 : n1;
+            const uint64_t c = pass == 0 ? c0 : c1;
+            const uint64_t v =
+                sort64<true>((uint32_t)lane < n ? ((uint64_t)key_of(__uint_as_float((uint32_t)c)) << 32) | (c >> 32) : 0ull);
+            const double e = (uint32_t)lane < n ? ak_mass(val_of(comp_key(v)), r.mx, Td) : 0.0;
+            const double cum = wave_scan_f64(e) + (pass == 0 ? r.above_c : r.above_d);
+            const double target = pass == 0 ? (double)p.top_p * r.S : r.u * tot + 0.0;
+            const uint64_t hit = __ballot((uint32_t)lane < n && cum >= target);
+            if (hit == 0ull) return false;
+            const int at = __ffsll((unsigned long long)hit) - 1;
+            const uint64_t x = read_lane(v, at);
+            if (pass == 0) {
+                xc = x;
+                tot = lane_f64(cum, at);
+                keep = (int)above + at + 1;
+            } else {
+                tok = (int)comp_id(x < xc ? xc : x);
+            }
+        }
+        return true;
+    }
 #pragma unroll 1
     for (int pass = r.cut ? 0 : 1; pass < 2; ++pass) {
         const int n = (int)(pass == 0 ? n0 : n1);
@@ -1353,8 +1389,10 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
     float tr = 0.0f, tc = 0.0f;                                // the bound: raw, capped
     bool go = true;
     AkRow ak = {};
+    SkDraw dr = {0.0, 0};
     if (ALL && every) {
-        go = ak_segment<NL, CAP>(v, mk, p, row, seg, nseg, seg_lo, ctr, list, penalise, pen_at, nf, sk_draw(a, row).u, ak, s);
+        dr = sk_draw(a, row);
+        go = ak_segment<NL, CAP>(v, mk, p, row, seg, nseg, seg_lo, ctr, list, penalise, pen_at, nf, dr.u, ak, s);
     } else if (!scan) {
         // the lane maxima, sorted in each wave, published at 16 ranks
         const uint32_t srt = sort64_desc_u32(key_of(lm));
@@ -1503,8 +1541,7 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
     }
     SK_TAG(13, 4);
     // ---- the row's end, by its last segment. (The lists are read at agent scope: past this CU's L1.)
-    SkDraw dr = {0.0, 0};
-    if (!greedy) dr = sk_draw(a, row);
+    if (!greedy && !(ALL && every)) dr = sk_draw(a, row);
     int tok = 0, keep = 1;
     // a greedy row's token (ferro keeps index 0 when its logit is NaN)
     auto greedy_end = [&](uint64_t top) {
@@ -1515,6 +1552,15 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
         }
     };
     const uint32_t slow = ld_agent(ctr + 34);                  // uniform
+    uint32_t n0 = 0u, n1 = 0u, above = 0u;
+    uint64_t c0 = 0ull, c1 = 0ull;
+    if (ALL && every) {                                        // (one round trip with the flags)
+        n0 = ld_agent(ctr + 38);
+        n1 = ld_agent(ctr + 39);
+        above = ld_agent(ctr + 37);
+        c0 = ld_agent(&list[lane]);
+        c1 = ld_agent(&list[AK_LIST + lane]);
+    }
     if (scan && slow == 0u) {
         if (w != 0) return;
         greedy_end(wave_max(lane < nseg ? ld_agent(&list[lane]) : 0ull));
@@ -1523,17 +1569,16 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
             ctr[35] = 0u;
         }
     } else if (ALL && every) {
-        const uint32_t n0 = ld_agent(ctr + 33), n1 = ld_agent(ctr + 36), above = ld_agent(ctr + 37);
         __syncthreads();
         if (tid == 0) {                                        // every segment has met and counted: left at 0
             ctr[0] = 0u;
-            for (int i = 32; i < 38; ++i) ctr[i] = 0u;
+            for (int i = 32; i < 40; ++i) ctr[i] = 0u;
             if (slow & 2u) atomicOr(a.err, FS_DEVERR_INTERNAL);
         }
         ulonglong2* rm = reinterpret_cast<ulonglong2*>(mk.mass + (int64_t)row * AK_BINS);
         for (int i = tid; i < AK_BINS / 2; i += SK_LT) rm[i] = make_ulonglong2(0ull, 0ull);
         if (slow != 0u || ak.plain || n0 > (uint32_t)AK_LIST || n1 > (uint32_t)AK_LIST ||
-            !ak_finish(list, n0, n1, above, ak, p, s, tok, keep))
+            !ak_finish(list, n0, n1, c0, c1, above, ak, p, s, tok, keep))
             ak_slow<CAP>(rowp, V, pen, win, pn, p, dr.u, s, tok, keep);
         if (w != 0) return;
     } else {
