@@ -34,14 +34,19 @@ KERNEL = "fs::segment_kernel"
 
 
 def kernel_of(w, route, cus=256, verify=False):
-    """The kernel a call of this workload launches, as the library routes it (fs_route_plan): fs_sample_batch_hp /
-    fs_verify_hp (route "host") pick the small-k kernel (its greedy-only form for all-greedy batches) where the batch
-    fits it, else the fused kernel; fs_sample_batch / fs_verify (route "device") always run the fused kernel."""
+    """The kernel a call of this workload launches, as the library routes it (fs_route_plan, fs_mid_k_plan):
+    fs_sample_batch_hp / fs_verify_hp (route "host") pick the small-k kernel (its greedy-only form for all-greedy
+    batches) where the batch fits it, then the mid-k kernel, else the fused kernel; fs_sample_batch / fs_verify
+    (route "device") always run the fused kernel."""
     fused = (KERNEL, "segments, then a merging workgroup per row, one grid")
     if route != "host":
         return fused
     from ferro_amd import _lib
     kind, nl, ns, per_cu = _lib.route_plan(cus, w.params, w.V, total_rows=w.B, verify=verify)
+    mid = _lib.mid_k_plan(cus, w.params, w.V, total_rows=w.B) if kind == 0 else None
+    if mid:
+        return (f"fs::mid_k_kernel<{mid[0]}>",
+                f"{mid[1]} segments of {1024 * mid[0]} logits per row, the last segment of a row merges it, one grid")
     if kind == 0:
         return (KERNEL, f"segments ({per_cu} per CU), then a merging workgroup per row, one grid")
     return (f"fs::small_k_kernel<{nl}>",

@@ -551,34 +551,42 @@ bool mid_k_choice(int cus, const fs_row_params* h, int64_t n, int64_t rows, int3
     return (int64_t)fs::XCDS * c.nseg * ((rows + fs::XCDS - 1) / fs::XCDS) <= 0x7fffffff;
 }
 
+// About 176 KB per row. FS_E_NOMEM leaves none of it allocated.
 int grow_mid(fs_context* c, size_t segs, size_t rows) {
-    if (segs > c->mk_segs) {
-        release(c, c->mk_qk);
-        c->mk_qk = nullptr; c->mk_segs = 0;
-        if (hipMalloc(&c->mk_qk, segs * fs::SK_NW * 16 * sizeof(uint32_t)) != hipSuccess) return FS_E_NOMEM;
-        c->mk_segs = segs;
+    if (segs <= c->mk_segs && rows <= c->mk_rows) return FS_OK;
+    segs = std::max(segs, c->mk_segs);
+    rows = std::max(rows, c->mk_rows);
+    auto drop = [&](auto*& p) {
+        release(c, p);
+        p = nullptr;
+    };
+    auto drop_all = [&]() {
+        drop(c->mk_qk); drop(c->mk_ctr); drop(c->mk_list); drop(c->mk_spill); drop(c->mk_mass);
+        c->mk_segs = c->mk_rows = 0;
+    };
+    drop_all();
+    if (hipMalloc(&c->mk_qk, segs * fs::SK_NW * 16 * sizeof(uint32_t)) != hipSuccess ||
+        hipMalloc(&c->mk_ctr, rows * fs::MK_CTR * sizeof(uint32_t)) != hipSuccess ||
+        hipMalloc(&c->mk_list, rows * fs::MK_LIST * sizeof(uint64_t)) != hipSuccess ||
+        hipMalloc(&c->mk_spill, rows * fs::MK_SPILL * sizeof(uint64_t)) != hipSuccess ||
+        hipMalloc(&c->mk_mass, rows * 2048 * sizeof(uint64_t)) != hipSuccess) {
+        (void)hipGetLastError();
+        drop_all();
+        return FS_E_NOMEM;
     }
-    if (rows > c->mk_rows) {
-        release(c, c->mk_ctr);
-        release(c, c->mk_list);
-        release(c, c->mk_spill);
-        release(c, c->mk_mass);
-        c->mk_mass = nullptr;
-        c->mk_ctr = nullptr; c->mk_list = nullptr; c->mk_spill = nullptr; c->mk_rows = 0;
-        if (hipMalloc(&c->mk_ctr, rows * fs::MK_CTR * sizeof(uint32_t)) != hipSuccess) return FS_E_NOMEM;
-        if (hipMemset(c->mk_ctr, 0, rows * fs::MK_CTR * sizeof(uint32_t)) != hipSuccess) return FS_E_HIP;
-        if (hipMalloc(&c->mk_list, rows * fs::MK_LIST * sizeof(uint64_t)) != hipSuccess) return FS_E_NOMEM;
-        if (hipMalloc(&c->mk_spill, rows * fs::MK_SPILL * sizeof(uint64_t)) != hipSuccess) return FS_E_NOMEM;
-        if (hipMalloc(&c->mk_mass, rows * 2048 * sizeof(uint64_t)) != hipSuccess) return FS_E_NOMEM;
-        if (hipMemset(c->mk_mass, 0, rows * 2048 * sizeof(uint64_t)) != hipSuccess) return FS_E_HIP;
-        c->mk_rows = rows;
+    if (hipMemset(c->mk_ctr, 0, rows * fs::MK_CTR * sizeof(uint32_t)) != hipSuccess ||
+        hipMemset(c->mk_mass, 0, rows * 2048 * sizeof(uint64_t)) != hipSuccess) {
+        drop_all();
+        return FS_E_HIP;
     }
+    c->mk_segs = segs;
+    c->mk_rows = rows;
     return FS_OK;
 }
 
 // Launches the mid-k kernel when the batch fits it; *used = false (nothing launched) otherwise. Under capture a
 // workspace that would have to grow leaves the batch to the fused kernel (no allocation in a capture that worked
-// without one).
+// without one), and so does one that the device has no room for.
 int launch_mid(fs_context* ctx, const fs::Args& a, const fs_row_params* h_params, hipStream_t st, bool& used) {
     used = false;
     std::lock_guard<std::mutex> g(ctx->mu);
@@ -597,11 +605,13 @@ int launch_mid(fs_context* ctx, const fs::Args& a, const fs_row_params* h_params
     rc = grow(ctx, 0, 0, streams);
     if (rc != FS_OK) return rc;
     rc = grow_mid(ctx, segs, (size_t)a.B);
+    if (rc == FS_E_NOMEM) return FS_OK;
     if (rc != FS_OK) return rc;
     if (cap) ctx->captured = true;
     fs::MkArgs m = {};
     m.a = row_args(ctx, a, ch.nseg);
-    m.ctr = ctx->mk_ctr; m.qk = ctx->mk_qk; m.list = ctx->mk_list; m.spill = ctx->mk_spill; m.mass = ctx->mk_mass; m.spins = ctx->merge_spins;
+    m.ctr = ctx->mk_ctr; m.qk = ctx->mk_qk; m.list = ctx->mk_list; m.spill = ctx->mk_spill;
+    m.mass = ctx->mk_mass; m.spins = ctx->merge_spins;
     const int64_t grid = (int64_t)fs::XCDS * ch.nseg * (((int64_t)a.B + fs::XCDS - 1) / fs::XCDS);
 #ifdef FS_TRACE
     if (ctx->trace && grid * fs::TRACE_W <= ctx->trace_cap) m.a.trace = ctx->trace;

@@ -331,3 +331,63 @@ def test_every_token_give_up_and_decode():
     otok, oacc = O.verify(xv, fed, ro, hist, off, p, uv)
     np.testing.assert_array_equal(tok.cpu().numpy(), otok)
     np.testing.assert_array_equal(acc.cpu().numpy(), oacc)
+
+
+@pytest.mark.parametrize("every", [False, True])
+@pytest.mark.parametrize("warm", [True, False])
+def test_mid_k_calls_in_a_graph(every, warm):
+    """fs_sample_batch_hp recorded into a graph and replayed, with eager calls of another size between the replays: the
+    counters, lists and mass bins are left as each replay needs them. A context that never ran such a batch takes the
+    fused kernel under capture (no allocation there): the same tokens."""
+    import ctypes
+    from ferro_amd._lib import lib
+    from test_gpu_graph import Call, P, check_clean, mixed
+    B, V = 40, 65536
+    ctx, other = F.sampler.Context(), F.sampler.Context()
+    ws = [mixed(31 + i, B, V) for i in range(3)]
+    for w in ws:
+        w.params["top_k"][w.params["top_k"] == 0] = 0 if every else 1500
+    calls = [Call(w, kcap=16) for w in ws]
+
+    def launch(i, c, st):
+        outs = (None, None) if every else (P(calls[i].ids), P(calls[i].probs))
+        rc = lib().fs_sample_batch_hp(c.h, P(calls[i].x), calls[i].x.stride(0), B if i < 2 else B // 2, V, P(calls[i].hist),
+                                      P(calls[i].hoff), P(calls[i].params),
+                                      ws[i].params.ctypes.data_as(ctypes.c_void_p), P(calls[i].u), P(calls[i].tok),
+                                      0 if every else 16, *outs, P(calls[i].keep), ctypes.c_void_p(st.cuda_stream))
+        assert rc == 0, rc
+
+    cur, side = torch.cuda.current_stream(), torch.cuda.Stream()
+    want = []
+    for i in range(2):
+        calls[i].poison()
+        launch(i, ctx if warm else other, cur)
+        torch.cuda.synchronize()
+        want.append(calls[i].out())
+    if not warm:                                       # (the fused kernel's workspace only)
+        F.sample_batch(calls[0].x[:, :V], ws[0].params, ws[0].u, hist=ws[0].hist, hist_off=ws[0].hist_off, ctx=ctx,
+                       route="device")
+        torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    side.wait_stream(cur)
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(g, stream=side):
+            for i in range(2):
+                launch(i, ctx, side)
+    cur.wait_stream(side)
+    torch.cuda.synchronize()
+    for rep in range(3):
+        for c in calls[:2]:
+            c.poison()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        for i in range(2):
+            got = calls[i].out()
+            for k in ("tok", "keep", "ids"):
+                np.testing.assert_array_equal(got[k], want[i][k], err_msg=f"replay {rep} call {i} {k}")
+            np.testing.assert_allclose(got["probs"], want[i]["probs"], rtol=1e-12)   # (sums in another order)
+        launch(2, ctx, cur)
+        torch.cuda.synchronize()
+        check_clean(ctx)
+    del g
