@@ -17,11 +17,11 @@
 // selects the row's exact top k from the logits alone (mk_slow).
 // Bound: HBM, one read of the logits, then the chain behind a row's last logits.
 // Measured against the fused kernel (running bounds, per-row merges of the segments' lists): 256 rows of 262144 logits
-// with k from 1 to 2048 and every penalty 124 us -> 79; 24 rows of 100003 logits, k 200, frequency / presence 35 -> 19.4;
-// 40 rows of a verification window over 262144 logits, k 50, repetition 26.5 -> 24.3.
+// with k from 1 to 2048 and every penalty 124 us -> 77; 24 rows of 100003 logits, k 200, frequency / presence 35 -> 19.5;
+// 40 rows of a verification window over 262144 logits, k 50, repetition 26.5 -> 24.7.
 // Rows with every token a candidate (ak_segment, ak_finish) stay in registers through all their passes; the fused kernel
 // reads such a row again for each, and gave flat ones to one workgroup: 32 rows of 65536 N(0, 2) logits at temperature 1
-// 51.4 us -> 23.0, 3 rows of 178740 507 -> 21, 64 rows of 262144 heavy-tailed logits with top-p 0.95 37.5 -> 35.1.
+// 51.5 us -> 23.5, 3 rows of 178740 507 -> 21, 64 rows of 262144 heavy-tailed logits with top-p 0.95 37.5 -> 35.7.
 #include "row_device.hpp"
 
 #include <type_traits>
