@@ -526,6 +526,9 @@ bool mid_k_choice(int cus, const fs_row_params* h, int64_t n, int64_t rows, int3
         const int64_t k = greedy ? 1 : ((p.top_k > 0 && p.top_k < V) ? p.top_k : V);
         if (k == V && k > fs::KMAX) {
             // every token a candidate: no candidate outputs and no min-p (its count and sum over the kept logits)
+            // (taken whatever the rows hold, which the host cannot see: rows whose mass is a few logits come out at 0.97 to
+            // 1.10 times the fused kernel's short list, 16 rows of 65536 18.3 us there and 18.9 here, 64 of 262144 36.9 and
+            // 33.7; rows with a body gain: 16 normal rows of 65536 at temperature 0.2 49.8 and 23.3)
             if (outputs || p.min_p > 0.0f) return false;
             c.all = true;
         } else {
