@@ -477,7 +477,9 @@ __global__ __launch_bounds__(SK_LT, 4) void small_k_kernel(const float* logits, 
             const uint32_t kb = tau > 0x007FFFFFu ? tau : 0x007FFFFFu;          // (the key of -inf is the lowest)
             const uint32_t step = lane < 32 ? 1u << lane : 0u, room = kb - 0x007FFFFFu;
             const float c = softcap_one(val_of(room > step ? kb - step : 0x007FFFFFu + (lane < 32 ? 0u : room)), cap);
-            tc = read_lane(c, 32);
+            // no bound (fewer than k numbers among the maxima counted, or one at -inf): every number is a candidate, a
+            // penalised one below -cap too
+            tc = room != 0u ? read_lane(c, 32) : tf;
             const uint64_t below = __ballot(lane < 32 && c < tc);
             tr = -__builtin_huge_valf();
             if (below) {

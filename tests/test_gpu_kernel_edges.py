@@ -125,6 +125,23 @@ def test_softcap_where_it_saturates(cap, scale):
     check(x, p, [list(W.zipf_ids(rng, V, 900)) for _ in range(6)], rng.random(6))
 
 
+@pytest.mark.parametrize("V,k", [(5, 0), (40, 0), (64, 0), (65, 40), (320, 64), (800, 64), (2080, 50)])
+@pytest.mark.parametrize("cap", [0.5, 30.0])
+def test_softcap_and_penalties_on_short_rows(V, k, cap):
+    """Rows too short for a bound from their lane maxima (every logit is then a candidate): penalised logits below -cap
+    are candidates too. Windows of one id, of most and of all ids; -inf and NaN among the logits."""
+    rng = np.random.default_rng(V)
+    x = (rng.standard_normal((6, V)) * (2 if cap < 1 else 40)).astype(np.float32)
+    x[4, rng.choice(V, V // 2, replace=False)] = -np.inf
+    x[5, rng.choice(V, V // 2, replace=False)] = np.nan
+    p = W.make_params(6, temperature=0.9, top_k=k, repetition_penalty=1.2)
+    p["softcap"] = cap
+    p["repetition_penalty"][3] = 2.0
+    p["top_p"][1] = 0.9
+    hists = [[int(x[0].argmin())], list(rng.permutation(V)[:V * 3 // 4]), *[list(range(V))] * 4]
+    check(x, p, hists, np.array([0.999, 0.6, 0.999, 0.5, 0.9, 0.7]))
+
+
 def mid_params(B, k, **kw):
     p = W.make_params(B, temperature=0.9, top_k=k, top_p=0.97, repetition_penalty=1.0)
     for f, v in kw.items():
