@@ -1430,7 +1430,7 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
                 const uint32_t kb = T > 0x007FFFFFu ? T : 0x007FFFFFu, room = kb - 0x007FFFFFu;
                 const uint32_t step = lane < 32 ? 1u << lane : 0u;
                 const float c = softcap_one(val_of(room > step ? kb - step : 0x007FFFFFu + (lane < 32 ? 0u : room)), pn.cap);
-                tc = read_lane(c, 32);
+                tc = room != 0u ? read_lane(c, 32) : tc;       // (no bound: every number, a penalised one below -cap too)
                 const uint64_t below = __ballot(lane < 32 && c < tc);
                 tr = -__builtin_huge_valf();
                 if (below) {

@@ -190,6 +190,23 @@ def test_mid_k_penalties(V, B, H):
     check(x, p, hists, rng.random(B), kcap=256)
 
 
+@pytest.mark.parametrize("V,k", [(320, 10), (2080, 65), (4100, 100)])
+@pytest.mark.parametrize("cap", [0.5, 30.0])
+def test_mid_k_softcap_and_penalties_without_a_bound(V, k, cap):
+    """Windows that hold every id (no logit is left to bound the row) or most, with penalties that take logits below
+    -cap: they stay candidates. -inf and NaN among the logits."""
+    rng = np.random.default_rng(V)
+    x = (rng.standard_normal((6, V)) * (2 if cap < 1 else 40)).astype(np.float32)
+    x[4, rng.choice(V, V // 2, replace=False)] = -np.inf
+    x[5, rng.choice(V, V // 2, replace=False)] = np.nan
+    p = mid_params(6, k, repetition_penalty=1.2, frequency_penalty=2.0)
+    p["softcap"] = cap
+    p["repetition_penalty"][3] = 2.0
+    p["frequency_penalty"][3] = 0.0
+    hists = [list(range(V)) * 20, list(rng.permutation(V)[:V * 3 // 4]) * 3, *[list(range(V))] * 4]
+    check(x, p, hists, rng.random(6), kcap=k)
+
+
 def test_mid_k_more_penalised_ids_than_the_spill_list():
     rng = np.random.default_rng(5)
     V, H = 262144, 40000
