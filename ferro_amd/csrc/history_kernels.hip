@@ -127,7 +127,7 @@ __global__ __launch_bounds__(LU_BLOCK) void lookup_draft_kernel(const int32_t* h
                         m = w[r + 2] == t[1] ? m : 1;
                         m = w[r + 3] == t[0] ? m : 0;
                         m = m < (int)nmax ? m : (int)nmax;
-                        if (c0 == 0) m = m < i0 + r ? m : i0 + r;     // no ids before the history's first
+                        if (c0 < LU_N) m = m < (int)c0 + i0 + r ? m : (int)c0 + i0 + r;   // no ids before the history's first
                         if (i0 + r < n && w[r + LU_N] != eos && m >= bm) { bm = m; bi = i0 + r; }
                     }
                 }

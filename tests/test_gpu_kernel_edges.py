@@ -66,6 +66,31 @@ def test_lookup_draft_tile_edges(L):
         np.testing.assert_array_equal(draft[s, :nd[s]], want)
 
 
+@pytest.mark.parametrize("L", [16385, 16386, 16387, 16388, 32769, 32771])
+def test_lookup_draft_before_the_history(L):
+    """A history's first ids are not preceded by anything: id 0 (what a tile holds there) does not complete a match.
+    Histories that end in 0s and their own first ids; a genuine shorter match elsewhere stays the one found."""
+    rng = np.random.default_rng(L)
+    hists, min_n = [], []
+    for n in (1, 2, 3, 4):
+        for lead in (0, 1, 2, 3):
+            h = rng.integers(1000, 1 << 20, L).astype(np.int32)
+            h[L - 4:] = 0
+            if lead:
+                h[L - lead:] = h[:lead]
+            if n == 2:
+                h[L // 2:L // 2 + 2] = h[L - 2:]
+            hists.append(h)
+            min_n.append(n)
+    hist, off = csr(hists)
+    draft, nd = F.lookup_draft(hist, off, 20, min_n=np.asarray(min_n, np.int32), eos_id=3, draft_ld=20)
+    draft, nd = draft.cpu().numpy(), nd.cpu().numpy()
+    for s, h in enumerate(hists):
+        want = O.lookup_draft(h, 20, eos=3, min_n=min_n[s])
+        assert nd[s] == len(want), (L, s)
+        np.testing.assert_array_equal(draft[s, :nd[s]], want)
+
+
 @pytest.mark.parametrize("H,V", [(511, 65536), (512, 65536), (513, 65536), (515, 262144), (516 + 8192, 262144),
                                  (517 + 8192 + 2048 + 3, 262144), (20011, 100004)])
 def test_long_windows_and_history_copies(H, V):
