@@ -1420,7 +1420,7 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
         SK_MARK(3);
         go = s.misc[5] != 0u;
         if (go) {
-            const uint32_t T = mk_bound<NL == 16 ? 1 : NL == 8 ? 2 : 4>(qk, nseg, k, s);
+            const uint32_t T = mk_bound<NL == 16 ? 1 : 2>(qk, nseg, k, s);
             SK_MARK(4);
             tc = T > 0x007FFFFFu ? val_of(T) : -__builtin_huge_valf();
             tr = tc;

@@ -545,7 +545,7 @@ bool mid_k_choice(int cus, const fs_row_params* h, int64_t n, int64_t rows, int3
     c.nl = 0;
     for (const int nl : {4, 8, 16}) {
         const int64_t seg = (int64_t)fs::SK_LT * nl * 4, n = ((int64_t)V + seg - 1) / seg;
-        if (n * nl > 256) continue;
+        if (n * nl > 256 || n > fs::MK_MAX_SEGS) continue;
         c.nl = nl;
         c.nseg = (int)n;
         if (rows * n <= 4 * (int64_t)cus) break;

@@ -267,7 +267,10 @@ int fs_error_word(fs_context* ctx, const int32_t** d_bits);
 
 /* The merge's bounded wait for a row's segments, in polls (0 = the default, 2^20: far above any segment's time).
  * A smaller limit makes merges give up (FS_DEVERR_INTERNAL) and compute their rows alone; FS_WAIT_GIVE_UP makes
- * every merge give up without polling: tests of that path. */
+ * every merge give up without polling: tests of that path. The segments of a row wait for each other in the mid-k
+ * kernel; their number is limited so that calls of several contexts on the four hardware queues a process has by default
+ * never fill an XCD with rows that are not dispatched whole. With more queues in use at once (GPU_MAX_HW_QUEUES, other
+ * processes) such rows may wait out this limit; their results are exact all the same. */
 #define FS_WAIT_GIVE_UP 0xFFFFFFFFu
 int fs_set_wait_limit(fs_context* ctx, uint32_t polls);
 

@@ -288,6 +288,31 @@ def test_mid_k_give_up_is_exact():
         assert F.device_error(ctx) == bits
 
 
+def test_mid_k_on_several_streams():
+    """Three contexts on three streams, calls of few rows with the most segments each (they wait for each other) in
+    flight together."""
+    rng = np.random.default_rng(21)
+    B, V = 9, 262144
+    x = torch.from_numpy(W.mixture_logits(rng, B, V)).cuda()
+    want, outs = [], []
+    cfg = [(mid_params(B, k), rng.random(B), F.sampler.Context(), torch.cuda.Stream()) for k in (100, 0, 300)]
+    cfg[1][0]["top_p"] = 0.9
+    for p, u, ctx, _ in cfg:
+        o = O.sample_batch(x.cpu().numpy(), np.zeros(0, np.int32), np.zeros(B + 1, np.int64), p, u, kcap=1, nthreads=NT)
+        want.append(o["tok"])
+        F.sample_batch(x, p, u, ctx=ctx)
+    torch.cuda.synchronize()
+    for _ in range(12):
+        for i, (p, u, ctx, st) in enumerate(cfg):
+            with torch.cuda.stream(st):
+                outs.append((i, F.sample_batch(x, p, u, ctx=ctx)["tok"]))
+    torch.cuda.synchronize()
+    for i, tok in outs:
+        np.testing.assert_array_equal(tok.cpu().numpy(), want[i])
+    for _, _, ctx, _ in cfg:
+        assert F.device_error(ctx) == 0
+
+
 def test_mid_k_decode_steps():
     """Decode steps the mid-k kernel takes: history copies, draws and appends beside k > 64 and frequency penalties."""
     rng = np.random.default_rng(12)
