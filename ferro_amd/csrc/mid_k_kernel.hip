@@ -22,6 +22,7 @@
 // Rows with every token a candidate (ak_segment, ak_finish) stay in registers through all their passes; the fused kernel
 // reads such a row again for each, and gave flat ones to one workgroup: 32 rows of 65536 N(0, 2) logits at temperature 1
 // 51.5 us -> 23.5, 3 rows of 178740 507 -> 21, 64 rows of 262144 heavy-tailed logits with top-p 0.95 37.5 -> 35.7.
+#include "exp_table.hpp"
 #include "row_device.hpp"
 
 #include <type_traits>
@@ -76,6 +77,7 @@ struct MkShared {
         uint32_t hist[MK_H];               // the bound's histograms; mk_slow's digits
         uint32_t rk[SK_LT];                // partial ranks of a short list
         uint32_t srt[SK_NW][WAVE];         // the waves' sorted lane maxima
+        double2 pow2[64];                  // every token a candidate: 2^(j/64) in two parts
     } h;
     union {
         uint32_t bmp[SK_LT * 2];           // one bit per logit of the window's ids: 64 bits per thread; mk_slow: by id
@@ -90,7 +92,6 @@ struct MkShared {
     double dmisc;
     uint64_t umisc[2];
     uint32_t gn[4];
-    double pow2[64];                       // every token a candidate: 2^(j/64)
 #ifdef FS_TRACE
     uint64_t trace_t[16];
 #endif
@@ -475,38 +476,6 @@ __device__ __forceinline__ void mk_softmax(const SkArgs& a, const fs_row_params&
 }
 
 // ---- every token a candidate (top_k = 0: k = V)
-// 2^(j/64), correctly rounded.
-__device__ double ak_pow2[64] = {
-    0x1.0000000000000p+0, 0x1.02c9a3e778061p+0, 0x1.059b0d3158574p+0, 0x1.0874518759bc8p+0,
-    0x1.0b5586cf9890fp+0, 0x1.0e3ec32d3d1a2p+0, 0x1.11301d0125b51p+0, 0x1.1429aaea92de0p+0,
-    0x1.172b83c7d517bp+0, 0x1.1a35beb6fcb75p+0, 0x1.1d4873168b9aap+0, 0x1.2063b88628cd6p+0,
-    0x1.2387a6e756238p+0, 0x1.26b4565e27cddp+0, 0x1.29e9df51fdee1p+0, 0x1.2d285a6e4030bp+0,
-    0x1.306fe0a31b715p+0, 0x1.33c08b26416ffp+0, 0x1.371a7373aa9cbp+0, 0x1.3a7db34e59ff7p+0,
-    0x1.3dea64c123422p+0, 0x1.4160a21f72e2ap+0, 0x1.44e086061892dp+0, 0x1.486a2b5c13cd0p+0,
-    0x1.4bfdad5362a27p+0, 0x1.4f9b2769d2ca7p+0, 0x1.5342b569d4f82p+0, 0x1.56f4736b527dap+0,
-    0x1.5ab07dd485429p+0, 0x1.5e76f15ad2148p+0, 0x1.6247eb03a5585p+0, 0x1.6623882552225p+0,
-    0x1.6a09e667f3bcdp+0, 0x1.6dfb23c651a2fp+0, 0x1.71f75e8ec5f74p+0, 0x1.75feb564267c9p+0,
-    0x1.7a11473eb0187p+0, 0x1.7e2f336cf4e62p+0, 0x1.82589994cce13p+0, 0x1.868d99b4492edp+0,
-    0x1.8ace5422aa0dbp+0, 0x1.8f1ae99157736p+0, 0x1.93737b0cdc5e5p+0, 0x1.97d829fde4e50p+0,
-    0x1.9c49182a3f090p+0, 0x1.a0c667b5de565p+0, 0x1.a5503b23e255dp+0, 0x1.a9e6b5579fdbfp+0,
-    0x1.ae89f995ad3adp+0, 0x1.b33a2b84f15fbp+0, 0x1.b7f76f2fb5e47p+0, 0x1.bcc1e904bc1d2p+0,
-    0x1.c199bdd85529cp+0, 0x1.c67f12e57d14bp+0, 0x1.cb720dcef9069p+0, 0x1.d072d4a07897cp+0,
-    0x1.d5818dcfba487p+0, 0x1.da9e603db3285p+0, 0x1.dfc97337b9b5fp+0, 0x1.e502ee78b3ff6p+0,
-    0x1.ea4afa2a490dap+0, 0x1.efa1bee615a27p+0, 0x1.f50765b6e4540p+0, 0x1.fa7c1819e90d8p+0};
-// exp(z), -40 < z <= 0, within 2.3e-16 (Tang's table method: z = n ln2/64 + r, the degree-5 polynomial of e^r - 1 on
-// |r| < ln2/128, the table's 2^(j/64)); the ocml function takes twice the instructions. pow2: the table in LDS.
-__device__ __forceinline__ double ak_exp(double z, const double* pow2) {
-    const double n = __builtin_rint(z * 0x1.71547652b82fep+6);
-    const int i = (int)n;
-    double r = __builtin_fma(-n, 0x1.62e42fee00000p-7, z);
-    r = __builtin_fma(-n, 0x1.a39ef35793c76p-39, r);
-    double q = __builtin_fma(r, 1.0 / 120.0, 1.0 / 24.0);
-    q = __builtin_fma(r, q, 1.0 / 6.0);
-    q = __builtin_fma(r, q, 0.5);
-    q = __builtin_fma(r * r, q, r);
-    const double t = pow2[i & 63];
-    return __builtin_ldexp(__builtin_fma(t, q, t), i >> 6);
-}
 __device__ __forceinline__ double ak_mass(float x, float mx, double Td) { return exp((double)(x - mx) / Td); }
 
 // A row's segments meet: arrive, then wait (bounded) for `target` arrivals. What the caller published is drained first.
@@ -753,7 +722,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     const double Td = (double)p.temperature, inv = 1.0 / Td;
     const float invf = 1.0f / p.temperature;
     r.u = u;
-    const uint64_t pow2 = ld_agent(reinterpret_cast<const uint64_t*>(ak_pow2) + lane);   // (it arrives behind the meeting)
+    const double2 pow2 = reinterpret_cast<const double2*>(exp_pow2)[lane];   // (it arrives behind the meeting)
     penalise();
     if (CAP && p.softcap > 0.0f) {
 #pragma unroll
@@ -805,7 +774,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     }
     if (!mk_meet(ctr, (uint32_t)nseg, mk.spins, s)) return false;
     SK_MARK(2);
-    if (tid < 64) s.pow2[tid] = __longlong_as_double((long long)pow2);   // (the barrier before the masses publishes it)
+    if (tid < 64) s.h.pow2[tid] = pow2;                        // (the barrier before the masses publishes it)
     {
         const uint64_t e = lane < nseg ? line[lane * 32] : 0xFFFFFFFFull;
         r.nv = wave_allreduce(lane < nseg ? (uint32_t)line[lane * 32 + 1] : 0u, add_u);
@@ -871,7 +840,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
             const double d = (double)(x - mx);                 // fp32 subtraction, as ferro; then d / Td, correctly rounded
             double z = d * inv;
             z = __builtin_fma(__builtin_fma(-z, Td, d), inv, z);
-            const double m = ak_exp(z, s.pow2);
+            const double m = exp_table(z, s.h.pow2);
             part += m;
             const uint64_t f = (uint64_t)__double_as_longlong(__builtin_fma(m, AK_FX, 0x1p52)) - 0x4330000000000000ull;
             atomicAdd(reinterpret_cast<unsigned long long*>(&s.u.a.mass[b]), (unsigned long long)f);
@@ -948,7 +917,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
             const double tgt = (double)p.top_p * r.S;
             ok = ak_locate(cum, row_mass, (uint64_t)(tgt * AK_FX), r.bc, before);
             r.above_c = (double)before / AK_FX;
-            const double most = ak_exp(-(double)(ok ? r.bc : 0) * (double)depth * (1.0 / AK_BINS), s.pow2) * (1.0 + 1e-4);
+            const double most = exp_table(-(double)(ok ? r.bc : 0) * (double)depth * (1.0 / AK_BINS), s.h.pow2) * (1.0 + 1e-4);
             const double thi = tgt + most < r.S ? tgt + most : r.S;
             if (ok) ok = ak_locate(cum, row_mass, (uint64_t)(u * tgt * (1.0 - 1e-12) * AK_FX), r.d0, before);
             r.above_d = (double)before / AK_FX;
