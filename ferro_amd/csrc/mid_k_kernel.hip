@@ -46,7 +46,7 @@ constexpr int AK_BINS = 2048;              // every token a candidate: mass bins
 constexpr int AK_STAGE = 1024;             // logits of the searched bins that a segment stages, per list
 constexpr int AK_LIST = MK_LCAP / 2;       // entries of a row's two lists of such logits
 constexpr float AK_DEPTH = 32.0f;          // temperatures below the maximum that the bins reach
-constexpr double AK_FX = 17592186044416.0; // 2^44: fixed-point mass scale (a mass is <= 1)
+constexpr double AK_FX = 17592186044416.0; // 2^44: fixed-point mass scale of ak_slow (a mass is <= 1)
 
 struct MkShared {
     // in turn: the window's 16-bit counts per logit of the segment (frequency / presence); the merge's sorted candidates
@@ -751,16 +751,22 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
         n += x == x ? 1u : 0u;
     }
     auto add_u = [](uint32_t x, uint32_t y) { return x + y; };
+    auto add_f = [](float x, float y) { return x + y; };
     auto add_d = [](double x, double y) { return x + y; };
     uint32_t kx = wave_max(key_of(hi)), kn = wave_min(lo == lo ? key_of(lo) : 0xFFFFFFFFu);
     n = wave_allreduce(n, add_u);
+    // two 128-byte lines per segment, one per meeting (a line is read by others only after the meeting it is written for)
+    uint64_t* line = reinterpret_cast<uint64_t*>(mk.qk) + ((int64_t)row * nseg) * 32;
+    // a bound of the wave's mass, relative to its maximum: its lane maxima's masses, times the most logits a lane has
+    const float wm = kx > 0x007FFFFFu ? val_of(kx) : -__builtin_huge_valf();
+    const float wb = wave_allreduce(hi > -__builtin_huge_valf() ? __expf((hi - wm) * invf) : 0.0f, add_f) *
+                     (float)(NL * 4 + (nf + WAVE - 1) / WAVE);
     if (lane == 0) {
         s.w64[w] = ((uint64_t)kx << 32) | kn;
         s.w32[w] = n;
+        line[seg * 32 + 2 + w] = ((uint64_t)__float_as_uint(wm) << 32) | __float_as_uint(wb);
     }
     __syncthreads();
-    // two 128-byte lines per segment, one per meeting (a line is read by others only after the meeting it is written for)
-    uint64_t* line = reinterpret_cast<uint64_t*>(mk.qk) + ((int64_t)row * nseg) * 32;
     if (tid == 0) {
 #pragma unroll
         for (int q = 1; q < SK_NW; ++q) {
@@ -775,14 +781,30 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     if (!mk_meet(ctr, (uint32_t)nseg, mk.spins, s)) return false;
     SK_MARK(2);
     if (tid < 64) s.h.pow2[tid] = pow2;                        // (the barrier before the masses publishes it)
+    uint64_t we[SK_NW];
     {
         const uint64_t e = lane < nseg ? line[lane * 32] : 0xFFFFFFFFull;
+#pragma unroll
+        for (int q = 0; q < SK_NW; ++q) we[q] = lane < nseg ? line[lane * 32 + 2 + q] : 0xFF800000ull << 32;
         r.nv = wave_allreduce(lane < nseg ? (uint32_t)line[lane * 32 + 1] : 0u, add_u);
         kx = wave_max((uint32_t)(e >> 32));
         kn = wave_min((uint32_t)e);
     }
     const float mx = val_of(kx), mn = val_of(kn);
     r.mx = mx;
+    // The bins' fixed-point scale, a power of two: the largest at which the row's mass fits 63 bits, by the segments' bounds
+    // (one per cent for their roundings), and at most 2^52 (a mass is <= 1). A spiky row (bound < 2048) sums its masses to
+    // 2^-53, as fp64 does; the flattest row the layout takes (262144 equal logits) to 2^-45.
+    float bound = 0.0f;
+#pragma unroll
+    for (int q = 0; q < SK_NW; ++q) {
+        const float x = __uint_as_float((uint32_t)(we[q] >> 32));
+        if (x > -__builtin_huge_valf()) bound += __uint_as_float((uint32_t)we[q]) * __expf((x - mx) * invf);
+    }
+    bound = wave_allreduce(bound, add_f) * 1.01f;
+    const int be = (int)((__float_as_uint(bound) >> 23) & 255u) - 126;          // bound < 2^be
+    const int fxe = __builtin_amdgcn_readfirstlane(63 - be < 52 ? 63 - be : 52);
+    const double fx = __builtin_ldexp(1.0, fxe), ifx = __builtin_ldexp(1.0, -fxe);
     float depth = (mx - mn) * invf;
     const bool tail = !(depth < AK_DEPTH);
     depth = tail ? AK_DEPTH : depth;
@@ -842,7 +864,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
             z = __builtin_fma(__builtin_fma(-z, Td, d), inv, z);
             const double m = exp_table(z, s.h.pow2);
             part += m;
-            const uint64_t f = (uint64_t)__double_as_longlong(__builtin_fma(m, AK_FX, 0x1p52)) - 0x4330000000000000ull;
+            const uint64_t f = (uint64_t)__double_as_longlong(__builtin_fma(m, fx, 0x1p52)) - 0x4330000000000000ull;
             atomicAdd(reinterpret_cast<unsigned long long*>(&s.u.a.mass[b]), (unsigned long long)f);
         } else if (x == x) {
             rest += __expf((x - mx) * invf);
@@ -915,17 +937,17 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
             // top-p keeps through its crossing candidate (sampler.cpp:44), so the kept total lies in [tgt, tgt + the
             // largest mass of bin bc]: the draw's bin at both ends
             const double tgt = (double)p.top_p * r.S;
-            ok = ak_locate(cum, row_mass, (uint64_t)(tgt * AK_FX), r.bc, before);
-            r.above_c = (double)before / AK_FX;
+            ok = ak_locate(cum, row_mass, (uint64_t)(tgt * fx), r.bc, before);
+            r.above_c = (double)before * ifx;
             const double most = exp_table(-(double)(ok ? r.bc : 0) * (double)depth * (1.0 / AK_BINS), s.h.pow2) * (1.0 + 1e-4);
             const double thi = tgt + most < r.S ? tgt + most : r.S;
-            if (ok) ok = ak_locate(cum, row_mass, (uint64_t)(u * tgt * (1.0 - 1e-12) * AK_FX), r.d0, before);
-            r.above_d = (double)before / AK_FX;
-            if (ok && !ak_locate(cum, row_mass, (uint64_t)(u * thi * (1.0 + 1e-12) * AK_FX), r.d1, before)) r.d1 = r.bc;
+            if (ok) ok = ak_locate(cum, row_mass, (uint64_t)(u * tgt * (1.0 - 1e-12) * fx), r.d0, before);
+            r.above_d = (double)before * ifx;
+            if (ok && !ak_locate(cum, row_mass, (uint64_t)(u * thi * (1.0 + 1e-12) * fx), r.d1, before)) r.d1 = r.bc;
             if (r.d1 > r.bc) r.d1 = r.bc;
         } else {
-            ok = ak_locate(cum, row_mass, (uint64_t)(u * r.S * AK_FX), r.d0, before);
-            r.above_d = (double)before / AK_FX;
+            ok = ak_locate(cum, row_mass, (uint64_t)(u * r.S * fx), r.d0, before);
+            r.above_d = (double)before * ifx;
             r.d1 = r.d0;
         }
         r.plain = !ok;                                         // past the binned mass: the row is selected alone

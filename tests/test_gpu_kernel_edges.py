@@ -375,6 +375,33 @@ def test_every_token_a_candidate(B, V, top_p):
     assert F.device_error() == 0
 
 
+def test_every_token_draws_next_to_a_boundary():
+    """Rows whose mass is ten logits, draws 6e-15 below and above the cumulative mass of each, computed in 80 bits. Ten
+    masses summed in fp64 (or in units of 2^-52), each within 0.52 ulp, are off by less than 5e-15 of a sum >= 1; units of
+    2^-44 would be off by up to 3e-14 each."""
+    if np.finfo(np.longdouble).nmant < 63:
+        pytest.skip("no 80-bit long double")
+    rng = np.random.default_rng(44)
+    B, V = 60, 40000
+    x = np.full((B, V), -90.0, np.float32)
+    p = mid_params(B, 0, temperature=1.0)
+    p["top_p"] = 1.0
+    u, want = np.zeros(B), np.zeros(B, np.int32)
+    for b in range(B):
+        at = rng.choice(V, 10, replace=False)
+        x[b, at] = rng.uniform(-2, 0, 10).astype(np.float32)
+        order = at[np.lexsort((at, -x[b, at]))]
+        m = np.exp((x[b, order] - x[b].max()).astype(np.longdouble))
+        c = np.cumsum(m)
+        total = c[-1] + (V - 10) * np.exp(np.longdouble(-90.0) - np.longdouble(x[b].max()))
+        j = int(rng.integers(2, 8))
+        above = b % 2
+        u[b] = float(c[j] / total * (1 + (6e-15 if above else -6e-15)))
+        want[b] = order[j + above]
+    out = F.sample_batch(torch.from_numpy(x).cuda(), p, u)
+    np.testing.assert_array_equal(out["tok"].cpu().numpy(), want)
+
+
 def test_every_token_give_up_and_decode():
     """Rows whose segments do not wait for each other are selected alone; decode steps and verification windows with
     top_k = 0."""
