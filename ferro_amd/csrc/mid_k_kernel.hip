@@ -315,12 +315,94 @@ __device__ __forceinline__ uint32_t mk_slow(const float* rowp, int V, int k, boo
     return s.misc[2];
 }
 
+// Sorts the ranges of s.u.m.top on the work list (s.prel: start, length; s.misc[3] of them) in place, descending: a
+// counting sort over the range's span, 1024 bins at a time, entries ranked within their bin; a bin of more than MK_HEAVY
+// goes back on the list (equal logits: the bins then spread their ids). Whole workgroup, after a barrier; ends with one.
+constexpr uint32_t MK_HEAVY = 64;
+__device__ __forceinline__ void mk_spread(MkShared& s) {
+    constexpr int RPT = MK_TOP / SK_LT;
+    const int tid = threadIdx.x;
+#pragma unroll 1
+    for (uint32_t work = s.misc[3]; work != 0u; work = s.misc[3]) {
+        const int lo = s.prel[2 * work - 2], n = s.prel[2 * work - 1];
+        uint64_t* t = s.u.m.top + lo;
+        uint64_t e[RPT], mn = ~0ull, mx = 0ull;
+        uint32_t at[RPT];
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int i = q * SK_LT + tid;
+            e[q] = i < n ? t[i] : 0ull;
+            if (i < n) {
+                mn = e[q] < mn ? e[q] : mn;
+                mx = e[q] > mx ? e[q] : mx;
+            }
+        }
+        *reinterpret_cast<uint4*>(&s.h.hist[4 * tid]) = make_uint4(0u, 0u, 0u, 0u);
+        mn = mk_min_u64(mn, s);
+        mx = mk_max_u64(mx, s);
+        if (tid == 0) s.misc[3] = work - 1u;                   // (every thread has read it)
+        const int bits = 64 - __clzll((long long)((mx - mn) | 1ull)), sh = bits > 10 ? bits - 10 : 0;
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            at[q] = 0u;
+            if (q * SK_LT + tid < n) {
+                const uint32_t b = (uint32_t)((mx - e[q]) >> sh);
+                at[q] = (b << 16) | atomicAdd(&s.h.hist[b], 1u);
+            }
+        }
+        __syncthreads();
+        const uint4 c = *reinterpret_cast<const uint4*>(&s.h.hist[4 * tid]);
+        uint32_t tot;
+        const uint32_t o0 = mk_excl_u32(c.x + c.y + c.z + c.w, s, tot), o1 = o0 + c.x, o2 = o1 + c.y, o3 = o2 + c.z;
+        *reinterpret_cast<uint4*>(&s.h.hist[4 * tid]) = make_uint4(o0, o1, o2, o3);
+        auto again = [&](uint32_t o, uint32_t m) {
+            if (m > MK_HEAVY) {
+                const uint32_t w = atomicAdd(&s.misc[3], 1u);
+                s.prel[2 * w] = (uint16_t)(lo + (int)o);
+                s.prel[2 * w + 1] = (uint16_t)m;
+            }
+        };
+        again(o0, c.x); again(o1, c.y); again(o2, c.z); again(o3, c.w);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < RPT; ++q)
+            if (q * SK_LT + tid < n) t[s.h.hist[at[q] >> 16] + (at[q] & 0xFFFFu)] = e[q];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int i = q * SK_LT + tid;
+            at[q] = 0u;
+            if (i < n) {
+                e[q] = t[i];
+                const uint32_t b = (uint32_t)((mx - e[q]) >> sh);
+                const uint32_t b0 = s.h.hist[b], b1 = b < (uint32_t)MK_H - 1u ? s.h.hist[b + 1] : (uint32_t)n;
+                uint32_t x = b0;
+                if (b1 - b0 > MK_HEAVY) x = (uint32_t)i;
+                else
+                    for (uint32_t j = b0; j < b1; ++j) x += t[j] > e[q] ? 1u : 0u;
+                at[q] = x;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < RPT; ++q)
+            if (q * SK_LT + tid < n) t[at[q]] = e[q];
+        __syncthreads();
+    }
+}
+
 // Sorts the row's list (n <= MK_LCAP composites in registers, 0: none) into s.u.m.top[0, min(n, k)), descending: a
 // counting sort over the span of the composites, of which only the bins that hold the first k are placed; entries rank
-// themselves within their bin. Returns false when those bins hold more than MK_TOP entries (hundreds of ties at the
-// k-th). Whole workgroup.
+// themselves within their bin, and bins of many entries (equal logits) are spread further first (ranked at once, rows of
+// logits rounded to whole numbers took 120 us: 32 rows of 262144, k 200; now 31). Returns false when the bins
+// that hold the first k have more than MK_TOP entries (hundreds of ties at the k-th). Whole workgroup.
+// In two parts (mk_sort_end does not depend on EPT: one copy of it for the kernel's instruction cache).
+struct MkSorted {
+    uint64_t cmx;                          // the largest composite; the bins' shift; entries placed, -1: too many
+    int sh, m;
+};
 template <int EPT>
-__device__ __forceinline__ bool mk_sort(const uint64_t (&v)[EPT], int n, int k, MkShared& s) {
+__device__ __forceinline__ MkSorted mk_sort(const uint64_t (&v)[EPT], int n, int k, MkShared& s) {
     const int tid = threadIdx.x;
     uint64_t cmn = ~0ull, cmx = 0ull;
 #pragma unroll
@@ -331,6 +413,7 @@ __device__ __forceinline__ bool mk_sort(const uint64_t (&v)[EPT], int n, int k, 
         }
     }
     for (int i = tid; i < MK_BINS; i += SK_LT) s.u.m.bins[i] = 0u;
+    if (tid == 0) s.misc[3] = 0u;                              // bins to spread
     cmn = mk_min_u64(cmn, s);
     cmx = mk_max_u64(cmx, s);
     const uint64_t span = cmx - cmn;
@@ -356,17 +439,22 @@ __device__ __forceinline__ bool mk_sort(const uint64_t (&v)[EPT], int n, int k, 
     }
     uint32_t tot;
     uint32_t off = mk_excl_u32(sum, s, tot);
-    if (tid == 0) s.misc[3] = (uint32_t)n;                     // entries in the bins that start before k
 #pragma unroll
     for (int j = 0; j < BPT; ++j) {
         s.u.m.bins[BPT * tid + j] = off;
         if (off < (uint32_t)k && off + c[j] >= (uint32_t)k) s.misc[4] = off + c[j];
+        if (off < (uint32_t)k && c[j] > MK_HEAVY && off + c[j] <= (uint32_t)MK_TOP) {
+            const uint32_t w = atomicAdd(&s.misc[3], 1u);
+            s.prel[2 * w] = (uint16_t)off;
+            s.prel[2 * w + 1] = (uint16_t)c[j];
+        }
         off += c[j];
     }
+    static_assert(2 * (MK_TOP / (int)MK_HEAVY) <= MK_PC, "the work list holds every heavy bin");
     if (tid == SK_LT - 1) s.u.m.bins[MK_BINS] = off;
     __syncthreads();
     const int m = n <= k ? n : (int)s.misc[4];
-    if (m > MK_TOP) return false;
+    if (m > MK_TOP) return {0ull, 0, -1};
 #pragma unroll
     for (int q = 0; q < EPT; ++q) {
         if (q * SK_LT + tid < n) {
@@ -375,26 +463,34 @@ __device__ __forceinline__ bool mk_sort(const uint64_t (&v)[EPT], int n, int k, 
         }
     }
     __syncthreads();
-    constexpr int TPT_ = EPT < MK_TOP / SK_LT ? EPT : MK_TOP / SK_LT;
-    uint64_t e[TPT_];
-    uint32_t r[TPT_];
+    return {cmx, sh, m};
+}
+__device__ __forceinline__ bool mk_sort_end(const MkSorted& o, int k, MkShared& s) {
+    constexpr int RPT = MK_TOP / SK_LT;
+    const int tid = threadIdx.x, m = o.m;
+    if (m < 0) return false;
+    if (s.misc[3] != 0u) mk_spread(s);
+    uint64_t e[RPT];
+    uint32_t r[RPT];
 #pragma unroll
-    for (int q = 0; q < TPT_; ++q) {
+    for (int q = 0; q < RPT; ++q) {
         const int i = q * SK_LT + tid;
         e[q] = 0ull;
         r[q] = 0xFFFFFFFFu;
         if (i < m) {
             e[q] = s.u.m.top[i];
-            const uint32_t b = (uint32_t)((cmx - e[q]) >> sh);
+            const uint32_t b = (uint32_t)((o.cmx - e[q]) >> o.sh);
             const uint32_t lo = s.u.m.bins[b], hi = s.u.m.bins[b + 1];
             uint32_t x = lo;
-            for (uint32_t j = lo; j < hi; ++j) x += s.u.m.top[j] > e[q] ? 1u : 0u;
+            if (hi - lo > MK_HEAVY) x = (uint32_t)i;           // (spread: in place already)
+            else
+                for (uint32_t j = lo; j < hi; ++j) x += s.u.m.top[j] > e[q] ? 1u : 0u;
             r[q] = x;
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < TPT_; ++q)
+    for (int q = 0; q < RPT; ++q)
         if (r[q] < (uint32_t)k) s.u.m.top[r[q]] = e[q];
     __syncthreads();
     return true;
@@ -1080,7 +1176,7 @@ __device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uin
 #pragma unroll
             for (int q = 0; q < EPT; ++q) e[q] = entry(q * SK_LT + tid);
             __syncthreads();
-            if (!mk_sort(e, n, n, s)) return false;
+            if (!mk_sort_end(mk_sort(e, n, n, s), n, s)) return false;
         }
         double cum;
         const double target = pass == 0 ? (double)p.top_p * r.S : r.u * tot + 0.0;
@@ -1659,8 +1755,11 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
                 __syncthreads();
                 sk_rank(cand, s.h.rk, (int)C, [&](uint32_t r, uint64_t c) { if (r < (uint32_t)k) s.u.m.top[r] = c; });
                 __syncthreads();
-            } else if (C <= 4u * SK_LT) sorted = sort_list(std::integral_constant<int, 4>{});
-            else sorted = sort_list(std::integral_constant<int, MK_LCAP / SK_LT>{});
+            } else {
+                const MkSorted o = C <= 4u * SK_LT ? sort_list(std::integral_constant<int, 4>{})
+                                                   : sort_list(std::integral_constant<int, MK_LCAP / SK_LT>{});
+                sorted = mk_sort_end(o, k, s);
+            }
             SK_MARK(7);
             if (sorted && greedy) {
                 if (w == 0) greedy_end(s.u.m.top[0]);

@@ -232,6 +232,28 @@ def test_mid_k_softcap_and_penalties_without_a_bound(V, k, cap):
     check(x, p, hists, rng.random(6), kcap=k)
 
 
+@pytest.mark.parametrize("k", [200, 1500, 2048])
+def test_mid_k_lists_of_equal_logits(k):
+    """Candidate lists of a few values: whole numbers, two neighbouring floats below one far larger logit (both fall in one
+    bin of the sort, their ids in one bin of the next), equal logits at neighbouring ids."""
+    rng = np.random.default_rng(k)
+    B, V = 5, 100000
+    x = np.full((B, V), -5.0, np.float32) + rng.random((B, V)).astype(np.float32)
+    x[0] = np.round(rng.standard_normal(V) * 2)
+    at = rng.permutation(V)
+    x[1, at[:1100]] = 3.0
+    x[1, at[1100:2100]] = np.nextafter(np.float32(3.0), np.float32(4.0))
+    x[1, 17] = 1e6
+    x[2, 5000:6000] = 2.0
+    x[2, 90000:90700] = 2.0
+    x[2, at[:90]] = 2.5
+    x[3, at[:2400]] = bf16_valued(x[3, at[:2400]] * 0.01 + 6)
+    x[4, at[:700]] = 1.0
+    x[4, at[700:1500]] = 2.0
+    x[4, at[1500:2300]] = 3.0
+    check(x, mid_params(B, k, temperature=2.0), [[]] * B, rng.random(B), kcap=2048)
+
+
 def test_mid_k_more_penalised_ids_than_the_spill_list():
     rng = np.random.default_rng(5)
     V, H = 262144, 40000

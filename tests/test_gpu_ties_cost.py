@@ -1,0 +1,69 @@
+"""Rows with many equal logits cost a small multiple of rows without (coarse logits, masks with a finite value): the whole
+device works on them, not one workgroup. Times of the same call on the same shapes, side by side; the bounds leave a
+factor of two over what was measured."""
+import ctypes
+import os
+import sys
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+
+from ferro_amd import workloads as W  # noqa: E402
+from ferro_amd._lib import lib  # noqa: E402
+import ferro_amd as F  # noqa: E402
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    yield
+    torch.cuda.synchronize()
+
+
+def P(t):
+    return ctypes.c_void_p(t.data_ptr())
+
+
+def time_us(x, k, top_p=0.95, **kw):
+    """Median over five blocks of eight calls."""
+    B, V = x.shape
+    p = W.make_params(B, temperature=0.8, top_k=k, top_p=top_p, repetition_penalty=1.0)
+    for f, v in kw.items():
+        p[f] = v
+    d = torch.from_numpy(x).cuda()
+    dp = torch.from_numpy(p.view(np.uint8).copy()).cuda()
+    u = torch.from_numpy(np.random.default_rng(1).random(B)).cuda()
+    hist = torch.arange(B * 64, dtype=torch.int32, device="cuda")
+    off = torch.arange(B + 1, dtype=torch.int64, device="cuda") * 64
+    tok = torch.empty(B, dtype=torch.int32, device="cuda")
+    ctx, st = F.sampler.Context(), torch.cuda.current_stream()
+
+    def call():
+        rc = lib().fs_sample_batch_hp(ctx.h, P(d), V, B, V, P(hist), P(off), P(dp), p.ctypes.data_as(ctypes.c_void_p),
+                                      P(u), P(tok), 0, None, None, None, ctypes.c_void_p(st.cuda_stream))
+        assert rc == 0
+    call()
+    torch.cuda.synchronize()
+    t = []
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(8):
+            call()
+        b.record()
+        b.synchronize()
+        t.append(a.elapsed_time(b) * 1e3 / 8)
+    assert F.device_error(ctx) == 0
+    return sorted(t)[2]
+
+
+def test_lists_of_equal_logits():
+    rng = np.random.default_rng(2)
+    x = (rng.standard_normal((32, 262144)) * 2).astype(np.float32)
+    plain, coarse = time_us(x, 200), time_us(np.round(x), 200)
+    assert coarse < 3.5 * plain, (plain, coarse)
