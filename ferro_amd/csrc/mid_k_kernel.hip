@@ -14,7 +14,8 @@
 //     places; the last segment to finish (an L2 ticket) sorts the list and samples the row.
 // The waiting is bounded and a row's segments are consecutive workgroups of one XCD, dispatched in order; a segment that
 // gives up (or a list that overflows: thousands of equal logits at the bound) marks the row, and its last segment then
-// selects the row's exact top k from the logits alone (mk_slow).
+// selects the row's exact top k from the logits alone (mk_slow). Equal logits at the bound in larger numbers than the list
+// takes are counted first (one meeting more), and only the row's first ones written.
 // Bound: HBM, one read of the logits, then the chain behind a row's last logits.
 // Measured against the fused kernel (running bounds, per-row merges of the segments' lists): 256 rows of 262144 logits
 // with k from 1 to 2048 and every penalty 124 us -> 77; 24 rows of 100003 logits, k 200, frequency / presence 35 -> 19.5;
@@ -173,9 +174,10 @@ __device__ __forceinline__ bool mk_locate(MkShared& s, uint32_t kk, uint32_t& b,
 
 // The row's bound from its segments' published keys (nseg * SK_NW lists of 16): the largest 20-bit prefix T (sign,
 // exponent, 11 mantissa bits) such that the weights of the keys at or above it add up to k, 1 when they do not. Two
-// histograms of ten key bits each in LDS. Whole workgroup; s.h.hist is zero on entry.
+// histograms of ten key bits each in LDS. sum: those weights' sum; need: what the keys of T's own prefix have to add.
+// Whole workgroup; s.h.hist is zero on entry.
 template <int NQ>
-__device__ __forceinline__ uint32_t mk_bound(const uint32_t* qk, int nseg, int k, MkShared& s) {
+__device__ __forceinline__ uint32_t mk_bound(const uint32_t* qk, int nseg, int k, MkShared& s, uint32_t& sum, uint32_t& need) {
     const int tid = threadIdx.x;
     const int n4 = nseg * SK_NW * 4;                           // 16-byte quarters of the lists
     uint4 e[NQ];
@@ -200,6 +202,7 @@ __device__ __forceinline__ uint32_t mk_bound(const uint32_t* qk, int nseg, int k
         add(e[r].w, pk >> 24, 0u, 0);
     }
     __syncthreads();
+    sum = need = 0u;
     if (!mk_locate(s, (uint32_t)k, hi, above)) return 1u;
     *reinterpret_cast<uint4*>(&s.h.hist[4 * tid]) = make_uint4(0u, 0u, 0u, 0u);   // (mk_locate's reads are over)
     __syncthreads();
@@ -212,8 +215,33 @@ __device__ __forceinline__ uint32_t mk_bound(const uint32_t* qk, int nseg, int k
     }
     __syncthreads();
     (void)mk_locate(s, (uint32_t)k - above, lo, above2);
+    sum = above + above2 + s.h.hist[lo];
+    need = (uint32_t)k - above - above2;
     const uint32_t T = (hi << 22) | (lo << 12);
     return T ? T : 1u;
+}
+
+// T's other twelve bits: the largest key such that the weights of the keys at or above it add up to k.
+__device__ __forceinline__ uint32_t mk_bound_exact(const uint32_t* qk, int nseg, uint32_t T, uint32_t need, MkShared& s) {
+    const int tid = threadIdx.x;
+    const uint32_t wgt = mk_rank(tid & 15) - ((tid & 15) ? mk_rank((tid & 15) - 1) : 0u);
+#pragma unroll 1
+    for (int sh = 2, bits = 10; sh >= 0; sh -= 2, bits = 2) {
+        __syncthreads();
+        *reinterpret_cast<uint4*>(&s.h.hist[4 * tid]) = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();
+#pragma unroll 1
+        for (int i = tid; i < nseg * SK_NW * 16; i += SK_LT) {
+            const uint32_t key = qk[i];
+            if (key >> (sh + bits) == T >> (sh + bits)) atomicAdd(&s.h.hist[(key >> sh) & ((1u << bits) - 1u)], wgt);
+        }
+        __syncthreads();
+        uint32_t b = 0u, above = 0u;
+        (void)mk_locate(s, need, b, above);
+        T |= b << sh;
+        need -= above;
+    }
+    return T;
 }
 
 // The row's window of history ids: na ids of the stream's history, then nb of the drafts fed before this row.
@@ -315,6 +343,42 @@ __device__ __forceinline__ uint32_t mk_slow(const float* rowp, int V, int k, boo
     return s.misc[2];
 }
 
+// Of the composites in registers (0: none) exactly the k largest, 0 in the place of the others, packed; there are at
+// least k. A radix select as mk_slow's, for lists that mk_sort does not take. Whole workgroup.
+template <int EPT>
+__device__ __forceinline__ void mk_trim(uint64_t (&e)[EPT], int k, MkShared& s) {
+    const int tid = threadIdx.x;
+    uint64_t prefix = 0ull, mask = 0ull;
+    uint32_t need = (uint32_t)k;
+#pragma unroll 1
+    for (int sh = 54;; sh -= 10) {
+        const int sft = sh < 0 ? 0 : sh;
+        const uint64_t dm = sh < 0 ? 0x3FFull >> -sh : 0x3FFull;
+        __syncthreads();
+        *reinterpret_cast<uint4*>(&s.h.hist[4 * tid]) = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < EPT; ++q)
+            if (e[q] != 0ull && (e[q] & mask) == prefix) atomicAdd(&s.h.hist[(uint32_t)(e[q] >> sft) & (uint32_t)dm], 1u);
+        __syncthreads();
+        uint32_t b = 0u, above = 0u;
+        (void)mk_locate(s, need, b, above);
+        need -= above;
+        prefix |= (uint64_t)b << sft;
+        mask |= dm << sft;
+        if (s.h.hist[b] == need || sh < 0) break;              // the whole bin is inside
+    }
+    if (tid == 0) s.misc[2] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < EPT; ++q)
+        if (e[q] != 0ull && (e[q] & mask) >= prefix) s.u.m.top[atomicAdd(&s.misc[2], 1u)] = e[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < EPT; ++q) e[q] = q * SK_LT + tid < k ? s.u.m.top[q * SK_LT + tid] : 0ull;
+    __syncthreads();
+}
+
 // Sorts the ranges of s.u.m.top on the work list (s.prel: start, length; s.misc[3] of them) in place, descending: a
 // counting sort over the range's span, 1024 bins at a time, entries ranked within their bin; a bin of more than MK_HEAVY
 // goes back on the list (equal logits: the bins then spread their ids). Whole workgroup, after a barrier; ends with one.
@@ -394,11 +458,11 @@ __device__ __forceinline__ void mk_spread(MkShared& s) {
 // Sorts the row's list (n <= MK_LCAP composites in registers, 0: none) into s.u.m.top[0, min(n, k)), descending: a
 // counting sort over the span of the composites, of which only the bins that hold the first k are placed; entries rank
 // themselves within their bin, and bins of many entries (equal logits) are spread further first (ranked at once, rows of
-// logits rounded to whole numbers took 120 us: 32 rows of 262144, k 200; now 31). Returns false when the bins
-// that hold the first k have more than MK_TOP entries (hundreds of ties at the k-th). Whole workgroup.
+// logits rounded to whole numbers took 120 us: 32 rows of 262144, k 200; now 31). Whole workgroup.
 // In two parts (mk_sort_end does not depend on EPT: one copy of it for the kernel's instruction cache).
 struct MkSorted {
-    uint64_t cmx;                          // the largest composite; the bins' shift; entries placed, -1: too many
+    uint64_t cmx;                          // the largest composite; the bins' shift; entries placed, -1: none, as the bins
+                                           // that hold the first k have more than MK_TOP (hundreds of ties at the k-th)
     int sh, m;
 };
 template <int EPT>
@@ -465,10 +529,9 @@ __device__ __forceinline__ MkSorted mk_sort(const uint64_t (&v)[EPT], int n, int
     __syncthreads();
     return {cmx, sh, m};
 }
-__device__ __forceinline__ bool mk_sort_end(const MkSorted& o, int k, MkShared& s) {
+__device__ __forceinline__ void mk_sort_end(const MkSorted& o, int k, MkShared& s) {
     constexpr int RPT = MK_TOP / SK_LT;
     const int tid = threadIdx.x, m = o.m;
-    if (m < 0) return false;
     if (s.misc[3] != 0u) mk_spread(s);
     uint64_t e[RPT];
     uint32_t r[RPT];
@@ -493,7 +556,6 @@ __device__ __forceinline__ bool mk_sort_end(const MkSorted& o, int k, MkShared& 
     for (int q = 0; q < RPT; ++q)
         if (r[q] < (uint32_t)k) s.u.m.top[r[q]] = e[q];
     __syncthreads();
-    return true;
 }
 
 // Softmax at temperature, min-p, top-p and the draw (sampler.cpp:37-49) over the k <= MK_K sorted candidates in
@@ -1176,7 +1238,7 @@ __device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uin
 #pragma unroll
             for (int q = 0; q < EPT; ++q) e[q] = entry(q * SK_LT + tid);
             __syncthreads();
-            if (!mk_sort_end(mk_sort(e, n, n, s), n, s)) return false;
+            mk_sort_end(mk_sort(e, n, n, s), n, s);            // (n <= AK_LIST: they all fit)
         }
         double cum;
         const double target = pass == 0 ? (double)p.top_p * r.S : r.u * tot + 0.0;
@@ -1474,7 +1536,8 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
     SK_MARK(1);
     const bool every = ALL && k > MK_K;                        // every token a candidate
     float tr = 0.0f, tc = 0.0f;                                // the bound: raw, capped
-    bool go = true;
+    float tb = 0.0f, tu = 0.0f;                                // a tied bound: its raw value, the first above its capped one
+    bool go = true, tied = false;
     AkRow ak = {};
     SkDraw dr = {0.0, 0};
     if (ALL && every) {
@@ -1507,10 +1570,19 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
         SK_MARK(3);
         go = s.misc[5] != 0u;
         if (go) {
-            const uint32_t T = mk_bound<NL == 16 ? 1 : 2>(qk, nseg, k, s);
+            uint32_t sum, need;
+            uint32_t T = mk_bound<NL == 16 ? 1 : 2>(qk, nseg, k, s, sum, need);
+            // Lane maxima without ties add up to k and a few more. More than an eighth over it, and the bound is one value
+            // of many logits (a masked vocabulary with fewer than k tokens allowed, coarse logits): where so many lanes
+            // reach it that the row's list may overflow (half of them, or 2048), the segments count them and take the
+            // first ones only. Below that the list takes them all, and is faster (32 rows of 262144 logits rounded to
+            // halves, k 50: 21 us, 28 counted). The same for every segment of the row.
+            const uint32_t lanes = (uint32_t)nseg * SK_LT, many = lanes < MK_LIST ? lanes / 2u : MK_LIST / 2u;
+            tied = sum > (uint32_t)(k + k / 8 + 48) && sum > many;
+            if (tied) T = mk_bound_exact(qk, nseg, T, need, s);
             SK_MARK(4);
             tc = T > 0x007FFFFFu ? val_of(T) : -__builtin_huge_valf();
-            tr = tc;
+            tr = tb = tc;
             if (CAP && pn.cap > 0.0f) {
                 // tc: the capped bound; tr: a raw value that every logit whose capped value reaches tc reaches. Lane
                 // l < 32 caps the value 2^l keys below the bound (lane 32 the bound): the first that falls below tc
@@ -1523,6 +1595,16 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
                 if (below) {
                     const uint32_t st = 1u << (__ffsll((unsigned long long)below) - 1);
                     tr = room > st ? val_of(kb - st) : tr;
+                }
+                if (tied) {                                    // as tr, on the other side
+                    const uint32_t up = 0xFF800000u - kb;      // (the key of inf is the highest)
+                    const float h = softcap_one(val_of(kb + (up > step ? step : up)), pn.cap);
+                    const uint64_t over_ = __ballot(lane < 32 && h > read_lane(c, 32));
+                    tu = __builtin_nanf("");
+                    if (over_) {
+                        const uint32_t st = 1u << (__ffsll((unsigned long long)over_) - 1);
+                        tu = val_of(kb + (up > st ? st : up));
+                    }
                 }
             }
         }
@@ -1549,20 +1631,72 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
         best = mk_max_u64(best, s);
         if (tid == 0) list[seg] = best;
     } else if (!every) {
+        uint64_t gm = 0ull;
+        if (tied) {
+            // Of the logits at the bound only the first can be among the row's top k: as many as the logits above it and
+            // those at it in earlier segments leave of k. The segments count both and meet once more. (Every logit of a
+            // tied row went to the list before, which overflowed: 32 rows of 262144 logits, 20 of them allowed, k 200:
+            // 2920 us with one workgroup per row selecting it, 637 on the fused kernel, now 50.)
+            // With a softcap, logits from tr up to tu have the bound's capped value: those not at the bound go to the list
+            // uncounted.
+            uint64_t eq = 0ull;
+            uint32_t n_up = 0u;
+#pragma unroll
+            for (int q = 0; q < NL; ++q) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    gm |= (uint64_t)(v[q][c] >= tr ? 1u : 0u) << (4 * q + c);
+                    eq |= (uint64_t)(v[q][c] == tb ? 1u : 0u) << (4 * q + c);
+                    if (CAP) n_up += v[q][c] >= tu ? 1u : 0u;
+                }
+            }
+            gm &= ~eq;
+            if (!capped) n_up = (uint32_t)__popcll(gm);
+            auto add = [](uint32_t x, uint32_t y) { return x + y; };
+            const uint32_t g = wave_allreduce(n_up, add);
+            if (lane == 0) s.w32[w] = g;
+#pragma unroll 1
+            for (int q = 0; q < NL; ++q) {                     // in the order of their ids: by q, then by wave
+                const uint32_t t = wave_allreduce((uint32_t)__popc((uint32_t)(eq >> (4 * q)) & 15u), add);
+                if (lane == 0) s.h.hist[q * SK_NW + w] = t;
+            }
+            __syncthreads();
+            const uint32_t t = lane < NL * SK_NW ? s.h.hist[lane] : 0u;
+            const uint32_t incl = wave_incl_scan_u32(t);
+            if (tid == WAVE - 1) {
+                ctr[64 + 2 * seg] = s.w32[0] + s.w32[1] + s.w32[2] + s.w32[3];
+                ctr[65 + 2 * seg] = incl;
+            }
+            go = mk_meet(ctr, 2u * (uint32_t)nseg, mk.spins, s);
+            const uint32_t above = wave_allreduce(lane < nseg ? ld_agent(ctr + 64 + 2 * lane) : 0u, add) +
+                                   wave_allreduce(lane < seg ? ld_agent(ctr + 65 + 2 * lane) : 0u, add);
+            const uint32_t left = above < (uint32_t)k ? (uint32_t)k - above : 0u;
+#pragma unroll 1
+            for (int q = 0; q < NL; ++q) {
+                const uint32_t nib = (uint32_t)(eq >> (4 * q)) & 15u, n = (uint32_t)__popc(nib);
+                uint32_t at = (uint32_t)__shfl((int)(incl - t), q * SK_NW + w) + wave_incl_scan_u32(n) - n;
+                for (int c = 0; c < 4; ++c)
+                    if ((nib >> c) & 1u) {
+                        if (at < left) gm |= 1ull << (4 * q + c);
+                        ++at;
+                    }
+            }
+        }
         if (go) {
             // the logits at or above the bound to the row's list, the penalised ones against the capped bound
             uint32_t np = 0u;
             for (uint32_t i = (uint32_t)lane; i < nf; i += WAVE) np += __uint_as_float((uint32_t)pen_at(i)) >= tc ? 1u : 0u;
-            uint64_t gm = 0ull;
+            if (!tied) {
 #pragma unroll
-            for (int q = 0; q < NL; ++q)                       // (most groups hold none)
-                if (__ballot(fmaxf(fmaxf(v[q][0], v[q][1]), fmaxf(v[q][2], v[q][3])) >= tr) != 0ull) {
+                for (int q = 0; q < NL; ++q)                   // (most groups hold none)
+                    if (__ballot(fmaxf(fmaxf(v[q][0], v[q][1]), fmaxf(v[q][2], v[q][3])) >= tr) != 0ull) {
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) gm |= (uint64_t)(v[q][c] >= tr ? 1u : 0u) << (4 * q + c);
-                }
-            if (tr == -__builtin_huge_valf()) {
-                // fewer than k finite lane maxima (a masked vocabulary): of the logits at -inf only this wave's first
-                // k ids can be among the row's top k
+                        for (int c = 0; c < 4; ++c) gm |= (uint64_t)(v[q][c] >= tr ? 1u : 0u) << (4 * q + c);
+                    }
+            }
+            if (!tied && tr == -__builtin_huge_valf()) {
+                // fewer than k lane maxima (NaN): of the logits at -inf only this wave's first k ids can be among the
+                // row's top k
                 uint64_t eq = 0ull;
 #pragma unroll
                 for (int q = 0; q < NL; ++q)
@@ -1681,9 +1815,8 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
             ctr[35] = 0u;
             if (slow & 2u) atomicOr(a.err, FS_DEVERR_INTERNAL);
         }
-        bool select = again;
-        for (;;) {
-            if (select) {
+        do {
+            if (again) {
                 C = mk_slow<CAP>(rowp, V, k, pen, win, pn, list, s);
                 capped_list = false;
             }
@@ -1746,9 +1879,13 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
                     for (int q = 0; q < EPT; ++q) e[q] = entry(e[q]);
                 }
                 __syncthreads();
-                return mk_sort(e, (int)C, k, s);
+                MkSorted o = mk_sort(e, (int)C, k, s);
+                if (EPT * SK_LT > MK_TOP && o.m < 0) {         // ties at the k-th
+                    mk_trim(e, k, s);
+                    o = mk_sort(e, k, k, s);
+                }
+                return o;
             };
-            bool sorted = true;
             if (C <= (uint32_t)SK_LT) {
                 uint64_t* cand = s.u.m.top + MK_TOP - SK_LT;
                 if ((uint32_t)tid < C) cand[tid] = entry(ld_agent(&list[tid]));
@@ -1758,23 +1895,15 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
             } else {
                 const MkSorted o = C <= 4u * SK_LT ? sort_list(std::integral_constant<int, 4>{})
                                                    : sort_list(std::integral_constant<int, MK_LCAP / SK_LT>{});
-                sorted = mk_sort_end(o, k, s);
+                mk_sort_end(o, k, s);
             }
             SK_MARK(7);
-            if (sorted && greedy) {
+            if (greedy) {
                 if (w == 0) greedy_end(s.u.m.top[0]);
                 break;
             }
-            if (sorted) {
-                mk_softmax(a, p, row, kk, dr.u, s, tok, keep);
-                break;
-            }
-            if (select) {                                      // (never: mk_slow leaves at most k <= MK_TOP entries)
-                if (tid == 0) atomicOr(a.err, FS_DEVERR_INTERNAL);
-                break;
-            }
-            select = true;
-        }
+            mk_softmax(a, p, row, kk, dr.u, s, tok, keep);
+        } while (false);
         if (w != 0) return;
     }
     SK_TAG(9, k);

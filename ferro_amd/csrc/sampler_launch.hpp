@@ -63,12 +63,13 @@ hipError_t launch_small_k(int nl, bool capped, bool all_greedy, unsigned grid, i
 // The mid-k kernel: the small-k kernel's arguments (lists and ticket unused) and its own workspace.
 constexpr int MK_LIST = 4096;              // entries of a row's candidate list
 constexpr int MK_SPILL = 16384;            // entries of a row's list of penalised logits past those its segments keep in LDS
-constexpr int MK_CTR = 64;                 // words of a row's counters
+constexpr int MK_CTR = 128;                // words of a row's counters; from 64 on two per segment
 // Segments per row, which wait for each other. A process has four hardware queues unless it asks for more, and each can
 // hold one row whose segments are not all dispatched: 4 * 31 workgroups waiting leave room on an XCD (32 CUs of four
 // workgroups), so calls of several contexts on several streams always go on. With 64 segments three calls could fill an
 // XCD and wait out their limit. It is faster, too: 16 rows of 262144 logits, k 100: 18.1 us with 64 segments, 14.3 with 32.
 constexpr int MK_MAX_SEGS = 32;
+static_assert(64 + 2 * MK_MAX_SEGS <= MK_CTR, "");
 struct MkArgs {
     SkArgs a;
     uint32_t* ctr;                         // [B][MK_CTR], left at 0

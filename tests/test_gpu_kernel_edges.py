@@ -254,6 +254,40 @@ def test_mid_k_lists_of_equal_logits(k):
     check(x, mid_params(B, k, temperature=2.0), [[]] * B, rng.random(B), kcap=2048)
 
 
+@pytest.mark.parametrize("B,V,k", [(9, 4100, 100), (9, 33000, 1000), (9, 100003, 70), (18, 100003, 2048), (9, 262144, 300),
+                                   (66, 262144, 600)])
+@pytest.mark.parametrize("cap", [0.0, 0.5, 30.0])
+def test_mid_k_bounds_of_equal_logits(B, V, k, cap):
+    """Rows whose k-th logit is one value of many: masks, coarse logits, one value; every third with penalties on tied ids,
+    zeros of both signs, NaN among them. With cap 0.5 most of the larger values share a capped value."""
+    rng = np.random.default_rng(V + k + B)
+    low = np.finfo(np.float32).min
+    x = (rng.standard_normal((B, V)) * 2).astype(np.float32)
+    hists = []
+    for b in range(B):
+        r, few = x[b], rng.random(V) < 20.0 / V
+        kind = b % 9
+        if kind in (0, 1, 2):
+            r[~few] = (-np.inf, -1e9, low)[kind]
+        elif kind == 3:
+            r[:] = rng.choice(np.array([0.0, -0.0, np.nan], np.float32), V)
+        elif kind == 4:
+            r[:] = (r > 1).astype(np.float32)
+        elif kind == 5:
+            r[:] = np.round(r)
+        elif kind == 6:
+            r[:] = np.round(r * 2) / 2
+        elif kind == 7:                                    # many values and one, each in one part of the row
+            r[: V // 2] = 3.0
+        else:
+            r[:] = np.where(rng.random(V) < 0.5, np.float32(7.0), np.nextafter(np.float32(7.0), np.float32(8.0)))
+        hists.append(rng.integers(0, V, 0 if b % 3 else 400).astype(np.int32))
+    p = mid_params(B, k, temperature=3.0, softcap=cap)
+    p["repetition_penalty"][::3], p["frequency_penalty"][::3] = 1.3, 0.25
+    p["top_p"][1::2] = 0.9
+    check(x, p, hists, rng.random(B), kcap=2048)
+
+
 def test_mid_k_more_penalised_ids_than_the_spill_list():
     rng = np.random.default_rng(5)
     V, H = 262144, 40000

@@ -67,3 +67,17 @@ def test_lists_of_equal_logits():
     x = (rng.standard_normal((32, 262144)) * 2).astype(np.float32)
     plain, coarse = time_us(x, 200), time_us(np.round(x), 200)
     assert coarse < 3.5 * plain, (plain, coarse)
+
+
+@pytest.mark.parametrize("k", [65, 1000, 2048])
+def test_bounds_of_equal_logits(k):
+    """Masks that allow fewer than k tokens, coarse logits, rows of one value: 1.6 to 2.8 times a row without ties here
+    (100 to 120 times when one workgroup selected such a row alone)."""
+    rng = np.random.default_rng(2)
+    x = (rng.standard_normal((32, 262144)) * 2).astype(np.float32)
+    plain = time_us(x, k)
+    few = rng.random(x.shape) < 1e-4
+    for name, y in (("mask", np.where(few, x, -np.inf)), ("finite mask", np.where(few, x, -1e9)), ("one value", x * 0),
+                    ("whole", np.round(x)), ("two", np.where(x > 1, 1.0, 0.0))):
+        t = time_us(y.astype(np.float32), k)
+        assert t < 6 * plain, (name, t, plain)
