@@ -46,6 +46,7 @@ __device__ __forceinline__ uint32_t mk_rank(int j) {
 constexpr int AK_BINS = 2048;              // every token a candidate: mass bins of a row
 constexpr int AK_STAGE = 1024;             // logits of the searched bins that a segment stages, per list
 constexpr int AK_LIST = MK_LCAP / 2;       // entries of a row's two lists of such logits
+constexpr int AK_VALS = 64;                // distinct values of the searched bins in a chunk of ak_values
 constexpr float AK_DEPTH = 32.0f;          // temperatures below the maximum that the bins reach
 constexpr double AK_FX = 17592186044416.0; // 2^44: fixed-point mass scale of ak_slow (a mass is <= 1)
 
@@ -71,7 +72,12 @@ struct MkShared {
         } g;
         struct {
             uint32_t cnt[SK_LT * 8 * 4 / 2];   // ak_slow: a chunk's counts beside a digit's masses
-            uint64_t mass[MK_H];
+            union {
+                uint64_t mass[MK_H];
+                struct {
+                    uint32_t key[AK_VALS], cnt[AK_VALS];
+                } val[2];                      // ak_values: a chunk's values of the crossing's, of the draw's bins
+            };
         } z;
     } u;
     union {
@@ -264,6 +270,24 @@ struct MkPen {
     }
 };
 
+// f(logit, place) for a chunk of n logits of a row that one workgroup selects alone: eight loads in flight per thread.
+template <class F>
+__device__ __forceinline__ void slow_each(const float* p, int n, F f) {
+#pragma unroll 1
+    for (int i0 = threadIdx.x; i0 < n; i0 += 8 * SK_LT) {
+        float x[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) x[q] = i0 + q * SK_LT < n ? p[i0 + q * SK_LT] : 0.0f;
+#pragma unroll 1
+        for (int q = 0; q < 8 && i0 + q * SK_LT < n; ++q) {
+            float l = x[0];
+#pragma unroll
+            for (int t = 1; t < 8; ++t) l = q == t ? x[t] : l;
+            f(l, i0 + q * SK_LT);
+        }
+    }
+}
+
 // The exact top k of a row, from its logits alone, by one workgroup: a radix select over the composites, ten bits at a
 // time (it stops where a digit's bin is wholly inside), then the composites at or above the k-th to the row's list.
 // The penalties are counted again chunk by chunk. Returns the list's length. For rows with thousands of equal logits at
@@ -304,15 +328,13 @@ __device__ __forceinline__ uint32_t mk_slow(const float* rowp, int V, int k, boo
                 }
                 __syncthreads();
             }
-#pragma unroll 1
-            for (int i = tid; i < n; i += SK_LT) {
-                float l = rowp[lo + i];
+            slow_each(rowp + lo, n, [&](float l, int i) {
                 if (CAP && pn.cap > 0.0f) l = softcap_one(l, pn.cap);
                 if (pen && ((s.b.bmp[i >> 5] >> (i & 31)) & 1u))
                     l = pn.apply(l, pn.fp_on ? (s.u.cnt[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu : 0u);
                 const uint32_t key = key_of(l);
                 const uint64_t c = comp_of(key, (uint32_t)(lo + i));
-                if (key == 0u) continue;
+                if (key == 0u) return;
                 if (gather) {
                     if ((c & mask) >= prefix) {
                         const uint32_t pos = atomicAdd(&s.misc[2], 1u);
@@ -321,7 +343,7 @@ __device__ __forceinline__ uint32_t mk_slow(const float* rowp, int V, int k, boo
                 } else if ((c & mask) == prefix) {
                     atomicAdd(&s.h.hist[(uint32_t)(c >> sft) & (uint32_t)dm], 1u);
                 }
-            }
+            });
         }
         __syncthreads();
         if (gather) break;
@@ -683,12 +705,17 @@ __device__ __forceinline__ bool ak_locate(const uint64_t* cum, const uint64_t* r
 }
 
 // The first of the n sorted candidates in s.u.w.top at which above + the masses so far reach the target, -1 when they do
-// not; *cum: the sum there. Whole workgroup.
+// not; *cum: the sum there. COUNTED: each stands for as many equal ones as its low 16 bits say. Whole workgroup.
+template <bool COUNTED>
 __device__ __forceinline__ int ak_walk(int n, double above, double target, float mx, double Td, MkShared& s, double& cum) {
     const int tid = threadIdx.x, per = (n + SK_LT - 1) / SK_LT, i0 = tid * per, i1 = i0 + per < n ? i0 + per : n;
     double* E = s.u.w.e;
 #pragma unroll 1
-    for (int i = tid; i < n; i += SK_LT) E[i] = ak_mass(val_of(comp_key(s.u.w.top[i])), mx, Td);
+    for (int i = tid; i < n; i += SK_LT) {
+        const uint64_t c = s.u.w.top[i];
+        const double m = ak_mass(val_of(comp_key(c)), mx, Td);
+        E[i] = COUNTED ? (double)((uint32_t)c & 0xFFFFu) * m : m;
+    }
     __syncthreads();
     double run = 0.0, all;
 #pragma unroll 1
@@ -753,14 +780,12 @@ __device__ __forceinline__ void ak_slow(const float* rowp, int V, bool pen, cons
                 }
                 __syncthreads();
             }
-#pragma unroll 1
-            for (int i = tid; i < n; i += SK_LT) {
-                float l = rowp[lo + i];
+            slow_each(rowp + lo, n, [&](float l, int i) {
                 if (CAP && pn.cap > 0.0f) l = softcap_one(l, pn.cap);
                 if (pen && ((s.b.bmp[i >> 5] >> (i & 31)) & 1u))
                     l = pn.apply(l, pn.fp_on ? (s.u.z.cnt[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu : 0u);
                 const uint32_t key = key_of(l);
-                if (key == 0u) continue;
+                if (key == 0u) return;
                 const uint64_t c = comp_of(key, (uint32_t)(lo + i));
                 if (phase == 0) {
                     mxc = c > mxc ? c : mxc;
@@ -775,7 +800,7 @@ __device__ __forceinline__ void ak_slow(const float* rowp, int V, bool pen, cons
                         atomicAdd(reinterpret_cast<unsigned long long*>(&s.u.z.mass[(uint32_t)(c >> sft) & (uint32_t)dm]),
                                   (unsigned long long)(m * AK_FX + 0.5));
                 }
-            }
+            });
         }
         __syncthreads();
         if (phase == 0) {
@@ -867,6 +892,8 @@ struct AkRow {
     double S, u, above_c, above_d;
     int bc, d0, d1;
     bool cut, plain;
+    float scale;                           // bins per unit below mx; 0 with plain: one value
+    bool tail;                             // the bins end above the row's minimum
 };
 // One segment of such a row: extremes, meet, masses into the row's 2048 bins (linear in the logit from the row's maximum
 // down to its minimum, or 32 temperatures below: about 500 logits in the fullest bin of a normal row of 262144 whatever
@@ -967,6 +994,8 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     const bool tail = !(depth < AK_DEPTH);
     depth = tail ? AK_DEPTH : depth;
     const float scale = (float)AK_BINS / (depth * p.temperature);
+    r.scale = mn < mx || !(mx < __builtin_huge_valf()) || !(mx > -__builtin_huge_valf()) ? scale : 0.0f;
+    r.tail = tail;
     r.plain = r.nv == 0u || !(mx < __builtin_huge_valf()) || !(mx > -__builtin_huge_valf()) || !(mn < mx) || !(scale > 0.0f) ||
               !(scale < __builtin_huge_valf());
     if (r.plain) return true;                                  // uniform over the row
@@ -1242,7 +1271,7 @@ __device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uin
         }
         double cum;
         const double target = pass == 0 ? (double)p.top_p * r.S : r.u * tot + 0.0;
-        const int at = ak_walk(n, pass == 0 ? r.above_c : r.above_d, target, r.mx, Td, s, cum);
+        const int at = ak_walk<false>(n, pass == 0 ? r.above_c : r.above_d, target, r.mx, Td, s, cum);
         if (at < 0) return false;
         const uint64_t c = s.u.w.top[at];
         if (pass == 0) {
@@ -1253,6 +1282,171 @@ __device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uin
             tok = (int)comp_id(c < xc ? xc : c);
         }
     }
+    return true;
+}
+
+// The row's end where the searched bins hold more logits than a list takes (coarse logits: equal values share a bin; a row of
+// one value): by its last segment, from the row's logits. Chunk by chunk the bins' values and how often each occurs (a
+// wave counts each value of its 64 logits at once); crossing and draw are located among the values, in the order of their
+// chunks, and the draw's id in its chunk. Returns false when a chunk holds more than AK_VALS values of a bin, or a target
+// lies outside. One workgroup, two passes: 32 rows of 262144 logits rounded to halves 10140 us with ak_slow, now 830
+// (2460 on the fused kernel).
+template <bool CAP>
+__device__ __forceinline__ bool ak_values(const float* rowp, int V, bool pen, const MkWin& win, const MkPen& pn, uint64_t* list,
+                                          uint32_t above, const AkRow& r, const fs_row_params& p, MkShared& s, int& tok,
+                                          int& keep) {
+    constexpr int PT = 32, CH = SK_LT * PT;                    // logits of a thread, of a chunk
+    const int tid = threadIdx.x, lane = lane_id();
+    const double Td = (double)p.temperature;
+    const bool one = r.plain;
+    const int bc = one ? 0 : r.bc, d0 = one ? 0 : r.d0, d1 = one ? 0 : r.d1;
+    const bool cut = p.top_p < 1.0f;
+    const double S = one ? (double)r.nv : r.S;
+    auto bin_of = [&](float x) {                               // as ak_segment's
+        const float t = (r.mx - x) * r.scale;
+        const int b = (int)fminf(t, (float)AK_BINS);
+        return t == t ? (r.tail ? b : (b < AK_BINS ? b : AK_BINS - 1)) : AK_BINS;
+    };
+    auto window = [&](int lo, int n) {                         // a chunk's window ids, with their counts
+        for (int i = tid; i < CH / 32; i += SK_LT) s.b.bmp[i] = 0u;
+        for (int i = tid; i < CH / 2; i += SK_LT) s.u.z.cnt[i] = 0u;
+        __syncthreads();
+#pragma unroll 1
+        for (int64_t i = tid; i < win.n(); i += SK_LT) {
+            const uint32_t rel = (uint32_t)win.at(i) - (uint32_t)lo;
+            if (rel < (uint32_t)n) {
+                atomicOr(&s.b.bmp[rel >> 5], 1u << (rel & 31u));
+                atomicAdd(&s.u.z.cnt[rel >> 1], 1u << ((rel & 1u) * 16u));
+            }
+        }
+        __syncthreads();
+    };
+    auto value = [&](float l, int i) {                         // i: in the chunk
+        if (CAP && pn.cap > 0.0f) l = softcap_one(l, pn.cap);
+        if (pen && ((s.b.bmp[i >> 5] >> (i & 31)) & 1u)) l = pn.apply(l, (s.u.z.cnt[i >> 1] >> ((i & 1) * 16)) & 0xFFFFu);
+        return l;
+    };
+    auto put = [&](int l, uint32_t key, uint32_t n) {          // open addressing
+        uint32_t h = (key * 0x9E3779B1u) >> 26;
+        static_assert(AK_VALS == 1 << (32 - 26) && AK_VALS == WAVE, "the hash gives a place; a lane per place");
+#pragma unroll 1
+        for (int i = 0; i < AK_VALS; ++i, h = (h + 1u) & (AK_VALS - 1u)) {
+            const uint32_t old = atomicCAS(&s.u.z.val[l].key[h], 0u, key);
+            if (old == 0u || old == key) {
+                atomicAdd(&s.u.z.val[l].cnt[h], n);
+                return;
+            }
+        }
+        s.gn[3] = 1u;
+    };
+    if (tid < 4) s.gn[tid] = 0u;                               // the lists' lengths; [3]: too many values
+#pragma unroll 1
+    for (int lo = 0, chunk = 0; lo < V; lo += CH, ++chunk) {
+        const int n = V - lo < CH ? V - lo : CH;
+        __syncthreads();
+        if (tid < 4 * AK_VALS) reinterpret_cast<uint32_t*>(s.u.z.val)[tid] = 0u;
+        if (pen) window(lo, n);
+        else __syncthreads();
+#pragma unroll 1
+        for (int q0 = 0; q0 < PT && s.gn[3] == 0u; q0 += 8) {
+            float x[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int i = (q0 + q) * SK_LT + tid;
+                x[q] = i < n ? rowp[lo + i] : __builtin_nanf("");
+            }
+#pragma unroll 1
+            for (int q = 0; q < 8; ++q) {
+                float y = x[0];
+#pragma unroll
+                for (int t = 1; t < 8; ++t) y = q == t ? x[t] : y;
+                y = value(y, (q0 + q) * SK_LT + tid);
+                const int b = bin_of(y);
+                const bool in_c = cut && b == bc, in_d = b >= d0 && b <= d1;
+                const uint32_t key = key_of(y);
+#pragma unroll 1
+                for (uint64_t left = __ballot(in_c || in_d); left != 0ull;) {
+                    const int first = __ffsll((unsigned long long)left) - 1;
+                    const uint64_t eq = __ballot(key == read_lane(key, first)) & left;
+                    if (lane == first) {
+                        if (in_c) put(0, key, (uint32_t)__popcll(eq));
+                        if (in_d) put(1, key, (uint32_t)__popcll(eq));
+                    }
+                    left &= ~eq;
+                }
+            }
+        }
+        __syncthreads();
+        // entries: the value's key, the chunk (descending), the count. (Waves 0 and 1: a list each.)
+        if (tid < 2 * WAVE) {
+            const int l = tid / WAVE;
+            const uint32_t key = s.u.z.val[l].key[lane];
+            const uint64_t has = __ballot(key != 0u);
+            const uint32_t at = s.gn[l] + (uint32_t)__popcll(has & ((1ull << lane) - 1ull));
+            if (key != 0u && at < (uint32_t)AK_LIST)
+                st_agent(&list[l * AK_LIST + at], ((uint64_t)key << 32) | ((uint32_t)(63 - chunk) << 16) | s.u.z.val[l].cnt[lane]);
+            if (lane == 0) s.gn[l] += (uint32_t)__popcll(has);
+        }
+    }
+    vm_drain();
+    __syncthreads();
+    const uint32_t n0 = s.gn[0], n1 = s.gn[1];
+    if (s.gn[3] != 0u || n0 > (uint32_t)AK_LIST || n1 > (uint32_t)AK_LIST) return false;
+    uint64_t xc = 0ull, c = 0ull;
+    double tot = S;
+    keep = (int)r.nv;
+#pragma unroll 1
+    for (int pass = cut ? 0 : 1; pass < 2; ++pass) {
+        const int n = (int)(pass == 0 ? n0 : n1);
+        if (n == 0) return false;
+        uint64_t e[AK_LIST / SK_LT];
+#pragma unroll
+        for (int q = 0; q < AK_LIST / SK_LT; ++q)
+            e[q] = q * SK_LT + tid < n ? ld_agent(&list[pass * AK_LIST + q * SK_LT + tid]) : 0ull;
+        __syncthreads();                                       // (the first pass's entries are spent)
+        mk_sort_end(mk_sort(e, n, n, s), n, s);
+        double cum;
+        const double target = pass == 0 ? (double)p.top_p * S : r.u * tot + 0.0;
+        const int at = ak_walk<true>(n, one ? 0.0 : pass == 0 ? r.above_c : r.above_d, target, r.mx, Td, s, cum);
+        if (at < 0) return false;
+        // the j-th of the entry's equal logits reaches the target; c becomes the entry's value and chunk above ~j
+        c = s.u.w.top[at];
+        const uint32_t cnt = (uint32_t)c & 0xFFFFu;
+        const double m = ak_mass(val_of(comp_key(c)), r.mx, Td), from = cum - (double)cnt * m;
+        const double want = ceil((target - from) / m);
+        uint32_t j = want >= (double)cnt ? cnt : want > 1.0 ? (uint32_t)want : 1u;
+        if (j > 1u && from + (double)(j - 1u) * m >= target) --j;
+        c = (c & ~0xFFFFull) | (0xFFFFull - j);
+        if (pass == 0) {
+            uint64_t before = 0ull;
+            for (int i = tid; i < at; i += SK_LT) before += s.u.w.top[i] & 0xFFFFull;
+            before = mk_reduce_u64(before, s, [](uint64_t x, uint64_t y) { return x + y; });
+            xc = c;
+            tot = from + (double)j * m;
+            keep = (int)above + (int)before + (int)j;
+        }
+    }
+    if (c < xc) c = xc;
+    // the id of its j-th logit
+    const int lo = (63 - (int)((c >> 16) & 0xFFFFull)) * CH, n = V - lo < CH ? V - lo : CH;
+    const uint32_t j = 0xFFFFu - ((uint32_t)c & 0xFFFFu);
+    __syncthreads();
+    if (pen) window(lo, n);
+    uint32_t eq = 0u;                                          // a bit per logit of the thread, which are neighbours here
+#pragma unroll 4
+    for (int q = 0; q < PT; ++q) {
+        const int i = tid * PT + q;
+        const float y = value(i < n ? rowp[lo + i] : __builtin_nanf(""), i);
+        eq |= (key_of(y) == comp_key(c) ? 1u : 0u) << q;
+    }
+    uint32_t all;
+    uint32_t before = mk_excl_u32((uint32_t)__popc(eq), s, all);
+    if (before < j && j <= before + (uint32_t)__popc(eq)) {
+        while (++before < j) eq &= eq - 1u;
+        s.misc[4] = (uint32_t)(lo + tid * PT + __ffs((int)eq) - 1);
+    }
+    __syncthreads();
+    tok = (int)s.misc[4];
     return true;
 }
 
@@ -1746,7 +1940,7 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
         }
     }
     if (over && lane == 0)                                     // too many penalised ids: the row is selected alone
-        __hip_atomic_fetch_or(ctr + 34, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_or(ctr + 34, 4u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     if (cp_on) sk_cp_store(a, cp, row, seg);
     SK_MARK(5);
     vm_drain();                                                // the candidates are in the L2
@@ -1798,9 +1992,12 @@ __global__ __launch_bounds__(SK_LT, 4) void mid_k_kernel(const float* logits, in
         }
         ulonglong2* rm = reinterpret_cast<ulonglong2*>(mk.mass + (int64_t)row * AK_BINS);
         for (int i = tid; i < AK_BINS / 2; i += SK_LT) rm[i] = make_ulonglong2(0ull, 0ull);
-        if (slow != 0u || ak.plain || n0 > (uint32_t)AK_LIST || n1 > (uint32_t)AK_LIST ||
-            !ak_finish(list, n0, n1, c0, c1, above, ak, p, s, tok, keep))
-            ak_slow<CAP>(rowp, V, pen, win, pn, p, dr.u, s, tok, keep);
+        const bool fits = n0 <= (uint32_t)AK_LIST && n1 <= (uint32_t)AK_LIST;
+        bool done = false;
+        if (slow == 0u && !ak.plain && fits) done = ak_finish(list, n0, n1, c0, c1, above, ak, p, s, tok, keep);
+        else if ((slow & ~1u) == 0u && (!ak.plain || (ak.nv != 0u && ak.scale == 0.0f)))
+            done = ak_values<CAP>(rowp, V, pen, win, pn, list, above, ak, p, s, tok, keep);
+        if (!done) ak_slow<CAP>(rowp, V, pen, win, pn, p, dr.u, s, tok, keep);
         if (w != 0) return;
     } else {
         uint32_t C = ld_agent(ctr + 33);

@@ -431,6 +431,51 @@ def test_every_token_a_candidate(B, V, top_p):
     assert F.device_error() == 0
 
 
+@pytest.mark.parametrize("B,V", [(9, 4100), (9, 33000), (18, 100003), (9, 262144), (66, 262144)])
+@pytest.mark.parametrize("cap", [0.0, 0.5])
+def test_every_token_of_few_values(B, V, cap):
+    """top_k = 0 on rows whose searched bins hold thousands of equal logits (located by value and count): one and two values,
+    whole numbers, halves, zeros of both signs, two values in parts of the row, narrow rows below one large logit; with
+    and without top-p, penalties on tied ids. With cap 0.5 most of the larger values share a capped value."""
+    rng = np.random.default_rng(V + B)
+    x = (rng.standard_normal((B, V)) * 2).astype(np.float32)
+    hists = []
+    for b in range(B):
+        r, kind = x[b], b % 9
+        if kind == 0:
+            r[:] = 1.5
+        elif kind == 1:
+            r[:] = (r > 1).astype(np.float32)
+        elif kind == 2:
+            r[:] = np.round(r)
+        elif kind == 3:
+            r[:] = np.round(r * 2) / 2
+        elif kind == 4:
+            r[:] = rng.choice(np.array([0.0, -0.0, np.nan, -40.0], np.float32), V)
+        elif kind == 5:
+            r[: V // 2] = 3.0
+        elif kind == 6:
+            r[:] = np.maximum(r, 0)
+        elif kind == 7:
+            r[:] = r * 0.01
+            r[V // 3] = 9.0
+        else:
+            r[rng.choice(V, V // 2, replace=False)] = -1e9
+        hists.append(rng.integers(0, V, 0 if b % 2 else 300).astype(np.int32))
+    p = mid_params(B, 0, temperature=0.9, softcap=cap)
+    p["top_p"] = np.where(np.arange(B) % 4 < 2, 0.9, 1.0)
+    p["repetition_penalty"][::2], p["frequency_penalty"][::4] = 1.3, 0.25
+    u = rng.random(B)
+    u[-1] = 0.0
+    hist, off = csr(hists)
+    out = F.sample_batch(torch.from_numpy(x).cuda(), p, u, hist=hist, hist_off=off)
+    torch.cuda.synchronize()
+    o = O.sample_batch(x, hist, off, p, u, kcap=1, nthreads=NT)
+    np.testing.assert_array_equal(out["tok"].cpu().numpy(), o["tok"])
+    np.testing.assert_array_equal(out["keep"].cpu().numpy(), o["keep"])
+    assert F.device_error() == 0
+
+
 def test_every_token_draws_next_to_a_boundary():
     """Rows whose mass is ten logits, draws 6e-15 below and above the cumulative mass of each, computed in 80 bits. Ten
     masses summed in fp64 (or in units of 2^-52), each within 0.52 ulp, are off by less than 5e-15 of a sum >= 1; units of
