@@ -476,6 +476,31 @@ def test_every_token_of_few_values(B, V, cap):
     assert F.device_error() == 0
 
 
+@pytest.mark.parametrize("mask", [-np.inf, -1e9, np.finfo(np.float32).min])
+def test_every_token_of_masked_rows_at_high_temperatures(mask):
+    """Tokens masked far below rows that are narrow in units of the temperature: the bins cover the other tokens."""
+    rng = np.random.default_rng(5)
+    B, V = 10, 100003
+    x = (rng.standard_normal((B, V)) * 2).astype(np.float32)
+    x[::2, ::100] = mask
+    x[1::2, :20000] = mask                           # whole segments of masked tokens
+    x[4, 77777] = 6 * 3.0 * 32                       # the others are below the bins of this row
+    x[5] = np.where(x[5] > 4, x[5], mask)
+    p = mid_params(B, 0, temperature=3.0)
+    p["temperature"][6:8] = 0.7, 20.0
+    p["top_p"] = np.where(np.arange(B) % 4 < 2, 0.9, 1.0)
+    p["repetition_penalty"][::3] = 1.2
+    hist, off = csr([rng.integers(0, V, 300).astype(np.int32) for _ in range(B)])
+    for _ in range(3):
+        u = rng.random(B)
+        out = F.sample_batch(torch.from_numpy(x).cuda(), p, u, hist=hist, hist_off=off)
+        torch.cuda.synchronize()
+        o = O.sample_batch(x, hist, off, p, u, kcap=1, nthreads=NT)
+        np.testing.assert_array_equal(out["tok"].cpu().numpy(), o["tok"])
+        np.testing.assert_array_equal(out["keep"].cpu().numpy(), o["keep"])
+    assert F.device_error() == 0
+
+
 def test_every_token_draws_next_to_a_boundary():
     """Rows whose mass is ten logits, draws 6e-15 below and above the cumulative mass of each, computed in 80 bits. Ten
     masses summed in fp64 (or in units of 2^-52), each within 0.52 ulp, are off by less than 5e-15 of a sum >= 1; units of
