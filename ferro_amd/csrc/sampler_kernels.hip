@@ -136,13 +136,13 @@ struct fs_context {
     size_t sk_slots = 0;
     uint32_t* sk_ticket = nullptr;  // small-k kernel: [rows] segment tickets, left at 0
     size_t sk_rows = 0;
-    uint32_t* mk_ctr = nullptr;     // mid-k kernel: [mk_rows][MK_CTR] counters, left at 0
-    uint64_t* mk_list = nullptr;    //   [mk_rows][MK_LIST] candidate lists
-    uint64_t* mk_spill = nullptr;   //   [mk_rows][MK_SPILL] penalised logits
-    uint64_t* mk_mass = nullptr;    //   [mk_rows][2048] mass bins, left at 0
-    size_t mk_rows = 0;
+    uint32_t* mk_ctr = nullptr;     // mid-k kernel: [mk_ctr_rows][MK_CTR] counters, left at 0
+    uint64_t* mk_list = nullptr;    //   [mk_list_rows][MK_LIST] candidate lists
+    uint64_t* mk_spill = nullptr;   //   [mk_spill_rows][MK_SPILL] penalised logits (batches with penalties)
+    uint64_t* mk_mass = nullptr;    //   [mk_mass_rows][2048] mass bins, left at 0 (batches with every token a candidate)
     uint32_t* mk_qk = nullptr;      //   [mk_segs][SK_NW][16] published lane maxima
-    size_t mk_segs = 0;
+    size_t mk_ctr_rows = 0, mk_list_rows = 0, mk_spill_rows = 0, mk_mass_rows = 0, mk_segs = 0;
+    int mk_wait = 0;                //   calls that still go without trying again after an allocation failed
     uint64_t* cand = nullptr;
     size_t cand_slots = 0;     // chunk slots of CAP entries
     uint32_t* meta = nullptr;
@@ -554,37 +554,51 @@ bool mid_k_choice(int cus, const fs_row_params* h, int64_t n, int64_t rows, int3
     return (int64_t)fs::XCDS * c.nseg * ((rows + fs::XCDS - 1) / fs::XCDS) <= 0x7fffffff;
 }
 
-// About 176 KB per row. FS_E_NOMEM leaves none of it allocated.
-int grow_mid(fs_context* c, size_t segs, size_t rows) {
-    if (segs <= c->mk_segs && rows <= c->mk_rows) return FS_OK;
-    segs = std::max(segs, c->mk_segs);
-    rows = std::max(rows, c->mk_rows);
-    auto drop = [&](auto*& p) {
-        release(c, p);
-        p = nullptr;
-    };
-    auto drop_all = [&]() {
-        drop(c->mk_qk); drop(c->mk_ctr); drop(c->mk_list); drop(c->mk_spill); drop(c->mk_mass);
-        c->mk_segs = c->mk_rows = 0;
-    };
-    drop_all();
-    if (hipMalloc(&c->mk_qk, segs * fs::SK_NW * 16 * sizeof(uint32_t)) != hipSuccess ||
-        hipMalloc(&c->mk_ctr, rows * fs::MK_CTR * sizeof(uint32_t)) != hipSuccess ||
-        hipMalloc(&c->mk_list, rows * fs::MK_LIST * sizeof(uint64_t)) != hipSuccess ||
-        hipMalloc(&c->mk_spill, rows * fs::MK_SPILL * sizeof(uint64_t)) != hipSuccess ||
-        hipMalloc(&c->mk_mass, rows * 2048 * sizeof(uint64_t)) != hipSuccess) {
-        (void)hipGetLastError();
-        drop_all();
-        return FS_E_NOMEM;
+// One buffer of the mid-k kernel's workspace: at least n elements of `per` words each, half as many again when it grows.
+// FS_E_NOMEM leaves the old one as it was.
+template <class T>
+int grow_buffer(fs_context* c, T*& p, size_t& cap, size_t n, size_t per, bool zero) {
+    if (n <= cap) return FS_OK;
+    T* q = nullptr;
+    size_t m = std::max(n, cap + cap / 2);
+    if (hipMalloc(&q, m * per * sizeof(T)) != hipSuccess) {
+        m = n;
+        if (hipMalloc(&q, m * per * sizeof(T)) != hipSuccess) {
+            (void)hipGetLastError();
+            return FS_E_NOMEM;
+        }
     }
-    if (hipMemset(c->mk_ctr, 0, rows * fs::MK_CTR * sizeof(uint32_t)) != hipSuccess ||
-        hipMemset(c->mk_mass, 0, rows * 2048 * sizeof(uint64_t)) != hipSuccess) {
-        drop_all();
+    if (zero && hipMemset(q, 0, m * per * sizeof(T)) != hipSuccess) {
+        (void)hipFree(q);
         return FS_E_HIP;
     }
-    c->mk_segs = segs;
-    c->mk_rows = rows;
+    release(c, p);
+    p = q;
+    cap = m;
     return FS_OK;
+}
+
+// Whether a call needs more than the context holds.
+bool mid_grows(const fs_context* c, const MidKChoice& ch, size_t rows) {
+    return rows * ch.nseg > c->mk_segs || rows > c->mk_ctr_rows || rows > c->mk_list_rows ||
+           (ch.may_pen && rows > c->mk_spill_rows) || (ch.all && rows > c->mk_mass_rows);
+}
+
+// About 33 KB per row, 128 KB more with penalties and 16 KB with every token a candidate. After a failed allocation the
+// next 64 calls that would have to grow don't try.
+int grow_mid(fs_context* c, const MidKChoice& ch, size_t rows) {
+    if (!mid_grows(c, ch, rows)) return FS_OK;
+    if (c->mk_wait > 0) {
+        --c->mk_wait;
+        return FS_E_NOMEM;
+    }
+    int rc = grow_buffer(c, c->mk_qk, c->mk_segs, rows * ch.nseg, fs::SK_NW * 16, false);
+    if (rc == FS_OK) rc = grow_buffer(c, c->mk_ctr, c->mk_ctr_rows, rows, fs::MK_CTR, true);
+    if (rc == FS_OK) rc = grow_buffer(c, c->mk_list, c->mk_list_rows, rows, fs::MK_LIST, false);
+    if (rc == FS_OK && ch.may_pen) rc = grow_buffer(c, c->mk_spill, c->mk_spill_rows, rows, fs::MK_SPILL, false);
+    if (rc == FS_OK && ch.all) rc = grow_buffer(c, c->mk_mass, c->mk_mass_rows, rows, 2048, true);
+    if (rc == FS_E_NOMEM) c->mk_wait = 64;
+    return rc;
 }
 
 // Launches the mid-k kernel when the batch fits it; *used = false (nothing launched) otherwise. Under capture a
@@ -601,13 +615,12 @@ int launch_mid(fs_context* ctx, const fs::Args& a, const fs_row_params* h_params
     if (!mid_k_choice(ctx->cus, h_params, verify ? (int64_t)a.n_streams : (int64_t)a.B, a.B, a.V,
                       a.cand_ids || a.cand_probs, ch))
         return FS_OK;
-    const size_t segs = (size_t)a.B * ch.nseg, streams = verify ? 3 * (size_t)a.n_streams : 0;
+    const size_t streams = verify ? 3 * (size_t)a.n_streams : 0;
     const bool cap = capturing(st);
-    if (cap && (segs > ctx->mk_segs || (size_t)a.B > ctx->mk_rows || streams > ctx->stream_cap || !ctx->err))
-        return FS_OK;
+    if (cap && (mid_grows(ctx, ch, (size_t)a.B) || streams > ctx->stream_cap || !ctx->err)) return FS_OK;
     rc = grow(ctx, 0, 0, streams);
     if (rc != FS_OK) return rc;
-    rc = grow_mid(ctx, segs, (size_t)a.B);
+    rc = grow_mid(ctx, ch, (size_t)a.B);
     if (rc == FS_E_NOMEM) return FS_OK;
     if (rc != FS_OK) return rc;
     if (cap) ctx->captured = true;

@@ -344,6 +344,25 @@ def test_mid_k_give_up_is_exact():
         assert F.device_error(ctx) == bits
 
 
+def test_mid_k_workspace_grows_by_need():
+    """One context: batches that grow by a row and by what they need (penalties, every token a candidate, more segments), a
+    small one after a large one."""
+    rng = np.random.default_rng(11)
+    ctx = F.sampler.Context()
+    for B, V, k, rep in ((2, 70000, 100, 1.0), (3, 70000, 100, 1.2), (4, 70000, 0, 1.0), (5, 200000, 0, 1.3), (1, 33000, 300, 1.1),
+                         (6, 33000, 70, 1.0), (7, 200000, 0, 1.2), (40, 33000, 90, 1.1), (3, 200000, 90, 1.1)):
+        x = (rng.standard_normal((B, V)) * 2).astype(np.float32)
+        p = mid_params(B, k, repetition_penalty=rep, frequency_penalty=0.01)
+        hist, off = csr([rng.integers(0, V, 900).astype(np.int32) for _ in range(B)])
+        u = rng.random(B)
+        out = F.sample_batch(torch.from_numpy(x).cuda(), p, u, hist=hist, hist_off=off, ctx=ctx)
+        torch.cuda.synchronize()
+        o = O.sample_batch(x, hist, off, p, u, kcap=1, nthreads=NT)
+        np.testing.assert_array_equal(out["tok"].cpu().numpy(), o["tok"])
+        np.testing.assert_array_equal(out["keep"].cpu().numpy(), o["keep"])
+        assert F.device_error(ctx) == 0
+
+
 def test_mid_k_on_several_streams():
     """Three contexts on three streams, calls of few rows with the most segments each (they wait for each other) in
     flight together."""
