@@ -601,10 +601,21 @@ int grow_mid(fs_context* c, const MidKChoice& ch, size_t rows) {
     return rc;
 }
 
+// The fused kernel's layout for a call (a.nseg, a.seg_tiles, a.balance, its grid) and the workspace it needs.
+int grow_fused(fs_context* ctx, fs::Args& a, int64_t rows, int64_t streams, int per_cu, int64_t* grid) {
+    int64_t items = 0;
+    const int rc = plan(ctx->cus, a, rows, items, *grid, 0, per_cu);
+    if (rc != FS_OK) return rc;
+    // verify: a 64-bit word per stream, then the 32-bit counters of streams longer than 32 rows
+    return grow(ctx, (size_t)(items > 0 ? items : 1), (size_t)rows, (size_t)(streams > 0 ? 3 * streams : 1));
+}
+
 // Launches the mid-k kernel when the batch fits it; *used = false (nothing launched) otherwise. Under capture a
 // workspace that would have to grow leaves the batch to the fused kernel (no allocation in a capture that worked
 // without one), and so does one that the device has no room for.
-int launch_mid(fs_context* ctx, const fs::Args& a, const fs_row_params* h_params, hipStream_t st, bool& used) {
+// per_cu: as launch's; the fused kernel's workspace grows as launch would grow it, so that a context warmed up with any
+// parameters of a shape allocates nothing when a call of that shape with others is recorded.
+int launch_mid(fs_context* ctx, const fs::Args& a, const fs_row_params* h_params, hipStream_t st, bool& used, int per_cu = 2) {
     used = false;
     std::lock_guard<std::mutex> g(ctx->mu);
     int rc = device_of(ctx);
@@ -618,7 +629,15 @@ int launch_mid(fs_context* ctx, const fs::Args& a, const fs_row_params* h_params
     const size_t streams = verify ? 3 * (size_t)a.n_streams : 0;
     const bool cap = capturing(st);
     if (cap && (mid_grows(ctx, ch, (size_t)a.B) || streams > ctx->stream_cap || !ctx->err)) return FS_OK;
-    rc = grow(ctx, 0, 0, streams);
+    if (!cap) {
+        fs::Args fused = a;
+        int64_t fused_grid = 0;
+        rc = grow_fused(ctx, fused, a.B, verify ? a.n_streams : 0, per_cu, &fused_grid);
+    }
+    if (rc == FS_E_NOMEM || rc == FS_E_INVALID) {   // (this kernel does not need it)
+        (void)hipGetLastError();
+        rc = grow(ctx, 0, 0, streams);
+    }
     if (rc != FS_OK) return rc;
     rc = grow_mid(ctx, ch, (size_t)a.B);
     if (rc == FS_E_NOMEM) return FS_OK;
@@ -643,11 +662,8 @@ int launch(fs_context* ctx, fs::Args a, int64_t rows, int64_t streams, hipStream
     std::lock_guard<std::mutex> g(ctx->mu);
     int rc = device_of(ctx);
     if (rc != FS_OK) return rc;
-    int64_t items = 0, seg_grid = 0;
-    rc = plan(ctx->cus, a, rows, items, seg_grid, 0, per_cu);
-    if (rc != FS_OK) return rc;
-    // verify: a 64-bit word per stream, then the 32-bit counters of streams longer than 32 rows
-    rc = grow(ctx, (size_t)(items > 0 ? items : 1), (size_t)rows, (size_t)(streams > 0 ? 3 * streams : 1));
+    int64_t seg_grid = 0;
+    rc = grow_fused(ctx, a, rows, streams, per_cu, &seg_grid);
     if (rc != FS_OK) return rc;
     if (capturing(st)) ctx->captured = true;
     a.cand = ctx->cand; a.meta = ctx->meta; a.rhist = ctx->rhist; a.rmass = ctx->rmass;
@@ -809,9 +825,10 @@ int fs_sample_batch_hp(fs_context* ctx, const float* d_logits, int64_t ld, int32
         bool used = false;
         rc = launch_small(ctx, a, h_params, (hipStream_t)stream, used);
         if (rc != FS_OK || used) return rc;
-        rc = launch_mid(ctx, a, h_params, (hipStream_t)stream, used);
+        const int per_cu = mixed_merges(h_params, B, V) ? 4 : 2;
+        rc = launch_mid(ctx, a, h_params, (hipStream_t)stream, used, per_cu);
         if (rc != FS_OK || used) return rc;
-        if (mixed_merges(h_params, B, V)) return launch(ctx, a, B, 0, (hipStream_t)stream, 4);
+        return launch(ctx, a, B, 0, (hipStream_t)stream, per_cu);
     }
     return launch(ctx, a, B, 0, (hipStream_t)stream);
 }

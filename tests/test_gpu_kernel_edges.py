@@ -647,3 +647,50 @@ def test_mid_k_calls_in_a_graph(every, warm):
         torch.cuda.synchronize()
         check_clean(ctx)
     del g
+
+
+@pytest.mark.parametrize("params", [dict(min_p=0.05, top_k=0), dict(top_k=3000)])
+def test_recorded_call_the_mid_k_kernel_refuses(params):
+    """A context warmed up with a batch of the mid-k kernel records the same shape with parameters that only the fused
+    kernel takes: its workspace is there, nothing is allocated in the capture."""
+    import ctypes
+    from ferro_amd._lib import lib
+    from test_gpu_graph import Call, P, check_clean, mixed
+    B, V = 24, 65536
+    ctx, other = F.sampler.Context(), F.sampler.Context()
+    warm, w = mixed(3, B, V), mixed(4, B, V)
+    warm.params["top_k"][:], warm.params["min_p"][:] = 0, 0.0
+    for f, v in params.items():
+        w.params[f][:] = v
+
+    def launch(c, wl, call, st):
+        rc = lib().fs_sample_batch_hp(c.h, P(call.x), call.x.stride(0), B, V, P(call.hist), P(call.hoff), P(call.params),
+                                      wl.params.ctypes.data_as(ctypes.c_void_p), P(call.u), P(call.tok), 0, None, None,
+                                      P(call.keep), ctypes.c_void_p(st.cuda_stream))
+        assert rc == 0, rc
+
+    cw, c = Call(warm, kcap=16), Call(w, kcap=16)
+    cur, side = torch.cuda.current_stream(), torch.cuda.Stream()
+    launch(ctx, warm, cw, cur)
+    launch(other, w, c, cur)
+    torch.cuda.synchronize()
+    want = c.out()
+    g = torch.cuda.CUDAGraph()
+    side.wait_stream(cur)
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(g, stream=side):
+            launch(ctx, w, c, side)
+    cur.wait_stream(side)
+    torch.cuda.synchronize()
+    for rep in range(3):
+        c.poison()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        got = c.out()
+        for k in ("tok", "keep"):
+            np.testing.assert_array_equal(got[k], want[k], err_msg=f"replay {rep} {k}")
+        launch(ctx, warm, cw, cur)
+        torch.cuda.synchronize()
+        check_clean(ctx)
+    del g
