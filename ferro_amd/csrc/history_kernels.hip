@@ -113,6 +113,7 @@ __global__ __launch_bounds__(LU_BLOCK) void lookup_draft_kernel(const int32_t* h
             for (int j = 0; j < LU_PER; ++j) ids[LU_N + j * LU_BLOCK + tid] = v[j];
             __syncthreads();
             int bm = -1, bi = 0;                         // this thread's longest match, the most recent of those
+            const int start = c0 < LU_N ? (int)c0 : LU_N;   // ids before the tile (no match reaches past the history's first)
 #pragma unroll
             for (int j = 0; j < LU_PER / LU_N; ++j) {
                 const int i0 = (j * LU_BLOCK + tid) * LU_N;
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(LU_BLOCK) void lookup_draft_kernel(const int32_t* h
                         m = w[r + 2] == t[1] ? m : 1;
                         m = w[r + 3] == t[0] ? m : 0;
                         m = m < (int)nmax ? m : (int)nmax;
-                        if (c0 < LU_N) m = m < (int)c0 + i0 + r ? m : (int)c0 + i0 + r;   // no ids before the history's first
+                        m = m < start + i0 + r ? m : start + i0 + r;
                         if (i0 + r < n && w[r + LU_N] != eos && m >= bm) { bm = m; bi = i0 + r; }
                     }
                 }
