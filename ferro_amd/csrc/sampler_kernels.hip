@@ -336,8 +336,11 @@ bool capturing(hipStream_t st) {
 // A batch whose rows cost very differently: rows sampled with 64 < k <= KMAX beside greedy or k <= 64 rows, none on
 // the whole-row path (k > KMAX), 16 to 64 rows per XCD (the balanced layout). The host copy of the parameters shows
 // the mix, and such batches take about four segments per CU instead of two, which gives the balanced layout finer
-// shares to apportion (B=256 x V=262144 with k from 1 to 2048: 119.7 -> 116.6-117.4 us). Uniform batches lose with
-// more segments (more lists to merge, a second round of workgroups).
+// shares to apportion. It is reached by batches the mid-k kernel does not take (more than 262144 logits, or too few for
+// their largest k). k spread evenly over 1 to 2048 by its logarithm, with two segments per CU and with four: 384 rows of
+// 262208 logits 224 us and 167, of 50000 106 and 88; but 256 rows of 262208 116 and 131, of 32000 89 and 96 (the rule dates
+// from 256 rows of 262144, which the mid-k kernel now has). Uniform batches lose with more segments (more lists to merge, a
+// second round of workgroups).
 bool mixed_merges(const fs_row_params* h, int64_t B, int32_t V) {
     const int64_t per_x = (B + fs::XCDS - 1) / fs::XCDS;
     if (per_x < 16 || per_x > fs::WAVE) return false;
@@ -511,7 +514,7 @@ int launch_small(fs_context* ctx, const fs::Args& a_in, const fs_row_params* h_p
 }
 
 // ---- mid-k kernel (fs_sample_batch_hp, fs_verify_hp, fs_decode_step_hp)
-// Every row greedy or sampling from k <= 2048 candidates, with any penalty. The row's bound comes from its lanes'
+// Every row greedy or sampling from k <= 2048 candidates or from every token, with any penalty. The row's bound comes from its lanes'
 // maxima (one per 4 * nl logits): twice as many as the largest k keep the candidates at about 1.4 k, and a row's
 // segments publish at most 64 lists of 16 per 4 * nl loads, which the bound's search reads in one round.
 struct MidKChoice {
@@ -526,9 +529,10 @@ bool mid_k_choice(int cus, const fs_row_params* h, int64_t n, int64_t rows, int3
         const int64_t k = greedy ? 1 : ((p.top_k > 0 && p.top_k < V) ? p.top_k : V);
         if (k == V && k > fs::KMAX) {
             // every token a candidate: no candidate outputs and no min-p (its count and sum over the kept logits)
-            // (taken whatever the rows hold, which the host cannot see: rows whose mass is a few logits come out at 0.97 to
-            // 1.10 times the fused kernel's short list, 16 rows of 65536 18.3 us there and 18.9 here, 64 of 262144 36.9 and
-            // 33.7; rows with a body gain: 16 normal rows of 65536 at temperature 0.2 49.8 and 23.3)
+            // (taken whatever the rows hold, which the host cannot see. Rows whose mass is a few logits take about as long as
+            // on the fused kernel with its short list: heavy-tailed logits at temperature 0.3, 1 row of 65536 19.1 us here
+            // and 18.4 there, 16 rows 19.2 and 19.1, 64 of 262144 33.5 and 36.4. Rows with a body gain: 16 rows of 65536
+            // N(0, 2) logits 24.0 and 28.3 at temperature 0.2, 27.5 and 62.4 at 1)
             if (outputs || p.min_p > 0.0f) return false;
             c.all = true;
         } else {

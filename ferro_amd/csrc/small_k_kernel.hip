@@ -9,7 +9,7 @@ namespace fs {
 // A separate kernel for batches whose every row is greedy or samples from k <= SK_K candidates with at most a
 // repetition penalty (no frequency / presence counts) - the serving batches of ferro's decode loop (server.cpp:603-606:
 // top-k 40-64 on every row). The host picks it from a host copy of the parameters (fs_sample_batch_hp). It has its own
-// register budget (it shares no code path with the fused kernel above), which lets it stream a row differently:
+// register budget (it shares no code path with the fused kernel), which lets it stream a row differently:
 //   - one workgroup of SK_LT threads per (row, segment): every load of the segment (NL float4 per thread) is issued at
 //     once, so the whole batch is requested at the start. The memory system serves the requests roughly in dispatch
 //     order, so a row's segments (consecutive workgroups) receive their data together, and rows finish one after

@@ -94,9 +94,9 @@ int fs_sample_batch(fs_context* ctx, const float* d_logits, int64_t ld, int32_t 
  * most 64 candidates (k = top_k, or V when top_k is 0) with no frequency / presence penalty run on a kernel made for
  * them (every segment's loads issued at once, bitonic sorts in registers; all-greedy batches a greedy-only form);
  * other batches whose every row is greedy, samples from at most 2048 candidates or, without min-p and candidate outputs,
- * from every token (k = V), with any penalty, run on the mid-k kernel (fs_mid_k_plan); of the rest, batches mixing rows of 64 < k <= 2048 with cheaper rows run fs_sample_batch's
- * kernel with about twice its segments; other batches, and h_params = NULL, run fs_sample_batch. fs_route_plan reports
- * the choice between the small-k kernel and the others. Same outputs as fs_sample_batch. h_params is read before the
+ * from every token (k = V), with any penalty, run on the mid-k kernel (fs_mid_k_plan); of the rest, batches mixing rows
+ * of 64 < k <= 2048 with cheaper rows run fs_sample_batch's kernel with about twice its segments; other batches, and
+ * h_params = NULL, run fs_sample_batch. fs_route_plan reports the choice between the small-k kernel and the others. Same outputs as fs_sample_batch. h_params is read before the
  * call returns. Under HIP graph capture a batch whose mid-k workspace would have to grow runs fs_sample_batch's kernel. */
 int fs_sample_batch_hp(fs_context* ctx, const float* d_logits, int64_t ld, int32_t B, int32_t V,
                        const int32_t* d_hist, const int64_t* d_hist_off, const fs_row_params* d_params,
@@ -111,15 +111,17 @@ int fs_small_k_plan(int32_t cus, int32_t B, int32_t V, int32_t* nl, int32_t* nse
 /* Host-only: the kernel fs_sample_batch_hp (verify = 0: n = total_rows = B row records) or fs_verify_hp (verify != 0:
  * n stream records over total_rows rows) launches for these host parameters, on a device with `cus` compute units
  * whose XCD count divides 8: *kernel 0 the mid-k kernel where fs_mid_k_plan gives it a layout, else the fused kernel
- * (*nseg segments per row, *per_cu segments per CU of the fused kernel's layout), 1 the small-k kernel, 2 its greedy-only form (*nl float4 loads per thread, *nseg segments per row). No
- * counterpart in the reference (a routing check for callers and tests). */
+ * (*nseg segments per row, *per_cu segments per CU of the fused kernel's layout), 1 the small-k kernel, 2 its greedy-only
+ * form (*nl float4 loads per thread, *nseg segments per row). No counterpart in the reference (a routing check for
+ * callers and tests). */
 int fs_route_plan(int32_t cus, const fs_row_params* h_params, int32_t n, int32_t total_rows, int32_t V,
                   int32_t verify, int32_t* kernel, int32_t* nl, int32_t* nseg, int32_t* per_cu);
 
 /* Host-only: the mid-k kernel's layout for a batch the small-k kernel does not take (arguments as fs_route_plan's): *nl
  * float4 loads per thread (segments of 1024 * nl logits) and *nseg segments per row; FS_E_LIMIT, and zeros, when the
  * batch does not fit it (a row of more than 2048 candidates that are not every token or with min-p, more than 262144
- * logits per row, or too few logits for the largest k). No counterpart in the reference (a planner check). */
+ * logits per row, or too few logits for the largest k). It assumes a call without candidate outputs: with them the launch
+ * takes no batch with top_k = 0 rows of more than 2048 logits. No counterpart in the reference (a planner check). */
 int fs_mid_k_plan(int32_t cus, const fs_row_params* h_params, int32_t n, int32_t total_rows, int32_t V, int32_t* nl,
                   int32_t* nseg);
 
