@@ -74,9 +74,10 @@ struct MkShared {
             uint32_t cnt[SK_LT * 8 * 4 / 2];   // ak_slow: a chunk's counts beside a digit's masses
             union {
                 uint64_t mass[MK_H];
+                uint64_t sub[2][MK_H];         // ak_values: masses within the crossing's bin, within the draw's
                 struct {
                     uint32_t key[AK_VALS], cnt[AK_VALS];
-                } val[2];                      // ak_values: a chunk's values of the crossing's, of the draw's bins
+                } val[2];                      //   a chunk's values of both, and how often each occurs
             };
         } z;
     } u;
@@ -1305,10 +1306,13 @@ __device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uin
 }
 
 // The row's end where the searched bins hold more logits than a list takes (coarse logits: equal values share a bin; a row of
-// one value): by its last segment, from the row's logits. Chunk by chunk the bins' values and how often each occurs (a
-// wave counts each value of its 64 logits at once); crossing and draw are located among the values, in the order of their
-// chunks, and the draw's id in its chunk. Returns false when a chunk holds more than AK_VALS values of a bin, or a target
-// lies outside. One workgroup, two passes: 32 rows of 262144 logits rounded to halves 10140 us with ak_slow, now 830
+// one value; rows narrow in units of the bins, with a logit far from the others): by its last segment, from the row's
+// logits. Chunk by chunk the bins' values and how often each occurs (a wave counts each value of its 64 logits at once);
+// crossing and draw are located among the values, in the order of their chunks, and the draw's id in its chunk. More than
+// AK_VALS values of a bin in a chunk: the bins' masses are summed again in 1024 parts of each, and the values are those of
+// the parts that hold crossing and draw (32 rows of 262144 N(0, 0.05) logits and one at 10: 12040 us with ak_slow, 1460;
+// 160 on the fused kernel, whose histogram is of keys). Returns false when a part holds too many, too, or a target lies outside. One
+// workgroup, two passes (four with the parts): 32 rows of 262144 logits rounded to halves 10140 us with ak_slow, now 830
 // (2460 on the fused kernel).
 template <bool CAP>
 __device__ __forceinline__ bool ak_values(const float* rowp, int V, bool pen, const MkWin& win, const MkPen& pn, uint64_t* list,
@@ -1325,6 +1329,20 @@ __device__ __forceinline__ bool ak_values(const float* rowp, int V, bool pen, co
         const float t = (r.mx - x) * r.scale;
         const int b = (int)fminf(t, (float)AK_BINS);
         return t == t ? (r.tail ? b : (b < AK_BINS ? b : AK_BINS - 1)) : AK_BINS;
+    };
+    // its part among those of the bins b0 .. b1 (never falls as the logit falls)
+    auto part_of = [&](float x, int b0, int b1) {
+        const float t = ((r.mx - x) * r.scale - (float)b0) * ((float)MK_H / (float)(b1 - b0 + 1));
+        return (int)fminf(fmaxf(t, 0.0f), (float)(MK_H - 1));
+    };
+    bool fine = false;                                         // the parts c0 and e0 .. e1 only
+    int c0 = 0, e0 = 0, e1 = 0;
+    double above_c = one ? 0.0 : r.above_c, above_d = one ? 0.0 : r.above_d;
+    auto in_crossing = [&](float x, int b) { return cut && b == bc && (!fine || part_of(x, bc, bc) == c0); };
+    auto in_draw = [&](float x, int b) {
+        if (b < d0 || b > d1) return false;
+        const int q = fine ? part_of(x, d0, d1) : 0;
+        return q >= e0 && q <= e1;
     };
     auto window = [&](int lo, int n) {                         // a chunk's window ids, with their counts
         for (int i = tid; i < CH / 32; i += SK_LT) s.b.bmp[i] = 0u;
@@ -1358,16 +1376,10 @@ __device__ __forceinline__ bool ak_values(const float* rowp, int V, bool pen, co
         }
         s.gn[3] = 1u;
     };
-    if (tid < 4) s.gn[tid] = 0u;                               // the lists' lengths; [3]: too many values
+    // f(final logit) for a chunk's logits, all lanes of a wave together (past the chunk: NaN), while go() holds
+    auto each = [&](int lo, int n, auto go, auto f) {
 #pragma unroll 1
-    for (int lo = 0, chunk = 0; lo < V; lo += CH, ++chunk) {
-        const int n = V - lo < CH ? V - lo : CH;
-        __syncthreads();
-        if (tid < 4 * AK_VALS) reinterpret_cast<uint32_t*>(s.u.z.val)[tid] = 0u;
-        if (pen) window(lo, n);
-        else __syncthreads();
-#pragma unroll 1
-        for (int q0 = 0; q0 < PT && s.gn[3] == 0u; q0 += 8) {
+        for (int q0 = 0; q0 < PT && go(); q0 += 8) {
             float x[8];
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
@@ -1379,38 +1391,134 @@ __device__ __forceinline__ bool ak_values(const float* rowp, int V, bool pen, co
                 float y = x[0];
 #pragma unroll
                 for (int t = 1; t < 8; ++t) y = q == t ? x[t] : y;
-                y = value(y, (q0 + q) * SK_LT + tid);
-                const int b = bin_of(y);
-                const bool in_c = cut && b == bc, in_d = b >= d0 && b <= d1;
-                const uint32_t key = key_of(y);
-#pragma unroll 1
-                for (uint64_t left = __ballot(in_c || in_d); left != 0ull;) {
-                    const int first = __ffsll((unsigned long long)left) - 1;
-                    const uint64_t eq = __ballot(key == read_lane(key, first)) & left;
-                    if (lane == first) {
-                        if (in_c) put(0, key, (uint32_t)__popcll(eq));
-                        if (in_d) put(1, key, (uint32_t)__popcll(eq));
-                    }
-                    left &= ~eq;
-                }
+                f(value(y, (q0 + q) * SK_LT + tid));
+            }
+        }
+    };
+    // The part in which the masses, from the first on, reach the target (in units), and the units before it: wave 0 looks at
+    // sixteen parts per lane. -1: they do not.
+    auto locate = [&](const uint64_t* m, uint64_t target, uint64_t& before) {
+        if (tid < WAVE) {
+            uint64_t h = 0ull;
+            for (int q = 0; q < MK_H / WAVE; ++q) h += m[lane * (MK_H / WAVE) + q];
+            uint64_t inc = h;
+#pragma unroll
+            for (int o = 1; o < WAVE; o <<= 1) {
+                const uint64_t y = __shfl_up(inc, o);
+                if (lane >= o) inc += y;
+            }
+            if (target == 0ull) target = 1ull;
+            const uint64_t hit = __ballot(inc >= target);
+            if (hit == 0ull) {
+                if (lane == 0) s.umisc[0] = ~0ull;
+            } else if (lane == __ffsll((unsigned long long)hit) - 1) {
+                uint64_t at = inc - h;
+                int q = lane * (MK_H / WAVE);
+                while (at + m[q] < target) at += m[q++];
+                s.umisc[0] = (uint64_t)q;
+                s.umisc[1] = at;
             }
         }
         __syncthreads();
-        // entries: the value's key, the chunk (descending), the count. (Waves 0 and 1: a list each.)
-        if (tid < 2 * WAVE) {
-            const int l = tid / WAVE;
-            const uint32_t key = s.u.z.val[l].key[lane];
-            const uint64_t has = __ballot(key != 0u);
-            const uint32_t at = s.gn[l] + (uint32_t)__popcll(has & ((1ull << lane) - 1ull));
-            if (key != 0u && at < (uint32_t)AK_LIST)
-                st_agent(&list[l * AK_LIST + at], ((uint64_t)key << 32) | ((uint32_t)(63 - chunk) << 16) | s.u.z.val[l].cnt[lane]);
-            if (lane == 0) s.gn[l] += (uint32_t)__popcll(has);
+        const int q = (int)s.umisc[0];
+        before = s.umisc[1];
+        __syncthreads();
+        return q;
+    };
+#pragma unroll 1
+    for (;;) {
+        if (tid < 4) s.gn[tid] = 0u;                               // the lists' lengths; [3]: too many values
+#pragma unroll 1
+        for (int lo = 0, chunk = 0; lo < V && (chunk == 0 || s.gn[3] == 0u); lo += CH, ++chunk) {
+            const int n = V - lo < CH ? V - lo : CH;
+            __syncthreads();
+            if (tid < 4 * AK_VALS) reinterpret_cast<uint32_t*>(s.u.z.val)[tid] = 0u;
+            if (pen) window(lo, n);
+            else __syncthreads();
+            each(lo, n, [&]() { return s.gn[3] == 0u; }, [&](float y) {
+                    const int b = bin_of(y);
+                    const bool in_c = in_crossing(y, b), in_d = in_draw(y, b);
+                    const uint32_t key = key_of(y);
+#pragma unroll 1
+                    for (uint64_t left = __ballot(in_c || in_d); left != 0ull;) {
+                        const int first = __ffsll((unsigned long long)left) - 1;
+                        const uint64_t eq = __ballot(key == read_lane(key, first)) & left;
+                        if (lane == first) {
+                            if (in_c) put(0, key, (uint32_t)__popcll(eq));
+                            if (in_d) put(1, key, (uint32_t)__popcll(eq));
+                        }
+                        left &= ~eq;
+                    }
+            });
+            __syncthreads();
+            // entries: the value's key, the chunk (descending), the count. (Waves 0 and 1: a list each.)
+            if (tid < 2 * WAVE) {
+                const int l = tid / WAVE;
+                const uint32_t key = s.u.z.val[l].key[lane];
+                const uint64_t has = __ballot(key != 0u);
+                const uint32_t at = s.gn[l] + (uint32_t)__popcll(has & ((1ull << lane) - 1ull));
+                if (key != 0u && at < (uint32_t)AK_LIST)
+                    st_agent(&list[l * AK_LIST + at],
+                             ((uint64_t)key << 32) | ((uint32_t)(63 - chunk) << 16) | s.u.z.val[l].cnt[lane]);
+                if (lane == 0) s.gn[l] += (uint32_t)__popcll(has);
+            }
         }
+        vm_drain();
+        __syncthreads();
+        if (s.gn[3] == 0u && s.gn[0] <= (uint32_t)AK_LIST && s.gn[1] <= (uint32_t)AK_LIST) break;
+        if (fine || one) return false;
+        // the masses again, in parts of the bins (in units that the row's mass is less than 2^63 of), and the crossing bin's
+        // counts
+        const int fxe = 62 - ilogb(S) < 52 ? 62 - ilogb(S) : 52;
+        const double fx = __builtin_ldexp(1.0, fxe), ifx = __builtin_ldexp(1.0, -fxe);
+        __syncthreads();
+        for (int i = tid; i < 2 * MK_H; i += SK_LT) s.u.z.sub[i / MK_H][i % MK_H] = 0ull;
+        *reinterpret_cast<uint4*>(&s.h.hist[4 * tid]) = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll 1
+        for (int lo = 0; lo < V; lo += CH) {
+            const int n = V - lo < CH ? V - lo : CH;
+            __syncthreads();
+            if (pen) window(lo, n);
+            each(lo, n, []() { return true; }, [&](float y) {
+                const int b = bin_of(y);
+                const bool in_c = cut && b == bc, in_d = b >= d0 && b <= d1;
+                if (in_c || in_d) {
+                    const unsigned long long m = (unsigned long long)(ak_mass(y, r.mx, Td) * fx + 0.5);
+                    if (in_c) {
+                        atomicAdd(reinterpret_cast<unsigned long long*>(&s.u.z.sub[0][part_of(y, bc, bc)]), m);
+                        atomicAdd(&s.h.hist[part_of(y, bc, bc)], 1u);
+                    }
+                    if (in_d) atomicAdd(reinterpret_cast<unsigned long long*>(&s.u.z.sub[1][part_of(y, d0, d1)]), m);
+                }
+            });
+        }
+        __syncthreads();
+        auto units = [&](double x) { return x > 0.0 ? (uint64_t)(x * fx) : 0ull; };
+        uint64_t before = 0ull;
+        double lo_t = r.u * S, hi_t = lo_t;                        // the draw, at both ends of the kept total
+        if (cut) {
+            const double tgt = (double)p.top_p * S;
+            c0 = locate(s.u.z.sub[0], units(tgt - above_c), before);
+            if (c0 < 0) return false;
+            above_c += (double)before * ifx;
+            uint32_t up = 0u;
+            for (int i = tid; i < c0; i += SK_LT) up += s.h.hist[i];
+            uint32_t ups;
+            (void)mk_excl_u32(up, s, ups);
+            above += ups;
+            // (a logit of the part has at most the mass at the part's upper end)
+            const double most = exp(-((double)bc + (double)c0 / MK_H) / ((double)r.scale * Td)) * (1.0 + 1e-4);
+            lo_t = r.u * tgt;
+            hi_t = r.u * (tgt + most < S ? tgt + most : S);
+        }
+        e1 = locate(s.u.z.sub[1], units(hi_t * (1.0 + 1e-12) - above_d), before);
+        if (e1 < 0) e1 = MK_H - 1;
+        e0 = locate(s.u.z.sub[1], units(lo_t * (1.0 - 1e-12) - above_d), before);
+        if (e0 < 0) return false;
+        above_d += (double)before * ifx;
+        fine = true;
     }
-    vm_drain();
-    __syncthreads();
     const uint32_t n0 = s.gn[0], n1 = s.gn[1];
-    if (s.gn[3] != 0u || n0 > (uint32_t)AK_LIST || n1 > (uint32_t)AK_LIST) return false;
     uint64_t xc = 0ull, c = 0ull;
     double tot = S;
     keep = (int)r.nv;
@@ -1426,7 +1534,7 @@ __device__ __forceinline__ bool ak_values(const float* rowp, int V, bool pen, co
         mk_sort_end(mk_sort(e, n, n, s), n, s);
         double cum;
         const double target = pass == 0 ? (double)p.top_p * S : r.u * tot + 0.0;
-        const int at = ak_walk<true>(n, one ? 0.0 : pass == 0 ? r.above_c : r.above_d, target, r.mx, Td, s, cum);
+        const int at = ak_walk<true>(n, pass == 0 ? above_c : above_d, target, r.mx, Td, s, cum);
         if (at < 0) return false;
         // the j-th of the entry's equal logits reaches the target; c becomes the entry's value and chunk above ~j
         c = s.u.w.top[at];
