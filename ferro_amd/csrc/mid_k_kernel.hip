@@ -943,10 +943,13 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     // A minimum far down (masked tokens) would spread the bins over a range without logits: the wave's minimum is then that
     // of its logits less than AK_DEPTH temperatures below its maximum; the others are none of the row's bins' either. (32
     // rows of 262144 N(0, 2) logits at temperature 3, one of a hundred at -inf: 11400 us, thousands per bin; now 53. Not
-    // for rows with tails: they spread over the bins anyway, and the second look cost 2 us of 36.)
+    // for rows with tails, which spread over the bins anyway, where the second look cost 2 us of 36: the minimum is very
+    // far down, or most lanes' maxima are near the wave's.)
     bool cut = false;
-    if (kx > 0x007FFFFFu && kn < kx && val_of(kn) < val_of(kx) - 32.0f * AK_DEPTH * p.temperature) {
-        const float low = val_of(kx) - AK_DEPTH * p.temperature;
+    const float low = val_of(kx) - AK_DEPTH * p.temperature;
+    if (kx > 0x007FFFFFu && kn < kx && val_of(kn) < low &&
+        (val_of(kn) < val_of(kx) - 32.0f * AK_DEPTH * p.temperature ||
+         __popcll(__ballot(hi > val_of(kx) - 0.5f * AK_DEPTH * p.temperature)) >= 48)) {
         auto above = [&](float x) { return x >= low ? x : __builtin_nanf(""); };
         lo = __builtin_nanf("");
 #pragma unroll
@@ -1010,14 +1013,15 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     const int be = (int)((__float_as_uint(bound) >> 23) & 255u) - 126;          // bound < 2^be
     const int fxe = __builtin_amdgcn_readfirstlane(63 - be < 52 ? 63 - be : 52);
     const double fx = __builtin_ldexp(1.0, fxe), ifx = __builtin_ldexp(1.0, -fxe);
-    float depth = (mx - mn) * invf * (cut ? 1.0001f : 1.0f);   // (the lowest in the last bin, whatever its place's rounding)
+    // (cut: the lowest in the last bin, whatever its place's rounding; one value and masked tokens: all in the first bin)
+    float depth = (mx - mn) * invf * (cut ? 1.0001f : 1.0f);
     const bool tail = cut || !(depth < AK_DEPTH);
-    depth = depth < AK_DEPTH ? depth : AK_DEPTH;
+    depth = depth < AK_DEPTH && !(cut && !(mn < mx)) ? depth : AK_DEPTH;
     const float scale = (float)AK_BINS / (depth * p.temperature);
-    r.scale = mn < mx || !(mx < __builtin_huge_valf()) || !(mx > -__builtin_huge_valf()) ? scale : 0.0f;
+    r.scale = cut || mn < mx || !(mx < __builtin_huge_valf()) || !(mx > -__builtin_huge_valf()) ? scale : 0.0f;
     r.tail = tail;
-    r.plain = r.nv == 0u || !(mx < __builtin_huge_valf()) || !(mx > -__builtin_huge_valf()) || !(mn < mx) || !(scale > 0.0f) ||
-              !(scale < __builtin_huge_valf());
+    r.plain = r.nv == 0u || !(mx < __builtin_huge_valf()) || !(mx > -__builtin_huge_valf()) || !(cut || mn < mx) ||
+              !(scale > 0.0f) || !(scale < __builtin_huge_valf());
     if (r.plain) return true;                                  // uniform over the row
     for (int i = tid; i < AK_BINS / 2; i += SK_LT) reinterpret_cast<ulonglong2*>(s.u.a.mass)[i] = make_ulonglong2(0ull, 0ull);
     __syncthreads();

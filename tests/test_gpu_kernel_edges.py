@@ -505,6 +505,10 @@ def test_every_token_of_masked_rows_at_high_temperatures(mask):
     x[1::2, :20000] = mask                           # whole segments of masked tokens
     x[4, 77777] = 6 * 3.0 * 32                       # the others are below the bins of this row
     x[5] = np.where(x[5] > 4, x[5], mask)
+    x[2] = np.where(x[2] > 0, np.float32(2.0), mask)  # one value, the others masked: thousands, and a few
+    x[3] = np.where(x[3] > 5.5, np.float32(2.0), mask)
+    x[8:, 50001] = -130.0                            # one token below the bins of the others, one above its range
+    x[9, 60000:] *= 0.01
     p = mid_params(B, 0, temperature=3.0)
     p["temperature"][6:8] = 0.7, 20.0
     p["top_p"] = np.where(np.arange(B) % 4 < 2, 0.9, 1.0)
