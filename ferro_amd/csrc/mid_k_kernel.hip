@@ -18,11 +18,11 @@
 // takes are counted first (one meeting more), and only the row's first ones written.
 // Bound: HBM, one read of the logits, then the chain behind a row's last logits.
 // Measured against the fused kernel (running bounds, per-row merges of the segments' lists): 256 rows of 262144 logits
-// with k from 1 to 2048 and every penalty 124 us -> 77; 24 rows of 100003 logits, k 200, frequency / presence 35 -> 19.5;
-// 40 rows of a verification window over 262144 logits, k 50, repetition 26.5 -> 24.7.
+// with k from 1 to 2048 and every penalty 124 us -> 75; 24 rows of 100003 logits, k 200, frequency / presence 35 -> 17.9;
+// 40 rows of a verification window over 262144 logits, k 50, repetition 26.5 -> 22.
 // Rows with every token a candidate (ak_segment, ak_finish) stay in registers through all their passes; the fused kernel
 // reads such a row again for each, and gave flat ones to one workgroup: 32 rows of 65536 N(0, 2) logits at temperature 1
-// 51.5 us -> 23.5, 3 rows of 178740 507 -> 21, 64 rows of 262144 heavy-tailed logits with top-p 0.95 37.5 -> 35.7.
+// 51.5 us -> 24.2, 3 rows of 178740 698 -> 28.6, 64 rows of 262144 heavy-tailed logits with top-p 0.95 37.5 -> 37.1.
 #include "exp_table.hpp"
 #include "row_device.hpp"
 
@@ -942,7 +942,7 @@ __device__ __forceinline__ bool ak_segment(float (&v)[NL][4], const MkArgs& mk, 
     uint32_t kx = wave_max(key_of(hi)), kn = wave_min(lo == lo ? key_of(lo) : 0xFFFFFFFFu);
     // A minimum far down (masked tokens) would spread the bins over a range without logits: the wave's minimum is then that
     // of its logits less than AK_DEPTH temperatures below its maximum; the others are none of the row's bins' either. (32
-    // rows of 262144 N(0, 2) logits at temperature 3, one of a hundred at -inf: 11400 us, thousands per bin; now 53. Not
+    // rows of 262144 N(0, 2) logits at temperature 3, one of a hundred at -inf: 6640 us, thousands per bin; now 54. Not
     // for rows with tails, which spread over the bins anyway, where the second look cost 2 us of 36: the minimum is very
     // far down, or most lanes' maxima are near the wave's.)
     bool cut = false;
@@ -1314,7 +1314,7 @@ __device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uin
 // logits. Chunk by chunk the bins' values and how often each occurs (a wave counts each value of its 64 logits at once);
 // crossing and draw are located among the values, in the order of their chunks, and the draw's id in its chunk. More than
 // AK_VALS values of a bin in a chunk: the bins' masses are summed again in 1024 parts of each, and the values are those of
-// the parts that hold crossing and draw (32 rows of 262144 N(0, 0.05) logits and one at 10: 12040 us with ak_slow, 1460;
+// the parts that hold crossing and draw (32 rows of 262144 N(0, 0.05) logits and one at 10: 9510 us with ak_slow, 1460;
 // 160 on the fused kernel, whose histogram is of keys). Returns false when a part holds too many, too, or a target lies outside. One
 // workgroup, two passes (four with the parts): 32 rows of 262144 logits rounded to halves 10140 us with ak_slow, now 830
 // (2460 on the fused kernel).

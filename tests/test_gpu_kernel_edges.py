@@ -150,6 +150,27 @@ def test_softcap_where_it_saturates(cap, scale):
     check(x, p, [list(W.zipf_ids(rng, V, 900)) for _ in range(6)], rng.random(6))
 
 
+@pytest.mark.parametrize("cap", [1.0, 30.0, 0.375])
+def test_softcap_never_decreases(cap):
+    """Over every float from -inf to inf: bounds taken over raw logits hold for the capped ones."""
+    import ctypes
+    from ferro_amd._lib import lib
+    chunk = 1 << 27
+    out = torch.empty(chunk, dtype=torch.float32, device="cuda")
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    last = None
+    for first in range(-0x7F800000, 0x7F800001, chunk):              # ascending floats: below 0 by their magnitude's bits
+        i = torch.arange(first, min(first + chunk, 0x7F800001), dtype=torch.int64, device="cuda")
+        x = torch.where(i < 0, -i, i).to(torch.int32).view(torch.float32)
+        x = torch.where(i < 0, -x, x).contiguous()
+        n = x.numel()
+        assert lib().fs_softcap_batch(ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(out.data_ptr()), n,
+                                      ctypes.c_float(cap), st) == 0
+        y = out[:n]
+        assert bool((y[1:] >= y[:-1]).all()) and (last is None or bool(y[0] >= last))
+        last = y[-1].clone()
+
+
 @pytest.mark.parametrize("V,k", [(5, 0), (40, 0), (64, 0), (65, 40), (320, 64), (800, 64), (2080, 50)])
 @pytest.mark.parametrize("cap", [0.5, 30.0])
 def test_softcap_and_penalties_on_short_rows(V, k, cap):
