@@ -184,7 +184,8 @@ __device__ __forceinline__ bool mk_locate(MkShared& s, uint32_t kk, uint32_t& b,
 // histograms of ten key bits each in LDS. sum: those weights' sum; need: what the keys of T's own prefix have to add.
 // Whole workgroup; s.h.hist is zero on entry.
 template <int NQ>
-__device__ __forceinline__ uint32_t mk_bound(const uint32_t* qk, int nseg, int k, MkShared& s, uint32_t& sum, uint32_t& need) {
+__device__ __forceinline__ uint32_t mk_bound(const uint32_t* qk, int nseg, int k, MkShared& s, uint32_t& sum,
+                                             uint32_t& need) {
     const int tid = threadIdx.x;
     const int n4 = nseg * SK_NW * 4;                           // 16-byte quarters of the lists
     uint4 e[NQ];
@@ -1315,9 +1316,9 @@ __device__ __forceinline__ bool ak_finish(const uint64_t* list, uint32_t n0, uin
 // crossing and draw are located among the values, in the order of their chunks, and the draw's id in its chunk. More than
 // AK_VALS values of a bin in a chunk: the bins' masses are summed again in 1024 parts of each, and the values are those of
 // the parts that hold crossing and draw (32 rows of 262144 N(0, 0.05) logits and one at 10: 9510 us with ak_slow, 1460;
-// 160 on the fused kernel, whose histogram is of keys). Returns false when a part holds too many, too, or a target lies outside. One
-// workgroup, two passes (four with the parts): 32 rows of 262144 logits rounded to halves 10140 us with ak_slow, now 830
-// (2460 on the fused kernel).
+// 160 on the fused kernel, whose histogram is of keys). Returns false when a part holds too many, too, or a target lies
+// outside. One workgroup, two passes (four with the parts): 32 rows of 262144 logits rounded to halves 10140 us with ak_slow,
+// now 830 (2460 on the fused kernel).
 template <bool CAP>
 __device__ __forceinline__ bool ak_values(const float* rowp, int V, bool pen, const MkWin& win, const MkPen& pn, uint64_t* list,
                                           uint32_t above, const AkRow& r, const fs_row_params& p, MkShared& s, int& tok,
